@@ -76,6 +76,14 @@ static unsigned decode_scale_lds(size_t group, int rb, int kt_per_wave) {
     return ((unsigned)(rb * kt_per_wave * (128 / (int)group) * 32) + 1023u) / 1024u * 1024u;
 }
 
+// x loads per k tile, four rows each, and the LDS bytes of a wave: its partial tiles, or its staged x tile where x goes
+// through LDS (kernels/decode.hip, REGION)
+static int decode_x_loads(size_t t) { return t <= 4 ? 1 : t <= 8 ? 2 : 4; }
+static unsigned decode_wave_lds(int rb, size_t t) {
+    const int xl = decode_x_loads(t);
+    return (unsigned)std::max(rb * 1024, xl > 1 ? (4 * xl + 1) * 256 : 0);
+}
+
 static int plan_decode(const DecodePlanIn& in, DecodePlan* out) {
     const int kt_n = (int)(in.k / 128);
     if (kt_n <= 0 || in.row_blocks == 0) return w4_fail(W4A16_ERR_SHAPE, "decode: empty linear");
@@ -117,9 +125,9 @@ static int plan_decode(const DecodePlanIn& in, DecodePlan* out) {
         if (P.nks > 1) P.waves = std::max(1, std::min(P.waves, kt_n / P.nks));
         P.kt_per_slice = (kt_n + P.nks - 1) / P.nks;
         P.kt_per_wave = (P.kt_per_slice + P.waves - 1) / P.waves;
-        // the split-K partial tiles [waves][rb][1 KiB]; then per wave the scales of its whole k slice (rb x tiles per
+        // per wave its partial tiles or staged x tile; then per wave the scales of its whole k slice (rb x tiles per
         // wave x groups per tile x 32 bytes, in whole 1 KiB DMA instructions); then the statistics staging area
-        P.shmem = (unsigned)(P.waves * rb * 1024) + (unsigned)P.waves * decode_scale_lds(in.group, rb, P.kt_per_wave) + in.extra_lds;
+        P.shmem = (unsigned)P.waves * decode_wave_lds(rb, in.t) + (unsigned)P.waves * decode_scale_lds(in.group, rb, P.kt_per_wave) + in.extra_lds;
         if (P.shmem <= 160u * 1024u) {
             *out = P;
             return 0;
@@ -255,7 +263,7 @@ static int launch_decode(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_t y,
     int waves = P.waves, nks = P.nks, kt_per_slice = P.kt_per_slice, kt_per_wave = P.kt_per_wave;
     const size_t blocks = P.blocks;
     // x loads per k tile: one serves up to 4 token rows, two up to 8, four up to 16 (kernels/decode.hip)
-    const int xl = t <= 4 ? 1 : t <= 8 ? 2 : 4;
+    const int xl = decode_x_loads(t);
     char sym[64];
     if (multi)
         snprintf(sym, sizeof sym, "w4a16_decode_g%zu_%s_multi_x%d", L.group, L.scale_bf16 ? "bf16" : "f16", xl);
@@ -307,7 +315,7 @@ static int launch_decode_glu(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_
     W4_TRY(plan_decode(in, &P));
     int waves = P.waves, nks = P.nks, kt_per_slice = P.kt_per_slice, kt_per_wave = P.kt_per_wave;
     const size_t blocks = P.blocks;
-    const int xl = t <= 4 ? 1 : t <= 8 ? 2 : 4;
+    const int xl = decode_x_loads(t);
     char sym[64];
     snprintf(sym, sizeof sym, "w4a16_decode_g%zu_%s_glu_x%d", L.group, L.scale_bf16 ? "bf16" : "f16", xl);
     uint64_t qt = L.q_tiled, st = L.s_tiled;

@@ -9,8 +9,13 @@
 //   * x: every vector-memory instruction costs the CU's address unit about as much as a full 1 KiB load however few
 //     lanes are live, so one B-operand load per MFMA would cost more than the weight stream.  For t <= 4 a single
 //     buffer load per k tile brings all four 32-k chunks (lane m fetches chunk m/4 of token m%4; lanes for tokens
-//     >= t are out of range: zeros, no traffic) and v_mov_b32_dpp row_shl moves chunk c to the token's column;
-//     t <= 8 takes two loads, t <= 16 four (no shuffles).  No LDS and no barrier on the streaming path;
+//     >= t are out of range: zeros, no traffic) and v_mov_b32_dpp row_shl moves chunk c to the token's column.
+//     From five rows on x arrives in whole rows of the k tile (16 lanes x 16 B per row, two loads up to t = 8, four up
+//     to 16) and is turned into B operands through a wave-private piece of LDS: a load in B-operand order, whose
+//     neighbouring lanes read different rows, occupies the address unit for 62 clocks against 18 for whole rows (L2-resident
+//     x, 16 waves per CU).  5120 x 34816 at t = 16: 27.0 -> 25.7 us, gated 32.4 -> 26.8; 5120 x 7168 8.9 -> 8.3;
+//     17408 x 5120 15.8 -> 15.1; at t = 8 level, gated 22.7 -> 21.3; up to t = 4 it costs 0.1 us and is not used.
+//     No barrier on the streaming path;
 //   * weights enter the MFMA as exact integers; the per-group scale multiplies the f32 group sum, so no weight is
 //     ever rounded to f16 (error vs the f32 lane contract is summation order only);
 //   * each wave keeps DEPTH k-tiles of loads in flight (register ring, software pipelined);
@@ -75,10 +80,12 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
                                             float* __restrict__ stats_out, int stat_rows, float* __restrict__ resid,
                                             const float* __restrict__ nw, int act_kind, float in_scale, float out_scale,
                                             DecodeMulti mo) {
-    extern __shared__ f4_t red[];  // [W][RB][64] partial tiles of the in-block split-K, then the waves' staged scales
+    extern __shared__ f4_t red[];  // [W][REGION] staged x, then partial tiles of the in-block split-K; the waves' staged scales
     constexpr int GPT = W4_TILE_K / G;  // scale groups per k tile
-    constexpr int C = 4 / XL;           // 32-k chunks (MFMAs) served by one x load
-    constexpr int TPL = 16 / C;         // token columns served by one x load
+    constexpr bool XLDS = XL > 1;       // x goes through LDS
+    constexpr int XROWS = 4 * XL;       // x rows of a staged k tile
+    // LDS bytes per wave: its staged x tile while it streams, its partial tiles afterwards
+    constexpr int REGION = XLDS && (XROWS + 1) * 256 > RB * 1024 ? (XROWS + 1) * 256 : RB * 1024;
     // The launch geometry (W waves per block, nks k slices over blockIdx.y, tiles per slice and per wave) arrives as
     // kernel arguments: read from the dispatch packet instead, the block size costs a second dependent memory round
     // trip and the balanced split two integer divisions before the first weight load can be issued, on every wave.
@@ -97,9 +104,13 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
 
     // Every load is a raw buffer load: an out-of-range offset returns zeros and costs no memory traffic, which
     // predicates token columns >= t without a branch.
-    // x load l of a tile: lane (m, g) fetches, for token m % TPL, the 8 halves of chunk l*C + m / TPL at k offset g*8
-    const int xtok = m % TPL, xchunk = m / TPL;
-    const unsigned xoff = xtok < t ? ((unsigned)xtok * (unsigned)ldx + (unsigned)(xchunk * 32 + g * 8)) * 2u : W4_OOB;
+    // x load l of a tile brings rows 4l..4l+3, 16 bytes per lane.  XLDS: 16 lanes to a row, to be re-ordered through LDS;
+    // otherwise (one load) lane (m, g) fetches, for token m % 4, the 8 halves of chunk m / 4 at k offset g*8.
+    const int xrow = XLDS ? lane >> 4 : m & 3, xpiece = XLDS ? lane & 15 : (m >> 2) * 4 + g;
+    unsigned xoff[XL];
+#pragma unroll
+    for (int l = 0; l < XL; l++)
+        xoff[l] = 4 * l + xrow < t ? ((unsigned)(4 * l + xrow) * (unsigned)ldx + (unsigned)xpiece * 8u) * 2u : W4_OOB;
     const unsigned q_bytes = (unsigned)row_blocks * (unsigned)kt_n * 1024u, s_bytes = (unsigned)row_blocks * (unsigned)kg_n * 32u,
                    x_bytes = ((unsigned)(t - 1) * (unsigned)ldx + (unsigned)k) * 2u;  // x rows are ldx halves apart
     f4_t acc[RB];
@@ -116,7 +127,7 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
     // zeros, no traffic).  AUX_PW bytes per wave, whole DMA instructions.
     const int aux_rb_bytes = kt_per_wave * (GPT * 32);
     const int AUX_PW = (RB * aux_rb_bytes + 1023) & ~1023;
-    char* const aux_lds = reinterpret_cast<char*>(red) + W * RB * 1024 + wave * AUX_PW;
+    char* const aux_lds = reinterpret_cast<char*>(red) + W * REGION + wave * AUX_PW;
     {
         const __amdgpu_buffer_rsrc_t sr_ = w4_make_rsrc(st, s_bytes);
         const int slice_bytes = (kt1 - kt0) * (GPT * 32);
@@ -129,6 +140,12 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
                                                      0, 0);
         }
     }
+
+    // LDS places of a staged x tile: the 16 bytes of row r, piece p (k = 8p.. of the tile) at p * (XROWS + 1) * 16 + r * 16,
+    // so that the 16 pieces of a row (one write) and the XROWS rows of a piece (a B operand's read) each fall into distinct
+    // banks.  MFMA w reads piece 4w + g of row m; columns past the staged rows repeat one and are never stored.
+    char* const x_put = reinterpret_cast<char*>(red) + wave * REGION + xpiece * (XROWS + 1) * 16 + xrow * 16;
+    const char* const x_get = reinterpret_cast<char*>(red) + wave * REGION + g * (XROWS + 1) * 16 + (m & (XROWS - 1)) * 16;
 
     // Per-tile addressing costs no vector ALU work: the lane part of every offset is loop invariant, the k-tile part
     // travels in the scalar offset operand, and a tile past the wave's range is switched off by a zero-length
@@ -143,21 +160,24 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
             s_.q[rb] = __builtin_amdgcn_raw_buffer_load_b128(qr_, qoff[rb], kt * 1024, 2 /* nt: read-once stream */);
 #pragma unroll
         for (int l = 0; l < XL; l++)
-            s_.x[l] = __builtin_amdgcn_raw_buffer_load_b128(xr_, xoff + (unsigned)(l * C * 32) * 2u, kt * (W4_TILE_K * 2), 0);
+            s_.x[l] = __builtin_amdgcn_raw_buffer_load_b128(xr_, xoff[l], kt * (W4_TILE_K * 2), 0);
     };
     // sc = this lane's view of the scales of the round's first tile: rows 4g..4g+3 of (row block rb, tile d of the round,
     // group gi) are the 8 bytes at sc + rb*aux_rb_bytes + (d*GPT + gi)*32
     auto compute = [&](const DecodeStage<RB, XL>& s_, const char* sc, int d) {
-        // B operand of MFMA w = chunk w of x for token column m: held by lane (m + (w % C) * TPL) of load w / C
+        // B operand of MFMA w = chunk w of x for token column m.  Through LDS: a wave's LDS operations run in order, so
+        // neither the reads of this tile's rows nor the next tile's writes need a wait of their own.
         u4_t xb[4];
+        if constexpr (XLDS) {
 #pragma unroll
-        for (int l = 0; l < XL; l++) {
-            xb[l * C] = s_.x[l];
-            if (C >= 2) xb[l * C + 1] = w4_row_shl<TPL>(s_.x[l]);
-            if (C == 4) {
-                xb[2] = w4_row_shl<2 * TPL>(s_.x[l]);
-                xb[3] = w4_row_shl<3 * TPL>(s_.x[l]);
-            }
+            for (int l = 0; l < XL; l++) *reinterpret_cast<u4_t*>(x_put + l * 64) = s_.x[l];
+#pragma unroll
+            for (int w = 0; w < 4; w++) xb[w] = *reinterpret_cast<const u4_t*>(x_get + w * (4 * (XROWS + 1) * 16));
+        } else {  // held by lane m + 4w
+            xb[0] = s_.x[0];
+            xb[1] = w4_row_shl<4>(s_.x[0]);
+            xb[2] = w4_row_shl<8>(s_.x[0]);
+            xb[3] = w4_row_shl<12>(s_.x[0]);
         }
 #pragma unroll
         for (int rb = 0; rb < RB; rb++) {
@@ -191,11 +211,12 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
     // 1/sqrt(mean + 1e-6).  The entries of token columns 0..3 are fetched here, ahead of the ring, by LDS DMA (no
     // registers held across the fill) into a staging area behind the scale slots, 64 entries per instruction, lane l
     // entry c*64 + l; once the first weight tiles are in flight lane l adds its entries, a butterfly adds the lanes
-    // (fixed order: the same bits on every run), and the factor is parked in the wave's own slot of `red`, which the
-    // in-block reduction never writes.  The epilogue multiplies the sums by it.  Further token quads and entries
-    // beyond the staging area (8 x 64) repeat the fetch inside input_scale.
+    // (fixed order: the same bits on every run), and the factor is parked at the start of the staging area.  The
+    // epilogue multiplies the sums by it.  Further token quads and entries beyond the staging area (8 x 64) repeat the
+    // fetch inside input_scale.
     typedef __attribute__((address_space(3))) char lds_char_t;
-    lds_char_t* const stage_lds = (lds_char_t*)(reinterpret_cast<char*>(red) + W * RB * 1024 + W * AUX_PW);
+    lds_char_t* const stage_lds = (lds_char_t*)(reinterpret_cast<char*>(red) + W * REGION + W * AUX_PW);
+    float* const park = reinterpret_cast<float*>(reinterpret_cast<char*>(red) + W * REGION + W * AUX_PW);
     const int stat_chunks = min((n_stats_in + 63) >> 6, 8);
     auto fetch_stats = [&](int c0, int qd) {
         const __amdgpu_buffer_rsrc_t sr_in = w4_make_rsrc(stats_in, (unsigned)n_stats_in * 64u);
@@ -205,7 +226,7 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
     };
     if (stats_in != nullptr && wave == 0) fetch_stats(0, 0);
     auto input_scale = [&]() {
-        const f4_t* const staged = reinterpret_cast<const f4_t*>(reinterpret_cast<char*>(red) + W * RB * 1024 + W * AUX_PW);
+        const f4_t* const staged = reinterpret_cast<const f4_t*>(reinterpret_cast<char*>(red) + W * REGION + W * AUX_PW);
         float mine = 0.f;
         for (int qd = 0; qd * 4 < t; qd++) {  // a quad of token columns at a time
             f4_t sum = {0.f, 0.f, 0.f, 0.f};
@@ -227,7 +248,7 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
                 if (m == qd * 4 + j) mine = v;
             }
         }
-        reinterpret_cast<float*>(red)[lane] = (float)(1.0 / sqrt((double)mine * (double)inv_cols_in + 1e-6));
+        park[lane] = (float)(1.0 / sqrt((double)mine * (double)inv_cols_in + 1e-6));
     };
 
     // One counted loop does the pipeline fill (round -1, compute skipped) and the steady state, so on every path
@@ -265,13 +286,13 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
     if (W > 1) {
         if (wave != 0) {
 #pragma unroll
-            for (int rb = 0; rb < RB; rb++) red[(wave * RB + rb) * 64 + lane] = acc[rb];
+            for (int rb = 0; rb < RB; rb++) red[wave * (REGION / 16) + rb * 64 + lane] = acc[rb];
         }
         __syncthreads();
         if (wave != 0) return;
         for (int w = 1; w < W; w++) {
 #pragma unroll
-            for (int rb = 0; rb < RB; rb++) acc[rb] += red[(w * RB + rb) * 64 + lane];
+            for (int rb = 0; rb < RB; rb++) acc[rb] += red[w * (REGION / 16) + rb * 64 + lane];
         }
     }
     if (nks > 1) {  // wave 0 only from here
@@ -324,7 +345,7 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
     // times 1/in_scale, y leaves as its true value times out_scale (both exact; 1 = none).  in_scale joins the input's
     // 1/rms ahead of everything that looks at the values (statistics, residual, activation); out_scale is applied last.
     if (stats_in != nullptr || in_scale != 1.0f) {
-        const float inv = (stats_in != nullptr ? reinterpret_cast<const float*>(red)[lane] : 1.0f) * in_scale;
+        const float inv = (stats_in != nullptr ? park[lane] : 1.0f) * in_scale;
 #pragma unroll
         for (int rb = 0; rb < RB; rb++)
 #pragma unroll
