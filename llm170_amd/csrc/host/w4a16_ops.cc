@@ -51,6 +51,11 @@ static int launch_lane(w4a16_ctx* ctx, uint64_t q, uint64_t s, uint64_t x, uint6
 // enough waves; a narrow output with a long k range (the 27B down projection, 320 row blocks x 136 k tiles) from seven
 // tokens on runs four row blocks per wave, which share the x loads, with the k slices across workgroups bringing the
 // workgroups back (t = 16: 21.6 -> 15.8 us, t = 12: 18.6 -> 14.9, t = 8: 14.2 -> 13.5; level at t = 6).
+// Outputs of at most one row block per CU (256 row blocks, n = 4096): one row block per wave x eight waves, so that every
+// CU has a workgroup, and no k slices (4096 x 4096 at t = 1 5.72 -> 4.80 us, t = 8 6.31 -> 5.19, t = 16 7.01 -> 6.24;
+// k = 11008 9.07 -> 7.64; 1024 x 4096 5.24 -> 4.48; at 384 row blocks the two shapes are within 5 % and at 448 two row
+// blocks win) — from seven rows with a long k two row blocks in four slices (2048 x 11008 at t = 16 8.75 -> 8.1,
+// 1024 x 8192 7.86 -> 6.7: the slices split the x loads, which grow with t).
 // k slices across workgroups (one launch; partial tiles and tickets in a workspace): only for a long k range over
 // fewer workgroups than CUs (the 27B down projection: 160 blocks x 136 k tiles): slices of about 16 k tiles, four waves
 // each (measured 12.4 -> 11.8 us at t = 1, 13.3 -> 12.4 us at t = 4).  Shorter k ranges lose more to the extra
@@ -88,6 +93,7 @@ static int plan_decode(const DecodePlanIn& in, DecodePlan* out) {
     const int kt_n = (int)(in.k / 128);
     if (kt_n <= 0 || in.row_blocks == 0) return w4_fail(W4A16_ERR_SHAPE, "decode: empty linear");
     const bool wide = in.row_blocks >= 1024;
+    const bool small = in.row_blocks <= (size_t)std::max(in.cu_count, 1);  // one row block per workgroup fits the chip at once
     const bool long_k_narrow = !wide && kt_n >= 64 && in.t >= 7;
     int rb;
     bool rb_auto = false;
@@ -97,11 +103,11 @@ static int plan_decode(const DecodePlanIn& in, DecodePlan* out) {
         rb = in.rows_per_wave / 16;
         if (rb != 1 && rb != 2 && rb != 4) return w4_fail(W4A16_ERR_ARG, "decode: rows_per_wave must be 16, 32 or 64");
     } else {
-        rb = wide ? (in.t <= 2 ? 1 : in.t <= 6 ? 2 : 4) : long_k_narrow ? 4 : 2;
+        rb = wide ? (in.t <= 2 ? 1 : in.t <= 6 ? 2 : 4) : small ? (long_k_narrow ? 2 : 1) : long_k_narrow ? 4 : 2;
         rb_auto = true;
     }
     while (!in.glu && rb > 1 && in.row_blocks < (size_t)rb) rb >>= 1;
-    const int waves_auto = in.glu ? (in.t > 8 || wide ? 4 : 8) : wide ? 4 : (in.t > 8 || long_k_narrow ? 4 : 8);
+    const int waves_auto = in.glu ? (in.t > 8 || wide ? 4 : 8) : wide ? 4 : small && rb == 1 ? 8 : (in.t > 8 || long_k_narrow ? 4 : 8);
     const int waves_want = std::max(1, std::min(std::min(in.waves_per_block ? in.waves_per_block : waves_auto, 8), kt_n));
     int nks_want = 1;
     bool nks_auto = false;
@@ -111,8 +117,8 @@ static int plan_decode(const DecodePlanIn& in, DecodePlan* out) {
     } else if (in.ksplit == 0) {
         nks_auto = true;
         const size_t blocks = in.glu ? in.row_blocks / 2 : (in.row_blocks + (size_t)rb - 1) / (size_t)rb;
-        if (blocks < (size_t)std::max(in.cu_count, 1) && kt_n >= 64) {
-            nks_want = std::min(kW4DecodeMaxKsplit, kt_n / 16);
+        if (blocks < (size_t)std::max(in.cu_count, 1) && kt_n >= 64 && !(small && rb == 1)) {
+            nks_want = std::min(small && !in.glu ? 4 : kW4DecodeMaxKsplit, kt_n / 16);
             waves_cap = 4;
         }
     }

@@ -1,0 +1,32 @@
+"""Decode launches of outputs with at most one 16-row block per CU (one row block per wave, eight waves; two row blocks in
+four k slices from seven rows with a long k) and x rows re-ordered through LDS (five to sixteen rows): the edges of those
+ranges against the lane-order oracle."""
+import numpy as np
+import pytest
+
+from llm170_amd import gen, ops, parity
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,k,group,t", [
+    (4096, 512, 128, 1), (4096, 512, 128, 16),   # the last size with one row block per workgroup
+    (4112, 512, 128, 9),                         # one row block more: two per wave
+    (17, 1024, 32, 5), (1, 128, 128, 8),         # a partial row block; fewer k tiles than waves
+    (96, 8192, 128, 6), (96, 8192, 128, 7),      # a long k: whole up to six rows, four slices from seven
+    (96, 8192, 32, 16), (80, 8320, 128, 13),     # 65 k tiles in four slices: the last one short
+])
+def test_small_outputs(orc, n, k, group, t):
+    print("small outputs", n, k, group, t, flush=True)
+    dec = ops.W4a16Dec()
+    try:
+        q, s, x = gen.make_linear(n, k, group, t, seed=n + k + t)
+        dec.upload_lin_g("s", q, s, n, k, group, False)
+        want = orc.gemm_lane(x, t, q, s, n, k, group)
+        for _ in range(2):  # the tickets of a split launch are left at zero
+            got = dec.gemv_host("s", x, t=t, path=ops.PATH_DECODE)
+            parity.assert_close(got, want, "n%d k%d g%d t%d" % (n, k, group, t))
+        got16 = dec.gemv_host("s", x, t=t, out_f16=True, path=ops.PATH_DECODE)
+        assert np.array_equal(got16, gen.f32_to_f16_bits(got))
+    finally:
+        dec.cc.close()
