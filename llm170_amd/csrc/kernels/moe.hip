@@ -778,36 +778,32 @@ MOE_FAMILY(w4a16_moe_g128_bf16, 128, true, 4)
 // ---------------------------------------------------------------------------------------------------- routing
 // Routing rule of the reference (w4a16_dec/mod.rs:168-185, device counterpart assets/moe.cu:686-759): softmax over all
 // experts, the k largest probabilities with ties to the lower index, weights renormalised by the selected sum.
-// One wave per token, n <= 1024 (16 experts per lane).  Selection runs on ONE unique, totally ordered 64-bit key per
-// expert — the probability's bit pattern (monotone for non-negative floats) above the complement of the expert index —
-// so "larger probability, then lower index" is a plain unsigned maximum: a round takes the lane's largest key, a
-// butterfly of unsigned maxima over the wave, and retires the winner by comparing keys (0 = absent or taken; no real
-// key is 0 because index complements are non-zero).
-__device__ __forceinline__ unsigned long long topk_wave_max(unsigned long long v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const unsigned lo = __shfl_xor((unsigned)v, off), hi = __shfl_xor((unsigned)(v >> 32), off);
-        const unsigned long long o = ((unsigned long long)hi << 32) | lo;
-        v = o > v ? o : v;
-    }
-    return v;
+// One wave per token, n <= 1024; the body is built for 2, 4 and 16 experts per lane (n <= 128, 256, 1024).  The kernel is
+// a chain of dependent wave-wide steps and nothing else, so a selection round is kept short: the probability's bit
+// pattern (monotone for non-negative floats) plus one is a 32-bit key, 0 for an absent or taken expert; a lane's largest
+// key, six v_max_u32 with DPP operands and one lane read give the round's probability, and one ballot per expert of a
+// lane, in index order, names the lowest index that holds it.  (Rounds on a 64-bit key with the index in its low half
+// and shuffles through LDS, always 16 experts per lane: 6.9 us at one token and 9.0 at 2048, 128 experts, top-8; this form
+// 3.4 and 3.5, of which 2.4 are the launch.)
+template <int CTRL>
+__device__ __forceinline__ unsigned topk_dpp_max(unsigned v) {
+    const unsigned o = __builtin_amdgcn_update_dpp(0u, v, CTRL, 0xF, 0xF, true);  // lanes without a source read 0
+    return o > v ? o : v;
 }
 
-extern "C" __global__ __launch_bounds__(256) void w4a16_moe_topk_t(const float* __restrict__ lg, int* __restrict__ idx,
-                                                                   float* __restrict__ wt, int t, int n, int k) {
-    constexpr int PER_LANE = 16;
+template <int PER_LANE>
+__device__ __forceinline__ void moe_topk_body(const float* __restrict__ logits, int* __restrict__ idx,
+                                              float* __restrict__ wt, int n, int k) {
     const int lane = threadIdx.x & 63;
-    const int token = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (token >= t) return;
-    const float* logits = lg + (size_t)token * n;
     float e[PER_LANE];
     float top = -INFINITY;
 #pragma unroll
     for (int j = 0; j < PER_LANE; j++) {
         const int i = lane + 64 * j;
         e[j] = i < n ? logits[i] : -INFINITY;
-        top = fmaxf(top, e[j]);
     }
+#pragma unroll
+    for (int j = 0; j < PER_LANE; j++) top = fmaxf(top, e[j]);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off));
     float total = 0.f;
@@ -818,27 +814,52 @@ extern "C" __global__ __launch_bounds__(256) void w4a16_moe_topk_t(const float* 
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) total += __shfl_xor(total, off);
-    unsigned long long key[PER_LANE];
+    unsigned key[PER_LANE];
 #pragma unroll
-    for (int j = 0; j < PER_LANE; j++) {
-        const unsigned i = (unsigned)(lane + 64 * j);
-        const float p = e[j] / total;
-        key[j] = i < (unsigned)n ? ((unsigned long long)__builtin_bit_cast(unsigned, p) << 32) | (unsigned long long)(~i) : 0ull;
-    }
-    float chosen_sum = 0.f, kept = 0.f;  // lane r keeps the r-th chosen probability (k <= 64)
+    for (int j = 0; j < PER_LANE; j++)
+        key[j] = lane + 64 * j < n ? __builtin_bit_cast(unsigned, e[j] / total) + 1u : 0u;
+    float chosen_sum = 0.f, kept = 0.f;  // lane r keeps the r-th chosen probability and expert (k <= 64)
+    int kept_i = 0;
     for (int r = 0; r < k; r++) {
-        unsigned long long best = 0ull;
+        unsigned best = key[0];
 #pragma unroll
-        for (int j = 0; j < PER_LANE; j++) best = key[j] > best ? key[j] : best;
-        best = topk_wave_max(best);
+        for (int j = 1; j < PER_LANE; j++) best = key[j] > best ? key[j] : best;
+        best = topk_dpp_max<0x111>(best);  // row_shr 1, 2, 4, 8: lane 15 of a row holds the row's maximum
+        best = topk_dpp_max<0x112>(best);
+        best = topk_dpp_max<0x114>(best);
+        best = topk_dpp_max<0x118>(best);
+        best = topk_dpp_max<0x142>(best);  // row_bcast 15, 31: lane 63 holds the wave's
+        best = topk_dpp_max<0x143>(best);
+        best = (unsigned)__builtin_amdgcn_readlane((int)best, 63);
+        int at = 0;
 #pragma unroll
-        for (int j = 0; j < PER_LANE; j++) key[j] = key[j] == best ? 0ull : key[j];
-        const float p = __builtin_bit_cast(float, (unsigned)(best >> 32));
-        if (lane == 0) idx[(size_t)token * k + r] = (int)(~(unsigned)best);
+        for (int j = PER_LANE - 1; j >= 0; j--) {  // the last that matches is the lowest j
+            const unsigned long long hit = __ballot(key[j] == best);
+            if (hit) at = 64 * j + __builtin_ctzll(hit);
+        }
+#pragma unroll
+        for (int j = 0; j < PER_LANE; j++) key[j] = lane + 64 * j == at ? 0u : key[j];
+        const float p = __builtin_bit_cast(float, best - 1u);
         kept = lane == r ? p : kept;
+        kept_i = lane == r ? at : kept_i;
         chosen_sum += p;
     }
-    if (lane < k) wt[(size_t)token * k + lane] = kept / chosen_sum;
+    if (lane < k) {
+        idx[lane] = kept_i;
+        wt[lane] = kept / chosen_sum;
+    }
+}
+
+extern "C" __global__ __launch_bounds__(256) void w4a16_moe_topk_t(const float* __restrict__ lg, int* __restrict__ idx,
+                                                                   float* __restrict__ wt, int t, int n, int k) {
+    const int token = blockIdx.x * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (token >= t) return;
+    const float* const logits = lg + (size_t)token * n;
+    int* const oi = idx + (size_t)token * k;
+    float* const ow = wt + (size_t)token * k;
+    if (n <= 128) moe_topk_body<2>(logits, oi, ow, n, k);
+    else if (n <= 256) moe_topk_body<4>(logits, oi, ow, n, k);
+    else moe_topk_body<16>(logits, oi, ow, n, k);
 }
 
 // Stable counting sort of slots by expert with every expert's run padded to a multiple of `block`
