@@ -103,6 +103,7 @@ static const char* const kMoeSyms[] = {W4_MOE_FAMILY("w4a16_moe_g32_f16"),
                                        "w4a16_moe_g128_bf16_down_sum1",
                                        "w4a16_moe_topk_t",
                                        "w4a16_moe_align",
+                                       "w4a16_moe_align_wide",
                                        "w4a16_moe_topk_sum_f16",
                                        nullptr};
 

@@ -184,9 +184,12 @@ extern "C" int w4a16_moe_align(w4a16_ctx* ctx, uint64_t idx_dev, size_t ns, size
         return w4_fail(W4A16_ERR_SHAPE, "moe_align: ns=%zu n_exp=%zu block=%zu", ns, n_exp, block);
     W4_TRY(w4_hip(hipSetDevice(ctx->device), "hipSetDevice"));
     int nsi = (int)ns, ni = (int)n_exp, bi = (int)block;
-    void* p[] = {&idx_dev, &nsi, &ni, &bi, &sorted_dev, &expert_ids_dev, &num_post_dev};
-    // LDS: 16 per-wave count rows, totals and offsets, one entry per expert each
-    return w4_launch(ctx, "w4a16_moe_align", 1, 1, 64 * kW4MoeAlignWaves, (unsigned)((kW4MoeAlignWaves + 2) * n_exp * 4), p);
+    // one workgroup per 2048 slots, at most 16 (each counts all slots; kernels/moe.hip).  LDS: 16 per-wave count rows,
+    // totals, offsets and (several workgroups) slots ahead, one entry per expert each
+    int wgs = (int)std::min<size_t>(16, (ns + 2047) / 2048);
+    void* p[] = {&idx_dev, &nsi, &ni, &bi, &sorted_dev, &expert_ids_dev, &num_post_dev, &wgs};
+    return w4_launch(ctx, wgs > 1 ? "w4a16_moe_align_wide" : "w4a16_moe_align", (unsigned)wgs, 1, 64 * kW4MoeAlignWaves,
+                     (unsigned)((kW4MoeAlignWaves + (wgs > 1 ? 3 : 2)) * n_exp * 4), p);
 }
 
 // ------------------------------------------------------------------------------------------------ FFN

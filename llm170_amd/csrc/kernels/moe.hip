@@ -863,30 +863,37 @@ extern "C" __global__ __launch_bounds__(256) void w4a16_moe_topk_t(const float* 
 }
 
 // Stable counting sort of slots by expert with every expert's run padded to a multiple of `block`
-// (assets/moe.cu:860-908 + 1599-1633 in one launch).  One workgroup of 1024 threads, n_exp <= 1024.
+// (assets/moe.cu:860-908 + 1599-1633 in one launch).  Workgroups of 1024 threads, n_exp <= 1024.
 //   sorted_ids: slot ids in expert order, padding = sentinel ns; expert_ids[b]: expert of segment b;
 //   num_post[0] = padded total, num_post[1] = number of distinct experts hit.
-// Wave w owns the contiguous slot range [w*chunk, (w+1)*chunk): per-wave counts, an exclusive prefix over the
-// waves per expert, a two-level scan over the experts' padded counts, then every wave places its slots in order.
-// An out-of-range expert id is dropped (its slot is never placed).
+// A workgroup owns a contiguous range of slots, its wave w the w-th chunk of it: per-wave counts, an exclusive prefix
+// over the waves per expert, a two-level scan over the experts' padded counts, then every wave places its slots in
+// order.  An out-of-range expert id is dropped (its slot is never placed).
+// The placement (a ballot per bit of the expert id for every 64 slots) is what a launch spends its time on, so beyond
+// 2048 slots it is spread over workgroups, about two steps of 64 slots per wave; each of them counts ALL slots (LDS atomics,
+// a fraction of the placement's cost), which gives it the number of slots ahead of its range per expert and the totals
+// without a second launch (128 experts: 4136 slots 7.4 -> 6.2 us, 16384 18.1 -> 7.7, 32768 32.8 -> 9.8).
 #define MOE_ALIGN_WAVES 16
 #define MOE_ALIGN_THREADS (64 * MOE_ALIGN_WAVES)
 #define MOE_ALIGN_KEEP 4  // 64-slot steps of a wave whose expert ids stay in registers between the two passes
-extern "C" __global__ __launch_bounds__(MOE_ALIGN_THREADS) void w4a16_moe_align(const int* __restrict__ idx, int ns,
-                                                                               int n_exp, int block,
-                                                                               int* __restrict__ sorted_ids,
-                                                                               int* __restrict__ expert_ids,
-                                                                               int* __restrict__ num_post) {
-    extern __shared__ unsigned align_lds[];  // cnt[WAVES][n_exp] (per wave count, then exclusive prefix over the waves),
-                                             // tot[n_exp], poff[n_exp]
+template <bool WIDE>
+__device__ __forceinline__ void moe_align_body(const int* __restrict__ idx, int ns, int n_exp, int block,
+                                               int* __restrict__ sorted_ids, int* __restrict__ expert_ids,
+                                               int* __restrict__ num_post, int wgs) {
+    extern __shared__ unsigned align_lds[];  // cnt[WAVES][n_exp] (per wave count, then the slots of the expert ahead
+                                             // of the wave's), tot[n_exp], poff[n_exp], WIDE: pre[n_exp] (slots ahead of the range)
     unsigned* const cnt = align_lds;
     unsigned* const tot = cnt + MOE_ALIGN_WAVES * n_exp;
     unsigned* const poff = tot + n_exp;
+    unsigned* const pre = poff + n_exp;
     __shared__ unsigned wsum[MOE_ALIGN_WAVES], whit[MOE_ALIGN_WAVES];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int i = tid; i < MOE_ALIGN_WAVES * n_exp; i += MOE_ALIGN_THREADS) cnt[i] = 0;
-    const int chunk = ((ns + MOE_ALIGN_WAVES * 64 - 1) / (MOE_ALIGN_WAVES * 64)) * 64;  // slots per wave, multiple of 64
-    const int j0 = wave * chunk, steps = chunk / 64;
+    for (int i = tid; i < (MOE_ALIGN_WAVES + (WIDE ? 3 : 0)) * n_exp; i += MOE_ALIGN_THREADS) cnt[i] = 0;
+    const int wg = WIDE ? (int)blockIdx.x : 0;
+    if (!WIDE) wgs = 1;
+    const int chunk = ((ns + wgs * MOE_ALIGN_WAVES * 64 - 1) / (wgs * MOE_ALIGN_WAVES * 64)) * 64;  // slots per wave, multiple of 64
+    const int lo = wg * MOE_ALIGN_WAVES * chunk, hi = min(ns, lo + MOE_ALIGN_WAVES * chunk);  // this workgroup's slots
+    const int j0 = lo + wave * chunk, steps = chunk / 64;
     int keep[MOE_ALIGN_KEEP];
 #pragma unroll
     for (int s = 0; s < MOE_ALIGN_KEEP; s++) {
@@ -911,6 +918,19 @@ extern "C" __global__ __launch_bounds__(MOE_ALIGN_THREADS) void w4a16_moe_align(
         const int e = expert_of(s);
         if (e >= 0) atomicAdd(&cnt[wave * n_exp + e], 1u);
     }
+    if (WIDE) {  // the other workgroups' slots, four loads in flight per thread
+        for (int j = tid; j < ns; j += 4 * MOE_ALIGN_THREADS) {
+            int e[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int ju = j + u * MOE_ALIGN_THREADS;
+                e[u] = ju < ns && (ju < lo || ju >= hi) ? idx[ju] : -1;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if ((unsigned)e[u] < (unsigned)n_exp) atomicAdd(j + u * MOE_ALIGN_THREADS < lo ? &pre[e[u]] : &tot[e[u]], 1u);
+        }
+    }
     __syncthreads();
     // thread i owns expert i: total over the waves, then a scan of the padded totals over all threads
     unsigned padded = 0, hits = 0;
@@ -918,11 +938,13 @@ extern "C" __global__ __launch_bounds__(MOE_ALIGN_THREADS) void w4a16_moe_align(
         const int e = tid;
         unsigned run = 0;
         if (e < n_exp) {
+            if (WIDE) run = pre[e];
             for (int w = 0; w < MOE_ALIGN_WAVES; w++) {
                 const unsigned c = cnt[w * n_exp + e];
                 cnt[w * n_exp + e] = run;
                 run += c;
             }
+            if (WIDE) run += tot[e];
             tot[e] = run;
         }
         padded = ((run + block - 1) / block) * block;
@@ -951,16 +973,25 @@ extern "C" __global__ __launch_bounds__(MOE_ALIGN_THREADS) void w4a16_moe_align(
     }
     const unsigned pos0 = base + incl - padded;
     if (tid < n_exp) poff[tid] = pos0;
-    // every position gets the padding sentinel first, coalesced; the slots are placed over it after the barrier (a
-    // workgroup barrier waits for the stores issued before it, so the order of the two writes to a position is fixed)
-    for (unsigned p = tid; p < all; p += MOE_ALIGN_THREADS) sorted_ids[p] = ns;
-    if (tid < n_exp)
-        for (unsigned b = 0; b < padded / block; b++) expert_ids[pos0 / block + b] = tid;
-    if (tid == 0) {
-        num_post[0] = (int)all;
-        num_post[1] = (int)allhit;
+    // Padding sentinels.  A workgroup alone writes one to every position, coalesced, and places the slots over them after
+    // the barrier (which waits for the stores issued before it, so the order of the two writes to a position is fixed);
+    // several write the padding behind every expert's run only, after the barrier.
+    if (!WIDE)
+        for (unsigned p = tid; p < all; p += MOE_ALIGN_THREADS) sorted_ids[p] = ns;
+    if (wg == 0) {
+        if (tid < n_exp)
+            for (unsigned b = 0; b < padded / block; b++) expert_ids[pos0 / block + b] = tid;
+        if (tid == 0) {
+            num_post[0] = (int)all;
+            num_post[1] = (int)allhit;
+        }
     }
     __syncthreads();
+    // padding sentinels of several workgroups: eight threads to an expert, experts dealt to the workgroups
+    for (int i = wg * MOE_ALIGN_THREADS + tid; WIDE && i < n_exp * 8; i += wgs * MOE_ALIGN_THREADS) {
+        const unsigned n_e = tot[i >> 3], end = ((n_e + block - 1) / block) * block;
+        for (unsigned p = n_e + (i & 7); p < end; p += 8) sorted_ids[poff[i >> 3] + p] = ns;
+    }
     // placement in slot order: every wave walks its range 64 slots at a time; rank among equal experts in the step.
     // The wave's row of cnt is private to it and LDS operations of one wave execute in order, so the loop needs no
     // workgroup barrier; the wave-scope fences keep the compiler from reordering the LDS accesses.
@@ -989,6 +1020,18 @@ extern "C" __global__ __launch_bounds__(MOE_ALIGN_THREADS) void w4a16_moe_align(
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
     }
+}
+
+// (Two kernels: the few instructions more cost the one-workgroup launch 0.35 of its 3.8 us.)
+extern "C" __global__ __launch_bounds__(MOE_ALIGN_THREADS) void w4a16_moe_align(const int* idx, int ns, int n_exp, int block,
+                                                                               int* sorted_ids, int* expert_ids,
+                                                                               int* num_post) {
+    moe_align_body<false>(idx, ns, n_exp, block, sorted_ids, expert_ids, num_post, 1);
+}
+extern "C" __global__ __launch_bounds__(MOE_ALIGN_THREADS) void w4a16_moe_align_wide(const int* idx, int ns, int n_exp,
+                                                                                    int block, int* sorted_ids,
+                                                                                    int* expert_ids, int* num_post, int wgs) {
+    moe_align_body<true>(idx, ns, n_exp, block, sorted_ids, expert_ids, num_post, wgs);
 }
 
 // out[t][c] = sum over the token's k slots of f16 c2[slot][c], added in slot order in f32 (assets/moe.cu:1662-1674).

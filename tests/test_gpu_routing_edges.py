@@ -33,3 +33,33 @@ def test_route_edges(dec, n, k, t):
     assert np.array_equal(idx, want_i)
     # exp and the softmax sum in another order than on the host: 16 f32 roundings at most along either
     assert np.max(np.abs(w - want_w) / np.maximum(want_w, 1e-30)) < 16 * 2.0**-23
+
+
+@pytest.mark.parametrize("ns,n_exp,block", [(2048, 128, 32), (2049, 128, 32), (4097, 128, 48), (32769, 128, 64),
+                                            (70000, 8, 64), (2500, 1024, 16)])
+@pytest.mark.parametrize("kind", ["random", "one expert", "dropped"])
+def test_align_edges(dec, ns, n_exp, block, kind):
+    print("align", ns, n_exp, block, kind, flush=True)
+    idx = np.random.default_rng(ns).integers(0, n_exp, ns).astype(np.int32)
+    if kind == "one expert":
+        idx[:] = n_exp - 1
+    if kind == "dropped":
+        idx[::3] = -1
+        idx[1::7] = n_exp
+    cc = dec.cc
+    cap_s, cap_e = ns + n_exp * block, ns // block + n_exp + 1
+    pi, ps, pe, pn = cc.to_device(idx), cc.alloc(cap_s * 4), cc.alloc(cap_e * 4), cc.alloc(8)
+    dec.moe_align(pi, ns, n_exp, block, ps, pe, pn)
+    n_post, hit = cc.d2h(pn, (2,), np.int32)
+    s, e = cc.d2h(ps, (cap_s,), np.int32), cc.d2h(pe, (cap_e,), np.int32)
+    for p in (pi, ps, pe, pn):
+        cc.free(p)
+    want_s, want_e = [], []
+    for x in range(n_exp):
+        run = np.flatnonzero(idx == x)
+        segs = -(-run.size // block)
+        want_s.append(np.concatenate([run, np.full(segs * block - run.size, ns)]))
+        want_e.append(np.full(segs, x))
+    want_s, want_e = np.concatenate(want_s), np.concatenate(want_e)
+    assert n_post == want_s.size and hit == np.unique(want_e).size
+    assert np.array_equal(s[:n_post], want_s) and np.array_equal(e[: want_e.size], want_e)
