@@ -780,7 +780,8 @@ MOE_FAMILY(w4a16_moe_g128_bf16, 128, true, 4)
 // experts, the k largest probabilities with ties to the lower index, weights renormalised by the selected sum.
 // One wave per token, n <= 1024; the body is built for 2, 4 and 16 experts per lane (n <= 128, 256, 1024).  The kernel is
 // a chain of dependent wave-wide steps and nothing else, so a selection round is kept short: the probability's bit
-// pattern (monotone for non-negative floats) plus one is a 32-bit key, 0 for an absent or taken expert; a lane's largest
+// pattern (monotone for non-negative floats; NaN of all ones held one lower) plus one is a 32-bit key, 0 for an absent or
+// taken expert; a lane's largest
 // key, six v_max_u32 with DPP operands and one lane read give the round's probability, and one ballot per expert of a
 // lane, in index order, names the lowest index that holds it.  (Rounds on a 64-bit key with the index in its low half
 // and shuffles through LDS, always 16 experts per lane: 6.9 us at one token and 9.0 at 2048, 128 experts, top-8; this form
@@ -817,7 +818,7 @@ __device__ __forceinline__ void moe_topk_body(const float* __restrict__ logits, 
     unsigned key[PER_LANE];
 #pragma unroll
     for (int j = 0; j < PER_LANE; j++)
-        key[j] = lane + 64 * j < n ? __builtin_bit_cast(unsigned, e[j] / total) + 1u : 0u;
+        key[j] = lane + 64 * j < n ? min(__builtin_bit_cast(unsigned, e[j] / total), 0xfffffffeu) + 1u : 0u;
     float chosen_sum = 0.f, kept = 0.f;  // lane r keeps the r-th chosen probability and expert (k <= 64)
     int kept_i = 0;
     for (int r = 0; r < k; r++) {

@@ -35,6 +35,24 @@ def test_route_edges(dec, n, k, t):
     assert np.max(np.abs(w - want_w) / np.maximum(want_w, 1e-30)) < 16 * 2.0**-23
 
 
+@pytest.mark.parametrize("bits", [0x7FC00000, 0xFFFFFFFF])
+def test_route_nan_row(dec, bits):
+    """A row with a NaN logit (also one of all ones, the largest bit pattern) still names k different experts."""
+    n, k, t = 128, 8, 2
+    lg = gen.normal_f32(5, (t, n))
+    lg.view(np.uint32)[0, :] = bits
+    lg.view(np.uint32)[1, 77] = bits
+    cc = dec.cc
+    pl, pi, pw = cc.to_device(lg), cc.alloc(t * k * 4), cc.alloc(t * k * 4)
+    dec.moe_route(pl, t, n, k, pi, pw)
+    idx, w = cc.d2h(pi, (t, k), np.int32), cc.d2h(pw, (t, k), np.float32)
+    for p in (pl, pi, pw):
+        cc.free(p)
+    assert np.all(np.isnan(w))
+    for row in idx:
+        assert np.unique(row).size == k and row.min() >= 0 and row.max() < n
+
+
 @pytest.mark.parametrize("ns,n_exp,block", [(2048, 128, 32), (2049, 128, 32), (4097, 128, 48), (32769, 128, 64),
                                             (70000, 8, 64), (2500, 1024, 16)])
 @pytest.mark.parametrize("kind", ["random", "one expert", "dropped"])
