@@ -166,13 +166,16 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
     // group gi) are the 8 bytes at sc + rb*aux_rb_bytes + (d*GPT + gi)*32
     auto compute = [&](const DecodeStage<RB, XL>& s_, const char* sc, int d) {
         // B operand of MFMA w = chunk w of x for token column m.  Through LDS: a wave's LDS operations run in order, so
-        // neither the reads of this tile's rows nor the next tile's writes need a wait of their own.
+        // neither the reads of this tile's rows nor the next tile's writes need a wait of their own; the wave-scope
+        // fences (no instructions) keep the compiler from reordering them, as lanes read what other lanes wrote.
         u4_t xb[4];
         if constexpr (XLDS) {
 #pragma unroll
             for (int l = 0; l < XL; l++) *reinterpret_cast<u4_t*>(x_put + l * 64) = s_.x[l];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
 #pragma unroll
             for (int w = 0; w < 4; w++) xb[w] = *reinterpret_cast<const u4_t*>(x_get + w * (4 * (XROWS + 1) * 16));
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
         } else {  // held by lane m + 4w
             xb[0] = s_.x[0];
             xb[1] = w4_row_shl<4>(s_.x[0]);
