@@ -105,12 +105,18 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
     // Every load is a raw buffer load: an out-of-range offset returns zeros and costs no memory traffic, which
     // predicates token columns >= t without a branch.
     // x load l of a tile brings rows 4l..4l+3, 16 bytes per lane.  XLDS: 16 lanes to a row, to be re-ordered through LDS;
-    // otherwise (one load) lane (m, g) fetches, for token m % 4, the 8 halves of chunk m / 4 at k offset g*8.
-    const int xrow = XLDS ? lane >> 4 : m & 3, xpiece = XLDS ? lane & 15 : (m >> 2) * 4 + g;
-    unsigned xoff[XL];
+    // otherwise (one load) lane (m, g) fetches, for token m % 4, the 8 halves of chunk m / 4 at k offset g*8.  (The one
+    // offset outside the array: its branch keeps the few small arguments a batch of their own ahead of the pointers;
+    // 16 launches of 27B layers at t = 4 take 0.6 us more without it.)
+    const int xrow = lane >> 4, xpiece = lane & 15;
+    const int xtok = m % 4, xchunk = m / 4;
+    const unsigned xoff1 = xtok < t ? ((unsigned)xtok * (unsigned)ldx + (unsigned)(xchunk * 32 + g * 8)) * 2u : W4_OOB;
+    unsigned xoff[XL] = {xoff1};
+    if constexpr (XLDS) {
 #pragma unroll
-    for (int l = 0; l < XL; l++)
-        xoff[l] = 4 * l + xrow < t ? ((unsigned)(4 * l + xrow) * (unsigned)ldx + (unsigned)xpiece * 8u) * 2u : W4_OOB;
+        for (int l = 0; l < XL; l++)
+            xoff[l] = 4 * l + xrow < t ? ((unsigned)(4 * l + xrow) * (unsigned)ldx + (unsigned)xpiece * 8u) * 2u : W4_OOB;
+    }
     const unsigned q_bytes = (unsigned)row_blocks * (unsigned)kt_n * 1024u, s_bytes = (unsigned)row_blocks * (unsigned)kg_n * 32u,
                    x_bytes = ((unsigned)(t - 1) * (unsigned)ldx + (unsigned)k) * 2u;  // x rows are ldx halves apart
     f4_t acc[RB];
@@ -214,12 +220,13 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
     // 1/sqrt(mean + 1e-6).  The entries of token columns 0..3 are fetched here, ahead of the ring, by LDS DMA (no
     // registers held across the fill) into a staging area behind the scale slots, 64 entries per instruction, lane l
     // entry c*64 + l; once the first weight tiles are in flight lane l adds its entries, a butterfly adds the lanes
-    // (fixed order: the same bits on every run), and the factor is parked at the start of the staging area.  The
-    // epilogue multiplies the sums by it.  Further token quads and entries beyond the staging area (8 x 64) repeat the
-    // fetch inside input_scale.
+    // (fixed order: the same bits on every run), and the factor is parked in the wave's own slot of `red`, which the
+    // in-block reduction never writes, or where that holds staged x at the start of the staging area.  The epilogue
+    // multiplies the sums by it.  Further token quads and entries beyond the staging area (8 x 64) repeat the fetch
+    // inside input_scale.
     typedef __attribute__((address_space(3))) char lds_char_t;
     lds_char_t* const stage_lds = (lds_char_t*)(reinterpret_cast<char*>(red) + W * REGION + W * AUX_PW);
-    float* const park = reinterpret_cast<float*>(reinterpret_cast<char*>(red) + W * REGION + W * AUX_PW);
+    float* const park = reinterpret_cast<float*>(reinterpret_cast<char*>(red) + (XLDS ? W * REGION + W * AUX_PW : 0));
     const int stat_chunks = min((n_stats_in + 63) >> 6, 8);
     auto fetch_stats = [&](int c0, int qd) {
         const __amdgpu_buffer_rsrc_t sr_in = w4_make_rsrc(stats_in, (unsigned)n_stats_in * 64u);
