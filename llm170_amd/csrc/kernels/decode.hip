@@ -539,10 +539,11 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
 #define DECODE_HI __attribute__((amdgpu_waves_per_eu(6, 6)))
 #define DECODE_MID __attribute__((amdgpu_waves_per_eu(5, 5)))
 #define DECODE_LO
-// rb1 at group 128: all three x widths fit the HI regime
+// rb1 at group 128: x1 and x2 fit HI, x4 MID (85 VGPRs; held to 80 it spills one, and a launch is up to 4 % longer:
+// 3072 x 1024 at t = 12 4.08 against 4.24 us, 4096 x 4096 at t = 16 6.20 against 6.31)
 #define DECODE_KERNEL_RB1(NAME, G, SBF)                                                       \
     DECODE_KERNEL_X(NAME, G, SBF, 1, 1, 24, DECODE_HI) DECODE_KERNEL_X(NAME, G, SBF, 1, 2, 24, DECODE_HI) \
-    DECODE_KERNEL_X(NAME, G, SBF, 1, 4, 24, DECODE_HI)
+    DECODE_KERNEL_X(NAME, G, SBF, 1, 4, 24, DECODE_MID)
 // rb2 at group 128: x1 fits HI, x2 MID
 #define DECODE_KERNEL_RB2_G128(NAME, SBF)                                                         \
     DECODE_KERNEL_X(NAME, 128, SBF, 2, 1, 24, DECODE_HI) DECODE_KERNEL_X(NAME, 128, SBF, 2, 2, 24, DECODE_MID) \

@@ -142,6 +142,22 @@ def test_code_objects_are_gfx950():
         assert blob[:4] == b"\x7fELF" and b"gfx950" in blob, asset
 
 
+def test_decode_kernels_use_no_scratch():
+    """Neither spilled registers nor a private segment in any decode kernel: a kernel with one makes its first launch
+    allocate scratch memory, and w4a16_lin_forward_noalloc launches every one of them."""
+    import subprocess
+    readelf = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-readelf")
+    notes = subprocess.run([readelf, "--notes", os.path.join(ROOT, "llm170_amd", "assets", "decode.hsaco")],
+                           capture_output=True, text=True, check=True, timeout=60).stdout
+    field = lambda key: re.findall(r"^\s+(?:- )?\.%s:\s+(\w+)\s*$" % key, notes, flags=re.M)
+    names = [n for n in field("name") if n.startswith("w4a16_")]
+    assert sorted(names) == sorted(ffi.manifest()["decode"])
+    for key in ("private_segment_fixed_size", "vgpr_spill_count", "sgpr_spill_count"):
+        values = field(key)
+        assert len(values) == len(names)
+        assert [(n, v) for n, v in zip(names, values) if v != "0"] == [], key
+
+
 def test_bench_refuses_more_than_one_gpu():
     """The bench measures one GPU's share; asked for more it says so and exits non-zero without touching a device."""
     import subprocess
