@@ -46,28 +46,14 @@ static const char* const kLayoutSyms[] = {"w4a16_tile_q",         "w4a16_tile_s"
                                           "w4a16_untile_s",       "w4a16_dump_tiled_f16",  "w4a16_dump_tiled_bf16",
                                           "w4a16_dump_raw_f16",   "w4a16_dump_raw_bf16",   "w4a16_row_norm_max_f16",
                                           "w4a16_row_norm_max_bf16", nullptr};
-static const char* const kDecodeSyms[] = {
-    "w4a16_decode_g128_f16_rb1_x1", "w4a16_decode_g128_f16_rb1_x2", "w4a16_decode_g128_f16_rb1_x4",
-    "w4a16_decode_g128_f16_rb2_x1", "w4a16_decode_g128_f16_rb2_x2", "w4a16_decode_g128_f16_rb2_x4",
-    "w4a16_decode_g128_f16_rb4_x1", "w4a16_decode_g128_f16_rb4_x2", "w4a16_decode_g128_f16_rb4_x4",
-    "w4a16_decode_g128_bf16_rb1_x1", "w4a16_decode_g128_bf16_rb1_x2", "w4a16_decode_g128_bf16_rb1_x4",
-    "w4a16_decode_g128_bf16_rb2_x1", "w4a16_decode_g128_bf16_rb2_x2", "w4a16_decode_g128_bf16_rb2_x4",
-    "w4a16_decode_g128_bf16_rb4_x1", "w4a16_decode_g128_bf16_rb4_x2", "w4a16_decode_g128_bf16_rb4_x4",
-    "w4a16_decode_g32_f16_rb1_x1", "w4a16_decode_g32_f16_rb1_x2", "w4a16_decode_g32_f16_rb1_x4",
-    "w4a16_decode_g32_f16_rb2_x1", "w4a16_decode_g32_f16_rb2_x2", "w4a16_decode_g32_f16_rb2_x4",
-    "w4a16_decode_g32_f16_rb4_x1", "w4a16_decode_g32_f16_rb4_x2", "w4a16_decode_g32_f16_rb4_x4",
-    "w4a16_decode_g32_bf16_rb1_x1", "w4a16_decode_g32_bf16_rb1_x2", "w4a16_decode_g32_bf16_rb1_x4",
-    "w4a16_decode_g32_bf16_rb2_x1", "w4a16_decode_g32_bf16_rb2_x2", "w4a16_decode_g32_bf16_rb2_x4",
-    "w4a16_decode_g32_bf16_rb4_x1", "w4a16_decode_g32_bf16_rb4_x2", "w4a16_decode_g32_bf16_rb4_x4",
-    "w4a16_decode_g128_f16_glu_x1", "w4a16_decode_g128_f16_glu_x2", "w4a16_decode_g128_f16_glu_x4",
-    "w4a16_decode_g128_bf16_glu_x1", "w4a16_decode_g128_bf16_glu_x2", "w4a16_decode_g128_bf16_glu_x4",
-    "w4a16_decode_g32_f16_glu_x1", "w4a16_decode_g32_f16_glu_x2", "w4a16_decode_g32_f16_glu_x4",
-    "w4a16_decode_g32_bf16_glu_x1", "w4a16_decode_g32_bf16_glu_x2", "w4a16_decode_g32_bf16_glu_x4",
-    "w4a16_decode_g128_f16_multi_x1", "w4a16_decode_g128_f16_multi_x2", "w4a16_decode_g128_f16_multi_x4",
-    "w4a16_decode_g128_bf16_multi_x1", "w4a16_decode_g128_bf16_multi_x2", "w4a16_decode_g128_bf16_multi_x4",
-    "w4a16_decode_g32_f16_multi_x1", "w4a16_decode_g32_f16_multi_x2", "w4a16_decode_g32_f16_multi_x4",
-    "w4a16_decode_g32_bf16_multi_x1", "w4a16_decode_g32_bf16_multi_x2", "w4a16_decode_g32_bf16_multi_x4",
-    nullptr};
+// one family: the row counts' builds of a kernel, x by direct loads where the name ends in d (kernels/decode.hip)
+#define W4_DECODE_FAMILY(P) P "_x1", P "_x2", P "_x4", P "_x2d", P "_x4d"
+#define W4_DECODE_SCALES(P)                                                                               \
+    W4_DECODE_FAMILY(P "_rb1"), W4_DECODE_FAMILY(P "_rb2"), W4_DECODE_FAMILY(P "_rb4"), W4_DECODE_FAMILY(P "_glu"), \
+        W4_DECODE_FAMILY(P "_multi")
+static const char* const kDecodeSyms[] = {W4_DECODE_SCALES("w4a16_decode_g128_f16"), W4_DECODE_SCALES("w4a16_decode_g128_bf16"),
+                                          W4_DECODE_SCALES("w4a16_decode_g32_f16"), W4_DECODE_SCALES("w4a16_decode_g32_bf16"),
+                                          nullptr};
 static const char* const kPrefillG128Syms[] = {
     "w4a16_prefill_g128_f16", "w4a16_prefill_g128_bf16", "w4a16_prefill_g128_f16_m64", "w4a16_prefill_g128_bf16_m64",
     "w4a16_prefill_g128_f16_m96", "w4a16_prefill_g128_bf16_m96", "w4a16_prefill_g128_f16_glu", "w4a16_prefill_g128_bf16_glu",

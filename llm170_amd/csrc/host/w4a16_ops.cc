@@ -61,8 +61,9 @@ static int launch_lane(w4a16_ctx* ctx, uint64_t q, uint64_t s, uint64_t x, uint6
 // each (measured 12.4 -> 11.8 us at t = 1, 13.3 -> 12.4 us at t = 4).  Shorter k ranges lose more to the extra
 // workgroups than they gain.
 // LDS: the waves' staged scales grow with the k tiles per wave (kernels/decode.hip).  A plan that would pass the 160 KiB
-// of a CU is shrunk — automatic row blocks per wave are halved first (keeps one launch without tickets), then the k
-// range is cut into more slices — and only a shape that fits in no such plan is refused.
+// of a CU takes x by direct loads (from five rows on: 1 KiB per row block and wave instead of up to 4.25 KiB for staged
+// x).  If it still does, it is shrunk — automatic row blocks per wave are halved first (keeps one launch without tickets),
+// then the k range is cut into more slices — and only a shape that fits in no such plan is refused.
 struct DecodePlanIn {
     size_t row_blocks = 0, k = 0, group = 128, t = 1;
     int cu_count = 256;
@@ -74,6 +75,8 @@ struct DecodePlan {
     int rb = 0, waves = 0, nks = 1, kt_per_slice = 0, kt_per_wave = 0;
     size_t blocks = 0;
     unsigned shmem = 0;
+    int x_loads = 1;     // x loads per k tile, four rows each
+    bool x_lds = false;  // x goes through LDS
 };
 
 // LDS bytes of one wave's staged scales (kernels/decode.hip, AUX_PW)
@@ -81,12 +84,9 @@ static unsigned decode_scale_lds(size_t group, int rb, int kt_per_wave) {
     return ((unsigned)(rb * kt_per_wave * (128 / (int)group) * 32) + 1023u) / 1024u * 1024u;
 }
 
-// x loads per k tile, four rows each, and the LDS bytes of a wave: its partial tiles, or its staged x tile where x goes
-// through LDS (kernels/decode.hip, REGION)
-static int decode_x_loads(size_t t) { return t <= 4 ? 1 : t <= 8 ? 2 : 4; }
-static unsigned decode_wave_lds(int rb, size_t t) {
-    const int xl = decode_x_loads(t);
-    return (unsigned)std::max(rb * 1024, xl > 1 ? (4 * xl + 1) * 256 : 0);
+// LDS bytes of a wave: its partial tiles, or its staged x tile where x goes through LDS (kernels/decode.hip, REGION)
+static unsigned decode_wave_lds(int rb, int x_loads, bool x_lds) {
+    return (unsigned)std::max(rb * 1024, x_lds ? (4 * x_loads + 1) * 256 : 0);
 }
 
 static int plan_decode(const DecodePlanIn& in, DecodePlan* out) {
@@ -133,7 +133,11 @@ static int plan_decode(const DecodePlanIn& in, DecodePlan* out) {
         P.kt_per_wave = (P.kt_per_slice + P.waves - 1) / P.waves;
         // per wave its partial tiles or staged x tile; then per wave the scales of its whole k slice (rb x tiles per
         // wave x groups per tile x 32 bytes, in whole 1 KiB DMA instructions); then the statistics staging area
-        P.shmem = (unsigned)P.waves * decode_wave_lds(rb, in.t) + (unsigned)P.waves * decode_scale_lds(in.group, rb, P.kt_per_wave) + in.extra_lds;
+        const unsigned other = (unsigned)P.waves * decode_scale_lds(in.group, rb, P.kt_per_wave) + in.extra_lds;
+        P.x_loads = in.t <= 4 ? 1 : in.t <= 8 ? 2 : 4;
+        P.x_lds = P.x_loads > 1;
+        if ((unsigned)P.waves * decode_wave_lds(rb, P.x_loads, P.x_lds) + other > 160u * 1024u) P.x_lds = false;
+        P.shmem = (unsigned)P.waves * decode_wave_lds(rb, P.x_loads, P.x_lds) + other;
         if (P.shmem <= 160u * 1024u) {
             *out = P;
             return 0;
@@ -243,6 +247,12 @@ struct DecodeMultiHost {
 };
 static_assert(sizeof(DecodeMultiHost) == 40, "DecodeMulti is three pointers and four ints");
 
+// Kernel of a plan: one x load per k tile serves up to 4 token rows, two up to 8, four up to 16 (kernels/decode.hip)
+static void decode_sym(char* sym, size_t cap, const W4Lin& L, const char* body, const DecodePlan& P) {
+    snprintf(sym, cap, "w4a16_decode_g%zu_%s_%s_x%d%s", L.group, L.scale_bf16 ? "bf16" : "f16", body, P.x_loads,
+             P.x_loads > 1 && !P.x_lds ? "d" : "");
+}
+
 static int launch_decode(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_t y, size_t t, int out_f16,
                          DecodeNorm* norm = nullptr, const DecodeWorkspace* fixed_ws = nullptr,
                          const DecodeMultiHost* multi = nullptr) {
@@ -268,13 +278,8 @@ static int launch_decode(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_t y,
     const int rb = P.rb;
     int waves = P.waves, nks = P.nks, kt_per_slice = P.kt_per_slice, kt_per_wave = P.kt_per_wave;
     const size_t blocks = P.blocks;
-    // x loads per k tile: one serves up to 4 token rows, two up to 8, four up to 16 (kernels/decode.hip)
-    const int xl = decode_x_loads(t);
     char sym[64];
-    if (multi)
-        snprintf(sym, sizeof sym, "w4a16_decode_g%zu_%s_multi_x%d", L.group, L.scale_bf16 ? "bf16" : "f16", xl);
-    else
-        snprintf(sym, sizeof sym, "w4a16_decode_g%zu_%s_rb%d_x%d", L.group, L.scale_bf16 ? "bf16" : "f16", rb, xl);
+    decode_sym(sym, sizeof sym, L, multi ? "multi" : rb == 1 ? "rb1" : rb == 2 ? "rb2" : "rb4", P);
     uint64_t qt = L.q_tiled, st = L.s_tiled;
     int row_blocks = (int)L.row_blocks, ki = (int)L.k, ni = (int)L.n, ti = (int)t, of = out_f16 ? 1 : 0;
     DecodeWorkspace W;
@@ -321,9 +326,8 @@ static int launch_decode_glu(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_
     W4_TRY(plan_decode(in, &P));
     int waves = P.waves, nks = P.nks, kt_per_slice = P.kt_per_slice, kt_per_wave = P.kt_per_wave;
     const size_t blocks = P.blocks;
-    const int xl = decode_x_loads(t);
     char sym[64];
-    snprintf(sym, sizeof sym, "w4a16_decode_g%zu_%s_glu_x%d", L.group, L.scale_bf16 ? "bf16" : "f16", xl);
+    decode_sym(sym, sizeof sym, L, "glu", P);
     uint64_t qt = L.q_tiled, st = L.s_tiled;
     int row_blocks = (int)L.row_blocks, ki = (int)L.k, ni = (int)L.n, ti = (int)t, of = 1;
     DecodeWorkspace W;

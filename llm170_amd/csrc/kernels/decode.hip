@@ -71,7 +71,8 @@ struct DecodeMulti {
 
 #define DECODE_ONE_OUTPUT (DecodeMulti{{0ull, 0ull, 0ull}, {0x7fffffff, 0x7fffffff, 0x7fffffff}, 0})
 
-template <int G, bool SBF, int RB, int DEPTH, int XL, bool GLU = false, bool MULTI = false>
+// X_LDS: x through LDS where XL > 1 (off: every lane loads its B operands itself, two or four loads per k tile).
+template <int G, bool SBF, int RB, int DEPTH, int XL, bool X_LDS, bool GLU = false, bool MULTI = false>
 __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const uint16_t* __restrict__ st,
                                             const uint16_t* __restrict__ x, void* __restrict__ y, int row_blocks,
                                             int k, int n, int t, int out_f16, f4_t* ws, int* tickets, int W, int nks,
@@ -82,8 +83,10 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
                                             DecodeMulti mo) {
     extern __shared__ f4_t red[];  // [W][REGION] staged x, then partial tiles of the in-block split-K; the waves' staged scales
     constexpr int GPT = W4_TILE_K / G;  // scale groups per k tile
-    constexpr bool XLDS = XL > 1;       // x goes through LDS
-    constexpr int XROWS = 4 * XL;       // x rows of a staged k tile
+    constexpr bool XLDS = X_LDS && XL > 1;  // x goes through LDS
+    constexpr int XROWS = 4 * XL;           // x rows of a staged k tile
+    constexpr int C = 4 / XL;               // direct loads: 32-k chunks (MFMAs) served by one x load,
+    constexpr int TPL = 16 / C;             // and the token columns it serves
     // LDS bytes per wave: its staged x tile while it streams, its partial tiles afterwards
     constexpr int REGION = XLDS && (XROWS + 1) * 256 > RB * 1024 ? (XROWS + 1) * 256 : RB * 1024;
     // The launch geometry (W waves per block, nks k slices over blockIdx.y, tiles per slice and per wave) arrives as
@@ -104,18 +107,21 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
 
     // Every load is a raw buffer load: an out-of-range offset returns zeros and costs no memory traffic, which
     // predicates token columns >= t without a branch.
-    // x load l of a tile brings rows 4l..4l+3, 16 bytes per lane.  XLDS: 16 lanes to a row, to be re-ordered through LDS;
-    // otherwise (one load) lane (m, g) fetches, for token m % 4, the 8 halves of chunk m / 4 at k offset g*8.  (The one
+    // XLDS: x load l of a tile brings rows 4l..4l+3, 16 bytes per lane, 16 lanes to a row, to be re-ordered through LDS;
+    // otherwise lane (m, g) fetches, for token m % TPL, the 8 halves of chunk l*C + m / TPL at k offset g*8.  (The one
     // offset outside the array: its branch keeps the few small arguments a batch of their own ahead of the pointers;
     // 16 launches of 27B layers at t = 4 take 0.6 us more without it.)
     const int xrow = lane >> 4, xpiece = lane & 15;
-    const int xtok = m % 4, xchunk = m / 4;
+    const int xtok = m % TPL, xchunk = m / TPL;
     const unsigned xoff1 = xtok < t ? ((unsigned)xtok * (unsigned)ldx + (unsigned)(xchunk * 32 + g * 8)) * 2u : W4_OOB;
     unsigned xoff[XL] = {xoff1};
     if constexpr (XLDS) {
 #pragma unroll
         for (int l = 0; l < XL; l++)
             xoff[l] = 4 * l + xrow < t ? ((unsigned)(4 * l + xrow) * (unsigned)ldx + (unsigned)xpiece * 8u) * 2u : W4_OOB;
+    } else {
+#pragma unroll
+        for (int l = 1; l < XL; l++) xoff[l] = xoff1 + (unsigned)(l * C * 32) * 2u;
     }
     const unsigned q_bytes = (unsigned)row_blocks * (unsigned)kt_n * 1024u, s_bytes = (unsigned)row_blocks * (unsigned)kg_n * 32u,
                    x_bytes = ((unsigned)(t - 1) * (unsigned)ldx + (unsigned)k) * 2u;  // x rows are ldx halves apart
@@ -182,11 +188,16 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
 #pragma unroll
             for (int w = 0; w < 4; w++) xb[w] = *reinterpret_cast<const u4_t*>(x_get + w * (4 * (XROWS + 1) * 16));
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-        } else {  // held by lane m + 4w
-            xb[0] = s_.x[0];
-            xb[1] = w4_row_shl<4>(s_.x[0]);
-            xb[2] = w4_row_shl<8>(s_.x[0]);
-            xb[3] = w4_row_shl<12>(s_.x[0]);
+        } else {  // chunk w is held by lane m + (w % C) * TPL of load w / C
+#pragma unroll
+            for (int l = 0; l < XL; l++) {
+                xb[l * C] = s_.x[l];
+                if constexpr (C >= 2) xb[l * C + 1] = w4_row_shl<TPL>(s_.x[l]);
+                if constexpr (C == 4) {
+                    xb[2] = w4_row_shl<2 * TPL>(s_.x[l]);
+                    xb[3] = w4_row_shl<3 * TPL>(s_.x[l]);
+                }
+            }
         }
 #pragma unroll
         for (int rb = 0; rb < RB; rb++) {
@@ -485,57 +496,44 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
 #define DECODE_DEPTH(BUDGET, G, RB, XL) \
     ((BUDGET / DECODE_STAGE_REGS(G, RB, XL)) < 2 ? 2 : (BUDGET / DECODE_STAGE_REGS(G, RB, XL)) > 8 ? 8 : (BUDGET / DECODE_STAGE_REGS(G, RB, XL)))
 
-#define DECODE_KERNEL_X(NAME, G, SBF, RB, XL, BUDGET, ATTR)                                                          \
-    extern "C" __global__ __launch_bounds__(512) ATTR void NAME##_x##XL(const u4_t* qt, const uint16_t* st,          \
-                                                                        const uint16_t* x, void* y, int row_blocks,  \
-                                                                        int k, int n, int t, int out_f16, f4_t* ws,  \
-                                                                        int* tickets, int waves, int nks,            \
-                                                                        int kt_per_slice, int kt_per_wave, int ldx,  \
-                                                                        const float* stats_in, int n_stats_in,       \
-                                                                        float inv_cols_in, float* stats_out,         \
-                                                                        int stat_rows, float* resid,                 \
-                                                                        const float* nw, int act_kind,               \
-                                                                        float in_scale, float out_scale) {           \
-        decode_body<G, SBF, RB, DECODE_DEPTH(BUDGET, G, RB, XL), XL>(                                                \
-            qt, st, x, y, row_blocks, k, n, t, out_f16, ws, tickets, waves, nks, kt_per_slice, kt_per_wave, ldx,     \
-            stats_in, n_stats_in, inv_cols_in, stats_out, stat_rows, resid, nw, act_kind, in_scale, out_scale,       \
-            DECODE_ONE_OUTPUT);                                                                                      \
+#define DECODE_PARAMS                                                                                                  \
+    const u4_t *qt, const uint16_t *st, const uint16_t *x, void *y, int row_blocks, int k, int n, int t, int out_f16,  \
+        f4_t *ws, int *tickets, int waves, int nks, int kt_per_slice, int kt_per_wave, int ldx, const float *stats_in, \
+        int n_stats_in, float inv_cols_in, float *stats_out, int stat_rows, float *resid, const float *nw,             \
+        int act_kind, float in_scale, float out_scale
+#define DECODE_ARGS                                                                                                    \
+    qt, st, x, y, row_blocks, k, n, t, out_f16, ws, tickets, waves, nks, kt_per_slice, kt_per_wave, ldx, stats_in,     \
+        n_stats_in, inv_cols_in, stats_out, stat_rows, resid, nw, act_kind, in_scale, out_scale
+
+#define DECODE_KERNEL_SYM(SYM, G, SBF, RB, XL, X_LDS, BUDGET, ATTR)                                                    \
+    extern "C" __global__ __launch_bounds__(512) ATTR void SYM(DECODE_PARAMS) {                                        \
+        decode_body<G, SBF, RB, DECODE_DEPTH(BUDGET, G, RB, XL), XL, X_LDS>(DECODE_ARGS, DECODE_ONE_OUTPUT);           \
     }
 // The same kernel with one output per part of a fused linear (two row blocks per wave): a symbol of its own, because
 // the 40 more bytes of kernel arguments cost every launch 0.2 us, whether it has parts or not (measured on the 27B
 // shapes at t = 1 and 4).
-#define DECODE_MULTI_KERNEL_X(NAME, G, SBF, XL, BUDGET, ATTR)                                                         \
-    extern "C" __global__ __launch_bounds__(512) ATTR void NAME##_x##XL(const u4_t* qt, const uint16_t* st,          \
-                                                                        const uint16_t* x, void* y, int row_blocks,  \
-                                                                        int k, int n, int t, int out_f16, f4_t* ws,  \
-                                                                        int* tickets, int waves, int nks,            \
-                                                                        int kt_per_slice, int kt_per_wave, int ldx,  \
-                                                                        const float* stats_in, int n_stats_in,       \
-                                                                        float inv_cols_in, float* stats_out,         \
-                                                                        int stat_rows, float* resid,                 \
-                                                                        const float* nw, int act_kind,               \
-                                                                        float in_scale, float out_scale,             \
-                                                                        DecodeMulti mo) {                            \
-        decode_body<G, SBF, 2, DECODE_DEPTH(BUDGET, G, 2, XL), XL, false, true>(                                     \
-            qt, st, x, y, row_blocks, k, n, t, out_f16, ws, tickets, waves, nks, kt_per_slice, kt_per_wave, ldx,     \
-            stats_in, n_stats_in, inv_cols_in, stats_out, stat_rows, resid, nw, act_kind, in_scale, out_scale, mo);  \
+#define DECODE_MULTI_KERNEL_SYM(SYM, G, SBF, XL, X_LDS, BUDGET, ATTR)                                                  \
+    extern "C" __global__ __launch_bounds__(512) ATTR void SYM(DECODE_PARAMS, DecodeMulti mo) {                        \
+        decode_body<G, SBF, 2, DECODE_DEPTH(BUDGET, G, 2, XL), XL, X_LDS, false, true>(DECODE_ARGS, mo);               \
     }
-#define DECODE_GLU_KERNEL_X(NAME, G, SBF, XL, BUDGET, ATTR)                                                           \
-    extern "C" __global__ __launch_bounds__(512) ATTR void NAME##_x##XL(const u4_t* qt, const uint16_t* st,          \
-                                                                        const uint16_t* x, void* y, int row_blocks,  \
-                                                                        int k, int n, int t, int out_f16, f4_t* ws,  \
-                                                                        int* tickets, int waves, int nks,            \
-                                                                        int kt_per_slice, int kt_per_wave, int ldx,  \
-                                                                        const float* stats_in, int n_stats_in,       \
-                                                                        float inv_cols_in, float* stats_out,         \
-                                                                        int stat_rows, float* resid,                 \
-                                                                        const float* nw, int act_kind,               \
-                                                                        float in_scale, float out_scale) {           \
-        decode_body<G, SBF, 2, DECODE_DEPTH(BUDGET, G, 2, XL), XL, true>(                                            \
-            qt, st, x, y, row_blocks, k, n, t, out_f16, ws, tickets, waves, nks, kt_per_slice, kt_per_wave, ldx,     \
-            stats_in, n_stats_in, inv_cols_in, stats_out, stat_rows, resid, nw, act_kind, in_scale, out_scale,       \
-            DECODE_ONE_OUTPUT);                                                                                      \
+#define DECODE_GLU_KERNEL_SYM(SYM, G, SBF, XL, X_LDS, BUDGET, ATTR)                                                    \
+    extern "C" __global__ __launch_bounds__(512) ATTR void SYM(DECODE_PARAMS) {                                        \
+        decode_body<G, SBF, 2, DECODE_DEPTH(BUDGET, G, 2, XL), XL, X_LDS, true>(DECODE_ARGS, DECODE_ONE_OUTPUT);       \
     }
+// _x<XL>: x through LDS (XL > 1).  _x<XL>d: x by direct loads, in the same register regime; for launches whose staged
+// scales leave no LDS for x (a wave's region is 1 KiB per row block instead of up to 4.25 KiB).
+#define DECODE_KERNEL_X(NAME, G, SBF, RB, XL, BUDGET, ATTR) \
+    DECODE_KERNEL_SYM(NAME##_x##XL, G, SBF, RB, XL, true, BUDGET, ATTR)
+#define DECODE_KERNEL_XD(NAME, G, SBF, RB, XL, BUDGET, ATTR) \
+    DECODE_KERNEL_SYM(NAME##_x##XL##d, G, SBF, RB, XL, false, BUDGET, ATTR)
+#define DECODE_MULTI_KERNEL_X(NAME, G, SBF, XL, BUDGET, ATTR) \
+    DECODE_MULTI_KERNEL_SYM(NAME##_x##XL, G, SBF, XL, true, BUDGET, ATTR)
+#define DECODE_MULTI_KERNEL_XD(NAME, G, SBF, XL, BUDGET, ATTR) \
+    DECODE_MULTI_KERNEL_SYM(NAME##_x##XL##d, G, SBF, XL, false, BUDGET, ATTR)
+#define DECODE_GLU_KERNEL_X(NAME, G, SBF, XL, BUDGET, ATTR) \
+    DECODE_GLU_KERNEL_SYM(NAME##_x##XL, G, SBF, XL, true, BUDGET, ATTR)
+#define DECODE_GLU_KERNEL_XD(NAME, G, SBF, XL, BUDGET, ATTR) \
+    DECODE_GLU_KERNEL_SYM(NAME##_x##XL##d, G, SBF, XL, false, BUDGET, ATTR)
 #define DECODE_HI __attribute__((amdgpu_waves_per_eu(6, 6)))
 #define DECODE_MID __attribute__((amdgpu_waves_per_eu(5, 5)))
 #define DECODE_LO
@@ -543,14 +541,17 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
 // 3072 x 1024 at t = 12 4.08 against 4.24 us, 4096 x 4096 at t = 16 6.20 against 6.31)
 #define DECODE_KERNEL_RB1(NAME, G, SBF)                                                       \
     DECODE_KERNEL_X(NAME, G, SBF, 1, 1, 24, DECODE_HI) DECODE_KERNEL_X(NAME, G, SBF, 1, 2, 24, DECODE_HI) \
-    DECODE_KERNEL_X(NAME, G, SBF, 1, 4, 24, DECODE_MID)
+    DECODE_KERNEL_X(NAME, G, SBF, 1, 4, 24, DECODE_MID) DECODE_KERNEL_XD(NAME, G, SBF, 1, 2, 24, DECODE_HI) \
+    DECODE_KERNEL_XD(NAME, G, SBF, 1, 4, 24, DECODE_HI)
 // rb2 at group 128: x1 fits HI, x2 MID
 #define DECODE_KERNEL_RB2_G128(NAME, SBF)                                                         \
     DECODE_KERNEL_X(NAME, 128, SBF, 2, 1, 24, DECODE_HI) DECODE_KERNEL_X(NAME, 128, SBF, 2, 2, 24, DECODE_MID) \
-    DECODE_KERNEL_X(NAME, 128, SBF, 2, 4, 64, DECODE_LO)
+    DECODE_KERNEL_X(NAME, 128, SBF, 2, 4, 64, DECODE_LO) DECODE_KERNEL_XD(NAME, 128, SBF, 2, 2, 24, DECODE_MID) \
+    DECODE_KERNEL_XD(NAME, 128, SBF, 2, 4, 64, DECODE_LO)
 #define DECODE_KERNEL_LO3(NAME, G, SBF, RB)                                                   \
     DECODE_KERNEL_X(NAME, G, SBF, RB, 1, 24, DECODE_LO) DECODE_KERNEL_X(NAME, G, SBF, RB, 2, 24, DECODE_LO) \
-    DECODE_KERNEL_X(NAME, G, SBF, RB, 4, 24, DECODE_LO)
+    DECODE_KERNEL_X(NAME, G, SBF, RB, 4, 24, DECODE_LO) DECODE_KERNEL_XD(NAME, G, SBF, RB, 2, 24, DECODE_LO) \
+    DECODE_KERNEL_XD(NAME, G, SBF, RB, 4, 24, DECODE_LO)
 
 DECODE_KERNEL_RB1(w4a16_decode_g128_f16_rb1, 128, false)
 DECODE_KERNEL_RB2_G128(w4a16_decode_g128_f16_rb2, false)
@@ -567,10 +568,12 @@ DECODE_KERNEL_LO3(w4a16_decode_g32_bf16_rb4, 32, true, 4)
 // one output per part of a fused linear
 #define DECODE_MULTI_G128(NAME, SBF)                                                                       \
     DECODE_MULTI_KERNEL_X(NAME, 128, SBF, 1, 24, DECODE_HI) DECODE_MULTI_KERNEL_X(NAME, 128, SBF, 2, 24, DECODE_MID) \
-    DECODE_MULTI_KERNEL_X(NAME, 128, SBF, 4, 64, DECODE_LO)
+    DECODE_MULTI_KERNEL_X(NAME, 128, SBF, 4, 64, DECODE_LO) DECODE_MULTI_KERNEL_XD(NAME, 128, SBF, 2, 24, DECODE_MID) \
+    DECODE_MULTI_KERNEL_XD(NAME, 128, SBF, 4, 64, DECODE_LO)
 #define DECODE_MULTI_G32(NAME, SBF)                                                                      \
     DECODE_MULTI_KERNEL_X(NAME, 32, SBF, 1, 24, DECODE_LO) DECODE_MULTI_KERNEL_X(NAME, 32, SBF, 2, 24, DECODE_LO) \
-    DECODE_MULTI_KERNEL_X(NAME, 32, SBF, 4, 24, DECODE_LO)
+    DECODE_MULTI_KERNEL_X(NAME, 32, SBF, 4, 24, DECODE_LO) DECODE_MULTI_KERNEL_XD(NAME, 32, SBF, 2, 24, DECODE_LO) \
+    DECODE_MULTI_KERNEL_XD(NAME, 32, SBF, 4, 24, DECODE_LO)
 DECODE_MULTI_G128(w4a16_decode_g128_f16_multi, false)
 DECODE_MULTI_G128(w4a16_decode_g128_bf16_multi, true)
 DECODE_MULTI_G32(w4a16_decode_g32_f16_multi, false)
@@ -578,10 +581,12 @@ DECODE_MULTI_G32(w4a16_decode_g32_bf16_multi, true)
 // fused gate|up with the SiLU*up epilogue (two row blocks per wave by construction)
 #define DECODE_GLU_G128(NAME, SBF)                                                                     \
     DECODE_GLU_KERNEL_X(NAME, 128, SBF, 1, 24, DECODE_HI) DECODE_GLU_KERNEL_X(NAME, 128, SBF, 2, 24, DECODE_MID) \
-    DECODE_GLU_KERNEL_X(NAME, 128, SBF, 4, 64, DECODE_LO)
+    DECODE_GLU_KERNEL_X(NAME, 128, SBF, 4, 64, DECODE_LO) DECODE_GLU_KERNEL_XD(NAME, 128, SBF, 2, 24, DECODE_MID) \
+    DECODE_GLU_KERNEL_XD(NAME, 128, SBF, 4, 64, DECODE_LO)
 #define DECODE_GLU_G32(NAME, SBF)                                                                    \
     DECODE_GLU_KERNEL_X(NAME, 32, SBF, 1, 24, DECODE_LO) DECODE_GLU_KERNEL_X(NAME, 32, SBF, 2, 24, DECODE_LO) \
-    DECODE_GLU_KERNEL_X(NAME, 32, SBF, 4, 24, DECODE_LO)
+    DECODE_GLU_KERNEL_X(NAME, 32, SBF, 4, 24, DECODE_LO) DECODE_GLU_KERNEL_XD(NAME, 32, SBF, 2, 24, DECODE_LO) \
+    DECODE_GLU_KERNEL_XD(NAME, 32, SBF, 4, 24, DECODE_LO)
 DECODE_GLU_G128(w4a16_decode_g128_f16_glu, false)
 DECODE_GLU_G128(w4a16_decode_g128_bf16_glu, true)
 DECODE_GLU_G32(w4a16_decode_g32_f16_glu, false)

@@ -79,6 +79,9 @@ def test_decode_plan_shrinks_to_fit_the_lds():
     assert p["rows_per_wave"] == 64, "group 128 needs a quarter of that and keeps four row blocks"
     p = ops.plan_decode(16384, 106496, 32, 8, glu=True)
     assert p["lds_bytes"] <= 160 * 1024 and p["k_slices"] >= 2, p
+    # staged x (4.25 KiB per wave from nine rows on) takes no shape away: it gives way to direct loads first
+    p = ops.plan_decode(16, 128 * 9216, 32, 16)
+    assert p["lds_bytes"] <= 160 * 1024 and p["k_slices"] == 8, p
     # nothing fits: a k range that even one row block per wave and eight slices cannot stage
     with pytest.raises(ops.W4a16Error) as e:
         ops.plan_decode(64, 128 * 20000, 32, 1)
