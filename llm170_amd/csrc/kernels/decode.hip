@@ -86,7 +86,7 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
     constexpr bool XLDS = X_LDS && XL > 1;  // x goes through LDS
     constexpr int XROWS = 4 * XL;           // x rows of a staged k tile
     constexpr int C = 4 / XL;               // direct loads: 32-k chunks (MFMAs) served by one x load,
-    constexpr int TPL = 16 / C;             // and the token columns it serves
+    constexpr int TPL = XLDS ? 4 : 16 / C;  // and the token columns it serves
     // LDS bytes per wave: its staged x tile while it streams, its partial tiles afterwards
     constexpr int REGION = XLDS && (XROWS + 1) * 256 > RB * 1024 ? (XROWS + 1) * 256 : RB * 1024;
     // The launch geometry (W waves per block, nks k slices over blockIdx.y, tiles per slice and per wave) arrives as

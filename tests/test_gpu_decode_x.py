@@ -55,3 +55,25 @@ def test_pinned_gated_shape_without_room_for_staged_x(dec):
         for p in (xd, gu, a, b):
             cc.free(p)
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("group,rows,t,direct", [
+    (128, 16, 5, True), (128, 32, 8, True), (128, 32, 9, True), (128, 32, 11, True), (128, 32, 12, False),
+    (32, 16, 8, True), (32, 32, 8, False), (32, 32, 9, True), (32, 64, 14, True), (32, 32, 15, False),
+])
+def test_few_waves_take_x_directly_with_the_same_bits(dec, group, rows, t, direct):
+    """One workgroup of four waves per CU at most: the rule's edges, and every row's bits as in the 16-row launch (x
+    through LDS), whose sums run in the same order."""
+    print("few waves", group, rows, t, flush=True)
+    n, k = 200, 1280  # a partial row block; ten k tiles on four waves
+    q, s, x = gen.make_linear(n, k, group, 16, seed=group + rows + t)
+    dec.upload_lin_g("few", q, s, n, k, group, False)
+    try:
+        dec.set_decode_shape(rows, 4)
+        want = dec.gemv_host("few", x, t=16, path=ops.PATH_DECODE)
+        assert dec.cc.last_launch_symbol().endswith("_rb%d_x4" % (rows // 16))
+        got = dec.gemv_host("few", np.ascontiguousarray(x[:t]), t=t, path=ops.PATH_DECODE)
+        assert dec.cc.last_launch_symbol().endswith("d") == direct
+    finally:
+        dec.set_decode_shape(0, 0)
+    assert np.array_equal(got.view(np.uint32), want[:t].view(np.uint32))

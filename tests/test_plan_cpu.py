@@ -69,6 +69,20 @@ def test_decode_plan_at_the_layer_shapes():
         assert p["lds_bytes"] <= 160 * 1024
 
 
+def test_decode_plan_takes_x_directly_where_few_waves_run():
+    """At most four waves per CU: a wave's LDS holds its partial tiles (2 KiB at two row blocks) and scales, not staged
+    x (4.25 KiB), up to the row count where staging wins; 5120 x 5120 is 160 workgroups of four waves."""
+    scales = {128: 4 * 1024, 32: 4 * 3 * 1024}  # 2 row blocks x 10 k tiles x (1 or 4) groups x 32 B, in whole KiB
+    for group, last in [(128, 11), (32, 14)]:
+        for t in (9, last, last + 1, 16):
+            p = ops.plan_decode(5120, 5120, group, t)
+            assert (p["rows_per_wave"], p["waves_per_block"], p["k_slices"]) == (32, 4, 1)
+            assert p["lds_bytes"] == 4 * (2048 if t <= last else 17 * 256) + scales[group], (group, t, p)
+    # twice the row blocks: two workgroups per CU, staged from nine rows on
+    p = ops.plan_decode(10240, 5120, 128, 9)
+    assert p["lds_bytes"] == 4 * 17 * 256 + scales[128], p
+
+
 def test_decode_plan_shrinks_to_fit_the_lds():
     """Group 32 with a long unsplit k: the staged scales of four row blocks per wave would pass 160 KiB (n = 16384,
     k = 53248, t = 8: 4 waves x 104 k tiles x 4 groups x 4 row blocks x 32 B = 213 KiB).  The plan halves the rows per
