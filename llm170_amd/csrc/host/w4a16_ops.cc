@@ -100,7 +100,9 @@ static int plan_decode(const DecodePlanIn& in, DecodePlan* out) {
     const int kt_n = (int)(in.k / 128);
     if (kt_n <= 0 || in.row_blocks == 0) return w4_fail(W4A16_ERR_SHAPE, "decode: empty linear");
     const bool wide = in.row_blocks >= 1024;
-    const bool small = in.row_blocks <= (size_t)std::max(in.cu_count, 1);  // one row block per workgroup fits the chip at once
+    // one row block per workgroup fits the chip at once; pinned rows (and a launch with one output per part) keep the
+    // slices of any narrow output
+    const bool small = !in.glu && !in.rows_per_wave && in.row_blocks <= (size_t)std::max(in.cu_count, 1);
     const bool long_k_narrow = !wide && kt_n >= 64 && in.t >= 7;
     int rb;
     bool rb_auto = false;
@@ -125,7 +127,7 @@ static int plan_decode(const DecodePlanIn& in, DecodePlan* out) {
         nks_auto = true;
         const size_t blocks = in.glu ? in.row_blocks / 2 : (in.row_blocks + (size_t)rb - 1) / (size_t)rb;
         if (blocks < (size_t)std::max(in.cu_count, 1) && kt_n >= 64 && !(small && rb == 1)) {
-            nks_want = std::min(small && !in.glu ? 4 : kW4DecodeMaxKsplit, kt_n / 16);
+            nks_want = std::min(small ? 4 : kW4DecodeMaxKsplit, kt_n / 16);
             waves_cap = 4;
         }
     }

@@ -30,3 +30,32 @@ def test_small_outputs(orc, n, k, group, t):
         assert np.array_equal(got16, gen.f32_to_f16_bits(got))
     finally:
         dec.cc.close()
+
+
+@pytest.mark.parametrize("t", [1, 8])
+def test_pinned_rows_keep_their_slices(t):
+    """32 rows per wave pinned, and the launch with one output per part (built for 32): a long k over few workgroups
+    runs in eight slices of four waves, at any row count, whatever the automatic row count would do."""
+    print("pinned rows", t, flush=True)
+    n, k = 512, 16384
+    dec = ops.W4a16Dec()
+    cc = dec.cc
+    try:
+        q, s, x = gen.make_linear(n, k, 128, t, seed=t)
+        dec.upload_lin_g("a", np.ascontiguousarray(q[:256]), np.ascontiguousarray(s[:256]), 256, k, 128, False)
+        dec.upload_lin_g("b", np.ascontiguousarray(q[256:]), np.ascontiguousarray(s[256:]), 256, k, 128, False)
+        dec.lin_fuse("ab", ["a", "b"])
+        xd, ya, yb = cc.to_device(x), cc.alloc(t * 256 * 4), cc.alloc(t * 256 * 4)
+        dec.lin_forward_multi("ab", xd, [ya, yb], t)
+        multi = np.concatenate([cc.d2h(ya, (t, 256), np.uint32), cc.d2h(yb, (t, 256), np.uint32)], axis=1)
+        dec.set_decode_shape(32, 0)
+        auto = dec.gemv_host("ab", x, t=t, path=ops.PATH_DECODE).view(np.uint32)
+        dec.set_decode_shape(32, 4)
+        sliced = {}
+        for slices in (4, 8):
+            dec.set_decode_ksplit(slices)
+            sliced[slices] = dec.gemv_host("ab", x, t=t, path=ops.PATH_DECODE).view(np.uint32)
+    finally:
+        dec.cc.close()
+    assert not np.array_equal(sliced[4], sliced[8])  # another order of the same sums
+    assert np.array_equal(auto, sliced[8]) and np.array_equal(multi, sliced[8])
