@@ -53,9 +53,20 @@ static int launch_lane(w4a16_ctx* ctx, uint64_t q, uint64_t s, uint64_t x, uint6
 // workgroups back (t = 16: 21.6 -> 15.8 us, t = 12: 18.6 -> 14.9, t = 8: 14.2 -> 13.5; level at t = 6).
 // Outputs of at most one row block per CU (256 row blocks, n = 4096): one row block per wave x eight waves, so that every
 // CU has a workgroup, and no k slices (4096 x 4096 at t = 1 5.72 -> 4.80 us, t = 8 6.31 -> 5.19, t = 16 7.01 -> 6.24;
-// k = 11008 9.07 -> 7.64; 1024 x 4096 5.24 -> 4.48; at 384 row blocks the two shapes are within 5 % and at 448 two row
-// blocks win) — from seven rows with a long k two row blocks in four slices (2048 x 11008 at t = 16 8.75 -> 8.1,
-// 1024 x 8192 7.86 -> 6.7: the slices split the x loads, which grow with t).
+// k = 8192 8.47 -> 6.58; at 384 row blocks the two shapes are within 5 % and at 448 two row blocks win).
+// Their k slices, from 64 k tiles on (figures: group 128, cold weights, best shape / unsplit one row block x eight waves
+// / two row blocks x four waves in slices of 16 k tiles, the rule of larger outputs).  A wave's k tiles follow each other at
+// about 0.29 us, so a slice pays once the tiles it saves outweigh the hand-over, which grows with the workgroups:
+//   t <= 4: 16 x 17408 t = 1 4.85 / 7.7 / 4.85; 512 x 9216 5.55 / 5.82 / 6.29, x 17408 6.40 / 8.16 / 7.07; 1024 x 9216
+//     5.84 (unsplit) / 6.50, x 17408 7.08 / 8.15 / 7.29; 2048 x 12288 6.90 (unsplit) / 7.70, x 17408 8.1 / 8.3 / 8.9; beyond 128
+//     row blocks unsplit wins throughout (3072 x 17408 8.7 / 9.9).
+//   t = 5, 6 (a k tile takes 0.39 us): 512 x 17408 t = 5 6.70 / 9.85 / 7.18; 1024 x 17408 7.29 / 9.85 / 7.40; 2048 x 10240
+//     7.4 (unsplit) / 7.4, x 17408 9.05 (two row blocks) / 10.1; a last generation of workgroups that is nearly empty loses
+//     (2064 x 16384, 520 workgroups: 9.49 unsplit, 10.4 in slices), so they have to fit two per CU or k be long.
+//   t >= 7: two row blocks share the x loads and the slices split them: 256 x 17408 t = 16 6.83 / 13.7 / 8.02 (four row
+//     blocks, the rule of larger outputs), 2048 x 11008 8.1 / 8.75; beyond 128 row blocks from nine rows on four row blocks,
+//     in as many slices as one workgroup per CU allows (group 128): 3072 x 16384 t = 16 10.4 against 11.9 in two row blocks
+//     and 11.5 in eight slices.  Row blocks 128 KiB apart (k = 16384) prefer that at 7 and 8 rows too (4096: 10.9 against 12.3).
 // k slices across workgroups (one launch; partial tiles and tickets in a workspace): only for a long k range over
 // fewer workgroups than CUs (the 27B down projection: 160 blocks x 136 k tiles): slices of about 16 k tiles, four waves
 // each (measured 12.4 -> 11.8 us at t = 1, 13.3 -> 12.4 us at t = 4).  Shorter k ranges lose more to the extra
@@ -65,8 +76,9 @@ static int launch_lane(w4a16_ctx* ctx, uint64_t q, uint64_t s, uint64_t x, uint6
 // what a launch waits for and the round trip shows, so direct loads stay up to the row count where their cost, which
 // grows with the rows, overtakes it (two row blocks x four waves, direct / through LDS: 5120 x 5120 group 128 t = 9 7.40 /
 // 7.72 us, t = 11 7.62 / 7.66, t = 12 7.88 / 7.81; group 32 t = 9 7.99 / 8.60, t = 14 8.51 / 8.52, t = 15 8.81 / 8.63;
-// 5120 x 2048 group 32 t = 9 5.10 / 5.44; up to eight rows 4096 x 4096 group 128 t = 5 6.39 / 6.62).  Two row blocks at
-// group 32 up to eight rows are the exception (5120 x 5120 t = 8 8.70 / 8.31; one row block t = 6 6.03 / 6.28).
+// 5120 x 2048 group 32 t = 9 5.10 / 5.44; up to eight rows 4096 x 4096 group 128 t = 5 6.39 / 6.62; four row blocks
+// 5120 x 5120 group 128 t = 12 9.75 / 9.93, t = 16 10.56 / 10.13, group 32 t = 16 11.49 / 12.08).  Two row blocks at group 32
+// up to eight rows are the exception (5120 x 5120 t = 8 8.70 / 8.31; one row block t = 6 6.03 / 6.28).
 // LDS: the waves' staged scales grow with the k tiles per wave (kernels/decode.hip).  A plan that would pass the 160 KiB
 // of a CU takes x by direct loads (from five rows on: 1 KiB per row block and wave instead of up to 4.25 KiB for staged
 // x).  If it still does, it is shrunk — automatic row blocks per wave are halved first (keeps one launch without tickets),
@@ -104,6 +116,31 @@ static int plan_decode(const DecodePlanIn& in, DecodePlan* out) {
     // slices of any narrow output
     const bool small = !in.glu && !in.rows_per_wave && in.row_blocks <= (size_t)std::max(in.cu_count, 1);
     const bool long_k_narrow = !wide && kt_n >= 64 && in.t >= 7;
+    // Row blocks per wave, waves and k slices of a small output with a long k
+    int small_rb = 1, small_waves = 8, small_slices = 1;
+    if (small && kt_n >= 64) {
+        const size_t cus = (size_t)std::max(in.cu_count, 1), rbs = in.row_blocks * 256 / cus;  // row blocks per 256 CUs
+        const int by16 = std::min(kW4DecodeMaxKsplit, kt_n / 16);  // slices of 16 k tiles, four per wave
+        auto shape = [&](int r, int w, int sl) { small_rb = r, small_waves = w, small_slices = sl; };
+        if (in.t >= 7) {
+            if (in.row_blocks == 1) shape(1, 4, by16);
+            else if (rbs <= 64) shape(2, 4, by16);
+            else if (rbs > 128 && in.group == 128 && (in.t > 8 ? kt_n >= 80 : kt_n % 128 == 0))
+                shape(4, 4, std::min(by16, (int)(cus / ((in.row_blocks + 3) / 4))));
+            else shape(2, 4, 4);
+        } else if (rbs <= 8) {
+            shape(1, 4, by16);
+        } else if (rbs <= 20 && kt_n >= 104) {
+            shape(2, 4, by16);
+        } else if (in.t <= 4) {
+            if (rbs <= 128 && kt_n >= (rbs <= 64 ? 56 + (int)rbs / 2 : 104)) shape(1, 4, 4);
+        } else if (rbs <= 64) {
+            shape(1, 8, 4);
+        } else if (rbs <= 192 && kt_n >= (rbs <= 112 ? 76 : 96) &&
+                   (kt_n > 128 || (in.row_blocks + 1) / 2 * (size_t)by16 <= 2 * cus)) {
+            shape(2, 4, by16);
+        }
+    }
     int rb;
     bool rb_auto = false;
     if (in.glu) {
@@ -112,7 +149,7 @@ static int plan_decode(const DecodePlanIn& in, DecodePlan* out) {
         rb = in.rows_per_wave / 16;
         if (rb != 1 && rb != 2 && rb != 4) return w4_fail(W4A16_ERR_ARG, "decode: rows_per_wave must be 16, 32 or 64");
     } else {
-        rb = wide ? (in.t <= 2 ? 1 : in.t <= 6 ? 2 : 4) : small ? (long_k_narrow ? 2 : 1) : long_k_narrow ? 4 : 2;
+        rb = wide ? (in.t <= 2 ? 1 : in.t <= 6 ? 2 : 4) : small ? small_rb : long_k_narrow ? 4 : 2;
         rb_auto = true;
     }
     while (!in.glu && rb > 1 && in.row_blocks < (size_t)rb) rb >>= 1;
@@ -126,8 +163,11 @@ static int plan_decode(const DecodePlanIn& in, DecodePlan* out) {
     } else if (in.ksplit == 0) {
         nks_auto = true;
         const size_t blocks = in.glu ? in.row_blocks / 2 : (in.row_blocks + (size_t)rb - 1) / (size_t)rb;
-        if (blocks < (size_t)std::max(in.cu_count, 1) && kt_n >= 64 && !(small && rb == 1)) {
-            nks_want = std::min(small ? 4 : kW4DecodeMaxKsplit, kt_n / 16);
+        if (small) {
+            nks_want = small_slices;
+            waves_cap = small_waves;
+        } else if (blocks < (size_t)std::max(in.cu_count, 1) && kt_n >= 64) {
+            nks_want = std::min(kW4DecodeMaxKsplit, kt_n / 16);
             waves_cap = 4;
         }
     }
@@ -145,7 +185,7 @@ static int plan_decode(const DecodePlanIn& in, DecodePlan* out) {
         const unsigned other = (unsigned)P.waves * decode_scale_lds(in.group, rb, P.kt_per_wave) + in.extra_lds;
         P.x_loads = in.t <= 4 ? 1 : in.t <= 8 ? 2 : 4;
         const bool few_waves = P.waves <= 4 && P.blocks * (size_t)P.nks <= (size_t)std::max(in.cu_count, 1);
-        const bool direct_x = P.x_loads == 2 ? in.group == 128 || rb != 2 : in.t <= (in.group == 128 ? 11u : 14u);
+        const bool direct_x = P.x_loads == 2 ? in.group == 128 || rb != 2 : in.t <= (rb == 4 ? (in.group == 128 ? 13u : 16u) : in.group == 128 ? 11u : 14u);
         P.x_lds = P.x_loads > 1 && !(few_waves && direct_x);
         if ((unsigned)P.waves * decode_wave_lds(rb, P.x_loads, P.x_lds) + other > 160u * 1024u) P.x_lds = false;
         P.shmem = (unsigned)P.waves * decode_wave_lds(rb, P.x_loads, P.x_lds) + other;

@@ -59,7 +59,8 @@ def test_pinned_gated_shape_without_room_for_staged_x(dec):
 
 @pytest.mark.parametrize("group,rows,t,direct", [
     (128, 16, 5, True), (128, 32, 8, True), (128, 32, 9, True), (128, 32, 11, True), (128, 32, 12, False),
-    (32, 16, 8, True), (32, 32, 8, False), (32, 32, 9, True), (32, 64, 14, True), (32, 32, 15, False),
+    (32, 16, 8, True), (32, 32, 8, False), (32, 32, 14, True), (32, 32, 15, False),
+    (128, 64, 13, True), (128, 64, 14, False),
 ])
 def test_few_waves_take_x_directly_with_the_same_bits(dec, group, rows, t, direct):
     """One workgroup of four waves per CU at most: the rule's edges, and every row's bits as in the 16-row launch (x

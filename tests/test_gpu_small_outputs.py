@@ -1,6 +1,6 @@
-"""Decode launches of outputs with at most one 16-row block per CU (one row block per wave, eight waves; two row blocks in
-four k slices from seven rows with a long k) and x rows re-ordered through LDS (five to sixteen rows): the edges of those
-ranges against the lane-order oracle."""
+"""Decode launches of outputs with at most one 16-row block per CU: one row block per wave, up to eight waves; a long k in
+slices, over one, two or four row blocks per wave; x rows re-ordered through LDS or loaded directly (five to sixteen
+rows).  The edges of those ranges against the lane-order oracle."""
 import numpy as np
 import pytest
 
@@ -13,8 +13,12 @@ pytestmark = pytest.mark.gpu
     (4096, 512, 128, 1), (4096, 512, 128, 16),   # the last size with one row block per workgroup
     (4112, 512, 128, 9),                         # one row block more: two per wave
     (17, 1024, 32, 5), (1, 128, 128, 8),         # a partial row block; fewer k tiles than waves
-    (96, 8192, 128, 6), (96, 8192, 128, 7),      # a long k: whole up to six rows, four slices from seven
+    (272, 4096, 128, 13), (272, 4096, 32, 6),    # eight waves of four k tiles: the load ring and staged x go round
+    (96, 8192, 128, 6), (96, 8192, 128, 7),      # a long k: one row block per wave up to six rows, two from seven
     (96, 8192, 32, 16), (80, 8320, 128, 13),     # 65 k tiles in four slices: the last one short
+    (16, 17408, 128, 4), (144, 17408, 32, 3),    # one row block; two per wave in eight slices
+    (528, 9472, 128, 2), (528, 9472, 32, 6),     # 74 k tiles in four slices of four and of eight waves
+    (1040, 9728, 128, 5), (2064, 10240, 128, 9), # two and four row blocks per wave, a partial last group
 ])
 def test_small_outputs(orc, n, k, group, t):
     print("small outputs", n, k, group, t, flush=True)

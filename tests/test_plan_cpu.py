@@ -69,6 +69,33 @@ def test_decode_plan_at_the_layer_shapes():
         assert p["lds_bytes"] <= 160 * 1024
 
 
+def test_decode_plan_of_small_outputs():
+    """At most one row block per CU (256): the edges of the rule for k slices.  A narrow output with a long k is split,
+    so that it does not stream its whole k from a few workgroups."""
+    want = {  # (n, k tiles, t) -> (rows per wave, waves, k slices)
+        (4096, 32, 1): (16, 8, 1), (4096, 32, 16): (16, 8, 1), (4112, 32, 1): (32, 8, 1),  # a row block more than CUs
+        (4096, 63, 16): (16, 8, 1), (4096, 64, 16): (32, 4, 4),                            # a long k from 64 tiles
+        (4096, 136, 6): (16, 8, 1), (4096, 136, 7): (32, 4, 4), (4096, 136, 9): (64, 4, 4), (4096, 128, 7): (64, 4, 4),
+        (16, 136, 1): (16, 4, 8), (16, 136, 16): (16, 4, 8), (16, 63, 1): (16, 8, 1),      # one row block
+        (128, 136, 4): (16, 4, 8), (144, 136, 4): (32, 4, 8), (336, 136, 4): (16, 4, 4),
+        (512, 71, 4): (16, 8, 1), (512, 72, 4): (16, 4, 4), (1024, 87, 1): (16, 8, 1), (1024, 88, 1): (16, 4, 4),
+        (2048, 103, 4): (16, 8, 1), (2048, 104, 4): (16, 4, 4), (2064, 136, 4): (16, 8, 1),
+        (1024, 64, 5): (16, 8, 4), (1040, 75, 6): (16, 8, 1), (1040, 76, 6): (32, 4, 4), (2304, 112, 5): (32, 4, 7),
+        (2064, 128, 5): (16, 8, 1), (2064, 136, 5): (32, 4, 8), (3088, 136, 5): (16, 8, 1),
+        (1024, 136, 8): (32, 4, 8), (1040, 136, 8): (32, 4, 4), (2304, 112, 16): (64, 4, 7), (2304, 79, 16): (32, 4, 4),
+    }
+    for (n, kt, t), (rows, waves, nks) in want.items():
+        p = ops.plan_decode(n, 128 * kt, 128, t)
+        assert (p["rows_per_wave"], p["waves_per_block"], p["k_slices"]) == (rows, waves, nks), (n, kt, t, p)
+    # no shape streams a long k from fewer waves than the 16-tile slices of four waves would bring, two row blocks each
+    for n in range(16, 1025, 16):
+        for kt in (104, 120, 136):
+            for t in range(1, 17):
+                p = ops.plan_decode(n, 128 * kt, 128, t)
+                blocks = -(-n // p["rows_per_wave"])
+                assert blocks * p["waves_per_block"] * p["k_slices"] >= -(-n // 64) * 4 * (kt // 16), (n, kt, t, p)
+
+
 def test_decode_plan_takes_x_directly_where_few_waves_run():
     """At most four waves per CU: a wave's LDS holds its partial tiles (2 KiB at two row blocks) and scales, not staged
     x (4.25 KiB), up to the row count where staging wins; 5120 x 5120 is 160 workgroups of four waves."""
