@@ -781,9 +781,8 @@ MOE_FAMILY(w4a16_moe_g128_bf16, 128, true, 4)
 // One wave per token, n <= 1024; the body is built for 2, 4 and 16 experts per lane (n <= 128, 256, 1024).  The kernel is
 // a chain of dependent wave-wide steps and nothing else, so a selection round is kept short: the probability's bit
 // pattern (monotone for non-negative floats; NaN of all ones held one lower) plus one is a 32-bit key, 0 for an absent or
-// taken expert; a lane's largest
-// key, six v_max_u32 with DPP operands and one lane read give the round's probability, and one ballot per expert of a
-// lane, in index order, names the lowest index that holds it.  (Rounds on a 64-bit key with the index in its low half
+// taken expert; a lane's largest key, six v_max_u32 with DPP operands and one lane read give the round's probability, and
+// one ballot per expert of a lane, in index order, names the lowest index that holds it.  (Rounds on a 64-bit key with the index in its low half
 // and shuffles through LDS, always 16 experts per lane: 6.9 us at one token and 9.0 at 2048, 128 experts, top-8; this form
 // 3.4 and 3.5, of which 2.4 are the launch.)
 template <int CTRL>
@@ -811,7 +810,7 @@ __device__ __forceinline__ void moe_topk_body(const float* __restrict__ logits, 
 #pragma unroll
     for (int j = 0; j < PER_LANE; j++) {
         e[j] = lane + 64 * j < n ? expf(e[j] - top) : 0.f;
-        total += e[j];  // lane-local sum in index order, then the butterfly: the order the host statement follows too
+        total += e[j];  // lane-local sum in index order, then the butterfly (the host statement adds all in index order)
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) total += __shfl_xor(total, off);
