@@ -72,13 +72,16 @@ static int launch_lane(w4a16_ctx* ctx, uint64_t q, uint64_t s, uint64_t x, uint6
 // each (measured 12.4 -> 11.8 us at t = 1, 13.3 -> 12.4 us at t = 4).  Shorter k ranges lose more to the extra
 // workgroups than they gain.
 // x from five rows on (kernels/decode.hip): through LDS, which saves the address unit work and adds an LDS round trip, about
-// 0.06 us, to every k tile of a wave.  With at most one workgroup of up to four waves per CU the address unit is not
-// what a launch waits for and the round trip shows, so direct loads stay up to the row count where their cost, which
-// grows with the rows, overtakes it (two row blocks x four waves, direct / through LDS: 5120 x 5120 group 128 t = 9 7.40 /
-// 7.72 us, t = 11 7.62 / 7.66, t = 12 7.88 / 7.81; group 32 t = 9 7.99 / 8.60, t = 14 8.51 / 8.52, t = 15 8.81 / 8.63;
-// 5120 x 2048 group 32 t = 9 5.10 / 5.44; up to eight rows 4096 x 4096 group 128 t = 5 6.39 / 6.62; four row blocks
-// 5120 x 5120 group 128 t = 12 9.75 / 9.93, t = 16 10.56 / 10.13, group 32 t = 16 11.49 / 12.08).  Two row blocks at group 32
-// up to eight rows are the exception (5120 x 5120 t = 8 8.70 / 8.31; one row block t = 6 6.03 / 6.28).
+// 0.06 us, to every k tile of a wave.  Where the address unit is not what a launch waits for, the round trip shows and
+// direct loads stay (us, direct / through LDS):
+//   * at most one workgroup of up to four waves per CU, up to the row count where the direct loads' cost, which grows with
+//     the rows, overtakes it: two row blocks, 5120 x 5120 group 128 t = 9 7.40 / 7.72, t = 11 7.62 / 7.66, t = 12 7.88 / 7.81;
+//     group 32 t = 9 7.99 / 8.60, t = 14 8.51 / 8.52, t = 15 8.81 / 8.63; 5120 x 2048 group 32 t = 9 5.10 / 5.44; 4096 x 4096
+//     group 128 t = 5 6.39 / 6.62; four row blocks, 5120 x 5120 group 128 t = 12 9.75 / 9.93, t = 16 10.56 / 10.13, group 32
+//     t = 16 11.49 / 12.08; but two row blocks at group 32 up to eight rows 8.70 / 8.31 (t = 8);
+//   * one workgroup of eight waves per CU, two row blocks at group 128, few rows and few k tiles per wave: gated 8192 x 1792
+//     at t = 5 and 6 4 to 5 % apart, 5120 x 2048 3 %, level at t + k tiles per wave = 10, 3 % the other way at t = 7, k = 8064;
+//   * four row blocks, five to eight rows, at most four k tiles per wave: 20480 x 2048 t = 7 3 % apart, level at k = 4096.
 // LDS: the waves' staged scales grow with the k tiles per wave (kernels/decode.hip).  A plan that would pass the 160 KiB
 // of a CU takes x by direct loads (from five rows on: 1 KiB per row block and wave instead of up to 4.25 KiB for staged
 // x).  If it still does, it is shrunk — automatic row blocks per wave are halved first (keeps one launch without tickets),
@@ -184,9 +187,14 @@ static int plan_decode(const DecodePlanIn& in, DecodePlan* out) {
         // wave x groups per tile x 32 bytes, in whole 1 KiB DMA instructions); then the statistics staging area
         const unsigned other = (unsigned)P.waves * decode_scale_lds(in.group, rb, P.kt_per_wave) + in.extra_lds;
         P.x_loads = in.t <= 4 ? 1 : in.t <= 8 ? 2 : 4;
-        const bool few_waves = P.waves <= 4 && P.blocks * (size_t)P.nks <= (size_t)std::max(in.cu_count, 1);
-        const bool direct_x = P.x_loads == 2 ? in.group == 128 || rb != 2 : in.t <= (rb == 4 ? (in.group == 128 ? 13u : 16u) : in.group == 128 ? 11u : 14u);
-        P.x_lds = P.x_loads > 1 && !(few_waves && direct_x);
+        const bool one_per_cu = P.blocks * (size_t)P.nks <= (size_t)std::max(in.cu_count, 1), g128 = in.group == 128;
+        bool direct_x;
+        if (P.x_loads == 2)
+            direct_x = (one_per_cu && P.waves <= 4 && (g128 || rb != 2)) || (rb == 4 && P.kt_per_wave <= 4) ||
+                       (one_per_cu && g128 && rb == 2 && (int)in.t + P.kt_per_wave <= 10);
+        else
+            direct_x = one_per_cu && P.waves <= 4 && in.t <= (rb == 4 ? (g128 ? 13u : 16u) : g128 ? 11u : 14u);
+        P.x_lds = P.x_loads > 1 && !direct_x;
         if ((unsigned)P.waves * decode_wave_lds(rb, P.x_loads, P.x_lds) + other > 160u * 1024u) P.x_lds = false;
         P.shmem = (unsigned)P.waves * decode_wave_lds(rb, P.x_loads, P.x_lds) + other;
         if (P.shmem <= 160u * 1024u) {

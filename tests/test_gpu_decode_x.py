@@ -57,20 +57,21 @@ def test_pinned_gated_shape_without_room_for_staged_x(dec):
     assert np.array_equal(got, want)
 
 
-@pytest.mark.parametrize("group,rows,t,direct", [
-    (128, 16, 5, True), (128, 32, 8, True), (128, 32, 9, True), (128, 32, 11, True), (128, 32, 12, False),
-    (32, 16, 8, True), (32, 32, 8, False), (32, 32, 14, True), (32, 32, 15, False),
-    (128, 64, 13, True), (128, 64, 14, False),
+@pytest.mark.parametrize("group,rows,waves,t,direct", [
+    (128, 16, 4, 5, True), (128, 32, 4, 8, True), (128, 32, 4, 9, True), (128, 32, 4, 11, True), (128, 32, 4, 12, False),
+    (32, 16, 4, 8, True), (32, 32, 4, 8, False), (32, 32, 4, 14, True), (32, 32, 4, 15, False),
+    (128, 64, 4, 13, True), (128, 64, 4, 14, False),
+    (128, 32, 8, 8, True), (32, 32, 8, 8, False), (128, 16, 8, 8, False), (32, 64, 8, 8, True), (128, 64, 8, 9, False),
 ])
-def test_few_waves_take_x_directly_with_the_same_bits(dec, group, rows, t, direct):
-    """One workgroup of four waves per CU at most: the rule's edges, and every row's bits as in the 16-row launch (x
-    through LDS), whose sums run in the same order."""
-    print("few waves", group, rows, t, flush=True)
-    n, k = 200, 1280  # a partial row block; ten k tiles on four waves
+def test_short_launches_take_x_directly_with_the_same_bits(dec, group, rows, waves, t, direct):
+    """One workgroup per CU at most and few k tiles per wave: the rule's edges, and every row's bits as in the 16-row
+    launch (x through LDS), whose sums run in the same order."""
+    print("short", group, rows, waves, t, flush=True)
+    n, k = 200, 1280  # a partial row block; ten k tiles on four or eight waves
     q, s, x = gen.make_linear(n, k, group, 16, seed=group + rows + t)
     dec.upload_lin_g("few", q, s, n, k, group, False)
     try:
-        dec.set_decode_shape(rows, 4)
+        dec.set_decode_shape(rows, waves)
         want = dec.gemv_host("few", x, t=16, path=ops.PATH_DECODE)
         assert dec.cc.last_launch_symbol().endswith("_rb%d_x4" % (rows // 16))
         got = dec.gemv_host("few", np.ascontiguousarray(x[:t]), t=t, path=ops.PATH_DECODE)

@@ -105,6 +105,12 @@ def test_decode_plan_takes_x_directly_where_few_waves_run():
             p = ops.plan_decode(5120, 5120, group, t)
             assert (p["rows_per_wave"], p["waves_per_block"], p["k_slices"]) == (32, 4, 1)
             assert p["lds_bytes"] == 4 * (2048 if t <= last else 17 * 256) + scales[group], (group, t, p)
+    # eight waves, five and six rows: staged x needs 2.25 KiB per wave; rows + k tiles per wave decide at group 128
+    for kt, t, group, direct in [(40, 5, 128, True), (48, 5, 128, False), (32, 6, 128, True), (40, 6, 128, False), (32, 5, 32, False)]:
+        p = ops.plan_decode(5120, 128 * kt, group, t)
+        assert (p["rows_per_wave"], p["waves_per_block"]) == (32, 8)
+        scales_w = -(-2 * (kt // 8) * (128 // group) * 32 // 1024) * 1024
+        assert p["lds_bytes"] == 8 * ((2048 if direct else 9 * 256) + scales_w), (kt, t, group, p)
     # twice the row blocks: two workgroups per CU, staged from nine rows on
     p = ops.plan_decode(10240, 5120, 128, 9)
     assert p["lds_bytes"] == 4 * 17 * 256 + scales[128], p
