@@ -52,8 +52,8 @@ static int launch_lane(w4a16_ctx* ctx, uint64_t q, uint64_t s, uint64_t x, uint6
 // tokens on runs four row blocks per wave, which share the x loads, with the k slices across workgroups bringing the
 // workgroups back (t = 16: 21.6 -> 15.8 us, t = 12: 18.6 -> 14.9, t = 8: 14.2 -> 13.5; level at t = 6).
 // Outputs of at most one row block per CU (256 row blocks, n = 4096): one row block per wave x eight waves, so that every
-// CU has a workgroup, and no k slices (4096 x 4096 at t = 1 5.72 -> 4.80 us, t = 8 6.31 -> 5.19, t = 16 7.01 -> 6.24;
-// k = 8192 8.47 -> 6.58; at 384 row blocks the two shapes are within 5 % and at 448 two row blocks win).
+// CU has a workgroup, and no k slices (4096 x 4096 at t = 1 5.77 -> 4.81 us, t = 8 6.31 -> 5.42, t = 16 7.29 -> 6.18;
+// k = 8192 8.58 -> 6.57; at 384 row blocks the two shapes are within 5 % and at 448 two row blocks win).
 // Their k slices, from 64 k tiles on (figures: group 128, cold weights, best shape / unsplit one row block x eight waves
 // / two row blocks x four waves in slices of 16 k tiles, the rule of larger outputs).  A wave's k tiles follow each other at
 // about 0.29 us, so a slice pays once the tiles it saves outweigh the hand-over, which grows with the workgroups:
@@ -64,7 +64,7 @@ static int launch_lane(w4a16_ctx* ctx, uint64_t q, uint64_t s, uint64_t x, uint6
 //     7.4 (unsplit) / 7.4, x 17408 9.05 (two row blocks) / 10.1; a last generation of workgroups that is nearly empty loses
 //     (2064 x 16384, 520 workgroups: 9.49 unsplit, 10.4 in slices), so they have to fit two per CU or k be long.
 //   t >= 7: two row blocks share the x loads and the slices split them: 256 x 17408 t = 16 6.83 / 13.7 / 8.02 (four row
-//     blocks, the rule of larger outputs), 2048 x 11008 8.1 / 8.75; beyond 128 row blocks from nine rows on four row blocks,
+//     blocks, the rule of larger outputs), 2048 x 11008 8.0 / 8.5; beyond 128 row blocks from nine rows on four row blocks,
 //     in as many slices as one workgroup per CU allows (group 128): 3072 x 16384 t = 16 10.4 against 11.9 in two row blocks
 //     and 11.5 in eight slices.  Row blocks 128 KiB apart (k = 16384) prefer that at 7 and 8 rows too (4096: 10.9 against 12.3).
 // k slices across workgroups (one launch; partial tiles and tickets in a workspace): only for a long k range over

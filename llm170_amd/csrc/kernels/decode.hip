@@ -13,9 +13,10 @@
 //     From five rows on x arrives in whole rows of the k tile (16 lanes x 16 B per row, two loads up to t = 8, four up
 //     to 16) and is turned into B operands through a wave-private piece of LDS: a load in B-operand order, whose
 //     neighbouring lanes read different rows, occupies the address unit for 62 clocks against 18 for whole rows (L2-resident
-//     x, 16 waves per CU).  5120 x 34816 at t = 16: 27.0 -> 25.7 us, gated 32.4 -> 26.8; 5120 x 7168 8.9 -> 8.3;
-//     17408 x 5120 15.8 -> 15.1; at t = 8 level, gated 22.7 -> 21.3; up to t = 4 it costs 0.1 us and is not used.
-//     No barrier on the streaming path;
+//     x, 16 waves per CU).  5120 x 34816 at t = 16: 29.3 -> 27.1 us, gated 36.1 -> 31.2; 5120 x 7168 9.5 -> 9.2;
+//     17408 x 5120 18.1 -> 16.6; at t = 8 24.4 -> 23.9, gated 26.6 -> 24.3; up to t = 4 it costs 0.1 us and is not used.
+//     Launches with too few waves or k tiles to hide the LDS round trip keep loads in B-operand order (t <= 8 two, t <= 16
+//     four per k tile); the host chooses.  No barrier on the streaming path;
 //   * weights enter the MFMA as exact integers; the per-group scale multiplies the f32 group sum, so no weight is
 //     ever rounded to f16 (error vs the f32 lane contract is summation order only);
 //   * each wave keeps DEPTH k-tiles of loads in flight (register ring, software pipelined);
@@ -520,8 +521,9 @@ __device__ __forceinline__ void decode_body(const u4_t* __restrict__ qt, const u
     extern "C" __global__ __launch_bounds__(512) ATTR void SYM(DECODE_PARAMS) {                                        \
         decode_body<G, SBF, 2, DECODE_DEPTH(BUDGET, G, 2, XL), XL, X_LDS, true>(DECODE_ARGS, DECODE_ONE_OUTPUT);       \
     }
-// _x<XL>: x through LDS (XL > 1).  _x<XL>d: x by direct loads, in the same register regime; for launches whose staged
-// scales leave no LDS for x (a wave's region is 1 KiB per row block instead of up to 4.25 KiB).
+// _x<XL>: x through LDS (XL > 1).  _x<XL>d: x by direct loads; for launches with too few waves or k tiles to hide the LDS
+// round trip, and those whose staged scales leave no LDS for x (a wave's region is 1 KiB per row block instead of up to
+// 4.25 KiB).
 #define DECODE_KERNEL_X(NAME, G, SBF, RB, XL, BUDGET, ATTR) \
     DECODE_KERNEL_SYM(NAME##_x##XL, G, SBF, RB, XL, true, BUDGET, ATTR)
 #define DECODE_KERNEL_XD(NAME, G, SBF, RB, XL, BUDGET, ATTR) \

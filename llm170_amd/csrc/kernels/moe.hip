@@ -783,8 +783,8 @@ MOE_FAMILY(w4a16_moe_g128_bf16, 128, true, 4)
 // pattern (monotone for non-negative floats; NaN of all ones held one lower) plus one is a 32-bit key, 0 for an absent or
 // taken expert; a lane's largest key, six v_max_u32 with DPP operands and one lane read give the round's probability, and
 // one ballot per expert of a lane, in index order, names the lowest index that holds it.  (Rounds on a 64-bit key with the index in its low half
-// and shuffles through LDS, always 16 experts per lane: 6.9 us at one token and 9.0 at 2048, 128 experts, top-8; this form
-// 3.4 and 3.5, of which 2.4 are the launch.)
+// and shuffles through LDS, always 16 experts per lane: 6.9 us at one token and 8.9 at 2048, 128 experts, top-8; this form
+// 2.8 and 3.4.)
 template <int CTRL>
 __device__ __forceinline__ unsigned topk_dpp_max(unsigned v) {
     const unsigned o = __builtin_amdgcn_update_dpp(0u, v, CTRL, 0xF, 0xF, true);  // lanes without a source read 0
@@ -872,7 +872,7 @@ extern "C" __global__ __launch_bounds__(256) void w4a16_moe_topk_t(const float* 
 // The placement (a ballot per bit of the expert id for every 64 slots) is what a launch spends its time on, so beyond
 // 2048 slots it is spread over workgroups, about two steps of 64 slots per wave; each of them counts ALL slots (LDS atomics,
 // a fraction of the placement's cost), which gives it the number of slots ahead of its range per expert and the totals
-// without a second launch (128 experts: 4136 slots 7.4 -> 6.2 us, 16384 18.1 -> 7.7, 32768 32.8 -> 9.8).
+// without a second launch (128 experts: 4136 slots 7.4 -> 6.0 us, 16384 18.1 -> 7.6, 32768 32.7 -> 9.6).
 #define MOE_ALIGN_WAVES 16
 #define MOE_ALIGN_THREADS (64 * MOE_ALIGN_WAVES)
 #define MOE_ALIGN_KEEP 4  // 64-slot steps of a wave whose expert ids stay in registers between the two passes
