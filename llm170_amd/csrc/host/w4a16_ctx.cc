@@ -68,13 +68,19 @@ static const char* const kPrefillSyms[] = {"w4a16_prefill_g32_f16", "w4a16_prefi
                                            "w4a16_moe_g128_f16_pf_glu", "w4a16_moe_g128_f16_pf_lin", "w4a16_moe_g128_bf16_pf_glu",
                                            "w4a16_moe_g128_bf16_pf_lin", "w4a16_moe_g32_f16_pf_glu", "w4a16_moe_g32_f16_pf_lin",
                                            "w4a16_moe_g32_bf16_pf_glu", "w4a16_moe_g32_bf16_pf_lin", nullptr};
+// waves along n and k of a workgroup (kernels/mid.hip); the split launch's n4k1 has no gated form
+#define W4_MID_BUILDS(P)                                                                                               \
+    P "_n1k4", P "_n1k4_glu", P "_n2k4", P "_n2k4_glu", P "_n3k4", P "_n3k4_glu", P "_n4k1", P "_n4k2", P "_n4k2_glu", \
+        P "_n5k2", P "_n5k2_glu"
+#define W4_MID_FAMILY(P) W4_MID_BUILDS(P "_t2"), W4_MID_BUILDS(P "_t3"), W4_MID_BUILDS(P "_t4")
+static const char* const kMidSyms[] = {W4_MID_FAMILY("w4a16_mid_g128_f16"), W4_MID_FAMILY("w4a16_mid_g128_bf16"),
+                                       W4_MID_FAMILY("w4a16_mid_g32_f16"), W4_MID_FAMILY("w4a16_mid_g32_bf16"), nullptr};
 static const char* const kUtilSyms[] = {"w4a16_fill0_u32", nullptr};
 static const char* const kGlueSyms[] = {"w4a16_rms_rescale_f16", "w4a16_silu_mul_f16", "w4a16_synth_q", "w4a16_synth_s",
                                         "w4a16_norm_resid", nullptr};
 #define W4_MOE_FAMILY(P)                                                                                      \
     P "_dec_glu_x1", P "_dec_glu_x4", P "_dec_lin_x1", P "_dec_lin_x4", P "_mm_glu_t1", P "_mm_glu_t2",       \
-        P "_mm_glu_t3", P "_mm_glu_t4", P "_mm_lin_t1", P "_mm_lin_t2", P "_mm_lin_t3", P "_mm_lin_t4",       \
-        P "_mm_lin_t1_ks", P "_mm_lin_t2_ks", P "_mm_lin_t3_ks", P "_mm_lin_t4_ks"
+        P "_mm_glu_t3", P "_mm_glu_t4", P "_mm_lin_t1", P "_mm_lin_t2", P "_mm_lin_t3", P "_mm_lin_t4"
 static const char* const kMoeSyms[] = {W4_MOE_FAMILY("w4a16_moe_g32_f16"),
                                        W4_MOE_FAMILY("w4a16_moe_g32_bf16"),
                                        W4_MOE_FAMILY("w4a16_moe_g128_f16"),
@@ -103,6 +109,7 @@ static const W4Asset kAssets[] = {
     {"decode", kDecodeSyms},
     {"prefill", kPrefillSyms},
     {"prefill_g128", kPrefillG128Syms},
+    {"mid", kMidSyms},
     {"moe", kMoeSyms},
     {"glue", kGlueSyms},
     {"util", kUtilSyms},

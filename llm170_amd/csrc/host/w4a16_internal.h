@@ -47,8 +47,6 @@ struct W4MoeScratch {
     size_t block = 0;
     uint64_t iota = 0, always = 0;  // direct mode: identity segment table and a "padded total" no slot index reaches
     size_t iota_cap = 0;            // entries
-    uint64_t zeros = 0;             // all-zero expert table for a dense linear run as one expert
-    size_t zeros_cap = 0;           // entries
 };
 
 // Scratch of the layer chain, grown on demand (reference: dchain / dx16 / dy buffers, w4a16_dec/buffers.rs).
@@ -116,7 +114,9 @@ constexpr int kW4TileK = 128;               // W4_TILE_K (w4a16_common.hpp)
 constexpr int kW4TileRows = 16;             // W4_TILE_ROWS
 constexpr int kW4LaneTt = 8;                // LANE_TT (lane.hip): tokens per pass of the lane-order kernel
 constexpr int kW4DecodeMaxKsplit = 8;       // W4_DECODE_MAX_KSPLIT (decode.hip)
-constexpr int kW4MoeMaxKsplit = 8;          // MOE_MAX_KSPLIT (moe.hip)
+constexpr int kW4MoeMaxKsplit = 8;          // MOE_MAX_KSPLIT (mid.hip)
+constexpr int kW4MidParts = 4;              // MID_PARTS (mid.hip): runs of a slice's k tiles that are summed on their own
+constexpr int kW4MidLdx = 136;              // MID_LDX (mid.hip): halves per x row staged through registers
 constexpr int kW4MoeLdx = 136;              // MOE_LDX (moe.hip): halves per staged x row
 constexpr int kW4MoeAlignWaves = 16;        // MOE_ALIGN_WAVES (moe.hip)
 constexpr int kW4RmsLanes = 1024;           // RMS_LANES (glue.hip)
@@ -138,8 +138,9 @@ int w4_find_lin(w4a16_ctx* ctx, const char* name, W4Lin** out);
 // carries the running unit s_prev / s_cur can take
 bool w4_scales_regular(const uint16_t* s, size_t count, int scale_bf16);
 int w4_ensure(w4a16_ctx* ctx, uint64_t* buf, size_t* cap, size_t bytes);
-// glu_act >= 0: L is a fused gate|up linear and y_dev receives f16 [t][n/2] = act(gate) * up on the f32 sums
-int w4_dense_grouped(w4a16_ctx* ctx, const W4Lin& L, uint64_t x_dev, uint64_t y_dev, size_t t, int out_f16, int glu_act = -1);
+// dense linear at 17..64 rows, or any number of rows (kernels/mid.hip).  glu_act >= 0: L is a fused gate|up linear and y_dev
+// receives f16 [t][n/2] = act(gate) * up on the f32 sums
+int w4_dense_mid(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_t y, size_t t, int out_f16, int glu_act = -1);
 int w4_lin_forward_fixed_ws(w4a16_ctx* ctx, const char* name, uint64_t x_dev, uint64_t y_dev, size_t t, int out_f16,
                             uint64_t ws, size_t ws_bytes, uint64_t tickets, size_t ticket_bytes);
 // per-device fixed scratch of the allocation-free entry point (w4a16_noalloc.hip)

@@ -1,4 +1,5 @@
-// MoE layer of libw4a16hip.so: expert arenas, routing, slot alignment and the routed-expert FFN.
+// MoE layer of libw4a16hip.so: expert arenas, routing, slot alignment and the routed-expert FFN; and the launch of dense
+// linears at a few dozen rows.
 // Stands in for build_marlin_moe_arenas (w4a16_dec/upload.rs:1116-1235), moe_topk (w4a16_dec/mod.rs:168-185),
 // moe_align_launch (moe/moe_align.rs:4-22) and marlin_moe_ffn_dev (kernels/marlin_moe.rs:290-422).
 #include <algorithm>
@@ -229,7 +230,7 @@ static size_t pick_block(const w4a16_ctx* ctx, size_t t, size_t ns, size_t n_exp
 
 static int launch_moe_gemm(w4a16_ctx* ctx, const W4Experts& E, bool glu, uint64_t x, size_t x_rows, size_t x_div,
                            uint64_t y, int y_f16, uint64_t topw, size_t ns, size_t block, size_t max_segs,
-                           uint64_t sorted, uint64_t eids, uint64_t npost, size_t nks = 1, bool tiled = false) {
+                           uint64_t sorted, uint64_t eids, uint64_t npost, bool tiled = false) {
     const size_t n = glu ? 2 * E.n_ff : E.h, k = glu ? E.h : E.n_ff;
     const size_t row_blocks = (n + 15) / 16, kt_n = k / 128;
     const size_t units = glu ? row_blocks / 2 : (row_blocks + 1) / 2;
@@ -239,11 +240,10 @@ static int launch_moe_gemm(w4a16_ctx* ctx, const W4Experts& E, bool glu, uint64_
     unsigned long long qs = glu ? E.q13_stride : E.q2_stride, ss = glu ? E.s13_stride : E.s2_stride;
     int xr = (int)x_rows, xd = (int)x_div, yf = y_f16, blk = (int)block, nsi = (int)ns, rbi = (int)row_blocks,
         ki = (int)k, ni = (int)n, nei = (int)E.n_exp;
-    uint64_t ws = 0, tk = 0;
     int waves = 0;  // set below, before the launch reads it
     int act_kind = ctx->moe_act_kind;  // read by the gate|up kernels only
     void* p[] = {&qa, &sa, &qs, &ss, &x, &xr, &xd, &y, &yf, &topw, &sorted, &eids, &npost, &blk, &nsi, &rbi, &ki, &ni, &nei,
-                 &ws, &tk, &waves, &act_kind};
+                 &waves, &act_kind};
     char sym[80];
     const char* fam = E.scale_bf16 ? "bf16" : "f16";
     if (tiled) {
@@ -267,96 +267,90 @@ static int launch_moe_gemm(w4a16_ctx* ctx, const W4Experts& E, bool glu, uint64_
     waves = ctx->moe_waves ? ctx->moe_waves : 4;
     waves = waves >= 8 ? 8 : 4;  // the x staging needs at least 4 waves
     const size_t blocks = max_segs * ((units + (size_t)waves - 1) / (size_t)waves);
-    nks = std::max<size_t>(1, std::min<size_t>(std::min<size_t>(nks, kW4MoeMaxKsplit), kt_n / 2));
-    if (nks > 1) {
-        // split over k across workgroups: partial tiles and per-(block, wave) tickets, shared with the decode kernel
-        W4_TRY(w4_ensure(ctx, &ctx->decode_ws, &ctx->decode_ws_cap, blocks * (size_t)waves * 2 * (size_t)tt * 1024 * nks));
-        if (blocks * (size_t)waves * 4 > ctx->decode_tickets_cap) {
-            W4_TRY(w4_ensure(ctx, &ctx->decode_tickets, &ctx->decode_tickets_cap,
-                             std::max<size_t>(blocks * (size_t)waves * 4, 16384)));
+    snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_mm_%s_t%d", E.group, fam, glu ? "glu" : "lin", tt);
+    const unsigned shmem = (unsigned)(2 * 16 * tt * kW4MoeLdx * 2);
+    return w4_launch(ctx, sym, (unsigned)blocks, 1, (unsigned)(waves * 64), shmem, p);
+}
+
+// Launch plan of the 17..64-row kernel (kernels/mid.hip): waves along n and k of a workgroup, k slices across workgroups.
+// Every shape gives the same bits for a given number of slices.  From sweeps of 19 widths x 7 k x t = 24, 40, 64 and both
+// groups (units = pairs of row blocks; figures us, group 128, cold weights; over the sweeps the plan loses 0.4 % to the best
+// shape of each, 15 % at worst):
+//   * up to one unit per CU (n = 8192): a wave per unit and four along k, every unit's workgroup on a CU of its own
+//     (5120 x 5120 t = 64 14.6, two units per workgroup 18.8);
+//   * k slices, whose hand-over costs about 3 us plus what grows with the workgroups: few units (64) from 32 k tiles on, four
+//     or eight slices (1024 x 4096 t = 40 9.8 -> 8.2, 512 x 17408 29.2 -> 11.2); up to 96 units two on a middling k; beyond,
+//     from 65 k tiles, four waves along n, so that the slices' workgroups re-read little x (5120 x 17408 t = 64 37.1 -> 29.1,
+//     t = 24 24.2 -> 20.4);
+//   * more units than CUs: the waves along n that leave the fullest CU the fewest units, a workgroup's start counting as 1.2
+//     units (gated 34816 x 5120 t = 64: five waves 34.5, four 49.2; 28672 x 4096: four 22.3, five 26.4; 22016 x 4096: three
+//     19.3, four 21.3; 16384 x 4096: two 17.1, three 18.6); a long k over little more units than CUs runs four slices
+//     (11008 x 17408 t = 64 54.9 -> 45.7).
+struct MidPlan {
+    int wn = 1, wk = kW4MidParts;
+    size_t nks = 1;
+};
+
+static MidPlan plan_mid(size_t units, size_t kt_n, size_t t, size_t cus, int ksplit, bool may_split) {
+    const size_t u = units * 256 / cus;  // per 256 CUs
+    MidPlan P;
+    if (may_split && ksplit > 0) {
+        P.nks = std::max<size_t>(1, std::min(std::min<size_t>((size_t)ksplit, kW4MoeMaxKsplit), kt_n / 2));
+        if (P.nks > 1 && u > 96) P.wn = 4, P.wk = 1;
+        if (P.nks > 1) return P;
+    } else if (may_split && ksplit == 0) {
+        if (u <= 64 && kt_n >= 32) P.nks = kt_n >= 128 || (u <= 32 && kt_n >= 64 && t > 32) ? 8 : 4;
+        else if (u > 64 && u <= 96 && kt_n >= 40 && kt_n <= 64) P.nks = 2;
+        else if (u > 64 && u <= 256 && (kt_n > 64 || (kt_n == 64 && t > 32 && u <= 160))) P = MidPlan{4, 1, 8};
+        else if (u > 256 && u <= 352 && kt_n >= 86) P = MidPlan{4, 1, 4};
+        if (P.nks > 1) return P;
+    }
+    if (u <= 256) return P;
+    double best = 1e30;
+    for (const MidPlan& c : {MidPlan{2, 4, 1}, MidPlan{3, 4, 1}, MidPlan{4, 2, 1}, MidPlan{5, 2, 1}}) {
+        const size_t wgs = (units + (size_t)c.wn - 1) / (size_t)c.wn;
+        const double cost = (double)((wgs + cus - 1) / cus) * (c.wn + 1.2);
+        if (cost < best) best = cost, P = c;
+    }
+    return P;
+}
+
+// glu_act >= 0: the linear is a fused gate|up projection and y receives f16 [t][n/2] = act(gate) * up on the f32 sums; the
+// gated launch never splits over k.
+int w4_dense_mid(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_t y, size_t t, int out_f16, int glu_act) {
+    const bool glu = glu_act >= 0;
+    if (!L.q_tiled) return w4_fail(W4A16_ERR_UNSUPPORTED, "stream: linear has no tiled copy (needs k %% 128 == 0)");
+    if (t > 0x7fffffffu / 2) return w4_fail(W4A16_ERR_SHAPE, "stream: t=%zu too large", t);
+    if (glu && L.n % 32 != 0) return w4_fail(W4A16_ERR_SHAPE, "stream glu: n=%zu must be a multiple of 32", L.n);
+    if (t * L.k * 2 >= 0x80000000ull || L.row_blocks * (L.k / 128) * 1024 >= 0x80000000ull)
+        return w4_fail(W4A16_ERR_SHAPE, "stream: x or the tiled weights reach 2 GiB, beyond the buffer-descriptor range");
+    const size_t units = glu ? L.row_blocks / 2 : (L.row_blocks + 1) / 2, cus = (size_t)std::max(ctx->cu_count, 1);
+    const size_t tt = t <= 32 ? 2 : t <= 48 ? 3 : 4, segs = (t + 16 * tt - 1) / (16 * tt);
+    const MidPlan P = plan_mid(units, L.k / 128, t, cus, ctx->decode_ksplit, !glu);
+    const size_t wn = (size_t)P.wn, wk = (size_t)P.wk, groups = (units + wn - 1) / wn, blocks = groups * segs;
+    uint64_t ws = 0, tk = 0;
+    if (P.nks > 1) {  // partial tiles and per-wave tickets, shared with the decode kernel
+        const size_t ws_need = blocks * wn * 2 * tt * 1024 * P.nks, tk_need = blocks * wn * wk * 4;
+        if (ws_need > 0xffffffffull) return w4_fail(W4A16_ERR_SHAPE, "stream: %zu bytes of partial tiles", ws_need);
+        W4_TRY(w4_ensure(ctx, &ctx->decode_ws, &ctx->decode_ws_cap, ws_need));
+        if (tk_need > ctx->decode_tickets_cap) {
+            W4_TRY(w4_ensure(ctx, &ctx->decode_tickets, &ctx->decode_tickets_cap, std::max<size_t>(tk_need, 16384)));
             W4_TRY(w4a16_memset0(ctx, ctx->decode_tickets, ctx->decode_tickets_cap));
         }
         ws = ctx->decode_ws;
         tk = ctx->decode_tickets;
     }
-    if (nks > 1 && glu) return w4_fail(W4A16_ERR_UNSUPPORTED, "moe: the gate|up kernel does not split over k");
-    snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_mm_%s_t%d%s", E.group, fam, glu ? "glu" : "lin", tt, nks > 1 ? "_ks" : "");
-    const unsigned shmem = (unsigned)(2 * 16 * tt * kW4MoeLdx * 2);
-    return w4_launch(ctx, sym, (unsigned)blocks, (unsigned)nks, (unsigned)(waves * 64), shmem, p);
-}
-
-// A dense linear at a few dozen rows through the LDS-staged grouped kernel: one "expert" (the linear itself), slot =
-// token, segments of up to 64 tokens.  Between the streaming decode kernel (t <= 16: x operands straight from global
-// memory) and the 128-row MFMA tiles of the prefill kernel, this regime is still bound by the weight stream, and the
-// grouped kernel shares each x tile among all waves of a workgroup through LDS.
-int w4_dense_grouped(w4a16_ctx* ctx, const W4Lin& L, uint64_t x_dev, uint64_t y_dev, size_t t, int out_f16, int glu_act) {
-    if (!L.q_tiled) return w4_fail(W4A16_ERR_UNSUPPORTED, "stream: linear has no tiled copy (needs k %% 128 == 0)");
-    if (t > 0x7fffffffu / 2) return w4_fail(W4A16_ERR_SHAPE, "stream: t=%zu too large", t);
-    W4MoeScratch& S = ctx->moe;
-    const size_t block = ctx->moe_block >= 16 ? (size_t)ctx->moe_block : t <= 16 ? 16 : t <= 32 ? 32 : t <= 48 ? 48 : 64;
-    const size_t segs = (t + block - 1) / block, padded = segs * block;
-    // identity slot table (entries >= t are the padding sentinel by themselves), all-zero expert table, padded total
-    if (S.iota_cap < padded) {
-        const size_t cap = std::max<size_t>(padded, 4096);
-        std::vector<int32_t> host(cap);
-        for (size_t i = 0; i < cap; i++) host[i] = (int32_t)i;
-        size_t bytes_cap = S.iota_cap * 4;
-        W4_TRY(w4_ensure(ctx, &S.iota, &bytes_cap, cap * 4));
-        W4_TRY(w4a16_h2d(ctx, S.iota, host.data(), cap * 4));
-        S.iota_cap = cap;
-    }
-    if (S.zeros_cap < segs) {
-        const size_t cap = std::max<size_t>(segs, 1024);
-        size_t bytes_cap = S.zeros_cap * 4;
-        W4_TRY(w4_ensure(ctx, &S.zeros, &bytes_cap, cap * 4));
-        W4_TRY(w4a16_memset0(ctx, S.zeros, cap * 4));
-        S.zeros_cap = cap;
-    }
-    if (!S.always) {
-        const int32_t big[2] = {0x7fffffff, 0};
-        W4_TRY(w4a16_alloc(ctx, 8, &S.always));
-        W4_TRY(w4a16_h2d(ctx, S.always, big, 8));
-    }
-    const bool glu = glu_act >= 0;
-    W4Experts E;
-    E.n_exp = 1;
-    E.group = L.group;
-    E.scale_bf16 = L.scale_bf16;
-    if (glu) {  // the linear is the "gate|up arena" of its one expert: n = 2 n_ff rows over k = h
-        if (L.n % 32 != 0) return w4_fail(W4A16_ERR_SHAPE, "stream glu: n=%zu must be a multiple of 32", L.n);
-        E.q13 = L.q_tiled;
-        E.s13 = L.s_tiled;
-        E.h = L.k;
-        E.n_ff = L.n / 2;
-    } else {
-        E.q2 = L.q_tiled;
-        E.s2 = L.s_tiled;
-        E.h = L.n;
-        E.n_ff = L.k;
-    }
-    // k slices until the launch has a few workgroups per CU
-    const size_t waves = ctx->moe_waves >= 8 ? 8 : 4, units = glu ? L.row_blocks / 2 : (L.row_blocks + 1) / 2;
-    const size_t groups = (units + waves - 1) / waves;
-    size_t nks = 1;
-    if (glu) {
-        nks = 1;  // the gated kernel does not split over k
-    } else if (ctx->decode_ksplit > 0) {
-        nks = (size_t)ctx->decode_ksplit;
-    } else if (ctx->decode_ksplit == 0) {
-        // only while the launch has fewer workgroups than CUs: the 27B down projection (40 unit groups) runs 8 slices
-        // (78 -> 22 us at t = 32), the wide gate|up (272 groups) none (slices cost it 1-3 us, measured)
-        while (groups * segs * nks < (size_t)std::max(ctx->cu_count, 1) && nks < 8) nks *= 2;
-    }
-    // the grid covers exactly `segs` segments, so the "padded total" may be the constant no segment start reaches
-    if (glu) {
-        // bit 1: the activation takes the f32 sums (the expert FFN rounds gate and up to f16 first)
-        const int keep = ctx->moe_act_kind;
-        ctx->moe_act_kind = glu_act | 2;
-        const int rc = launch_moe_gemm(ctx, E, true, x_dev, t, 1, y_dev, 1, 0, t, block, segs, S.iota, S.zeros, S.always, 1);
-        ctx->moe_act_kind = keep;
-        return rc;
-    }
-    return launch_moe_gemm(ctx, E, false, x_dev, t, 1, y_dev, out_f16, 0, t, block, segs, S.iota, S.zeros, S.always, nks);
+    char sym[64];
+    snprintf(sym, sizeof sym, "w4a16_mid_g%zu_%s_t%zu_n%dk%d%s", L.group, L.scale_bf16 ? "bf16" : "f16", tt, P.wn, P.wk, glu ? "_glu" : "");
+    // staged x (two buffers of unpadded rows; a lone wave along n: one of padded rows), overlaid by the groups' results; then,
+    // where a wave sums several parts, its slot for the finished ones (kernels/mid.hip: XB, OB)
+    const size_t xb = wk * 16 * tt * (wn > 1 ? 2 * 256 : 2 * (size_t)kW4MidLdx), tiles = wk * wn * 2 * tt * 1024;
+    const size_t shmem = std::max(xb, wk > 1 ? tiles : 0) + (P.wk < kW4MidParts ? tiles : 0);
+    uint64_t qt = L.q_tiled, st = L.s_tiled;
+    int row_blocks = (int)L.row_blocks, ki = (int)L.k, ni = (int)L.n, ti = (int)t, of = out_f16 ? 1 : 0, act = glu ? glu_act : 0,
+        nksi = (int)P.nks, gp = (int)groups;
+    void* params[] = {&qt, &st, &x, &y, &row_blocks, &ki, &ni, &ti, &of, &act, &ws, &tk, &nksi, &gp};
+    return w4_launch(ctx, sym, (unsigned)blocks, (unsigned)P.nks, (unsigned)(wn * wk * 64), (unsigned)shmem, params);
 }
 
 // Direct mode for decode steps: no alignment pass.  The gate|up GEMM runs one segment per slot — the segment table is
@@ -446,10 +440,10 @@ extern "C" int w4a16_moe_ffn_act(w4a16_ctx* ctx, const char* name, uint64_t x_de
     W4_TRY(w4a16_moe_align(ctx, idx_dev, ns, E->n_exp, block, S.sorted, S.expert_ids, S.num_post));
     // gate|up with the SiLU*up epilogue: slot j reads token j / top_k
     W4_TRY(launch_moe_gemm(ctx, *E, true, x_dev, t, top_k, S.act, 1, 0, ns, block, max_segs, S.sorted, S.expert_ids,
-                           S.num_post, 1, tiled));
+                           S.num_post, tiled));
     // down, multiplied by the routing weight: slot j reads act row j
     W4_TRY(launch_moe_gemm(ctx, *E, false, S.act, ns, 1, S.c2, 1, wt_dev, ns, block, max_segs, S.sorted, S.expert_ids,
-                           S.num_post, 1, tiled));
+                           S.num_post, tiled));
     int ti = (int)t, hi = (int)E->h, ki = (int)top_k;
     void* p[] = {&S.c2, &y_dev, &ti, &hi, &ki};
     return w4_launch(ctx, "w4a16_moe_topk_sum_f16", std::min<unsigned>(ceil_div(t * E->h / (E->h % 8 == 0 ? 8 : 1), 256), 4096), 1, 256, 0, p);

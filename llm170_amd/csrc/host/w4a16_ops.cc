@@ -874,7 +874,7 @@ extern "C" int w4a16_lin_forward(w4a16_ctx* ctx, const char* name, uint64_t x_de
         case W4A16_PATH_PREFILL:
             return launch_prefill(ctx, *L, x_dev, y_dev, t, out_f16);
         case W4A16_PATH_STREAM:
-            return w4_dense_grouped(ctx, *L, x_dev, y_dev, t, out_f16);
+            return w4_dense_mid(ctx, *L, x_dev, y_dev, t, out_f16);
         default:
             return w4_fail(W4A16_ERR_ARG, "lin_forward %s: unknown path %d", name, path);
     }
@@ -919,7 +919,7 @@ extern "C" int w4a16_lin_forward_glu_act(w4a16_ctx* ctx, const char* name, uint6
     // (and for scales the MFMA kernel cannot divide by), the tiled MFMA GEMM above — each with the gated epilogue
     if (L->n % 32 != 0) return w4_fail(W4A16_ERR_SHAPE, "lin_forward_glu %s: n=%zu must be a multiple of 32", name, L->n);
     if (!L->q_tiled) return w4_fail(W4A16_ERR_UNSUPPORTED, "lin_forward_glu %s: linear has no tiled copy (needs k %% 128 == 0)", name);
-    if (t <= 64 || !L->scales_regular) return w4_dense_grouped(ctx, *L, x_dev, y_f16_dev, t, 1, act);
+    if (t <= 64 || !L->scales_regular) return w4_dense_mid(ctx, *L, x_dev, y_f16_dev, t, 1, act);
     return launch_prefill(ctx, *L, x_dev, y_f16_dev, t, 1, act);
 }
 

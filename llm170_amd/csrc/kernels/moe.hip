@@ -71,10 +71,8 @@ __device__ __forceinline__ void moe_store(f4_t a0, f4_t a1, int slot, int q, int
         h4_t o;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            // expert FFN: gate and up are f16 tensors in the reference and are rounded first; a dense gated linear
-            // (bit 1 of act_kind) applies the activation to the f32 sums, like the separate element-wise kernel
-            float g = (act_kind & 2) ? a0[i] : moe_round_f16(a0[i]), up = (act_kind & 2) ? a1[i] : moe_round_f16(a1[i]);
-            float v = w4_act_mul(g, up, act_kind & 1);
+            // gate and up are f16 tensors in the reference and are rounded first
+            float v = w4_act_mul(moe_round_f16(a0[i]), moe_round_f16(a1[i]), act_kind);
             asm volatile("" : "+v"(v));  // the product is rounded to f32 before the f16 conversion
             o[i] = (_Float16)v;
         }
@@ -115,11 +113,8 @@ __device__ __forceinline__ void moe_store(f4_t a0, f4_t a1, int slot, int q, int
 //   y: GLU -> f16 [ns][n/2]; LIN -> f16 or f32 [ns][n].  topw: null or f32 [ns] (LIN only).
 //   sorted_ids[seg*blk + i]: slot id or the sentinel ns; expert_ids[seg]; num_post[0] = padded slot total.
 //   A segment whose expert id is outside 0..n_exp-1 is skipped (its slots stay unwritten).
-//   ws / tickets: workspace and zeroed counters of a launch split over k across workgroups (gridDim.y slices; the
-//   LDS-staged kernel only): [slice][block][wave][2*TT] partial tiles, one counter per (block, wave).
-//   act_kind (GLU only): bit 0: 0 = silu(gate) * up (w4a16_moe_act_silu_f16), 1 = the tanh form of gelu on the gate
-//   (w4a16_moe_act_gelu_f16, assets/moe.cu:1635-1647); bit 1: gate and up enter the activation as f32 sums (a dense
-//   gated linear) instead of being rounded to f16 first (the expert FFN).
+//   act_kind (GLU only): 0 = silu(gate) * up (w4a16_moe_act_silu_f16), 1 = the tanh form of gelu on the gate
+//   (w4a16_moe_act_gelu_f16, assets/moe.cu:1635-1647).
 //   wpb: waves per block (the block size, as an argument: read from the dispatch packet it costs one more dependent
 //   scalar-cache miss before the first weight load).
 #define MOE_PARAMS                                                                                                  \
@@ -127,9 +122,9 @@ __device__ __forceinline__ void moe_store(f4_t a0, f4_t a1, int slot, int q, int
         unsigned long long s_stride, const uint16_t *__restrict__ x, int x_rows, int x_div, void *__restrict__ y,   \
         int y_f16, const float *__restrict__ topw, const int *__restrict__ sorted_ids,                              \
         const int *__restrict__ expert_ids, const int *__restrict__ num_post, int blk, int ns, int row_blocks, int k, \
-        int n, int n_exp, f4_t *ws, int *tickets, int wpb, int act_kind
+        int n, int n_exp, int wpb, int act_kind
 #define MOE_ARGS \
-    qa, sa, q_stride, s_stride, x, x_rows, x_div, y, y_f16, topw, sorted_ids, expert_ids, num_post, blk, ns, row_blocks, k, n, n_exp, ws, tickets, wpb, act_kind
+    qa, sa, q_stride, s_stride, x, x_rows, x_div, y, y_f16, topw, sorted_ids, expert_ids, num_post, blk, ns, row_blocks, k, n, n_exp, wpb, act_kind
 
 // ---------------------------------------------------------------------------------------------------- moe_dec
 template <int RB, int XL>
@@ -435,14 +430,9 @@ struct MoeMmStage {
     u2_t s[RB];
 };
 
-#define MOE_MAX_KSPLIT 8  // k slices across workgroups; the host clamps to this
-
 // One block = (segment of blk = 16*TT slots, group of W units); wave w owns unit group*W + w over the whole k range.
-// KS: the launch may be split over k across workgroups (dense linears run as one expert; the expert FFN never splits, and
-// its kernels are built without the epilogue that costs them registers).
-// TT: the 16-slot blocks of the segment this workgroup multiplies (those that hold a slot); TTMAX: the blocks of a full
-// segment, which size a wave's share of the split-k workspace.
-template <int G, bool SBF, bool GLU, int TT, int TTMAX, int DEPTH, bool KS>
+// TT: the 16-slot blocks of the segment this workgroup multiplies (those that hold a slot).
+template <int G, bool SBF, bool GLU, int TT, int DEPTH>
 __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
     extern __shared__ _Float16 xs[];  // [2][16*TT][MOE_LDX]
     constexpr int GPT = W4_TILE_K / G;
@@ -468,8 +458,6 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
     const int u = min(u_raw, units - 1);
     if ((unsigned)e >= (unsigned)n_exp) return;  // uniform for the block, before any barrier
     const int kt_n = k / W4_TILE_K, kg_n = kt_n * GPT;
-    const int nks = KS ? (int)gridDim.y : 1, ky = KS ? (int)blockIdx.y : 0;  // k slices across workgroups
-    const int kt_lo = (kt_n * ky) / nks, kt_hi = (kt_n * (ky + 1)) / nks;
     const int c = lane & 15, q = lane >> 4;
     const int rbA = GLU ? u : 2 * u, rbB = GLU ? u + units : min(2 * u + 1, row_blocks - 1);
     const bool haveB = GLU || 2 * u + 1 < row_blocks;
@@ -498,7 +486,7 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
 #pragma unroll
         for (int p = 0; p < TT; p++)
             r[p] = __builtin_amdgcn_raw_buffer_load_b128(
-                xr, (kt < kt_hi && xg_off[p] != W4_OOB) ? xg_off[p] + (unsigned)kt * (W4_TILE_K * 2u) : W4_OOB, 0, 0);
+                xr, (kt < kt_n && xg_off[p] != W4_OOB) ? xg_off[p] + (unsigned)kt * (W4_TILE_K * 2u) : W4_OOB, 0, 0);
     };
     auto store_x = [&](const u4_t (&r)[TT], int buf) {
         _Float16* base = xs + buf * (ROWS * MOE_LDX);
@@ -514,7 +502,7 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
                               (unsigned)rbB * (unsigned)kg_n * 32u + sg + (unsigned)q * 8u};
     MoeMmStage<2> stage[DEPTH];
     auto load_w = [&](MoeMmStage<2>& s_, int kt) {
-        const bool live = kt < kt_hi;
+        const bool live = kt < kt_n;
 #pragma unroll
         for (int rb = 0; rb < 2; rb++)
             s_.q[rb] = __builtin_amdgcn_raw_buffer_load_b128(qr, live ? qoff[rb] + (unsigned)kt * 1024u : W4_OOB, 0, 2);
@@ -627,26 +615,26 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
         group(std::integral_constant<int, 7>{});
     };
 
-    // prologue: the slice's first x tile into LDS buffer 0, the second in registers (both loads issued before the first
+    // prologue: the first x tile into LDS buffer 0, the second in registers (both loads issued before the first
     // is stored: the first tile's registers are free again before the accumulators are live), DEPTH weight stages in
     // flight
     {
         u4_t first[TT];
-        load_x(first, kt_lo);
-        load_x(xreg, kt_lo + 1);
+        load_x(first, 0);
+        load_x(xreg, 1);
 #pragma unroll
-        for (int d = 0; d < DEPTH; d++) load_w(stage[d], kt_lo + d);
+        for (int d = 0; d < DEPTH; d++) load_w(stage[d], d);
         store_x(first, 0);
     }
     __syncthreads();
     int xb = 0;  // LDS buffer of the tile being multiplied
-    for (int kt0 = kt_lo; kt0 < kt_hi; kt0 += DEPTH) {
+    for (int kt0 = 0; kt0 < kt_n; kt0 += DEPTH) {
 #pragma unroll
         for (int d = 0; d < DEPTH; d++) {
             const int kt = kt0 + d;
             // a wave that holds a landed tile issues ahead of the waves that are queueing loads (about 1 % at every T)
             __builtin_amdgcn_s_setprio(1);
-            if (kt < kt_hi) {
+            if (kt < kt_n) {
                 if constexpr (G == 32 && TT <= 3) compute32(stage[d], xb);
                 else compute(stage[d], xb);
             }
@@ -660,53 +648,6 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
     }
 
     if (!active) return;
-    if (KS && nks > 1) {
-        // every wave on its own: park the partial tiles (device-scope stores), draw the (block, wave) ticket, and the
-        // wave that draws the last one adds the slices in slice order and stores.  The hand-over is the one of the
-        // dense decode kernel (decode.hip): write-through stores completed before the agent-scope ticket atomic,
-        // cache-bypassing loads behind an agent-scope acquire fence in the wave that drew the last ticket; the slice
-        // offset travels in the vector offset (scalar offset 0) so that the compiler inserts the wait state a write to
-        // the data registers of a 16-byte store needs, and the tiles stay live until the stores have completed.
-        constexpr unsigned PER_WAVE = 2u * TTMAX * 1024u;
-        const unsigned per_slice = gridDim.x * (unsigned)W * PER_WAVE;
-        const __amdgpu_buffer_rsrc_t wr = w4_make_rsrc(ws, per_slice * (unsigned)nks);
-        const unsigned mine = (blockIdx.x * (unsigned)W + (unsigned)wave) * PER_WAVE + (unsigned)lane * 16u;
-        const unsigned park = mine + (unsigned)ky * per_slice;
-        constexpr int DEV = 16;  // cache policy: device scope
-#pragma unroll
-        for (int rb = 0; rb < 2; rb++)
-#pragma unroll
-            for (int tt = 0; tt < TT; tt++)
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4_t, acc[rb][tt]), wr,
-                                                       park + (unsigned)(rb * TT + tt) * 1024u, 0, DEV);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#pragma unroll
-        for (int rb = 0; rb < 2; rb++)
-#pragma unroll
-            for (int tt = 0; tt < TT; tt++) asm volatile("" ::"v"(acc[rb][tt]));
-        int ticket = 0;
-        int* const tk = tickets + blockIdx.x * W + wave;
-        if (lane == 0) ticket = __hip_atomic_fetch_add(tk, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        ticket = __builtin_amdgcn_readfirstlane(ticket);
-        if (ticket != nks - 1) return;
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-#pragma unroll
-        for (int rb = 0; rb < 2; rb++)
-#pragma unroll
-            for (int tt = 0; tt < TT; tt++) {
-                f4_t part[MOE_MAX_KSPLIT];  // all slices in flight at once; slices past nks: zero-length descriptor, zeros
-#pragma unroll
-                for (int s_ = 0; s_ < MOE_MAX_KSPLIT; s_++)
-                    part[s_] = __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(
-                                                            s_ < nks ? wr : w4_make_rsrc(ws, 0u),
-                                                            mine + (unsigned)(rb * TT + tt) * 1024u, s_ * per_slice, DEV));
-                f4_t sum = part[0];
-#pragma unroll
-                for (int s_ = 1; s_ < MOE_MAX_KSPLIT; s_++) sum += part[s_];
-                acc[rb][tt] = sum;
-            }
-        if (lane == 0) __hip_atomic_store(tk, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
 #pragma unroll
     for (int tt = 0; tt < TT; tt++) {
         const int slot = sorted_ids[seg * blk + tt * 16 + c];
@@ -720,20 +661,20 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
 // 16-slot block tells whether the block holds any: the workgroup runs the body built for the blocks that do, and the
 // MFMAs, scaled sums and x rows of all-padding blocks are never issued (128 experts, top-8, T = 512: runs of 32 +- 6
 // slots in 48-slot segments, every other expert fills two blocks of three).
-template <int G, bool SBF, bool GLU, int TT, int DEPTH, bool KS>
+template <int G, bool SBF, bool GLU, int TT, int DEPTH>
 __device__ __forceinline__ void moe_mm_entry(MOE_PARAMS) {
     if constexpr (TT == 1) {
-        moe_mm_body<G, SBF, GLU, 1, 1, DEPTH, KS>(MOE_ARGS);
+        moe_mm_body<G, SBF, GLU, 1, DEPTH>(MOE_ARGS);
     } else {
         const int units = GLU ? row_blocks >> 1 : (row_blocks + 1) >> 1;
         const int seg = blockIdx.x / ((units + wpb - 1) / wpb);
         int live = 1;
 #pragma unroll
         for (int p = 1; p < TT; p++) live += sorted_ids[seg * blk + 16 * p] < ns ? 1 : 0;
-        if (live == 1) moe_mm_body<G, SBF, GLU, 1, TT, DEPTH, KS>(MOE_ARGS);
-        else if (TT == 2 || live == 2) moe_mm_body<G, SBF, GLU, 2, TT, DEPTH, KS>(MOE_ARGS);
-        else if (TT == 3 || live == 3) moe_mm_body<G, SBF, GLU, TT >= 3 ? 3 : 2, TT, DEPTH, KS>(MOE_ARGS);
-        else moe_mm_body<G, SBF, GLU, TT, TT, DEPTH, KS>(MOE_ARGS);
+        if (live == 1) moe_mm_body<G, SBF, GLU, 1, DEPTH>(MOE_ARGS);
+        else if (TT == 2 || live == 2) moe_mm_body<G, SBF, GLU, 2, DEPTH>(MOE_ARGS);
+        else if (TT == 3 || live == 3) moe_mm_body<G, SBF, GLU, TT >= 3 ? 3 : 2, DEPTH>(MOE_ARGS);
+        else moe_mm_body<G, SBF, GLU, TT, DEPTH>(MOE_ARGS);
     }
 }
 
@@ -741,9 +682,9 @@ __device__ __forceinline__ void moe_mm_entry(MOE_PARAMS) {
     extern "C" __global__ __launch_bounds__(512) void NAME(MOE_PARAMS) {              \
         moe_dec_body<G, SBF, GLU, XL, DEPTH>(MOE_ARGS);                               \
     }
-#define MOE_MM_KERNEL(NAME, G, SBF, GLU, TT, DEPTH, KS)                               \
+#define MOE_MM_KERNEL(NAME, G, SBF, GLU, TT, DEPTH)                                   \
     extern "C" __global__ __launch_bounds__(512) void NAME(MOE_PARAMS) {              \
-        moe_mm_entry<G, SBF, GLU, TT, DEPTH, KS>(MOE_ARGS);                           \
+        moe_mm_entry<G, SBF, GLU, TT, DEPTH>(MOE_ARGS);                               \
     }
 // Ring depths, from sweeps on the 128-expert shape: the one-slot segments of the direct mode run best with two k tiles
 // in flight per wave (T = 4..12: 9-11 % faster than four: fewer registers, more waves resident at once); so do the
@@ -754,18 +695,14 @@ __device__ __forceinline__ void moe_mm_entry(MOE_PARAMS) {
     MOE_DEC_KERNEL(PFX##_dec_glu_x4, G, SBF, true, 4, 2)     \
     MOE_DEC_KERNEL(PFX##_dec_lin_x1, G, SBF, false, 1, 2)    \
     MOE_DEC_KERNEL(PFX##_dec_lin_x4, G, SBF, false, 4, 2)    \
-    MOE_MM_KERNEL(PFX##_mm_glu_t1, G, SBF, true, 1, DMM, false)    \
-    MOE_MM_KERNEL(PFX##_mm_glu_t2, G, SBF, true, 2, DMM, false)    \
-    MOE_MM_KERNEL(PFX##_mm_glu_t3, G, SBF, true, 3, DMM, false)    \
-    MOE_MM_KERNEL(PFX##_mm_glu_t4, G, SBF, true, 4, DMM, false)    \
-    MOE_MM_KERNEL(PFX##_mm_lin_t1, G, SBF, false, 1, DMM, false)   \
-    MOE_MM_KERNEL(PFX##_mm_lin_t2, G, SBF, false, 2, DMM, false)   \
-    MOE_MM_KERNEL(PFX##_mm_lin_t3, G, SBF, false, 3, DMM, false)   \
-    MOE_MM_KERNEL(PFX##_mm_lin_t4, G, SBF, false, 4, DMM, false)   \
-    MOE_MM_KERNEL(PFX##_mm_lin_t1_ks, G, SBF, false, 1, DMM, true) \
-    MOE_MM_KERNEL(PFX##_mm_lin_t2_ks, G, SBF, false, 2, DMM, true) \
-    MOE_MM_KERNEL(PFX##_mm_lin_t3_ks, G, SBF, false, 3, DMM, true) \
-    MOE_MM_KERNEL(PFX##_mm_lin_t4_ks, G, SBF, false, 4, DMM, true)
+    MOE_MM_KERNEL(PFX##_mm_glu_t1, G, SBF, true, 1, DMM)    \
+    MOE_MM_KERNEL(PFX##_mm_glu_t2, G, SBF, true, 2, DMM)    \
+    MOE_MM_KERNEL(PFX##_mm_glu_t3, G, SBF, true, 3, DMM)    \
+    MOE_MM_KERNEL(PFX##_mm_glu_t4, G, SBF, true, 4, DMM)    \
+    MOE_MM_KERNEL(PFX##_mm_lin_t1, G, SBF, false, 1, DMM)   \
+    MOE_MM_KERNEL(PFX##_mm_lin_t2, G, SBF, false, 2, DMM)   \
+    MOE_MM_KERNEL(PFX##_mm_lin_t3, G, SBF, false, 3, DMM)   \
+    MOE_MM_KERNEL(PFX##_mm_lin_t4, G, SBF, false, 4, DMM)
 
 #ifndef MOE_G32_DEPTH
 #define MOE_G32_DEPTH 2

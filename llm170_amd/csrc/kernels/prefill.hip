@@ -466,13 +466,12 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
     }
 
 // Grouped kernels for the expert FFN: same arguments as the streaming grouped kernels of moe.hip (blk must be 64, the
-// rows of a block tile; ws, tickets and wpb are unused).
+// rows of a block tile; wpb is unused).
 #define PREFILL_MOE_KERNEL(NAME, G, SBF, MODE)                                                                          \
     extern "C" __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(3, 3))) void NAME(            \
         const char* qa, const char* sa, unsigned long long q_stride, unsigned long long s_stride, const uint16_t* x,      \
         int x_rows, int x_div, void* y, int y_f16, const float* topw, const int* sorted_ids, const int* expert_ids,      \
-        const int* num_post, int blk, int ns, int row_blocks, int k, int n, int n_exp, f4_t* ws, int* tickets, int wpb,  \
-        int act_kind) {                                                                                                  \
+        const int* num_post, int blk, int ns, int row_blocks, int k, int n, int n_exp, int wpb, int act_kind) {                                                                                                  \
         PfGroup<MODE> gp;                                                                                                \
         gp.sorted_ids = sorted_ids;                                                                                      \
         gp.expert_ids = expert_ids;                                                                                      \
@@ -485,7 +484,7 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
         gp.x_div = x_div;                                                                                                \
         gp.n_exp = n_exp;                                                                                                \
         gp.act_kind = act_kind;                                                                                          \
-        (void)blk, (void)ws, (void)tickets, (void)wpb;                                                                   \
+        (void)blk, (void)wpb;                                                                   \
         prefill_body<G, SBF, 2, MODE>(reinterpret_cast<const u4_t*>(qa), reinterpret_cast<const uint16_t*>(sa), x, y,    \
                                       row_blocks, k, n, 0, y_f16, 1, 1, gp);                                             \
     }
