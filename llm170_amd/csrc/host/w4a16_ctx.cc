@@ -44,6 +44,7 @@ static const char* const kLaneSyms[] = {"w4a16_lane_g128_f16", "w4a16_lane_g128_
                                         "w4a16_lane_g32_bf16", nullptr};
 static const char* const kLayoutSyms[] = {"w4a16_tile_q",         "w4a16_tile_s",          "w4a16_untile_q",
                                           "w4a16_untile_s",       "w4a16_dump_tiled_f16",  "w4a16_dump_tiled_bf16",
+                                          "w4a16_tile_s_f16",
                                           "w4a16_dump_raw_f16",   "w4a16_dump_raw_bf16",   "w4a16_row_norm_max_f16",
                                           "w4a16_row_norm_max_bf16", nullptr};
 // one family: the row counts' builds of a kernel, x by direct loads where the name ends in d (kernels/decode.hip)

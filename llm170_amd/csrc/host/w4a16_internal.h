@@ -36,6 +36,7 @@ struct W4Experts {
     int scale_bf16 = 0;
     size_t q13_stride = 0, s13_stride = 0, q2_stride = 0, s2_stride = 0;  // bytes per expert
     bool scales_regular = true;  // same rule as W4Lin::scales_regular, over both arenas: the MFMA-tiled grouped kernels need it
+    bool tiled_bf16 = false;  // the arenas hold bf16 scales (bf16 scales that f16 holds exactly are stored as f16)
 };
 
 // Scratch of the MoE FFN, grown on demand (reference: moe_msorted / moe_mexp / moe_mnpost / moe_mact / moe_mc2,
@@ -116,8 +117,7 @@ constexpr int kW4LaneTt = 8;                // LANE_TT (lane.hip): tokens per pa
 constexpr int kW4DecodeMaxKsplit = 8;       // W4_DECODE_MAX_KSPLIT (decode.hip)
 constexpr int kW4MoeMaxKsplit = 8;          // MOE_MAX_KSPLIT (mid.hip)
 constexpr int kW4MidParts = 4;              // MID_PARTS (mid.hip): runs of a slice's k tiles that are summed on their own
-constexpr int kW4MidLdx = 136;              // MID_LDX (mid.hip): halves per x row staged through registers
-constexpr int kW4MoeLdx = 136;              // MOE_LDX (moe.hip): halves per staged x row
+constexpr int kW4MoeLdx = 136;              // MOE_LDX (mid.hip): halves per x row staged through registers
 constexpr int kW4MoeAlignWaves = 16;        // MOE_ALIGN_WAVES (moe.hip)
 constexpr int kW4RmsLanes = 1024;           // RMS_LANES (glue.hip)
 constexpr int kW4PfBn = 256;                // PF_BN (prefill.hip): block tile columns
@@ -137,6 +137,8 @@ int w4_find_lin(w4a16_ctx* ctx, const char* name, W4Lin** out);
 // true when every scale of `count` u16 entries is finite, non-zero and (bf16) inside [2^-60, 2^60]: what a kernel that
 // carries the running unit s_prev / s_cur can take
 bool w4_scales_regular(const uint16_t* s, size_t count, int scale_bf16);
+// true when every one of `count` bf16 scales is zero or a normal f16 number (2^-14 .. 2^16, 8 significant bits)
+bool w4_bf16_fits_f16(const uint16_t* s, size_t count);
 int w4_ensure(w4a16_ctx* ctx, uint64_t* buf, size_t* cap, size_t bytes);
 // dense linear at 17..64 rows, or any number of rows (kernels/mid.hip).  glu_act >= 0: L is a fused gate|up linear and y_dev
 // receives f16 [t][n/2] = act(gate) * up on the f32 sums

@@ -22,7 +22,7 @@ static void free_experts(w4a16_ctx* ctx, W4Experts& E) {
 
 // Tile one projection of every expert: raw [n_exp][n][k/8] + [n_exp][n][k/group] on the host -> arena on the device.
 static int tile_arena(w4a16_ctx* ctx, const void* q, const void* s, size_t n_exp, size_t n, size_t k, size_t group,
-                      uint64_t* q_arena, uint64_t* s_arena, size_t* q_stride, size_t* s_stride) {
+                      bool to_f16, uint64_t* q_arena, uint64_t* s_arena, size_t* q_stride, size_t* s_stride) {
     const size_t row_blocks = (n + 15) / 16, kt_n = k / 128, kg_n = k / group;
     const size_t q_raw_e = n * (k / 2), s_raw_e = n * kg_n * 2;
     *q_stride = row_blocks * kt_n * 1024;
@@ -45,7 +45,7 @@ static int tile_arena(w4a16_ctx* ctx, const void* q, const void* s, size_t n_exp
             void* pq[] = {&qr, &qt, &ni, &ki, &rbi};
             rc = w4_launch(ctx, "w4a16_tile_q", ceil_div(*q_stride / 4, 256), 1, 256, 0, pq);
             void* ps[] = {&sr, &st, &ni, &kgi, &rbi};
-            if (!rc) rc = w4_launch(ctx, "w4a16_tile_s", ceil_div(*s_stride / 2, 256), 1, 256, 0, ps);
+            if (!rc) rc = w4_launch(ctx, to_f16 ? "w4a16_tile_s_f16" : "w4a16_tile_s", ceil_div(*s_stride / 2, 256), 1, 256, 0, ps);
         }
         if (!rc) rc = w4a16_sync(ctx);  // the staging buffer is reused by the next batch
     }
@@ -83,8 +83,12 @@ extern "C" int w4a16_upload_experts(w4a16_ctx* ctx, const char* name, size_t n_e
     // whose every scale that kernel can divide by (the streaming kernels only multiply by scales and take any)
     E.scales_regular = w4_scales_regular(static_cast<const uint16_t*>(s13), s13_bytes / 2, scale_bf16) &&
                        w4_scales_regular(static_cast<const uint16_t*>(s2), s2_bytes / 2, scale_bf16);
-    int rc = tile_arena(ctx, q13, s13, n_experts, 2 * n_ff, h, group, &E.q13, &E.s13, &E.q13_stride, &E.s13_stride);
-    if (!rc) rc = tile_arena(ctx, q2, s2, n_experts, h, n_ff, group, &E.q2, &E.s2, &E.q2_stride, &E.s2_stride);
+    // bf16 scales that f16 holds exactly are stored as f16: the f16 kernels read the same values without a conversion per scale
+    const bool to_f16 = scale_bf16 && w4_bf16_fits_f16(static_cast<const uint16_t*>(s13), s13_bytes / 2) &&
+                        w4_bf16_fits_f16(static_cast<const uint16_t*>(s2), s2_bytes / 2);
+    E.tiled_bf16 = scale_bf16 && !to_f16;
+    int rc = tile_arena(ctx, q13, s13, n_experts, 2 * n_ff, h, group, to_f16, &E.q13, &E.s13, &E.q13_stride, &E.s13_stride);
+    if (!rc) rc = tile_arena(ctx, q2, s2, n_experts, h, n_ff, group, to_f16, &E.q2, &E.s2, &E.q2_stride, &E.s2_stride);
     if (rc) {
         const std::string keep = w4_err_save();
         free_experts(ctx, E);
@@ -129,7 +133,7 @@ extern "C" int w4a16_experts_dequant_dump(w4a16_ctx* ctx, const char* name, int 
     uint64_t st = (which == 0 ? E->s13 + expert * E->s13_stride : E->s2 + expert * E->s2_stride);
     int ni = (int)n, ki = (int)k, gi = (int)E->group, rbi = (int)((n + 15) / 16);
     void* p[] = {&qt, &st, &out_f32_dev, &ni, &ki, &gi, &rbi};
-    return w4_launch(ctx, E->scale_bf16 ? "w4a16_dump_tiled_bf16" : "w4a16_dump_tiled_f16",
+    return w4_launch(ctx, E->tiled_bf16 ? "w4a16_dump_tiled_bf16" : "w4a16_dump_tiled_f16",
                      ceil_div((size_t)rbi * (k / 128) * 256, 256), 1, 256, 0, p);
 }
 
@@ -245,14 +249,14 @@ static int launch_moe_gemm(w4a16_ctx* ctx, const W4Experts& E, bool glu, uint64_
     void* p[] = {&qa, &sa, &qs, &ss, &x, &xr, &xd, &y, &yf, &topw, &sorted, &eids, &npost, &blk, &nsi, &rbi, &ki, &ni, &nei,
                  &waves, &act_kind};
     char sym[80];
-    const char* fam = E.scale_bf16 ? "bf16" : "f16";
+    const char* fam = E.tiled_bf16 ? "bf16" : "f16";
     if (tiled) {
         // MFMA-tiled grouped kernel (kernels/prefill.hip, MODE 1 / 2): block tile = one 64-slot segment x 256 columns
         // (gate|up: 128 gate + the 128 matching up columns); LDS = two x stages of 64 rows x 64 k and the slot ids
         if (block != 64) return w4_fail(W4A16_ERR_ARG, "moe: the tiled grouped kernel needs 64-slot segments (got %zu)", block);
-        if (max_segs > 65535) return w4_fail(W4A16_ERR_SHAPE, "moe: %zu segments exceed the grid", max_segs);
         const size_t cols = glu ? E.n_ff : n, per_tile = glu ? 128 : 256;
         snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_pf_%s", E.group, fam, glu ? "glu" : "lin");
+        if (max_segs > 65535) return w4_fail(W4A16_ERR_SHAPE, "moe: %zu segments exceed the grid", max_segs);
         return w4_launch(ctx, sym, (unsigned)((cols + per_tile - 1) / per_tile), (unsigned)max_segs, 256, 2 * 64 * 64 * 2 + 256, p);
     }
     if (block <= 16) {
@@ -268,7 +272,7 @@ static int launch_moe_gemm(w4a16_ctx* ctx, const W4Experts& E, bool glu, uint64_
     waves = waves >= 8 ? 8 : 4;  // the x staging needs at least 4 waves
     const size_t blocks = max_segs * ((units + (size_t)waves - 1) / (size_t)waves);
     snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_mm_%s_t%d", E.group, fam, glu ? "glu" : "lin", tt);
-    const unsigned shmem = (unsigned)(2 * 16 * tt * kW4MoeLdx * 2);
+    const unsigned shmem = (unsigned)(2 * 16 * tt * 256);  // two x tiles of 128 k
     return w4_launch(ctx, sym, (unsigned)blocks, 1, (unsigned)(waves * 64), shmem, p);
 }
 
@@ -344,7 +348,7 @@ int w4_dense_mid(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_t y, size_t 
     snprintf(sym, sizeof sym, "w4a16_mid_g%zu_%s_t%zu_n%dk%d%s", L.group, L.scale_bf16 ? "bf16" : "f16", tt, P.wn, P.wk, glu ? "_glu" : "");
     // staged x (two buffers of unpadded rows; a lone wave along n: one of padded rows), overlaid by the groups' results; then,
     // where a wave sums several parts, its slot for the finished ones (kernels/mid.hip: XB, OB)
-    const size_t xb = wk * 16 * tt * (wn > 1 ? 2 * 256 : 2 * (size_t)kW4MidLdx), tiles = wk * wn * 2 * tt * 1024;
+    const size_t xb = wk * 16 * tt * (wn > 1 ? 2 * 256 : 2 * (size_t)kW4MoeLdx), tiles = wk * wn * 2 * tt * 1024;
     const size_t shmem = std::max(xb, wk > 1 ? tiles : 0) + (P.wk < kW4MidParts ? tiles : 0);
     uint64_t qt = L.q_tiled, st = L.s_tiled;
     int row_blocks = (int)L.row_blocks, ki = (int)L.k, ni = (int)L.n, ti = (int)t, of = out_f16 ? 1 : 0, act = glu ? glu_act : 0,
@@ -393,7 +397,7 @@ static int moe_ffn_direct(w4a16_ctx* ctx, const char* name, const W4Experts& E, 
     int tk = (int)top_k, nsi = (int)ns, rbi = (int)row_blocks, ki = (int)E.n_ff, ni = (int)E.h, nei = (int)E.n_exp;
     void* p[] = {&qa, &sa, &qs, &ss, &S.act, &idx_dev, &wt_dev, &y_dev, &tk, &nsi, &rbi, &ki, &ni, &nei};
     char sym[80];
-    snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_down_sum%s", E.group, E.scale_bf16 ? "bf16" : "f16", rbu == 1 ? "1" : "");
+    snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_down_sum%s", E.group, E.tiled_bf16 ? "bf16" : "f16", rbu == 1 ? "1" : "");
     return w4_launch(ctx, sym, (unsigned)(t * units), 1, (unsigned)(top_k * 64), (unsigned)(top_k * rbu * 64 * 16), p);
 }
 

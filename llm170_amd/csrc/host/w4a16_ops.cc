@@ -654,6 +654,14 @@ bool w4_scales_regular(const uint16_t* sp, size_t count, int scale_bf16) {
     return true;
 }
 
+bool w4_bf16_fits_f16(const uint16_t* sp, size_t count) {
+    for (size_t i = 0; i < count; i++) {
+        const unsigned e = (sp[i] >> 7) & 0xFFu;  // biased exponent, 127 = 2^0; an infinity or NaN has 255
+        if ((e < 127u - 14u || e > 127u + 15u) && (sp[i] & 0x7FFFu) != 0) return false;
+    }
+    return true;
+}
+
 static void free_lin(w4a16_ctx* ctx, W4Lin& L) {
     (void)w4a16_free(ctx, L.q_raw);
     (void)w4a16_free(ctx, L.s_raw);

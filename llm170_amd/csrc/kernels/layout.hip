@@ -41,6 +41,21 @@ extern "C" __global__ __launch_bounds__(256) void w4a16_tile_s(const uint16_t* _
     st[id] = row < n ? s[(size_t)row * kg_n + kg] : (uint16_t)0;
 }
 
+// The same from bf16 scales that f16 holds exactly, stored as f16: the same values for the f16 kernels.
+extern "C" __global__ __launch_bounds__(256) void w4a16_tile_s_f16(const uint16_t* __restrict__ s,
+                                                                   uint16_t* __restrict__ st, int n, int kg_n,
+                                                                   int row_blocks) {
+    const size_t total = (size_t)row_blocks * kg_n * 16;
+    const size_t id = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (id >= total) return;
+    const int r = id & 15;
+    const size_t rest = id >> 4;
+    const int kg = rest % kg_n, nb = rest / kg_n;
+    const int row = nb * 16 + r;
+    const float v = row < n ? w4_scale_to_f32<true>(s[(size_t)row * kg_n + kg]) : 0.f;
+    st[id] = __builtin_bit_cast(uint16_t, (_Float16)v);
+}
+
 // Inverse of w4a16_tile_q: one thread per operand-format word q[row][kw].
 extern "C" __global__ __launch_bounds__(256) void w4a16_untile_q(const uint32_t* __restrict__ qt,
                                                                  uint32_t* __restrict__ q, int n, int k) {

@@ -21,7 +21,7 @@
 // 19.2 / 14.6; 5120 x 2048 group 32 t = 37 13.1 / 7.6; 17408 x 5120 t = 64 32.7 / 28.0; 512 x 17408 t = 40 20.7 / 11.2.
 #include "w4a16_common.hpp"
 
-#define MID_LDX 136  // halves per staged x row: 128 + 8 padding (272-byte stride: 16-lane b128 reads hit all banks once)
+#define MOE_LDX 136  // halves per staged x row: 128 + 8 padding (272-byte stride: 16-lane b128 reads hit all banks once)
 #define MOE_MAX_KSPLIT 8  // k slices across workgroups; the host clamps to this
 #define MID_PARTS 4       // runs of a slice's k tiles, each summed from zero
 
@@ -96,7 +96,7 @@ __device__ __forceinline__ void mid_body(MID_PARAMS) {
         const int piece = WN > 1 ? c ^ (r & 15) : c;
         xoff[l] = row < t ? ((unsigned)row * (unsigned)k + (unsigned)piece * 8u) * 2u : W4_OOB;
     }
-    constexpr int LDX = WN > 1 ? 128 : MID_LDX;
+    constexpr int LDX = WN > 1 ? 128 : MOE_LDX;
     _Float16* const xg = xs + kg * (NBUF * ROWS * LDX);
     _Float16* const x_put = xg + (4 * wn + q) * LDX + c * 8;
     unsigned x_get[4];  // halves: operand of MFMA w, row c of a 16-row block

@@ -12,8 +12,8 @@
 //       - moe_dec (segments of <= 4 or <= 16 slots, decode steps): HBM streaming, in-block split-K over the waves,
 //         x gathered straight from global memory (one load + DPP row shifts for <= 4 slots);
 //       - moe_mm (segments of 16..64 slots, prefill chunks): the waves of a block take different output rows of the
-//         same segment and share the gathered x rows through LDS (double buffered, one k tile per stage), so x is
-//         fetched once per block instead of once per wave.
+//         same segment and share the gathered x rows through LDS (LDS DMA, double buffered, one k tile per stage), so x
+//         is fetched once per block instead of once per wave.
 //   * decode steps of at most four tokens skip the alignment: the gate|up GEMM runs one segment per slot (segment table
 //     = identity, expert table = idx itself) and moe_down_sum does the down projection of a token's experts, the
 //     routing-weight multiply, the f16 rounding and the slot-order sum in one launch — two launches per FFN;
@@ -25,8 +25,6 @@
 #include <type_traits>
 
 #include "w4a16_common.hpp"
-
-#define MOE_LDX 136  // halves per staged x row: 128 + 8 padding (272-byte stride: 16-lane b128 reads hit all banks once)
 
 template <int W>
 __device__ __forceinline__ unsigned w4_quad_bcast(unsigned v) {
@@ -432,9 +430,9 @@ struct MoeMmStage {
 
 // One block = (segment of blk = 16*TT slots, group of W units); wave w owns unit group*W + w over the whole k range.
 // TT: the 16-slot blocks of the segment this workgroup multiplies (those that hold a slot).
-template <int G, bool SBF, bool GLU, int TT, int DEPTH>
+template <int G, bool SBF, bool GLU, int TT>
 __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
-    extern __shared__ _Float16 xs[];  // [2][16*TT][MOE_LDX]
+    extern __shared__ _Float16 xs[];  // [2][16*TT][128]
     constexpr int GPT = W4_TILE_K / G;
     constexpr int ROWS = 16 * TT;
     const int tid = threadIdx.x, lane = tid & 63, W = wpb;
@@ -442,13 +440,12 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
     const int units = GLU ? row_blocks >> 1 : (row_blocks + 1) >> 1;
     const int groups = (units + W - 1) / W;
     const int seg = blockIdx.x / groups, grp = blockIdx.x % groups;
-    // the table reads (padded total, the segment's expert, this thread's slot ids) are issued together, ahead of the
-    // tests that use them (see moe_dec_body)
-    const int rows_pp = 4 * W;
+    // the table reads (padded total, the segment's expert, this lane's slot ids) are issued together, ahead of the tests that
+    // use them (see moe_dec_body); x load p of wave w brings rows 4 * (w + p * W) ..+3 of the segment, 16 lanes to a row
     int np = num_post[0], e = expert_ids[seg];
     int slot_of[TT];
 #pragma unroll
-    for (int p = 0; p < TT; p++) slot_of[p] = sorted_ids[seg * blk + min(p * rows_pp + (tid >> 4), ROWS - 1)];
+    for (int p = 0; p < TT; p++) slot_of[p] = sorted_ids[seg * blk + min(4 * (wave + p * W) + (lane >> 4), ROWS - 1)];
     asm volatile("" : "+s"(np), "+s"(e));
 #pragma unroll
     for (int p = 0; p < TT; p++) asm volatile("" : "+v"(slot_of[p]));
@@ -462,53 +459,46 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
     const int rbA = GLU ? u : 2 * u, rbB = GLU ? u + units : min(2 * u + 1, row_blocks - 1);
     const bool haveB = GLU || 2 * u + 1 < row_blocks;
 
-    const __amdgpu_buffer_rsrc_t qr =
-        w4_make_rsrc(qa + (unsigned long long)e * q_stride, (unsigned)row_blocks * (unsigned)kt_n * 1024u);
-    const __amdgpu_buffer_rsrc_t sr =
-        w4_make_rsrc(sa + (unsigned long long)e * s_stride, (unsigned)row_blocks * (unsigned)kg_n * 32u);
-    const __amdgpu_buffer_rsrc_t xr = w4_make_rsrc(x, (unsigned)x_rows * (unsigned)k * 2u);
+    const char* const qe = qa + (unsigned long long)e * q_stride;
+    const char* const se = sa + (unsigned long long)e * s_stride;
+    const unsigned q_bytes = (unsigned)row_blocks * (unsigned)kt_n * 1024u, s_bytes = (unsigned)row_blocks * (unsigned)kg_n * 32u;
 
-    // x staging: one k tile of the segment's rows = ROWS x 256 B; 16 threads cover a row, 4*W rows per pass
+    // x staging: one k tile of the segment's rows, gathered straight into LDS by DMA (no registers held), rows of 256 B whose
+    // 16-byte chunks are swizzled, chunk p of row r at position p ^ (r & 15), so that the 16 rows of a B operand's read fall
+    // into distinct banks.  W >= 4: at most TT loads per wave.
     unsigned xg_off[TT];
-    int xl_off[TT];
 #pragma unroll
     for (int p = 0; p < TT; p++) {
-        const int row = p * rows_pp + (tid >> 4);
-        const int slot = row < ROWS ? slot_of[p] : ns;
-        xg_off[p] = slot < ns ? ((unsigned)(slot / x_div) * (unsigned)k + (unsigned)(tid & 15) * 8u) * 2u : W4_OOB;
-        xl_off[p] = row < ROWS ? row * MOE_LDX + (tid & 15) * 8 : -1;
+        const int row = 4 * (wave + p * W) + q, slot = row < ROWS ? slot_of[p] : ns;
+        xg_off[p] = slot < ns ? ((unsigned)(slot / x_div) * (unsigned)k + (unsigned)((c ^ (row & 15)) * 8)) * 2u : W4_OOB;
     }
-    // x tiles travel global -> registers -> LDS two k tiles ahead of their use: the gathered rows come from L2 with a
-    // latency longer than one k tile of compute.  One register set: an iteration stores the tile loaded in the previous
-    // one and then loads the next into the same registers.
-    u4_t xreg[TT];
-    auto load_x = [&](u4_t (&r)[TT], int kt) {
+    typedef __attribute__((address_space(3))) char lds_char_t;
+    auto load_x = [&](int kt, int buf) {
+        const __amdgpu_buffer_rsrc_t xr = w4_make_rsrc(x, kt < kt_n ? (unsigned)x_rows * (unsigned)k * 2u : 0u);
 #pragma unroll
         for (int p = 0; p < TT; p++)
-            r[p] = __builtin_amdgcn_raw_buffer_load_b128(
-                xr, (kt < kt_n && xg_off[p] != W4_OOB) ? xg_off[p] + (unsigned)kt * (W4_TILE_K * 2u) : W4_OOB, 0, 0);
+            if (wave + p * W < 4 * TT)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    xr, (__attribute__((address_space(3))) void*)((lds_char_t*)xs + (buf * ROWS + 4 * (wave + p * W)) * 256), 16, xg_off[p],
+                    kt * (W4_TILE_K * 2), 0, 0);
     };
-    auto store_x = [&](const u4_t (&r)[TT], int buf) {
-        _Float16* base = xs + buf * (ROWS * MOE_LDX);
+    unsigned x_get[4];  // halves: operand of MFMA w, row c of a 16-row block
 #pragma unroll
-        for (int p = 0; p < TT; p++)
-            if (xl_off[p] >= 0) *reinterpret_cast<u4_t*>(base + xl_off[p]) = r[p];
-    };
+    for (int w = 0; w < 4; w++) x_get[w] = (unsigned)(c * 128 + ((w * 4 + q) ^ c) * 8);
 
     const unsigned qoff[2] = {(unsigned)rbA * (unsigned)kt_n * 1024u + (unsigned)lane * 16u,
                               (unsigned)rbB * (unsigned)kt_n * 1024u + (unsigned)lane * 16u};
     const unsigned sg = G == 32 ? (unsigned)(lane & 3) * 32u : 0u;
     const unsigned soff[2] = {(unsigned)rbA * (unsigned)kg_n * 32u + sg + (unsigned)q * 8u,
                               (unsigned)rbB * (unsigned)kg_n * 32u + sg + (unsigned)q * 8u};
-    MoeMmStage<2> stage[DEPTH];
+    MoeMmStage<2> stage[2];
     auto load_w = [&](MoeMmStage<2>& s_, int kt) {
         const bool live = kt < kt_n;
+        const __amdgpu_buffer_rsrc_t qr = w4_make_rsrc(qe, live ? q_bytes : 0u), sr = w4_make_rsrc(se, live ? s_bytes : 0u);
 #pragma unroll
-        for (int rb = 0; rb < 2; rb++)
-            s_.q[rb] = __builtin_amdgcn_raw_buffer_load_b128(qr, live ? qoff[rb] + (unsigned)kt * 1024u : W4_OOB, 0, 2);
+        for (int rb = 0; rb < 2; rb++) s_.q[rb] = __builtin_amdgcn_raw_buffer_load_b128(qr, qoff[rb], kt * 1024, 2);
 #pragma unroll
-        for (int rb = 0; rb < 2; rb++)
-            s_.s[rb] = __builtin_amdgcn_raw_buffer_load_b64(sr, live ? soff[rb] + (unsigned)kt * (GPT * 32u) : W4_OOB, 0, 0);
+        for (int rb = 0; rb < 2; rb++) s_.s[rb] = __builtin_amdgcn_raw_buffer_load_b64(sr, soff[rb], kt * (GPT * 32), 0);
     };
 
     f4_t acc[2][TT];
@@ -518,14 +508,14 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
         for (int tt = 0; tt < TT; tt++) acc[rb][tt] = (f4_t){0.f, 0.f, 0.f, 0.f};
 
     auto compute = [&](const MoeMmStage<2>& s_, int buf) {
-        const _Float16* xb = xs + buf * (ROWS * MOE_LDX) + c * MOE_LDX + q * 8;
+        const _Float16* xb = xs + buf * (ROWS * 128);
         const f4_t zero = {0.f, 0.f, 0.f, 0.f};
         f4_t part[2][TT];
         auto step = [&](auto wc) {
             constexpr int w = decltype(wc)::value;
             h8_t b[TT];
 #pragma unroll
-            for (int tt = 0; tt < TT; tt++) b[tt] = *reinterpret_cast<const h8_t*>(xb + tt * 16 * MOE_LDX + w * 32);
+            for (int tt = 0; tt < TT; tt++) b[tt] = *reinterpret_cast<const h8_t*>(xb + x_get[w] + tt * 16 * 128);
 #pragma unroll
             for (int rb = 0; rb < 2; rb++) {
                 // G = 32 (segments of 64 slots only; smaller ones run compute32 below): every 32-k group's products are
@@ -572,11 +562,11 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
     // live at a time.  128 experts, top-8: T = 64 77.6 -> 76.1 us, T = 512 117.9 -> 115.6 us; with four blocks the
     // extra registers cost a wave per SIMD (T = 1024 +2 %), so 64-slot segments keep the plain order.
     auto compute32 = [&](const MoeMmStage<2>& s_, int buf) {
-        const _Float16* xb = xs + buf * (ROWS * MOE_LDX) + c * MOE_LDX + q * 8;
+        const _Float16* xb = xs + buf * (ROWS * 128);
         const f4_t zero = {0.f, 0.f, 0.f, 0.f};
         h8_t b[TT];
 #pragma unroll
-        for (int tt = 0; tt < TT; tt++) b[tt] = *reinterpret_cast<const h8_t*>(xb + tt * 16 * MOE_LDX);
+        for (int tt = 0; tt < TT; tt++) b[tt] = *reinterpret_cast<const h8_t*>(xb + x_get[0] + tt * 16 * 128);
         h8_t a = w4_deq8(s_.q[0][0]);
         auto group = [&](auto gc) {
             constexpr int g = decltype(gc)::value, w = g >> 1, rb = g & 1;
@@ -592,7 +582,7 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
                 constexpr int w2 = (g + 1) >> 1, rb2 = (g + 1) & 1;
                 if constexpr (w2 != w) {
 #pragma unroll
-                    for (int tt = 0; tt < TT; tt++) b[tt] = *reinterpret_cast<const h8_t*>(xb + tt * 16 * MOE_LDX + w2 * 32);
+                    for (int tt = 0; tt < TT; tt++) b[tt] = *reinterpret_cast<const h8_t*>(xb + x_get[w2] + tt * 16 * 128);
                 }
                 a = w4_deq8(s_.q[rb2][w2]);
                 asm volatile("" : "+v"(a));
@@ -615,35 +605,28 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
         group(std::integral_constant<int, 7>{});
     };
 
-    // prologue: the first x tile into LDS buffer 0, the second in registers (both loads issued before the first
-    // is stored: the first tile's registers are free again before the accumulators are live), DEPTH weight stages in
-    // flight
-    {
-        u4_t first[TT];
-        load_x(first, 0);
-        load_x(xreg, 1);
-#pragma unroll
-        for (int d = 0; d < DEPTH; d++) load_w(stage[d], d);
-        store_x(first, 0);
-    }
+    // one k tile ahead: its DMA and weights are issued ahead of this tile's MFMAs and waited for (vmcnt 0) at the barrier
+    // that ends them.  Few registers, many waves: x in flight in registers and weights two (group 32) or four (group 128) tiles
+    // ahead, the wait for x behind the youngest weights, were slower throughout (128 experts, us per FFN: group 32 f16 T = 64
+    // 75.6 -> 70.7, T = 517 117 -> 113; group 128 T = 64 74.9 -> 67.4, T = 517 111.5 -> 98.5).
+    load_x(0, 0);
+    load_w(stage[0], 0);
     __syncthreads();
-    int xb = 0;  // LDS buffer of the tile being multiplied
-    for (int kt0 = 0; kt0 < kt_n; kt0 += DEPTH) {
+    for (int kt0 = 0; kt0 < kt_n; kt0 += 2) {
 #pragma unroll
-        for (int d = 0; d < DEPTH; d++) {
+        for (int d = 0; d < 2; d++) {
             const int kt = kt0 + d;
+            load_x(kt + 1, d ^ 1);  // out of range past the last tile: zeros, no traffic
+            load_w(stage[d ^ 1], kt + 1);
+            __builtin_amdgcn_sched_barrier(0);
             // a wave that holds a landed tile issues ahead of the waves that are queueing loads (about 1 % at every T)
             __builtin_amdgcn_s_setprio(1);
             if (kt < kt_n) {
-                if constexpr (G == 32 && TT <= 3) compute32(stage[d], xb);
-                else compute(stage[d], xb);
+                if constexpr (G == 32 && TT <= 3) compute32(stage[d], d);
+                else compute(stage[d], d);
             }
             __builtin_amdgcn_s_setprio(0);
-            load_w(stage[d], kt + DEPTH);
-            store_x(xreg, xb ^ 1);  // tile kt+1, loaded an iteration ago, into the buffer tile kt-1 was read from
-            load_x(xreg, kt + 2);   // out of range past the last tile: zeros, no traffic
             __syncthreads();
-            xb ^= 1;
         }
     }
 
@@ -661,20 +644,20 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
 // 16-slot block tells whether the block holds any: the workgroup runs the body built for the blocks that do, and the
 // MFMAs, scaled sums and x rows of all-padding blocks are never issued (128 experts, top-8, T = 512: runs of 32 +- 6
 // slots in 48-slot segments, every other expert fills two blocks of three).
-template <int G, bool SBF, bool GLU, int TT, int DEPTH>
+template <int G, bool SBF, bool GLU, int TT>
 __device__ __forceinline__ void moe_mm_entry(MOE_PARAMS) {
     if constexpr (TT == 1) {
-        moe_mm_body<G, SBF, GLU, 1, DEPTH>(MOE_ARGS);
+        moe_mm_body<G, SBF, GLU, 1>(MOE_ARGS);
     } else {
         const int units = GLU ? row_blocks >> 1 : (row_blocks + 1) >> 1;
         const int seg = blockIdx.x / ((units + wpb - 1) / wpb);
         int live = 1;
 #pragma unroll
         for (int p = 1; p < TT; p++) live += sorted_ids[seg * blk + 16 * p] < ns ? 1 : 0;
-        if (live == 1) moe_mm_body<G, SBF, GLU, 1, DEPTH>(MOE_ARGS);
-        else if (TT == 2 || live == 2) moe_mm_body<G, SBF, GLU, 2, DEPTH>(MOE_ARGS);
-        else if (TT == 3 || live == 3) moe_mm_body<G, SBF, GLU, TT >= 3 ? 3 : 2, DEPTH>(MOE_ARGS);
-        else moe_mm_body<G, SBF, GLU, TT, DEPTH>(MOE_ARGS);
+        if (live == 1) moe_mm_body<G, SBF, GLU, 1>(MOE_ARGS);
+        else if (TT == 2 || live == 2) moe_mm_body<G, SBF, GLU, 2>(MOE_ARGS);
+        else if (TT == 3 || live == 3) moe_mm_body<G, SBF, GLU, TT >= 3 ? 3 : 2>(MOE_ARGS);
+        else moe_mm_body<G, SBF, GLU, TT>(MOE_ARGS);
     }
 }
 
@@ -682,35 +665,31 @@ __device__ __forceinline__ void moe_mm_entry(MOE_PARAMS) {
     extern "C" __global__ __launch_bounds__(512) void NAME(MOE_PARAMS) {              \
         moe_dec_body<G, SBF, GLU, XL, DEPTH>(MOE_ARGS);                               \
     }
-#define MOE_MM_KERNEL(NAME, G, SBF, GLU, TT, DEPTH)                                   \
+#define MOE_MM_KERNEL(NAME, G, SBF, GLU, TT)                                          \
     extern "C" __global__ __launch_bounds__(512) void NAME(MOE_PARAMS) {              \
-        moe_mm_entry<G, SBF, GLU, TT, DEPTH>(MOE_ARGS);                               \
+        moe_mm_entry<G, SBF, GLU, TT>(MOE_ARGS);                                      \
     }
-// Ring depths, from sweeps on the 128-expert shape: the one-slot segments of the direct mode run best with two k tiles
-// in flight per wave (T = 4..12: 9-11 % faster than four: fewer registers, more waves resident at once); so do the
-// segments of up to 16 slots (5 % faster than three).  The LDS-staged kernels keep two (group 32) or four (group 128);
-// the LDS buffer of a k tile alternates on its own, whatever the ring depth.
-#define MOE_FAMILY(PFX, G, SBF, DMM)                             \
+// Ring depths of the streaming kernels, from sweeps on the 128-expert shape: the one-slot segments of the direct mode run
+// best with two k tiles in flight per wave (T = 4..12: 9-11 % faster than four: fewer registers, more waves resident at
+// once); so do the segments of up to 16 slots (5 % faster than three).
+#define MOE_FAMILY(PFX, G, SBF)                             \
     MOE_DEC_KERNEL(PFX##_dec_glu_x1, G, SBF, true, 1, 2)     \
     MOE_DEC_KERNEL(PFX##_dec_glu_x4, G, SBF, true, 4, 2)     \
     MOE_DEC_KERNEL(PFX##_dec_lin_x1, G, SBF, false, 1, 2)    \
     MOE_DEC_KERNEL(PFX##_dec_lin_x4, G, SBF, false, 4, 2)    \
-    MOE_MM_KERNEL(PFX##_mm_glu_t1, G, SBF, true, 1, DMM)    \
-    MOE_MM_KERNEL(PFX##_mm_glu_t2, G, SBF, true, 2, DMM)    \
-    MOE_MM_KERNEL(PFX##_mm_glu_t3, G, SBF, true, 3, DMM)    \
-    MOE_MM_KERNEL(PFX##_mm_glu_t4, G, SBF, true, 4, DMM)    \
-    MOE_MM_KERNEL(PFX##_mm_lin_t1, G, SBF, false, 1, DMM)   \
-    MOE_MM_KERNEL(PFX##_mm_lin_t2, G, SBF, false, 2, DMM)   \
-    MOE_MM_KERNEL(PFX##_mm_lin_t3, G, SBF, false, 3, DMM)   \
-    MOE_MM_KERNEL(PFX##_mm_lin_t4, G, SBF, false, 4, DMM)
+    MOE_MM_KERNEL(PFX##_mm_glu_t1, G, SBF, true, 1)    \
+    MOE_MM_KERNEL(PFX##_mm_glu_t2, G, SBF, true, 2)    \
+    MOE_MM_KERNEL(PFX##_mm_glu_t3, G, SBF, true, 3)    \
+    MOE_MM_KERNEL(PFX##_mm_glu_t4, G, SBF, true, 4)    \
+    MOE_MM_KERNEL(PFX##_mm_lin_t1, G, SBF, false, 1)   \
+    MOE_MM_KERNEL(PFX##_mm_lin_t2, G, SBF, false, 2)   \
+    MOE_MM_KERNEL(PFX##_mm_lin_t3, G, SBF, false, 3)   \
+    MOE_MM_KERNEL(PFX##_mm_lin_t4, G, SBF, false, 4)
 
-#ifndef MOE_G32_DEPTH
-#define MOE_G32_DEPTH 2
-#endif
-MOE_FAMILY(w4a16_moe_g32_f16, 32, false, MOE_G32_DEPTH)
-MOE_FAMILY(w4a16_moe_g32_bf16, 32, true, MOE_G32_DEPTH)
-MOE_FAMILY(w4a16_moe_g128_f16, 128, false, 4)
-MOE_FAMILY(w4a16_moe_g128_bf16, 128, true, 4)
+MOE_FAMILY(w4a16_moe_g32_f16, 32, false)
+MOE_FAMILY(w4a16_moe_g32_bf16, 32, true)
+MOE_FAMILY(w4a16_moe_g128_f16, 128, false)
+MOE_FAMILY(w4a16_moe_g128_bf16, 128, true)
 
 // ---------------------------------------------------------------------------------------------------- routing
 // Routing rule of the reference (w4a16_dec/mod.rs:168-185, device counterpart assets/moe.cu:686-759): softmax over all

@@ -441,3 +441,41 @@ def test_moe_direct_mode_out_of_range_expert_contributes_zero(dec, orc, small_ex
     ok_wt = np.array([[0.5, 0.0], [0.5, 0.5]], np.float32)
     ref = orc.moe_ffn(x, ok_idx, ok_wt, q13, s13, q2, s2, h, n_ff, 32, False)
     assert parity.compare(y, ref["y"])["rel_l2"] < 1e-3
+
+
+@pytest.mark.parametrize("t", [3, 20, 70, 200, 600])
+def test_bf16_arenas_inside_and_outside_the_f16_range(dec, orc, t):
+    """bf16 scales that f16 holds exactly (zero, 2^-14 .. 2^16, negative ones among them) are stored as f16 and run the f16
+    kernels: same dequantised weights and the same result bits as arenas whose one scale beyond the range, in a row of an expert
+    no slot reaches, keeps them in bf16; direct mode, segments of 16 to 64 slots with ragged ends, MFMA-tiled."""
+    E, h, n_ff, k, group = 8, 256, 128, 2, 32
+    q13, s13, q2, s2 = gen.make_experts(E, h, n_ff, group, seed=gen.GATE_SEED + 91)
+    s13, s2 = _bf16_scales(s13), _bf16_scales(s2)
+    s13[1, 5, 2], s2[2, 7, 1] = 0x3880, 0xB8FF             # 2^-14, the smallest normal f16; -(2 - 2^-7) 2^-14
+    if t < 600:
+        s13[2, 9, 0], s2[3, 11, 3] = 0x0000, 0x8000        # zeros (the MFMA-tiled kernels are not for them)
+    edge13 = s13.copy()
+    edge13[0, 1, 1] = 0x477F                               # (2 - 2^-7) 2^15 = 65280, below f16's 65504
+    out13 = s13.copy()
+    out13[0, 1, 1] = 0x3800                                # 2^-15: an f16 subnormal, kept in bf16
+    x = gen.normal_f16(78, (t, h))
+    lg = gen.router_logits(t, E, seed=6)
+    lg[:, 0] = -30.0                                       # expert 0 is never chosen
+    idx, wt = ops.moe_topk(lg, k)
+    assert not np.any(idx == 0)
+    dec.upload_experts("in", q13, s13, q2, s2, E, h, n_ff, group, True)
+    dec.upload_experts("edge", q13, edge13, q2, s2, E, h, n_ff, group, True)
+    dec.upload_experts("out", q13, out13, q2, s2, E, h, n_ff, group, True)
+    for name, s in (("edge", edge13), ("out", out13)):
+        for e in (0, 1, 2, 3):
+            want = orc.dequant_matrix(q13[e], s[e], 2 * n_ff, h, group, True)
+            assert np.array_equal(dec.experts_dequant(name, 0, e), want)  # value by value; a zero's sign may differ
+            assert np.array_equal(dec.experts_dequant(name, 1, e), orc.dequant_matrix(q2[e], s2[e], h, n_ff, group, True))
+    runs = [_run_ffn(dec, name, x, idx, wt, t, k, h) for name in ("in", "edge", "out")]
+    if t == 600:
+        assert runs[0][3] == 64
+    for r in runs[1:]:
+        assert np.array_equal(r[0].view(np.uint32), runs[0][0].view(np.uint32)) and np.array_equal(r[1], runs[0][1])
+    y, act, c2, _ = runs[0]
+    if c2 is not None:
+        _check_ffn(orc, y, act, c2, x, idx, wt, q13, s13, q2, s2, h, n_ff, group, True, "bf16 in f16 range t%d" % t)
