@@ -121,7 +121,8 @@ constexpr int kW4MoeLdx = 136;              // MOE_LDX (mid.hip): halves per x r
 constexpr int kW4MoeAlignWaves = 16;        // MOE_ALIGN_WAVES (moe.hip)
 constexpr int kW4RmsLanes = 1024;           // RMS_LANES (glue.hip)
 constexpr int kW4PfBn = 256;                // PF_BN (prefill.hip): block tile columns
-constexpr int kW4PfKs = 64;                 // PF_KS (prefill.hip): k per LDS stage
+constexpr int kW4PfKs = 128;                // PF_KS (prefill.hip): k per LDS stage
+constexpr int kW4PfMoeIdsAt = 36864;        // PF_MOE_IDS_AT (prefill.hip): LDS bytes ahead of the grouped kernels' slot ids
 constexpr int kW4PfThreads = 256;           // PF_THREADS (prefill.hip)
 
 int w4_fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));

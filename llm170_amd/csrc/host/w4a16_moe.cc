@@ -256,8 +256,9 @@ static int launch_moe_gemm(w4a16_ctx* ctx, const W4Experts& E, bool glu, uint64_
         if (block != 64) return w4_fail(W4A16_ERR_ARG, "moe: the tiled grouped kernel needs 64-slot segments (got %zu)", block);
         const size_t cols = glu ? E.n_ff : n, per_tile = glu ? 128 : 256;
         snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_pf_%s", E.group, fam, glu ? "glu" : "lin");
-        if (max_segs > 65535) return w4_fail(W4A16_ERR_SHAPE, "moe: %zu segments exceed the grid", max_segs);
-        return w4_launch(ctx, sym, (unsigned)((cols + per_tile - 1) / per_tile), (unsigned)max_segs, 256, 2 * 64 * 64 * 2 + 256, p);
+        const size_t blocks = (max_segs + 7) / 8 * 8 * ((cols + per_tile - 1) / per_tile);
+        if (blocks > 0x7fffffffu) return w4_fail(W4A16_ERR_SHAPE, "moe: %zu segments exceed the grid", max_segs);
+        return w4_launch(ctx, sym, (unsigned)blocks, 1, 256, kW4PfMoeIdsAt + 64 * 8, p);
     }
     if (block <= 16) {
         // in-block split-K: each wave needs at least one k tile
@@ -418,11 +419,13 @@ extern "C" int w4a16_moe_ffn_act(w4a16_ctx* ctx, const char* name, uint64_t x_de
         return w4_fail(W4A16_ERR_SHAPE, "moe_ffn %s: t=%zu top_k=%zu experts=%zu", name, t, top_k, E->n_exp);
     W4_TRY(w4_hip(hipSetDevice(ctx->device), "hipSetDevice"));
     const size_t ns = t * top_k;
-    // From a mean run of 96 slots per expert on, 64-slot segments are mostly full and the MFMA-tiled grouped kernel
-    // (one segment x 256 columns per workgroup, x through LDS, 32x32x16 tiles) takes over from the streaming kernels.
+    // Where 64-slot segments are mostly full the MFMA-tiled grouped kernel (one segment x 256 columns per workgroup, x through
+    // LDS, 32x32x16 tiles) takes over from the streaming kernels.  Mean run per expert from which it wins: 68 slots (us per FFN,
+    // streaming / tiled: group 32, 128 experts top-8 h 2048 n_ff 768, T = 850 163 / 160, T = 1024 201 / 184; 32 experts top-4
+    // n_ff 1024 T = 512 80 / 83, T = 600 96 / 88; group 128, 64 experts top-6 n_ff 1408 T = 600 133 / 134, T = 700 155 / 152).
     if (ctx->moe_tiled > 0 && !E->scales_regular)
         return w4_fail(W4A16_ERR_UNSUPPORTED, "moe_ffn %s: the MFMA-tiled grouped kernels were requested (set_moe_tiled 1) but the experts hold a zero, non-finite or out-of-range scale; the streaming kernels serve them", name);
-    const bool tiled = ctx->moe_tiled > 0 || (ctx->moe_tiled == 0 && ctx->moe_block == 0 && E->scales_regular && ns >= 96 * E->n_exp);
+    const bool tiled = ctx->moe_tiled > 0 || (ctx->moe_tiled == 0 && ctx->moe_block == 0 && E->scales_regular && ns >= 68 * E->n_exp);
     const size_t block = tiled ? 64 : pick_block(ctx, t, ns, E->n_exp, top_k);
     if (block != 1 && block != 4 && block != 16 && block != 32 && block != 48 && block != 64)
         return w4_fail(W4A16_ERR_ARG, "moe_ffn %s: segment size %zu not in {1,4,16,32,48,64}", name, block);

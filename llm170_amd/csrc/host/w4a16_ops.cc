@@ -577,8 +577,8 @@ static int launch_prefill(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_t y
     const size_t grid = ((supers + 7) / 8) * (sup_m * sup_n) * 8;
     char sym[64];
     snprintf(sym, sizeof sym, "w4a16_prefill_g%zu_%s%s%s", L.group, L.scale_bf16 ? "bf16" : "f16", bm == 64 ? "_m64" : bm == 96 ? "_m96" : "", glu ? "_glu" : "");
-    // two stages of bm rows x PF_KS halves, then bm words (row factors of the dense kernels)
-    const unsigned shmem = (unsigned)(2 * bm * kW4PfKs * 2 + bm * 4);
+    // two stages of bm rows x PF_KS halves (the 96-row tile: half of that), then bm words (row factors)
+    const unsigned shmem = (unsigned)(2 * bm * (bm == 96 ? kW4PfKs / 2 : kW4PfKs) * 2 + bm * 4);
     uint64_t qt = L.q_tiled, st = L.s_tiled;
     int row_blocks = (int)L.row_blocks, ki = (int)L.k, ni = (int)L.n, ti = (int)t, of = (out_f16 || glu) ? 1 : 0;
     int spm = (int)sup_m, spn = (int)sup_n, act = glu ? glu_act : 0, glu_i = glu ? 1 : 0;

@@ -4,9 +4,11 @@
 //   * workgroup = 4 waves along n, block tile 128 (m) x 256 (n), wave tile 128 x 64 = 4 x 2 MFMA tiles of 32 x 32 with
 //     f32 accumulators in arch VGPRs (128 registers); two workgroups per CU, so one block's barriers and LDS writes
 //     overlap the other's MFMAs;
-//   * x (the A operand) is staged through LDS in k slabs of 64, double buffered, by LDS DMA (buffer_load ... lds:
-//     no staging registers, no ds_write); rows are unpadded and their 16-byte chunks swizzled by row so the
-//     ds_read_b128 fragment reads are bank-conflict free; rows >= t come from out-of-range loads (zeros);
+//   * x (the A operand) is staged through LDS a k tile at a time (in the 96-row tile, whose registers leave no room for the
+//     addresses, half of one), double buffered, by LDS DMA (buffer_load ... lds: no staging registers, no ds_write), one
+//     barrier per stage; stages of 64 k: 5120 x 34816 gated t = 300 113.5 -> 111.0 us, t = 4096 1158 -> 1151, 17408 x 5120
+//     t = 4096 618 -> 609; rows are unpadded and their 16-byte chunks swizzled by row so the ds_read_b128 fragment reads are
+//     bank-conflict free; rows >= t come from out-of-range loads (zeros);
 //   * the weights (B operand) never touch LDS: the tiled layout of w4a16_common.hpp already is the MFMA B layout —
 //     lane (n = l % 32, khalf = l / 32) reads 16 B of tile lane g = 2h + khalf, r = n % 16 of its row block, dword w of
 //     which is the k16 block (w, h) of the k tile — so each wave fetches its 64 x 128 weights with four coalesced
@@ -33,9 +35,9 @@ __device__ __forceinline__ float pf_ratio(float s_prev, float s_cur) {
 }
 
 #define PF_BN 256
-#define PF_KS 64          // k per LDS stage
-#define PF_LDA 64         // halves per staged x row (unpadded; chunks swizzled)
+#define PF_KS 128         // k per LDS stage, half of that in the 96-row tile
 #define PF_THREADS 256
+#define PF_MOE_IDS_AT 36864  // grouped: LDS bytes ahead of the slot ids, the larger of the two stages and four padded f16 tiles
 
 // MI = 32-row MFMA tiles along m per wave: 4 (block tile 128 x 256, 128 accumulator registers, two workgroups per CU) or
 // 2 (64 x 256, 64 registers, three workgroups per CU) for a few dozen to a couple of hundred rows, where 128-row tiles
@@ -66,6 +68,7 @@ struct PfGroup {
     const float* topw;
     unsigned long long q_stride, s_stride;  // bytes per expert
     int ns, x_rows, x_div, n_exp, act_kind;
+    int m0, n0, expert;  // the block tile: first position in sorted_ids, first column, expert
 };
 
 // Epilogue options of the dense kernels (MODE 0 and 3), the prefill-regime form of what the decode kernel does for a
@@ -91,9 +94,11 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
                                              const uint16_t* __restrict__ x, void* __restrict__ y, int row_blocks,
                                              int k, int n, int t, int out_f16, int sup_m, int sup_n,
                                              const PfGroup<MODE> gp = PfGroup<MODE>(), const PfEpi epi = PfEpi()) {
-    extern __shared__ _Float16 lds[];  // 2 stages x [PF_BM][PF_LDA]; then PF_BM ints: slot ids (grouped) / row factors (dense)
+    extern __shared__ _Float16 lds[];  // 2 stages x [PF_BM][KS]; then per row: factors (dense) / slot ids, weights (grouped)
     constexpr int GPT = W4_TILE_K / G;
-    constexpr int PF_BM = 32 * MI, PF_STAGE_BYTES = PF_BM * PF_LDA * 2;
+    constexpr int PF_BM = 32 * MI, KS = MI == 3 ? PF_KS / 2 : PF_KS;
+    constexpr int PF_STAGE_BYTES = PF_BM * KS * 2, CPR = KS / 8;  // 16-byte chunks per staged x row
+    constexpr int NA = PF_BM * CPR / PF_THREADS, SPT = W4_TILE_K / KS;  // x loads per thread and stage, stages per k tile
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wn = wave;  // 4 waves along n
@@ -118,16 +123,10 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
         m0 = tm * PF_BM;
         n0 = tn * (MODE == 3 ? PF_BN / 2 : PF_BN);
     } else {
-        // grouped: blockIdx.x = column tile (fastest, so the tiles of a segment run together and share its x rows
-        // through the L2), blockIdx.y = segment.  Gate|up tiles span 128 gate and the 128 matching up columns.
-        const int seg = blockIdx.y;
-        m0 = seg * PF_BM;  // position in sorted_ids
-        if (m0 >= gp.num_post[0]) return;
-        const int e = gp.expert_ids[seg];
-        if ((unsigned)e >= (unsigned)gp.n_exp) return;
-        qt = reinterpret_cast<const u4_t*>(reinterpret_cast<const char*>(qt) + (size_t)e * gp.q_stride);
-        st = reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(st) + (size_t)e * gp.s_stride);
-        n0 = blockIdx.x * (MODE == 1 ? PF_BN / 2 : PF_BN);
+        m0 = gp.m0;
+        n0 = gp.n0;
+        qt = reinterpret_cast<const u4_t*>(reinterpret_cast<const char*>(qt) + (size_t)gp.expert * gp.q_stride);
+        st = reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(st) + (size_t)gp.expert * gp.s_stride);
     }
 
     const unsigned ldx = DENSE && epi.ldx ? (unsigned)epi.ldx : (unsigned)k;  // halves between x rows
@@ -136,16 +135,16 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
     const __amdgpu_buffer_rsrc_t sr = w4_make_rsrc(st, (unsigned)row_blocks * (unsigned)kg_n * 32u);
 
     // ---- x staging by LDS DMA (buffer_load ... lds: global -> LDS without passing through registers).  A stage is
-    // PF_BM rows x 64 k = PF_BM * 8 chunks of 16 B, 4 per thread; one instruction of a wave fills 1 KiB of LDS, lane i
-    // at byte 16*i, so rows are 128 B apart without padding.  To keep the fragment reads conflict free the chunks of a
-    // row are stored swizzled: chunk position p of row r holds k chunk p ^ (r & 7) — the lane that fills position p
+    // PF_BM rows x KS k = PF_BM * CPR chunks of 16 B; one instruction of a wave fills 1 KiB of LDS, lane i at byte 16*i,
+    // so rows are 2 KS bytes apart without padding.  To keep the fragment reads conflict free the chunks of a
+    // row are stored swizzled: chunk position p of row r holds k chunk p ^ (r % CPR) — the lane that fills position p
     // simply fetches that k chunk.  Rows >= t fetch out of range: zeros.
     typedef __attribute__((address_space(3))) char lds_char_t;
     lds_char_t* const lds_base = (lds_char_t*)lds;
-    unsigned xa_off[MI];  // PF_BM * 8 chunks over 256 threads
+    unsigned xa_off[NA];
 #pragma unroll
-    for (int i = 0; i < MI; i++) {
-        const int c = tid + i * PF_THREADS, row = c >> 3, kc = (c & 7) ^ (row & 7);
+    for (int i = 0; i < NA; i++) {
+        const int c = tid + i * PF_THREADS, row = c / CPR, kc = (c % CPR) ^ (row % CPR);
         if (DENSE) {
             xa_off[i] = (m0 + row < t) ? ((unsigned)(m0 + row) * ldx + (unsigned)kc * 8u) * 2u : W4_OOB;
         } else {
@@ -153,8 +152,13 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
             xa_off[i] = id < gp.ns ? ((unsigned)(id / gp.x_div) * (unsigned)k + (unsigned)kc * 8u) * 2u : W4_OOB;
         }
     }
-    int* const seg_ids = reinterpret_cast<int*>(lds_base + 2 * PF_STAGE_BYTES);
-    if (!DENSE && tid < PF_BM) seg_ids[tid] = gp.sorted_ids[m0 + tid];  // visible after the first barrier
+    int* const seg_ids = reinterpret_cast<int*>(lds_base + (DENSE ? 2 * PF_STAGE_BYTES : PF_MOE_IDS_AT));
+    float* const seg_w = reinterpret_cast<float*>(seg_ids + PF_BM);
+    if (!DENSE && tid < PF_BM) {  // visible after the first barrier
+        const int id = gp.sorted_ids[m0 + tid];
+        seg_ids[tid] = id;
+        if (MODE == 2) seg_w[tid] = gp.topw != nullptr && id < gp.ns ? gp.topw[id] : 1.0f;
+    }
     // Dense, input statistics given: the 1/rms factor of this block's PF_BM input rows, once, into the same LDS words
     // (thread r < PF_BM owns row m0 + r: entries added in index order with eight loads in flight — the same bits on
     // every run; consecutive threads read consecutive floats of an entry).  Read back in the epilogue.
@@ -178,10 +182,10 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
     }
     auto load_a = [&](int s, int buf) {
 #pragma unroll
-        for (int i = 0; i < MI; i++)
+        for (int i = 0; i < NA; i++)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
                 xr, (__attribute__((address_space(3))) void*)(lds_base + buf * PF_STAGE_BYTES + (i * PF_THREADS + wave * 64) * 16),
-                16, xa_off[i], s * (PF_KS * 2), 0, 0);
+                16, xa_off[i], s * (KS * 2), 0, 0);
     };
 
     // ---- weights: lane (nl = l % 32, khalf = l / 32); per n sub-tile ni and half h one dwordx4 per k tile
@@ -224,24 +228,24 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
     // block covers k tiles [kt_lo, kt_hi) and writes an f32 partial; a second launch adds the partials in order
     const int kt_lo = DENSE ? (kt_n * (int)blockIdx.y) / (int)gridDim.y : 0,
               kt_hi = DENSE ? (kt_n * ((int)blockIdx.y + 1)) / (int)gridDim.y : kt_n;
-    const int stages = 2 * kt_hi;
+    const int stages = SPT * kt_hi;
     constexpr bool PF_WAVE_PRIO = G == 128;  // wave priority over a stage's MFMAs (see the k loop)
 
-    load_a(2 * kt_lo, 0);
+    load_a(SPT * kt_lo, 0);
     load_b(bq, sc, kt_lo);
     __syncthreads();  // the compiler waits for the LDS DMA (vmcnt) ahead of the barrier
 
     for (int kt = kt_lo; kt < kt_hi; kt++) {
 #pragma unroll
-        for (int half = 0; half < 2; half++) {
-            const int s = kt * 2 + half;
+        for (int half = 0; half < SPT; half++) {
+            const int s = kt * SPT + half;
             // stage s+1 goes into the buffer that stage s-1 was read from: every wave is past the barrier that ended it
-            if (s + 1 < stages) load_a(s + 1, (s + 1) & 1);
+            if (s + 1 < stages) load_a(s + 1, (s + 1 - SPT * kt_lo) & 1);
             if (half == 0 && kt + 1 < kt_hi) load_b(bqn, scn, kt + 1);
-            const _Float16* abuf = lds + (s & 1) * (PF_BM * PF_LDA) + a_row * PF_LDA;
+            const _Float16* abuf = lds + ((s - SPT * kt_lo) & 1) * (PF_BM * KS) + a_row * KS;
 #pragma unroll
-            for (int kbl = 0; kbl < 4; kbl++) {
-                const int kb = half * 4 + kbl, w = kb >> 1, h = kb & 1;
+            for (int kbl = 0; kbl < KS / 16; kbl++) {
+                const int kb = half * (KS / 16) + kbl, w = kb >> 1, h = kb & 1;
                 // Group boundary: re-express the accumulators in the next group's scale.
                 //   group 128: the multiply is done at the END of a k tile, tile by tile right after each tile's last
                 //   MFMA of the group, with the scale of the next k tile (already loaded), so the VALU work of tile j
@@ -272,7 +276,7 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
                 h8_t a[MI];
 #pragma unroll
                 for (int mi = 0; mi < MI; mi++)
-                    a[mi] = *reinterpret_cast<const h8_t*>(abuf + mi * 32 * PF_LDA + (((kbl * 2 + khalf) ^ (nl & 7)) * 8));
+                    a[mi] = *reinterpret_cast<const h8_t*>(abuf + mi * 32 * KS + (((kbl * 2 + khalf) ^ (nl % CPR)) * 8));
                 const bool last128 = G == 128 && kb == 7;  // branch free: the last k tile multiplies by 1
                 float next_ratio[2] = {1.f, 1.f};
                 if (last128) {
@@ -313,42 +317,40 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
     }
 
     // ---- epilogue: y[m][n] = acc * unit; D register e of lane (nl, khalf) is row 8*(e/4) + 4*khalf + e%4, column nl
-    if (MODE == 1) {
-        const int n_ff = n >> 1, col = n0 + wn * 32 + nl;
-        if (col >= n_ff) return;
+    if (!DENSE) {
+        // Grouped: the wave's f16 tile goes through its own part of the stages' LDS (free after the last barrier, a wave's LDS
+        // operations run in order) and out in 16-byte pieces of whole row segments: one store per 1 KiB instead of 2 bytes per
+        // lane; the routing weights were fetched once per row, not once per element.  128 experts top-8 h 2048 n_ff 768,
+        // T = 2048: down projection 126 -> 85 us, gate|up level (its stores cost 17 us, the activation keeps them busy).
+        constexpr int COLS = MODE == 1 ? 32 : 64, LD = COLS + 8, PER_ROW = COLS / 8;
+        const int n_out = MODE == 1 ? n >> 1 : n, col = n0 + wn * COLS;
+        if (col >= n_out) return;  // uniform for the wave (n_out % 64 == 0)
+        _Float16* const tile = lds + wave * (PF_BM * LD);
 #pragma unroll
         for (int mi = 0; mi < MI; mi++) {
 #pragma unroll
             for (int e = 0; e < 16; e++) {
-                const int slot = seg_ids[mi * 32 + 8 * (e >> 2) + 4 * khalf + (e & 3)];
-                if (slot < gp.ns) {
+                const int r = mi * 32 + 8 * (e >> 2) + 4 * khalf + (e & 3);
+                if (MODE == 1) {
                     const float gt = (float)(_Float16)(acc[mi][0][e] * unit[0]), up = (float)(_Float16)(acc[mi][1][e] * unit[1]);
-                    reinterpret_cast<_Float16*>(y)[(size_t)slot * n_ff + col] = (_Float16)w4_act_mul(gt, up, gp.act_kind);
-                }
-            }
-        }
-        return;
-    }
-    if (MODE == 2) {
+                    tile[r * LD + nl] = (_Float16)w4_act_mul(gt, up, gp.act_kind);
+                } else {
+                    const float w = seg_w[r];
 #pragma unroll
-        for (int ni = 0; ni < 2; ni++) {
-            const int col = n0 + wn * 64 + ni * 32 + nl;
-            if (col >= n) continue;
-#pragma unroll
-            for (int mi = 0; mi < MI; mi++) {
-#pragma unroll
-                for (int e = 0; e < 16; e++) {
-                    const int slot = seg_ids[mi * 32 + 8 * (e >> 2) + 4 * khalf + (e & 3)];
-                    if (slot < gp.ns) {
-                        float v = acc[mi][ni][e] * unit[ni];
-                        if (gp.topw != nullptr) v *= gp.topw[slot];
-                        if (out_f16)
-                            reinterpret_cast<_Float16*>(y)[(size_t)slot * n + col] = (_Float16)v;
-                        else
-                            reinterpret_cast<float*>(y)[(size_t)slot * n + col] = v;
+                    for (int ni = 0; ni < 2; ni++) {
+                        float v = acc[mi][ni][e] * unit[ni] * w;
+                        asm volatile("" : "+v"(v));  // the product is rounded to f32 before the f16 conversion
+                        tile[r * LD + ni * 32 + nl] = (_Float16)v;
                     }
                 }
             }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+#pragma unroll
+        for (int i = 0; i < PF_BM * PER_ROW / 64; i++) {
+            const int r = i * (64 / PER_ROW) + lane / PER_ROW, piece = lane % PER_ROW, slot = seg_ids[r];
+            const u4_t v = *reinterpret_cast<const u4_t*>(tile + r * LD + piece * 8);
+            if (slot < gp.ns) *reinterpret_cast<u4_t*>(reinterpret_cast<_Float16*>(y) + (size_t)slot * n_out + col + piece * 8) = v;
         }
         return;
     }
@@ -465,9 +467,27 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
         prefill_body<G, SBF, MI, 3>(qt, st, x, y, row_blocks, k, n, t, out_f16, sup_m, sup_n, gp, epi);                \
     }
 
+// Block tile of a grouped workgroup.  Every XCD (block b runs on XCD b % 8) takes an eighth of the live 64-slot segments in
+// order, column tiles fastest, so that the segments of one expert's run fetch its weights, and the column tiles of a segment
+// its x rows, into one L2 at about the same time (128 experts, T = 2048: -3 %).  Gate|up tiles span 128 gate and the 128
+// matching up columns.  A segment whose second half is padding (its slots are a prefix of it) runs the 32-row body: an expert's
+// last segment is partly filled (T = 1536 246 -> 225 us per FFN, T = 2048 284 -> 264).
+template <int MODE>
+__device__ __forceinline__ bool pf_moe_tile(PfGroup<MODE>& gp, const int* num_post, int n, int* rows) {
+    const int tiles = MODE == 1 ? ((n >> 1) + PF_BN / 2 - 1) / (PF_BN / 2) : (n + PF_BN - 1) / PF_BN;
+    const int segs = num_post[0] / 64, xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+    const int seg = segs * xcd / 8 + j / tiles;
+    if (seg >= segs * (xcd + 1) / 8) return false;
+    gp.m0 = seg * 64;
+    gp.n0 = (j % tiles) * (MODE == 1 ? PF_BN / 2 : PF_BN);
+    gp.expert = gp.expert_ids[seg];
+    *rows = gp.sorted_ids[gp.m0 + 32] < gp.ns ? 64 : 32;
+    return (unsigned)gp.expert < (unsigned)gp.n_exp;
+}
+
 // Grouped kernels for the expert FFN: same arguments as the streaming grouped kernels of moe.hip (blk must be 64, the
 // rows of a block tile; wpb is unused).
-#define PREFILL_MOE_KERNEL(NAME, G, SBF, MODE)                                                                          \
+#define PREFILL_MOE_KERNEL(NAME, G, SBF, MODE)                                                                        \
     extern "C" __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(3, 3))) void NAME(            \
         const char* qa, const char* sa, unsigned long long q_stride, unsigned long long s_stride, const uint16_t* x,      \
         int x_rows, int x_div, void* y, int y_f16, const float* topw, const int* sorted_ids, const int* expert_ids,      \
@@ -485,8 +505,12 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
         gp.n_exp = n_exp;                                                                                                \
         gp.act_kind = act_kind;                                                                                          \
         (void)blk, (void)wpb;                                                                   \
-        prefill_body<G, SBF, 2, MODE>(reinterpret_cast<const u4_t*>(qa), reinterpret_cast<const uint16_t*>(sa), x, y,    \
-                                      row_blocks, k, n, 0, y_f16, 1, 1, gp);                                             \
+        int rows;                                                                                                        \
+        if (!pf_moe_tile<MODE>(gp, num_post, n, &rows)) return;                                                          \
+        const u4_t* qt = reinterpret_cast<const u4_t*>(qa);                                                              \
+        const uint16_t* st = reinterpret_cast<const uint16_t*>(sa);                                                      \
+        if (rows <= 32) prefill_body<G, SBF, 1, MODE>(qt, st, x, y, row_blocks, k, n, 0, y_f16, 1, 1, gp);         \
+        else prefill_body<G, SBF, 2, MODE>(qt, st, x, y, row_blocks, k, n, 0, y_f16, 1, 1, gp);                    \
     }
 
 // This file builds two code objects.  Compiled on its own it holds everything but the dense group-128 kernels;
