@@ -55,12 +55,15 @@ static const char* const kLayoutSyms[] = {"w4a16_tile_q",         "w4a16_tile_s"
 static const char* const kDecodeSyms[] = {W4_DECODE_SCALES("w4a16_decode_g128_f16"), W4_DECODE_SCALES("w4a16_decode_g128_bf16"),
                                           W4_DECODE_SCALES("w4a16_decode_g32_f16"), W4_DECODE_SCALES("w4a16_decode_g32_bf16"),
                                           nullptr};
+#define W4_PREFILL_KG(P) P "_m64_n2k4", P "_m64_n3k4", P "_m64_n2k4_glu", P "_m64_n3k4_glu"
 static const char* const kPrefillG128Syms[] = {
+    W4_PREFILL_KG("w4a16_prefill_g128_f16"), W4_PREFILL_KG("w4a16_prefill_g128_bf16"),
     "w4a16_prefill_g128_f16", "w4a16_prefill_g128_bf16", "w4a16_prefill_g128_f16_m64", "w4a16_prefill_g128_bf16_m64",
     "w4a16_prefill_g128_f16_m96", "w4a16_prefill_g128_bf16_m96", "w4a16_prefill_g128_f16_glu", "w4a16_prefill_g128_bf16_glu",
     "w4a16_prefill_g128_f16_m64_glu", "w4a16_prefill_g128_bf16_m64_glu", "w4a16_prefill_g128_f16_m96_glu",
     "w4a16_prefill_g128_bf16_m96_glu", nullptr};
-static const char* const kPrefillSyms[] = {"w4a16_prefill_g32_f16", "w4a16_prefill_g32_bf16", "w4a16_prefill_g32_f16_m64",
+static const char* const kPrefillSyms[] = {W4_PREFILL_KG("w4a16_prefill_g32_f16"), W4_PREFILL_KG("w4a16_prefill_g32_bf16"),
+                                           "w4a16_prefill_g32_f16", "w4a16_prefill_g32_bf16", "w4a16_prefill_g32_f16_m64",
                                            "w4a16_prefill_g32_bf16_m64", "w4a16_prefill_splitk_sum", "w4a16_prefill_splitk_finish",
                                            "w4a16_prefill_g32_f16_glu", "w4a16_prefill_g32_bf16_glu",
                                            "w4a16_prefill_g32_f16_m64_glu", "w4a16_prefill_g32_bf16_m64_glu",

@@ -417,32 +417,34 @@ struct PrefillSuper {
 struct PrefillPlan {
     size_t bm, nks;
     PrefillSuper sup;
-    double us;  // the price it won with
+    double us;       // the price it won with
+    size_t wnw = 0;  // 2 or 3: the k-group build with 64 * wnw columns per block tile; 0: the 256-column tiles
 };
+
+// Super-tile shape for a grid of tiles_m x tiles_n block tiles: sup_m <= 8 along m, sup_n in {8, 4, 2, 1} along n.
+// Super-tiles are dealt round-robin to the 8 XCDs (m fastest), so every candidate is priced by the block tiles its
+// busiest XCD ends up with — counted exactly, partial super-tiles at the edges included — and the shape with the
+// lightest busiest XCD wins, the larger one on ties for L2 reuse.  (A fixed 8 along m left 10 tile rows as 8 + 2:
+// the XCDs that drew the 2-row super-tiles idled, 298 against 227 us on the down projection at t = 1280.)
+static PrefillSuper prefill_super(size_t tiles_m, size_t tiles_n) {
+    PrefillSuper best{std::min<size_t>(8, tiles_m), 8, 0, ~(size_t)0};
+    for (size_t cm = std::min<size_t>(8, tiles_m); cm >= 1; cm--) {
+        for (size_t cn : {8, 4, 2, 1}) {
+            const size_t sm = (tiles_m + cm - 1) / cm, sn = (tiles_n + cn - 1) / cn, sp = sm * sn;
+            size_t per_xcd[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+            for (size_t sidx = 0; sidx < sp; sidx++)
+                per_xcd[sidx & 7] += std::min(cm, tiles_m - (sidx % sm) * cm) * std::min(cn, tiles_n - (sidx / sm) * cn);
+            const size_t load = *std::max_element(per_xcd, per_xcd + 8);
+            if (load < best.load || (load == best.load && cm * cn > best.sup_m * best.sup_n)) best = PrefillSuper{cm, cn, sp, load};
+        }
+    }
+    return best;
+}
 
 static PrefillPlan plan_prefill(size_t t, size_t n, size_t k, size_t group, size_t cus, int tile_m_forced, int ksplit_forced,
                                 bool glu = false) {
     // a gated launch tiles the n/2 output columns by 128 (each block tile holds the matching 128 up columns as well)
     const size_t tiles_n = glu ? (n / 2 + kW4PfBn / 2 - 1) / (kW4PfBn / 2) : (n + kW4PfBn - 1) / kW4PfBn, kt_n = k / 128;
-    // Super-tile shape for a grid of tiles_m x tiles_n block tiles: sup_m <= 8 along m, sup_n in {8, 4, 2, 1} along n.
-    // Super-tiles are dealt round-robin to the 8 XCDs (m fastest), so every candidate is priced by the block tiles its
-    // busiest XCD ends up with — counted exactly, partial super-tiles at the edges included — and the shape with the
-    // lightest busiest XCD wins, the larger one on ties for L2 reuse.  (A fixed 8 along m left 10 tile rows as 8 + 2:
-    // the XCDs that drew the 2-row super-tiles idled, 298 against 227 us on the down projection at t = 1280.)
-    auto super_for = [&](size_t tiles_m) {
-        PrefillSuper best{std::min<size_t>(8, tiles_m), 8, 0, ~(size_t)0};
-        for (size_t cm = std::min<size_t>(8, tiles_m); cm >= 1; cm--) {
-            for (size_t cn : {8, 4, 2, 1}) {
-                const size_t sm = (tiles_m + cm - 1) / cm, sn = (tiles_n + cn - 1) / cn, sp = sm * sn;
-                size_t per_xcd[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-                for (size_t sidx = 0; sidx < sp; sidx++)
-                    per_xcd[sidx & 7] += std::min(cm, tiles_m - (sidx % sm) * cm) * std::min(cn, tiles_n - (sidx / sm) * cn);
-                const size_t load = *std::max_element(per_xcd, per_xcd + 8);
-                if (load < best.load || (load == best.load && cm * cn > best.sup_m * best.sup_n)) best = PrefillSuper{cm, cn, sp, load};
-            }
-        }
-        return best;
-    };
     // Price of a launch in microseconds, from measurements on MI355X (grids of exactly 256 x j workgroups of each tile,
     // k = 17408 and 5120).  A CU holds c workgroups at once (3 of the 64-row tile, 2 of the 128-row tile); j workgroups
     // per CU (of the busiest XCD) run as floor(j / c) full generations, `full` microseconds per k tile each, and a last
@@ -478,7 +480,7 @@ static PrefillPlan plan_prefill(size_t t, size_t n, size_t k, size_t group, size
         if (tile_m_forced && (size_t)tile_m_forced != rows) continue;
         if (rows == 96 && group != 128 && !tile_m_forced) continue;  // the group-32 builds of that tile spill: only when pinned
         const size_t tiles_m = (t + rows - 1) / rows;
-        const PrefillSuper sup = super_for(tiles_m);
+        const PrefillSuper sup = prefill_super(tiles_m, tiles_n);
         const size_t forced = ksplit_forced > 0 ? std::max<size_t>(1, std::min<size_t>((size_t)ksplit_forced, kt_n / 4)) : 0;
         for (size_t cand : {1, 2, 3, 4, 6, 8}) {
             const size_t nks = forced ? forced : cand;  // a pinned slice count is the only candidate
@@ -491,6 +493,35 @@ static PrefillPlan plan_prefill(size_t t, size_t n, size_t k, size_t group, size
             if (nks > 1) us += 6.0 + (double)nks * (double)t * (double)n * 8.0 / 9.76e6;
             if (us < best.us) best = PrefillPlan{rows, nks, sup, us};
         }
+    }
+    return best;
+}
+
+// Narrow outputs at a few dozen to some hundred rows: a workgroup of the 64-row tile over 128 or 192 columns whose waves also
+// form four k groups (kernels/prefill.hip, _n2k4 / _n3k4).  It fills a CU by itself without partial sums in memory, a second
+// launch or a workspace, but keeps only 8 or 12 waves there, so it is a candidate only where the grid is one generation (a block
+// tile per CU at most; beyond that it loses: 5120 x 5120 t = 450 over 128 columns 48 us, 46 for the plan above).  Both sides
+// measured with weights from memory, 1489 shapes per group size (15 widths 512..22016, k = 640..11008, t = 17..1500), the plan
+// above / this one in us: group 128 5120 x 5120 t = 300 34.7 / 28.3, 7168 x 5120 t = 300 48.0 / 33.5 (192 columns), 4096 x 2048
+// t = 300 24.5 / 13.6, 1024 x 640 t = 100 13.8 / 7.9, group 32 5120 x 2048 t = 300 31.9 / 17.3; not chosen: 5120 x 5120 t = 65
+// 22.7 / 23.7, 5120 x 17408 t = 128 43 / 74.
+// The price (fitted to the same sweep, 5 % rms): a fixed cost and one per k tile of a group's run, each growing with the part
+// of the chip in use.  The other plan's price is corrected before the two are compared, so that the choice is level or gains
+// at every shape of the sweep (2 %, the noise): + 3 us where its k range is whole (its fixed cost is low by 3..5 us at short k),
+// x 0.72 for up to four slices of up to four k tiles (they overlap better than priced), x 0.88 otherwise at group 128, whose
+// constants it was fitted with, 0.98 at group 32.  -13 % on average over the sweep; 1.6 % above the best choice for each shape.
+static PrefillPlan plan_prefill_groups(const PrefillPlan& tiles, size_t t, size_t n, size_t k, size_t group, size_t cus) {
+    static const double price[2][2][4] = {{{4.6, 1.86, 1.0, 0.39}, {5.45, 2.13, 1.28, 0.65}},  // group 128: 128, 192 columns
+                                          {{4.7, 2.53, 1.1, 0.27}, {5.4, 3.16, 1.4, 0.44}}};    // group 32
+    const size_t kt_n = k / 128, tiles_m = (t + 63) / 64, run = (kt_n + 3) / 4;
+    PrefillPlan best = tiles;
+    double us = tiles.nks == 1 ? tiles.us + 3.0 : tiles.us * (tiles.nks <= 4 && (kt_n + tiles.nks - 1) / tiles.nks <= 4 ? 0.72 : group == 32 ? 0.98 : 0.88);
+    for (size_t w : {2, 3}) {
+        const size_t tiles_n = (n + 64 * w - 1) / (64 * w);  // gated: as many pairs of 32 w gate and up columns
+        if (tiles_m * tiles_n > cus) continue;
+        const double* c = price[group == 32][w - 2];
+        const double full = (double)(tiles_m * tiles_n) / (double)cus, p = c[0] + c[2] * full + (c[1] + c[3] * full) * (double)run;
+        if (p < us) us = p, best = PrefillPlan{64, 1, prefill_super(tiles_m, tiles_n), p, w};
     }
     return best;
 }
@@ -567,25 +598,31 @@ static int launch_prefill(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_t y
         const auto key = std::make_tuple(t, L.n, L.k, ctx->prefill_tile_m + (glu ? 1000 : 0), ksplit);
         const auto hit = ctx->prefill_plans.find(key);
         if (hit != ctx->prefill_plans.end()) {
-            plan = PrefillPlan{hit->second[0], hit->second[1], PrefillSuper{hit->second[2], hit->second[3], hit->second[4], 0}, 0.0};
+            plan = PrefillPlan{hit->second[0], hit->second[1], PrefillSuper{hit->second[2], hit->second[3], hit->second[4], 0}, 0.0, hit->second[5]};
         } else {
             plan = plan_prefill(t, L.n, L.k, L.group, (size_t)std::max(ctx->cu_count, 1), ctx->prefill_tile_m, ksplit, glu);
-            ctx->prefill_plans[key] = {plan.bm, plan.nks, plan.sup.sup_m, plan.sup.sup_n, plan.sup.supers};
+            if (ctx->prefill_tile_m == 0 && ctx->prefill_ksplit == 0)  // a pinned tile or slice count names the 256-column tiles
+                plan = plan_prefill_groups(plan, t, L.n, L.k, L.group, (size_t)std::max(ctx->cu_count, 1));
+            ctx->prefill_plans[key] = {plan.bm, plan.nks, plan.sup.sup_m, plan.sup.sup_n, plan.sup.supers, plan.wnw};
         }
     }
     const size_t bm = plan.bm, nks = plan.nks, sup_m = plan.sup.sup_m, sup_n = plan.sup.sup_n, supers = plan.sup.supers;
     const size_t grid = ((supers + 7) / 8) * (sup_m * sup_n) * 8;
     char sym[64];
-    snprintf(sym, sizeof sym, "w4a16_prefill_g%zu_%s%s%s", L.group, L.scale_bf16 ? "bf16" : "f16", bm == 64 ? "_m64" : bm == 96 ? "_m96" : "", glu ? "_glu" : "");
-    // two stages of bm rows x PF_KS halves (the 96-row tile: half of that), then bm words (row factors)
-    const unsigned shmem = (unsigned)(2 * bm * (bm == 96 ? kW4PfKs / 2 : kW4PfKs) * 2 + bm * 4);
+    snprintf(sym, sizeof sym, "w4a16_prefill_g%zu_%s%s%s%s", L.group, L.scale_bf16 ? "bf16" : "f16", bm == 64 ? "_m64" : bm == 96 ? "_m96" : "",
+             plan.wnw == 2 ? "_n2k4" : plan.wnw == 3 ? "_n3k4" : "", glu ? "_glu" : "");
+    // two stages of bm rows x PF_KS halves (the 96-row tile: half of that), then a word per thread (row factors); k groups: two
+    // stages each, overlaid by the sums they hand over (12 shares of a wave's four 1 KiB tiles per 64 columns)
+    const size_t stages = 2 * bm * (bm == 96 ? kW4PfKs / 2 : kW4PfKs) * 2;
+    const unsigned threads = plan.wnw ? (unsigned)(plan.wnw * 256) : kW4PfThreads;
+    const unsigned shmem = (unsigned)(plan.wnw ? std::max<size_t>(4 * stages, plan.wnw * 12 * 4 * 1024) : stages) + threads * 4;
     uint64_t qt = L.q_tiled, st = L.s_tiled;
     int row_blocks = (int)L.row_blocks, ki = (int)L.k, ni = (int)L.n, ti = (int)t, of = (out_f16 || glu) ? 1 : 0;
     int spm = (int)sup_m, spn = (int)sup_n, act = glu ? glu_act : 0, glu_i = glu ? 1 : 0;
     if (nks == 1) {
         if (norm && epi.stats_out) norm->n_stats_out = ((size_t)epi.stat_cols + 63) / 64;  // one entry per wave's 64 columns
         void* params[] = {&qt, &st, &x, &y, &row_blocks, &ki, &ni, &ti, &of, &spm, &spn, &act, &epi};
-        return w4_launch(ctx, sym, (unsigned)grid, 1, kW4PfThreads, shmem, params);
+        return w4_launch(ctx, sym, (unsigned)grid, 1, threads, shmem, params);
     }
     if (L.n % (glu ? 8 : 4) != 0) return w4_fail(W4A16_ERR_UNSUPPORTED, "prefill: split-K needs n %% %d == 0", glu ? 8 : 4);
     const size_t count = t * L.n;

@@ -89,19 +89,22 @@ struct PfEpi {
     float inv_cols_in, in_scale, out_scale;
 };
 
-template <int G, bool SBF, int MI, int MODE = 0>
+template <int G, bool SBF, int MI, int MODE = 0, int WNW = 4, int KG = 1>
 __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const uint16_t* __restrict__ st,
                                              const uint16_t* __restrict__ x, void* __restrict__ y, int row_blocks,
                                              int k, int n, int t, int out_f16, int sup_m, int sup_n,
                                              const PfGroup<MODE> gp = PfGroup<MODE>(), const PfEpi epi = PfEpi()) {
-    extern __shared__ _Float16 lds[];  // 2 stages x [PF_BM][KS]; then per row: factors (dense) / slot ids, weights (grouped)
+    extern __shared__ _Float16 lds[];  // 2 stages x [PF_BM][KS]; then row factors, a word per thread (dense) / slot ids, weights (grouped)
     constexpr int GPT = W4_TILE_K / G;
+    constexpr int BN = 64 * WNW, GT = 64 * WNW;  // block tile columns, threads of a k group
     constexpr int PF_BM = 32 * MI, KS = MI == 3 ? PF_KS / 2 : PF_KS;
     constexpr int PF_STAGE_BYTES = PF_BM * KS * 2, CPR = KS / 8;  // 16-byte chunks per staged x row
-    constexpr int NA = PF_BM * CPR / PF_THREADS, SPT = W4_TILE_K / KS;  // x loads per thread and stage, stages per k tile
+    constexpr int NA = (PF_BM * CPR + GT - 1) / GT, SPT = W4_TILE_K / KS;  // x loads per thread and stage, stages per k tile
+    // LDS: per k group two stages of x, overlaid by what the groups hand over at the end; then a word per thread
+    constexpr int HAND = KG > 1 ? KG * (KG - 1) * WNW * MI * 2 * 1024 : 0, XB = KG * 2 * PF_STAGE_BYTES, LDS_ROWS_AT = XB > HAND ? XB : HAND;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wn = wave;  // 4 waves along n
+    const int wn = KG > 1 ? wave % WNW : wave, kg = KG > 1 ? wave / WNW : 0;
     const int kt_n = k / W4_TILE_K, kg_n = kt_n * GPT;
 
     // XCD-aware tile numbering.  Block b runs on XCD b % 8 and is the (b / 8)-th block of that XCD; consecutive
@@ -112,7 +115,7 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
     constexpr bool DENSE = MODE == 0 || MODE == 3, PAIRED = MODE == 1 || MODE == 3;  // PAIRED: gate and up columns per wave
     if (DENSE) {
         const int tiles_m = (t + PF_BM - 1) / PF_BM,
-                  tiles_n = MODE == 3 ? ((n >> 1) + PF_BN / 2 - 1) / (PF_BN / 2) : (n + PF_BN - 1) / PF_BN;
+                  tiles_n = MODE == 3 ? ((n >> 1) + BN / 2 - 1) / (BN / 2) : (n + BN - 1) / BN;
         const int sm_n = (tiles_m + sup_m - 1) / sup_m, sn_n = (tiles_n + sup_n - 1) / sup_n;
         const int per = sup_m * sup_n;
         const int j = blockIdx.x >> 3;
@@ -121,7 +124,7 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
         const int tm = (super % sm_n) * sup_m + within % sup_m, tn = (super / sm_n) * sup_n + within / sup_m;
         if (tm >= tiles_m || tn >= tiles_n) return;
         m0 = tm * PF_BM;
-        n0 = tn * (MODE == 3 ? PF_BN / 2 : PF_BN);
+        n0 = tn * (MODE == 3 ? BN / 2 : BN);
     } else {
         m0 = gp.m0;
         n0 = gp.n0;
@@ -144,7 +147,7 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
     unsigned xa_off[NA];
 #pragma unroll
     for (int i = 0; i < NA; i++) {
-        const int c = tid + i * PF_THREADS, row = c / CPR, kc = (c % CPR) ^ (row % CPR);
+        const int c = wn * 64 + lane + i * GT, row = c / CPR, kc = (c % CPR) ^ (row % CPR);
         if (DENSE) {
             xa_off[i] = (m0 + row < t) ? ((unsigned)(m0 + row) * ldx + (unsigned)kc * 8u) * 2u : W4_OOB;
         } else {
@@ -152,40 +155,48 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
             xa_off[i] = id < gp.ns ? ((unsigned)(id / gp.x_div) * (unsigned)k + (unsigned)kc * 8u) * 2u : W4_OOB;
         }
     }
-    int* const seg_ids = reinterpret_cast<int*>(lds_base + (DENSE ? 2 * PF_STAGE_BYTES : PF_MOE_IDS_AT));
+    int* const seg_ids = reinterpret_cast<int*>(lds_base + (DENSE ? LDS_ROWS_AT : PF_MOE_IDS_AT));
     float* const seg_w = reinterpret_cast<float*>(seg_ids + PF_BM);
     if (!DENSE && tid < PF_BM) {  // visible after the first barrier
         const int id = gp.sorted_ids[m0 + tid];
         seg_ids[tid] = id;
         if (MODE == 2) seg_w[tid] = gp.topw != nullptr && id < gp.ns ? gp.topw[id] : 1.0f;
     }
-    // Dense, input statistics given: the 1/rms factor of this block's PF_BM input rows, once, into the same LDS words
-    // (thread r < PF_BM owns row m0 + r: entries added in index order with eight loads in flight — the same bits on
-    // every run; consecutive threads read consecutive floats of an entry).  Read back in the epilogue.
-    float* const row_fac = reinterpret_cast<float*>(lds_base + 2 * PF_STAGE_BYTES);
-    if (DENSE && epi.stats_in != nullptr && tid < PF_BM) {
-        const int row = m0 + tid;
+    // Dense, input statistics given: the row factors of this block's PF_BM input rows, through a word per thread behind the
+    // stages.  The entries of a row are dealt to RP threads, eight loads in flight each, while the first stage of x and weights
+    // is on its way (one thread per row ahead of those loads: a chain of up to n / 512 loads in which nothing else runs); the
+    // thread of part 0 adds the parts after the first barrier and leaves the factor for the epilogue in its own word.  The
+    // order of the additions is fixed: the same bits on every run.
+    constexpr int RP = GT * KG / PF_BM;
+    float* const row_fac = reinterpret_cast<float*>(lds_base + LDS_ROWS_AT);
+    const bool has_stats = DENSE && epi.stats_in != nullptr;
+    auto sum_stats = [&]() {
+        const int row = tid % PF_BM, part = tid / PF_BM;
+        if (part >= RP) return;
+        const float* const sp = epi.stats_in + min(m0 + row, t - 1);
         float sum = 0.f;
-        if (row < t) {
-            const float* sp = epi.stats_in + row;
-            int e = 0;
-            for (; e + 8 <= epi.n_stats_in; e += 8) {
-                float v[8];
+        for (int e = part; e < epi.n_stats_in; e += 8 * RP) {
+            float v[8];
 #pragma unroll
-                for (int j = 0; j < 8; j++) v[j] = sp[(size_t)(e + j) * epi.ld_stats];
+            for (int j = 0; j < 8; j++) v[j] = sp[(size_t)min(e + j * RP, epi.n_stats_in - 1) * epi.ld_stats];
 #pragma unroll
-                for (int j = 0; j < 8; j++) sum += v[j];
-            }
-            for (; e < epi.n_stats_in; e++) sum += sp[(size_t)e * epi.ld_stats];
+            for (int j = 0; j < 8; j++) sum += e + j * RP < epi.n_stats_in ? v[j] : 0.f;
         }
+        row_fac[tid] = sum;
+    };
+    auto make_factor = [&]() {
+        float sum = row_fac[tid];
+#pragma unroll
+        for (int p = 1; p < RP; p++) sum += row_fac[p * PF_BM + tid];
         row_fac[tid] = (float)(1.0 / sqrt((double)sum * (double)epi.inv_cols_in + 1e-6)) * epi.in_scale;
-    }
+    };
     auto load_a = [&](int s, int buf) {
 #pragma unroll
         for (int i = 0; i < NA; i++)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                xr, (__attribute__((address_space(3))) void*)(lds_base + buf * PF_STAGE_BYTES + (i * PF_THREADS + wave * 64) * 16),
-                16, xa_off[i], s * (KS * 2), 0, 0);
+            if (PF_BM * CPR % GT == 0 || i * GT + wn * 64 < PF_BM * CPR)  // uniform for the wave
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    xr, (__attribute__((address_space(3))) void*)(lds_base + (kg * 2 + buf) * PF_STAGE_BYTES + (i * GT + wn * 64) * 16),
+                    16, xa_off[i], s * (KS * 2), 0, 0);
     };
 
     // ---- weights: lane (nl = l % 32, khalf = l / 32); per n sub-tile ni and half h one dwordx4 per k tile
@@ -226,23 +237,43 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
     const int a_row = nl;  // + mi * 32
     // split-K over gridDim.y (narrow outputs at moderate t, where the tile grid alone cannot fill the chip): this
     // block covers k tiles [kt_lo, kt_hi) and writes an f32 partial; a second launch adds the partials in order
-    const int kt_lo = DENSE ? (kt_n * (int)blockIdx.y) / (int)gridDim.y : 0,
-              kt_hi = DENSE ? (kt_n * ((int)blockIdx.y + 1)) / (int)gridDim.y : kt_n;
+    // KG > 1: the k range is dealt to the groups of the workgroup's waves instead, contiguous runs of equal length (the last
+    // shorter or empty); every group runs as many iterations, for the barriers, and skips those past its run
+    const int kt_a = DENSE && KG == 1 ? (kt_n * (int)blockIdx.y) / (int)gridDim.y : 0,
+              kt_b = DENSE && KG == 1 ? (kt_n * ((int)blockIdx.y + 1)) / (int)gridDim.y : kt_n;
+    const int per = (kt_b - kt_a + KG - 1) / KG;
+    const int kt_lo = kt_a + kg * per, kt_hi = KG > 1 ? min(kt_b, kt_lo + per) : kt_b;
     const int stages = SPT * kt_hi;
     constexpr bool PF_WAVE_PRIO = G == 128;  // wave priority over a stage's MFMAs (see the k loop)
 
-    load_a(SPT * kt_lo, 0);
-    load_b(bq, sc, kt_lo);
+    if (KG == 1 || kt_lo < kt_hi) {
+        load_a(SPT * kt_lo, 0);
+        load_b(bq, sc, kt_lo);
+    }
+    if (has_stats) sum_stats();
     __syncthreads();  // the compiler waits for the LDS DMA (vmcnt) ahead of the barrier
+    if (has_stats && tid < PF_BM) make_factor();  // read after the barriers of the k loop
+    if (KG > 1) {
+        // The first weights are waited for here: pending at the loop's head they make its first use wait, in every iteration,
+        // for as many loads as were just issued.
+#pragma unroll
+        for (int ni = 0; ni < 2; ni++) {
+#pragma unroll
+            for (int h = 0; h < 2; h++) asm volatile("" : "+v"(bq[ni][h]));
+#pragma unroll
+            for (int gi = 0; gi < GPT; gi++) asm volatile("" : "+v"(sc[ni][gi]));
+        }
+    }
 
-    for (int kt = kt_lo; kt < kt_hi; kt++) {
+    for (int kt = kt_lo; kt < kt_lo + per; kt++) {
 #pragma unroll
         for (int half = 0; half < SPT; half++) {
             const int s = kt * SPT + half;
             // stage s+1 goes into the buffer that stage s-1 was read from: every wave is past the barrier that ended it
             if (s + 1 < stages) load_a(s + 1, (s + 1 - SPT * kt_lo) & 1);
             if (half == 0 && kt + 1 < kt_hi) load_b(bqn, scn, kt + 1);
-            const _Float16* abuf = lds + ((s - SPT * kt_lo) & 1) * (PF_BM * KS) + a_row * KS;
+            const _Float16* abuf = lds + (kg * 2 + ((s - SPT * kt_lo) & 1)) * (PF_BM * KS) + a_row * KS;
+            if (KG == 1 || kt < kt_hi)  // uniform for the wave
 #pragma unroll
             for (int kbl = 0; kbl < KS / 16; kbl++) {
                 const int kb = half * (KS / 16) + kbl, w = kb >> 1, h = kb & 1;
@@ -278,6 +309,9 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
                 for (int mi = 0; mi < MI; mi++)
                     a[mi] = *reinterpret_cast<const h8_t*>(abuf + mi * 32 * KS + (((kbl * 2 + khalf) ^ (nl % CPR)) * 8));
                 const bool last128 = G == 128 && kb == 7;  // branch free: the last k tile multiplies by 1
+                // The next scales' arithmetic stays here: moved up by the scheduler it waits for loads just issued (the 64-row
+                // f16 build did so after the second MFMA: 2048 x 11008 t = 256 28.2 us instead of 26.2).
+                if (MI == 2 && last128) __builtin_amdgcn_sched_barrier(0x9c);  // SALU, MFMA and memory may cross, VALU may not
                 float next_ratio[2] = {1.f, 1.f};
                 if (last128) {
                     const bool more = kt + 1 < kt_hi;
@@ -316,7 +350,50 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
         }
     }
 
+    f4_t own[MI][2];  // KG > 1: the finished sums of this group's rows
+    if constexpr (KG > 1) {
+        // Add the groups' sums, in group order: group g takes rows 8g + 4 khalf ..+3 of every 32 (accumulator registers 4g..4g+3),
+        // gets them from the other groups through LDS and runs the epilogue for them.
+        static_assert(KG == 4, "a group's share is four accumulator registers");
+        f4_t* const hand = reinterpret_cast<f4_t*>(lds_base);  // [share][other group][wave along n][tile][lane]
+        auto at = [&](int share, int from) { return ((share * (KG - 1) + (from < share ? from : from - 1)) * WNW + wn) * (MI * 2 * 64) + lane; };
+#pragma unroll
+        for (int g = 0; g < KG; g++) {
+            if (g == kg) continue;
+#pragma unroll
+            for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+                for (int ni = 0; ni < 2; ni++) {
+                    const f4_t v = {acc[mi][ni][4 * g] * unit[ni], acc[mi][ni][4 * g + 1] * unit[ni], acc[mi][ni][4 * g + 2] * unit[ni],
+                                    acc[mi][ni][4 * g + 3] * unit[ni]};
+                    hand[at(g, kg) + (mi * 2 + ni) * 64] = v;
+                }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int g = 0; g < KG; g++) {
+            if (g != kg) continue;
+#pragma unroll
+            for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+                for (int ni = 0; ni < 2; ni++) {
+                    const f4_t mine = {acc[mi][ni][4 * g] * unit[ni], acc[mi][ni][4 * g + 1] * unit[ni], acc[mi][ni][4 * g + 2] * unit[ni],
+                                acc[mi][ni][4 * g + 3] * unit[ni]};
+                    f4_t sum;
+#pragma unroll
+                    for (int from = 0; from < KG; from++) {
+                        const f4_t v = from == g ? mine : hand[at(g, from) + (mi * 2 + ni) * 64];
+                        sum = from == 0 ? v : sum + v;
+                    }
+                    own[mi][ni] = sum;
+                }
+        }
+    }
+
     // ---- epilogue: y[m][n] = acc * unit; D register e of lane (nl, khalf) is row 8*(e/4) + 4*khalf + e%4, column nl
+    constexpr int NE = KG > 1 ? 4 : 16;  // registers of a 32-row tile that this wave finishes
+    auto value = [&](int mi, int ni, int e) { return KG > 1 ? own[mi][ni][e] : acc[mi][ni][e] * unit[ni]; };
+    auto row_of = [&](int mi, int e) { return m0 + mi * 32 + 8 * (KG > 1 ? kg : e >> 2) + 4 * khalf + (e & 3); };
     if (!DENSE) {
         // Grouped: the wave's f16 tile goes through its own part of the stages' LDS (free after the last barrier, a wave's LDS
         // operations run in order) and out in 16-byte pieces of whole row segments: one store per 1 KiB instead of 2 bytes per
@@ -355,20 +432,20 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
         return;
     }
     // x arrived as its true value times 1/in_scale and (with input statistics) un-normalised: one factor per row
-    const bool use_fac = DENSE && (epi.stats_in != nullptr || (epi.in_scale != 1.0f && epi.in_scale != 0.0f));
-    if (MODE == 3 && gridDim.y == 1) {
+    const bool use_fac = DENSE && (has_stats || (epi.in_scale != 1.0f && epi.in_scale != 0.0f));
+    if (MODE == 3 && (KG > 1 || gridDim.y == 1)) {
         const int n_ff = n >> 1, col = n0 + wn * 32 + nl;
         if (col >= n_ff) return;
 #pragma unroll
         for (int mi = 0; mi < MI; mi++) {
 #pragma unroll
-            for (int e = 0; e < 16; e++) {
-                const int row = m0 + mi * 32 + 8 * (e >> 2) + 4 * khalf + (e & 3);
+            for (int e = 0; e < NE; e++) {
+                const int row = row_of(mi, e);
                 if (row < t) {
-                    float gt = acc[mi][0][e] * unit[0], up = acc[mi][1][e] * unit[1];
+                    float gt = value(mi, 0, e), up = value(mi, 1, e);
                     asm volatile("" : "+v"(gt), "+v"(up));  // the sums are rounded to f32 as the separate launch stores them
                     if (use_fac) {
-                        const float f = epi.stats_in != nullptr ? row_fac[row - m0] : epi.in_scale;
+                        const float f = has_stats ? row_fac[row - m0] : epi.in_scale;
                         gt *= f;
                         up *= f;
                     }
@@ -384,7 +461,7 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
         }
         return;
     }
-    if (gridDim.y > 1) {  // partial (f32) of a split launch: w4a16_prefill_splitk_sum finishes (activation, epilogue options)
+    if (KG == 1 && gridDim.y > 1) {  // partial (f32) of a split launch: w4a16_prefill_splitk_sum finishes (activation, epilogue options)
         y = reinterpret_cast<float*>(y) + (size_t)blockIdx.y * (size_t)t * (size_t)n;
 #pragma unroll
         for (int ni = 0; ni < 2; ni++) {
@@ -404,45 +481,69 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
     // MODE 0, whole k range: y = acc * unit, then the optional parts in the order of the decode kernel's epilogue — row
     // factor, residual stream, statistics of what continues, norm weight, power-of-two hand-over factor
     const bool plain = !use_fac && epi.resid == nullptr && epi.stats_out == nullptr && epi.nw == nullptr && (epi.out_scale == 1.0f || epi.out_scale == 0.0f);
+    // The residual stream's values and norm weights are fetched ahead of the stores that the compiler may not move them across:
+    // a wait per four rows (k groups: one in all) instead of one per element.
+    int col[2];
+    float nwv[2] = {1.f, 1.f};
 #pragma unroll
-    for (int mi = 0; mi < MI; mi++) {
+    for (int ni = 0; ni < 2; ni++) {
+        col[ni] = n0 + wn * 64 + ni * 32 + nl;
+        if (epi.nw != nullptr) nwv[ni] = epi.nw[min(col[ni], n - 1)];
+    }
+    constexpr int MB = KG > 1 ? MI : 1;  // tiles per batch of four rows
 #pragma unroll
-        for (int e = 0; e < 16; e++) {
-            const int row = m0 + mi * 32 + 8 * (e >> 2) + 4 * khalf + (e & 3);
-            float p = 0.f;  // this lane's share of the row's sum of squares
-            if (row < t) {
-                const float f = !use_fac ? 1.0f : epi.stats_in != nullptr ? row_fac[row - m0] : epi.in_scale;
+    for (int mb = 0; mb < MI * NE; mb += 4 * MB) {
+        const int m_at = mb / NE, e_at = mb % NE;
+        float rv[MB][4][2];
+        if (epi.resid != nullptr) {
 #pragma unroll
-                for (int ni = 0; ni < 2; ni++) {
-                    const int col = n0 + wn * 64 + ni * 32 + nl;
-                    if (col >= n) continue;
-                    float v = acc[mi][ni][e] * unit[ni];
-                    if (!plain) {
-                        asm volatile("" : "+v"(v));
-                        if (use_fac) v *= f;
-                        if (epi.resid != nullptr) {
-                            float* const rp = epi.resid + (size_t)row * n + col;
-                            v += *rp;
-                            *rp = v;
+            for (int i = 0; i < MB; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+#pragma unroll
+                    for (int ni = 0; ni < 2; ni++)
+                        rv[i][e][ni] = epi.resid[(size_t)min(row_of(m_at + i, e_at + e), t - 1) * n + min(col[ni], n - 1)];
+        }
+#pragma unroll
+        for (int i = 0; i < MB; i++) {
+            const int mi = m_at + i;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int row = row_of(mi, e_at + e);
+                float p = 0.f;  // this lane's share of the row's sum of squares
+                if (row < t) {
+                    const float f = !use_fac ? 1.0f : has_stats ? row_fac[row - m0] : epi.in_scale;
+#pragma unroll
+                    for (int ni = 0; ni < 2; ni++) {
+                        if (col[ni] >= n) continue;
+                        const size_t at = (size_t)row * n + col[ni];
+                        float v = value(mi, ni, e_at + e);
+                        if (!plain) {
+                            asm volatile("" : "+v"(v));
+                            if (use_fac) v *= f;
+                            if (epi.resid != nullptr) {
+                                v += rv[i][e][ni];
+                                epi.resid[at] = v;
+                            }
+                            if (col[ni] < epi.stat_cols) p = __builtin_fmaf(v, v, p);
+                            if (epi.nw != nullptr) v *= nwv[ni];
+                            if (epi.out_scale != 1.0f && epi.out_scale != 0.0f) {
+                                v *= epi.out_scale;
+                                asm volatile("" : "+v"(v));  // rounded to f32 on its own, not fused into the f16 conversion
+                            }
                         }
-                        if (col < epi.stat_cols) p = __builtin_fmaf(v, v, p);
-                        if (epi.nw != nullptr) v *= epi.nw[col];
-                        if (epi.out_scale != 1.0f && epi.out_scale != 0.0f) {
-                            v *= epi.out_scale;
-                            asm volatile("" : "+v"(v));  // rounded to f32 on its own, not fused into the f16 conversion
-                        }
+                        if (out_f16)
+                            reinterpret_cast<_Float16*>(y)[at] = (_Float16)v;
+                        else
+                            reinterpret_cast<float*>(y)[at] = v;
                     }
-                    if (out_f16)
-                        reinterpret_cast<_Float16*>(y)[(size_t)row * n + col] = (_Float16)v;
-                    else
-                        reinterpret_cast<float*>(y)[(size_t)row * n + col] = v;
                 }
-            }
-            if (epi.stats_out != nullptr) {  // uniform: the 32 lanes of a row (same khalf) add up in a fixed order
+                if (epi.stats_out != nullptr) {  // uniform: the 32 lanes of a row (same khalf) add up in a fixed order
 #pragma unroll
-                for (int off = 16; off > 0; off >>= 1) p += __shfl_xor(p, off);
-                if (nl == 0 && row < t && n0 + wn * 64 < epi.stat_cols)
-                    epi.stats_out[(size_t)((n0 + wn * 64) >> 6) * epi.ld_stats + row] = p;
+                    for (int off = 16; off > 0; off >>= 1) p += __shfl_xor(p, off);
+                    if (nl == 0 && row < t && n0 + wn * 64 < epi.stat_cols)
+                        epi.stats_out[(size_t)((n0 + wn * 64) >> 6) * epi.ld_stats + row] = p;
+                }
             }
         }
     }
@@ -485,6 +586,28 @@ __device__ __forceinline__ bool pf_moe_tile(PfGroup<MODE>& gp, const int* num_po
     return (unsigned)gp.expert < (unsigned)gp.n_exp;
 }
 
+// k-group kernels, for outputs too narrow to fill the chip with 256-column tiles: 64 rows x 64 WNW columns, WNW waves along n times
+// four k groups in one workgroup (8 or 12 waves, 128 or 144 KiB of LDS: one workgroup per CU).  What bounds these launches is
+// not the matrix pipe but a chain per k tile (x by DMA, barrier, 16 MFMAs a wave) too few waves are there to hide, plus, when
+// k slices filled the chip instead, writing the slices' f32 sums to memory and a second launch that adds them.  Here each group
+// walks a quarter of k with x stages of its own, the groups' sums meet in LDS in group order (same bits on every run), and each
+// group runs the epilogue, options included, for a quarter of the rows.  5120 x 5120 t = 300 34.7 -> 28.3 us (200
+// workgroups instead of 400 and a second launch), 4096 x 2048 t = 300 24.5 -> 13.6, group 32 5120 x 2048 t = 300 31.9 -> 17.3.
+// One wave along n (64 columns) needs twice the waves for the same x traffic and won 0.3 % over the range: not built.
+#define PREFILL_KG_KERNEL(NAME, G, SBF, WNW, MODE)                                                                    \
+    extern "C" __global__ __launch_bounds__(64 * WNW * 4) __attribute__((amdgpu_waves_per_eu(WNW, WNW))) void NAME(       \
+        const u4_t* qt, const uint16_t* st, const uint16_t* x, void* y, int row_blocks, int k, int n, int t,          \
+        int out_f16, int sup_m, int sup_n, int act_kind, PfEpi epi) {                                                  \
+        PfGroup<MODE> gp;                                                                                              \
+        gp.act_kind = act_kind;                                                                                        \
+        prefill_body<G, SBF, 2, MODE, WNW, 4>(qt, st, x, y, row_blocks, k, n, t, out_f16, sup_m, sup_n, gp, epi);      \
+    }
+#define PREFILL_KG_FAMILY(PFX, G, SBF)                    \
+    PREFILL_KG_KERNEL(PFX##_m64_n2k4, G, SBF, 2, 0)       \
+    PREFILL_KG_KERNEL(PFX##_m64_n3k4, G, SBF, 3, 0)       \
+    PREFILL_KG_KERNEL(PFX##_m64_n2k4_glu, G, SBF, 2, 3)   \
+    PREFILL_KG_KERNEL(PFX##_m64_n3k4_glu, G, SBF, 3, 3)
+
 // Grouped kernels for the expert FFN: same arguments as the streaming grouped kernels of moe.hip (blk must be 64, the
 // rows of a block tile; wpb is unused).
 #define PREFILL_MOE_KERNEL(NAME, G, SBF, MODE)                                                                        \
@@ -514,7 +637,7 @@ __device__ __forceinline__ bool pf_moe_tile(PfGroup<MODE>& gp, const int* num_po
     }
 
 // This file builds two code objects.  Compiled on its own it holds everything but the dense group-128 kernels;
-// prefill_g128.hip includes it with PF_DENSE_G128 defined and holds those twelve, built with the backend's max-ILP
+// prefill_g128.hip includes it with PF_DENSE_G128 defined and holds those (the k-group ones as well), built with the backend's max-ILP
 // instruction scheduler (5120 x 34816 at M = 4096: 1.204 -> 1.193 ms, the other layer shapes -0.2...-0.6 %; the
 // group-32 builds spill registers under that scheduler and keep the default).
 #ifdef PF_DENSE_G128
@@ -530,6 +653,8 @@ PREFILL_GLU_KERNEL(w4a16_prefill_g128_f16_m64_glu, 128, false, 2, 3)
 PREFILL_GLU_KERNEL(w4a16_prefill_g128_bf16_m64_glu, 128, true, 2, 3)
 PREFILL_GLU_KERNEL(w4a16_prefill_g128_f16_m96_glu, 128, false, 3, 3)
 PREFILL_GLU_KERNEL(w4a16_prefill_g128_bf16_m96_glu, 128, true, 3, 3)
+PREFILL_KG_FAMILY(w4a16_prefill_g128_f16, 128, false)
+PREFILL_KG_FAMILY(w4a16_prefill_g128_bf16, 128, true)
 #else
 // y[i] = sum over the nks partials of a split-K launch, added in split order in f32; f32 or f16 out.
 // glu != 0: the partials are those of a fused gate|up linear, [slices][t][n]; y is f16 [t][n/2] = act(g) * u on the
@@ -639,6 +764,8 @@ PREFILL_GLU_KERNEL(w4a16_prefill_g32_f16_m64_glu, 32, false, 2, 3)
 PREFILL_GLU_KERNEL(w4a16_prefill_g32_bf16_m64_glu, 32, true, 2, 3)
 PREFILL_GLU_KERNEL(w4a16_prefill_g32_f16_m96_glu, 32, false, 3, 3)
 PREFILL_GLU_KERNEL(w4a16_prefill_g32_bf16_m96_glu, 32, true, 3, 3)
+PREFILL_KG_FAMILY(w4a16_prefill_g32_f16, 32, false)
+PREFILL_KG_FAMILY(w4a16_prefill_g32_bf16, 32, true)
 PREFILL_MOE_KERNEL(w4a16_moe_g128_f16_pf_glu, 128, false, 1)
 PREFILL_MOE_KERNEL(w4a16_moe_g128_f16_pf_lin, 128, false, 2)
 PREFILL_MOE_KERNEL(w4a16_moe_g128_bf16_pf_glu, 128, true, 1)
