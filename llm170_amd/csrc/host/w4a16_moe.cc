@@ -327,8 +327,10 @@ int w4_dense_mid(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_t y, size_t 
     if (!L.q_tiled) return w4_fail(W4A16_ERR_UNSUPPORTED, "stream: linear has no tiled copy (needs k %% 128 == 0)");
     if (t > 0x7fffffffu / 2) return w4_fail(W4A16_ERR_SHAPE, "stream: t=%zu too large", t);
     if (glu && L.n % 32 != 0) return w4_fail(W4A16_ERR_SHAPE, "stream glu: n=%zu must be a multiple of 32", L.n);
-    if (t * L.k * 2 >= 0x80000000ull || L.row_blocks * (L.k / 128) * 1024 >= 0x80000000ull)
-        return w4_fail(W4A16_ERR_SHAPE, "stream: x or the tiled weights reach 2 GiB, beyond the buffer-descriptor range");
+    // x is switched off row by row with an offset of 2 GiB; weights only by an empty descriptor, so they may fill all of its range
+    if (t * L.k * 2 >= 0x80000000ull) return w4_fail(W4A16_ERR_SHAPE, "stream: x reaches 2 GiB, beyond the buffer-descriptor range");
+    if (L.row_blocks * (L.k / 128) * 1024 > 0xffffffffull)
+        return w4_fail(W4A16_ERR_SHAPE, "stream: tiled weights of 4 GiB or more exceed the buffer-descriptor range");
     const size_t units = glu ? L.row_blocks / 2 : (L.row_blocks + 1) / 2, cus = (size_t)std::max(ctx->cu_count, 1);
     const size_t tt = t <= 32 ? 2 : t <= 48 ? 3 : 4, segs = (t + 16 * tt - 1) / (16 * tt);
     const MidPlan P = plan_mid(units, L.k / 128, t, cus, ctx->decode_ksplit, !glu);

@@ -120,3 +120,25 @@ def test_pinned_slices_agree_with_slice_launches(dec):
     finally:
         dec.set_decode_ksplit(0)
     assert np.array_equal(got, want.view(np.uint32))
+
+
+def test_weights_between_2_and_4_gib(dec):
+    """Offsets into the tiled weights are unsigned 32-bit: rows on both sides of 2 GiB, and the last, against float64.
+    Bound: f32 sums of k terms err by less than k * 2^-24 of the sum of the terms' magnitudes, far more than they do."""
+    n, k, t, rng = 131088, 33024, 20, np.random.default_rng(85)
+    q = np.tile(rng.integers(0, 2**32, (n // 16, k // 8), dtype=np.uint32), (16, 1))
+    q[::16, 0] = np.arange(n // 16, dtype=np.uint32)  # rows of the copies differ
+    s = np.tile(rng.uniform(0.002, 0.02, (n // 16, k // 128)).astype(np.float16), (16, 1)).view(np.uint16)
+    x = rng.standard_normal((t, k)).astype(np.float16)
+    dec.upload_lin_g("mid2g", q, s, n, k, 128, False)
+    mark = 2**31 // (k // 2)
+    rows = np.r_[0:16, mark - 32:mark + 32, n - 48:n]
+    w = ((q[rows][:, :, None] >> (4 * np.arange(8, dtype=np.uint32))) & 15).reshape(len(rows), k).astype(np.float64) - 8
+    w *= np.repeat(s[rows].view(np.float16).astype(np.float64), 128, axis=1)
+    got, sym = _run(dec, x.view(np.uint16), n, t, t * n, lambda xd, yd: dec.lin_forward("mid2g", xd, yd, t))
+    dec.upload_lin_g("mid2g", q[:16], s[:16], 16, k, 128, False)  # the big copy is freed
+    assert sym.startswith("w4a16_mid_g128_f16_t2_")
+    y = got.view(np.float32).reshape(t, n)[:, rows]
+    bound = k * 2.0**-24 * (np.abs(x.astype(np.float64)) @ np.abs(w).T)
+    assert np.all(np.abs(y - x.astype(np.float64) @ w.T) <= bound)
+    assert np.all(y != 0)
