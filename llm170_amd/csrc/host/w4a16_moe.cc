@@ -291,13 +291,16 @@ static int launch_moe_gemm(w4a16_ctx* ctx, const W4Experts& E, bool glu, uint64_
 //     units (gated 34816 x 5120 t = 64: five waves 34.5, four 49.2; 28672 x 4096: four 22.3, five 26.4; 22016 x 4096: three
 //     19.3, four 21.3; 16384 x 4096: two 17.1, three 18.6); a long k over little more units than CUs runs four slices
 //     (11008 x 17408 t = 64 54.9 -> 45.7).
+//   * more than 64 rows (scales the MFMA-tiled kernel cannot divide by): the units of all segments count, since k slices pay for
+//     workgroups the grid lacks and cost their workspace and hand-over where it has them (5120 x 17408 t = 512: 130 us in eight
+//     slices, 100 whole with x shared by five waves; t = 192: 53 whole, 49 in four slices; 1024 x 8192 t = 512 37 / 20).
 struct MidPlan {
     int wn = 1, wk = kW4MidParts;
     size_t nks = 1;
 };
 
-static MidPlan plan_mid(size_t units, size_t kt_n, size_t t, size_t cus, int ksplit, bool may_split) {
-    const size_t u = units * 256 / cus;  // per 256 CUs
+static MidPlan plan_mid(size_t units, size_t segs, size_t kt_n, size_t t, size_t cus, int ksplit, bool may_split) {
+    const size_t u = units * segs * 256 / cus;  // per 256 CUs
     MidPlan P;
     if (may_split && ksplit > 0) {
         P.nks = std::max<size_t>(1, std::min(std::min<size_t>((size_t)ksplit, kW4MoeMaxKsplit), kt_n / 2));
@@ -307,13 +310,13 @@ static MidPlan plan_mid(size_t units, size_t kt_n, size_t t, size_t cus, int ksp
         if (u <= 64 && kt_n >= 32) P.nks = kt_n >= 128 || (u <= 32 && kt_n >= 64 && t > 32) ? 8 : 4;
         else if (u > 64 && u <= 96 && kt_n >= 40 && kt_n <= 64) P.nks = 2;
         else if (u > 64 && u <= 256 && (kt_n > 64 || (kt_n == 64 && t > 32 && u <= 160))) P = MidPlan{4, 1, 8};
-        else if (u > 256 && u <= 352 && kt_n >= 86) P = MidPlan{4, 1, 4};
+        else if (u > 256 && (segs > 1 ? u <= 512 && kt_n >= 128 : u <= 352 && kt_n >= 86)) P = MidPlan{4, 1, 4};
         if (P.nks > 1) return P;
     }
     if (u <= 256) return P;
     double best = 1e30;
     for (const MidPlan& c : {MidPlan{2, 4, 1}, MidPlan{3, 4, 1}, MidPlan{4, 2, 1}, MidPlan{5, 2, 1}}) {
-        const size_t wgs = (units + (size_t)c.wn - 1) / (size_t)c.wn;
+        const size_t wgs = (units + (size_t)c.wn - 1) / (size_t)c.wn * segs;
         const double cost = (double)((wgs + cus - 1) / cus) * (c.wn + 1.2);
         if (cost < best) best = cost, P = c;
     }
@@ -333,7 +336,7 @@ int w4_dense_mid(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_t y, size_t 
         return w4_fail(W4A16_ERR_SHAPE, "stream: tiled weights of 4 GiB or more exceed the buffer-descriptor range");
     const size_t units = glu ? L.row_blocks / 2 : (L.row_blocks + 1) / 2, cus = (size_t)std::max(ctx->cu_count, 1);
     const size_t tt = t <= 32 ? 2 : t <= 48 ? 3 : 4, segs = (t + 16 * tt - 1) / (16 * tt);
-    const MidPlan P = plan_mid(units, L.k / 128, t, cus, ctx->decode_ksplit, !glu);
+    const MidPlan P = plan_mid(units, segs, L.k / 128, t, cus, ctx->decode_ksplit, !glu);
     const size_t wn = (size_t)P.wn, wk = (size_t)P.wk, groups = (units + wn - 1) / wn, blocks = groups * segs;
     uint64_t ws = 0, tk = 0;
     if (P.nks > 1) {  // partial tiles and per-wave tickets, shared with the decode kernel

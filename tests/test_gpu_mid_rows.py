@@ -70,8 +70,27 @@ def test_rows_beyond_a_segment(dec, t):
         want, _ = _run(dec, x, n, t, t * n, lambda xd, yd: dec.lin_forward("mid", xd, yd, t, path=ops.PATH_LANE))
         got, _ = _run(dec, x, n, t, t * n, lambda xd, yd: dec.lin_forward("mid", xd, yd, t, path=ops.PATH_STREAM))
         parity.assert_close(got.view(np.float32).reshape(t, n), want.view(np.float32).reshape(t, n), "segments t%d" % t)
-        one, _ = _run(dec, x, n, 64, 64 * n, lambda xd, yd: dec.lin_forward("mid", xd, yd, 64, path=ops.PATH_STREAM))
-        assert np.array_equal(one, got[:64 * n])  # a row's sums do not depend on the rows around it
+        # k whole, or in a given number of slices (which follows the size of the grid), a row's sums do not depend on the rows around it
+        try:
+            for nks in (-1, 4):
+                dec.set_decode_ksplit(nks)
+                got, _ = _run(dec, x, n, t, t * n, lambda xd, yd: dec.lin_forward("mid", xd, yd, t, path=ops.PATH_STREAM))
+                parity.assert_close(got.view(np.float32).reshape(t, n), want.view(np.float32).reshape(t, n), "segments t%d" % t)
+                one, _ = _run(dec, x, n, 64, 64 * n, lambda xd, yd: dec.lin_forward("mid", xd, yd, 64, path=ops.PATH_STREAM))
+                assert np.array_equal(one, got[:64 * n])
+        finally:
+            dec.set_decode_ksplit(0)
+
+
+def test_many_segments_stay_whole_along_k(dec):
+    """Slices of k are for a grid that does not fill the chip: ten segments do, and need no workspace."""
+    n, k, t = 4104, 8448, 640
+    q, s, x = gen.make_linear(n, k, 128, t, seed=86)
+    dec.upload_lin_g("mid", q, s, n, k, 128, False)
+    want, _ = _run(dec, x, n, t, t * n, lambda xd, yd: dec.lin_forward("mid", xd, yd, t, path=ops.PATH_LANE))
+    got, sym = _run(dec, x, n, t, t * n, lambda xd, yd: dec.lin_forward("mid", xd, yd, t, path=ops.PATH_STREAM))
+    assert sym.endswith("_t4_n3k4")
+    parity.assert_close(got.view(np.float32).reshape(t, n), want.view(np.float32).reshape(t, n), "ten segments")
 
 
 @pytest.mark.parametrize("n,k,group,build", [(64, 384, 32, "n1k4"), (16448, 640, 128, "n3k4"), (8256, 1408, 128, "n2k4"),
