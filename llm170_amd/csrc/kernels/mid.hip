@@ -17,8 +17,9 @@
 // Sums: a slice's k tiles are cut into MID_PARTS runs, each summed from zero and added in order.  WK groups take whole runs, so
 // every launch shape gives the same bits, and so do the gated and the plain launch and a slice of a split one.
 // Measured against the grouped expert kernel that served these rows before (us, before / now): gated 34816 x 5120 t = 64
-// 51.4 / 34.4, t = 32 34.1 / 26.2; gated 22016 x 4096 t = 64 30.3 / 19.3; 16384 x 4096 t = 40 22.4 / 14.0; 5120 x 5120 t = 64
-// 19.2 / 14.6; 5120 x 2048 group 32 t = 37 13.1 / 7.6; 17408 x 5120 t = 64 32.7 / 28.0; 512 x 17408 t = 40 20.7 / 11.2.
+// 49.8 / 34.7, t = 32 34.3 / 27.8; gated 22016 x 4096 t = 64 30.3 / 20.9; 16384 x 4096 t = 40 21.7 / 15.5; 5120 x 5120 t = 64
+// 18.6 / 14.5; 5120 x 2048 group 32 t = 37 12.8 / 7.1; 17408 x 5120 t = 64 35.8 / 24.9; 512 x 17408 t = 40 20.4 / 10.7.
+// (The full wait at the barriers costs the gated 34816 x 5120 at t = 64 1 us, the other shapes of the timing cases nothing.)
 #include "w4a16_common.hpp"
 
 #define MOE_LDX 136  // halves per staged x row: 128 + 8 padding (272-byte stride: 16-lane b128 reads hit all banks once)
@@ -206,7 +207,7 @@ __device__ __forceinline__ void mid_body(MID_PARAMS) {
         // barrier that ends them
         load_x(kt0, 0);
         load_w(stage[0], kt0);
-        __syncthreads();
+        w4_dma_barrier();
         for (int i0 = 0; i0 < iters; i0 += 2) {
 #pragma unroll
             for (int d = 0; d < 2; d++) {
@@ -216,7 +217,7 @@ __device__ __forceinline__ void mid_body(MID_PARAMS) {
                 __builtin_amdgcn_sched_barrier(0);
                 if (kt < kt1) compute(stage[d], d);
                 if (PPW > 1 && --left == 0 && done < PPW - 1) part_end();
-                __syncthreads();
+                w4_dma_barrier();
             }
         }
     } else {

@@ -611,7 +611,7 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
     // 75.6 -> 70.7, T = 517 117 -> 113; group 128 T = 64 74.9 -> 67.4, T = 517 111.5 -> 98.5).
     load_x(0, 0);
     load_w(stage[0], 0);
-    __syncthreads();
+    w4_dma_barrier();
     for (int kt0 = 0; kt0 < kt_n; kt0 += 2) {
 #pragma unroll
         for (int d = 0; d < 2; d++) {
@@ -626,7 +626,7 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
                 else compute(stage[d], d);
             }
             __builtin_amdgcn_s_setprio(0);
-            __syncthreads();
+            w4_dma_barrier();
         }
     }
 

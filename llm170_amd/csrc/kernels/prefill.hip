@@ -251,7 +251,7 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
         load_b(bq, sc, kt_lo);
     }
     if (has_stats) sum_stats();
-    __syncthreads();  // the compiler waits for the LDS DMA (vmcnt) ahead of the barrier
+    w4_dma_barrier();
     if (has_stats && tid < PF_BM) make_factor();  // read after the barriers of the k loop
     if (KG > 1) {
         // The first weights are waited for here: pending at the loop's head they make its first use wait, in every iteration,
@@ -339,7 +339,7 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
                         for (int mi = 0; mi < MI; mi++) acc[mi][ni] *= next_ratio[ni];
                 }
             }
-            __syncthreads();
+            w4_dma_barrier();
         }
 #pragma unroll
         for (int ni = 0; ni < 2; ni++) {

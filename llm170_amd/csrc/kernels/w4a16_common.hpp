@@ -65,6 +65,14 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t w4_make_rsrc(const void* base,
 }
 #define W4_OOB 0x80000000u  // a byte offset no buffer here reaches
 
+// Barrier behind LDS DMA (buffer_load ... lds): everything this wave has loaded has landed before any wave passes.  The wait is
+// written out: ahead of a plain barrier the compiler waits for the DMA with a counter wherever it can tell the younger loads
+// apart (weights issued behind x: vmcnt(3)), and a counted wait has let readers see LDS rows that had not arrived.
+__device__ __forceinline__ void w4_dma_barrier() {
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0); the other counters are left alone
+    __syncthreads();
+}
+
 // IEEE binary16 bits -> f32 by integer manipulation (subnormals normalised, Inf/NaN payload shifted), the routine
 // the reference uses on both host and device (crates/core/src/quant/deq.rs:4-27).
 __device__ __forceinline__ float w4_half_bits_to_f32(unsigned h) {
