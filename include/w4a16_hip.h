@@ -190,6 +190,10 @@ int w4a16_lin_forward(w4a16_ctx* ctx, const char* name, uint64_t x_dev, uint64_t
  * kernel of w4a16_lin_forward_glu.  Out pointers may be NULL. */
 int w4a16_plan_decode(size_t n, size_t k, size_t group, size_t t, int cu_count, int glu, int* rows_per_wave,
                       int* waves_per_block, int* k_slices, size_t* lds_bytes);
+/* The launch plan of the streaming path at 17..64 rows (W4A16_PATH_STREAM; any t) with every setting automatic: waves of a
+ * workgroup along the output and along k, and k slices across workgroups.  `glu` != 0 plans the gated launch of
+ * w4a16_lin_forward_glu (never split over k).  Needs neither a context nor a GPU.  Out pointers may be NULL. */
+int w4a16_plan_stream(size_t n, size_t k, size_t t, int cu_count, int glu, int* waves_n, int* waves_k, int* k_slices);
 /* The launch plan of the prefill path (W4A16_PATH_PREFILL) for t rows: out = {block tile rows (64, 96 or 128), k slices,
  * super-tile rows, super-tile columns, super-tile count}; `tile_rows` and `k_slices` pin a choice as
  * w4a16_set_prefill_tile / w4a16_set_prefill_ksplit do (0 = automatic); *price_us (may be NULL) receives the model's

@@ -72,10 +72,10 @@ static const char* const kPrefillSyms[] = {W4_PREFILL_KG("w4a16_prefill_g32_f16"
                                            "w4a16_moe_g128_f16_pf_glu", "w4a16_moe_g128_f16_pf_lin", "w4a16_moe_g128_bf16_pf_glu",
                                            "w4a16_moe_g128_bf16_pf_lin", "w4a16_moe_g32_f16_pf_glu", "w4a16_moe_g32_f16_pf_lin",
                                            "w4a16_moe_g32_bf16_pf_glu", "w4a16_moe_g32_bf16_pf_lin", nullptr};
-// waves along n and k of a workgroup (kernels/mid.hip); the split launch's n4k1 has no gated form
+// waves along n and k of a workgroup (kernels/mid.hip)
 #define W4_MID_BUILDS(P)                                                                                               \
-    P "_n1k4", P "_n1k4_glu", P "_n2k4", P "_n2k4_glu", P "_n3k4", P "_n3k4_glu", P "_n4k1", P "_n4k2", P "_n4k2_glu", \
-        P "_n5k2", P "_n5k2_glu"
+    P "_n1k4", P "_n1k4_glu", P "_n2k4", P "_n2k4_glu", P "_n3k4", P "_n3k4_glu", P "_n4k1", P "_n4k1_glu", P "_n4k2", \
+        P "_n4k2_glu", P "_n5k2", P "_n5k2_glu"
 #define W4_MID_FAMILY(P) W4_MID_BUILDS(P "_t2"), W4_MID_BUILDS(P "_t3"), W4_MID_BUILDS(P "_t4")
 static const char* const kMidSyms[] = {W4_MID_FAMILY("w4a16_mid_g128_f16"), W4_MID_FAMILY("w4a16_mid_g128_bf16"),
                                        W4_MID_FAMILY("w4a16_mid_g32_f16"), W4_MID_FAMILY("w4a16_mid_g32_bf16"), nullptr};

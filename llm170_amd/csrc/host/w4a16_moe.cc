@@ -278,49 +278,78 @@ static int launch_moe_gemm(w4a16_ctx* ctx, const W4Experts& E, bool glu, uint64_
 }
 
 // Launch plan of the 17..64-row kernel (kernels/mid.hip): waves along n and k of a workgroup, k slices across workgroups.
-// Every shape gives the same bits for a given number of slices.  From sweeps of 19 widths x 7 k x t = 24, 40, 64 and both
-// groups (units = pairs of row blocks; figures us, group 128, cold weights; over the sweeps the plan loses 0.4 % to the best
-// shape of each, 15 % at worst):
+// Every shape gives the same bits for a given number of slices.  Units are pairs of row blocks, those of all segments of a launch
+// beyond 64 rows.  Fitted to sweeps of every shape with cold weights (28 widths 512..28672, 20 k 2048..20480, t = 20..64, both
+// groups: 1632 points, over which it loses 0.6 % to the best shape, 20 % at worst; 424 at 72..1024 rows, 1.1 %).  Against the
+// kernel before this one it is slower by more than 2 % at 32 of 2944 shapes, 8 % at worst, and 32 % faster on average.  Figures:
+// us, group 128, what it takes / the other.
 //   * up to one unit per CU (n = 8192): a wave per unit and four along k, every unit's workgroup on a CU of its own
-//     (5120 x 5120 t = 64 14.6, two units per workgroup 18.8);
-//   * k slices, whose hand-over costs about 3 us plus what grows with the workgroups: few units (64) from 32 k tiles on, four
-//     or eight slices (1024 x 4096 t = 40 9.8 -> 8.2, 512 x 17408 29.2 -> 11.2); up to 96 units two on a middling k; beyond,
-//     from 65 k tiles, four waves along n, so that the slices' workgroups re-read little x (5120 x 17408 t = 64 37.1 -> 29.1,
-//     t = 24 24.2 -> 20.4);
-//   * more units than CUs: the waves along n that leave the fullest CU the fewest units, a workgroup's start counting as 1.2
-//     units (gated 34816 x 5120 t = 64: five waves 34.5, four 49.2; 28672 x 4096: four 22.3, five 26.4; 22016 x 4096: three
-//     19.3, four 21.3; 16384 x 4096: two 17.1, three 18.6); a long k over little more units than CUs runs four slices
-//     (11008 x 17408 t = 64 54.9 -> 45.7).
-//   * more than 64 rows (scales the MFMA-tiled kernel cannot divide by): the units of all segments count, since k slices pay for
-//     workgroups the grid lacks and cost their workspace and hand-over where it has them (5120 x 17408 t = 512: 130 us in eight
-//     slices, 100 whole with x shared by five waves; t = 192: 53 whole, 49 in four slices; 1024 x 8192 t = 512 37 / 20).
+//     (5120 x 5120 t = 64 15.3, two units per workgroup 18.8);
+//   * k slices of those where the CUs are many times the units, whose hand-over costs about 3 us: up to 64 units four, from a k
+//     on that falls with the token blocks (1280 x 3584 t = 20 7.0 / 7.5 whole, 704 x 2560 t = 56 9.1 / 9.8), up to 32 with a
+//     long k eight (512 x 17408 t = 40 11.2); up to 128 two, where the launch still is one workgroup per CU (2560 x 9216 t = 24
+//     11.8 / 15.4 in eight slices of four units, 4096 x 17408 t = 24 19.7 / 22.0);
+//   * else the lower price, in k tiles of a unit on the fullest CU.  k whole: a workgroup's start counts as 1.2 units (34816 x
+//     5120 gated t = 64: five waves along n 34.5, four 49.2; 28672 x 4096: four 24.7, five 26.4).  Workgroups of four units
+//     that walk k alone, where many of them share a CU (32 KiB of LDS at two token blocks, 48 at three, 64 at four: five, three,
+//     two per CU, at least two to hide each other's latency): 7168 x 5120 t = 1024 93 / 110.  Those in k slices, all resident at once,
+//     if the chip is not full without; their hand-over counts 55 and 4 for every unit and slice per CU.  13824 x 17408 t = 40
+//     47.3 in four slices / 56.7 whole (eight are not resident: 58.8), t = 64 53.8 / 63.1; 9216 x 13312 t = 24 26.4 in eight /
+//     33.9; 28672 x 20480 t = 56 97.7 in two / 110.  Between 129 and 256 units and 66..94 k tiles slices come up to 18 % too
+//     early at two token blocks (4104 x 8448 t = 20 15.8 / 13.4 whole).
 struct MidPlan {
     int wn = 1, wk = kW4MidParts;
     size_t nks = 1;
 };
 
 static MidPlan plan_mid(size_t units, size_t segs, size_t kt_n, size_t t, size_t cus, int ksplit, bool may_split) {
-    const size_t u = units * segs * 256 / cus;  // per 256 CUs
+    const size_t u = units * segs * 256 / cus, tt = t <= 32 ? 2 : t <= 48 ? 3 : 4;  // units per 256 CUs; token blocks
     MidPlan P;
     if (may_split && ksplit > 0) {
         P.nks = std::max<size_t>(1, std::min(std::min<size_t>((size_t)ksplit, kW4MoeMaxKsplit), kt_n / 2));
         if (P.nks > 1 && u > 96) P.wn = 4, P.wk = 1;
         if (P.nks > 1) return P;
-    } else if (may_split && ksplit == 0) {
-        if (u <= 64 && kt_n >= 32) P.nks = kt_n >= 128 || (u <= 32 && kt_n >= 64 && t > 32) ? 8 : 4;
-        else if (u > 64 && u <= 96 && kt_n >= 40 && kt_n <= 64) P.nks = 2;
-        else if (u > 64 && u <= 256 && (kt_n > 64 || (kt_n == 64 && t > 32 && u <= 160))) P = MidPlan{4, 1, 8};
-        else if (u > 256 && (segs > 1 ? u <= 512 && kt_n >= 128 : u <= 352 && kt_n >= 86)) P = MidPlan{4, 1, 4};
-        if (P.nks > 1) return P;
     }
-    if (u <= 256) return P;
+    const bool slices = may_split && ksplit == 0;
+    if (u <= 64) {
+        if (slices && kt_n >= 18 && kt_n * tt >= 56) P.nks = u <= 32 && kt_n * tt >= 120 ? 8 : 4;
+        return P;
+    }
+    if (u <= 128) {
+        if (slices && u > 96 && tt == 4 && kt_n >= 80) return MidPlan{4, 1, 8};
+        if (slices && kt_n * tt >= u + 4) P.nks = 2;
+        return P;
+    }
     double best = 1e30;
-    for (const MidPlan& c : {MidPlan{2, 4, 1}, MidPlan{3, 4, 1}, MidPlan{4, 2, 1}, MidPlan{5, 2, 1}}) {
-        const size_t wgs = (units + (size_t)c.wn - 1) / (size_t)c.wn * segs;
-        const double cost = (double)((wgs + cus - 1) / cus) * (c.wn + 1.2);
+    auto take = [&](const MidPlan& c, double per_k_tile, double once) {
+        const double cost = (double)kt_n * per_k_tile + once;
         if (cost < best) best = cost, P = c;
+    };
+    if (u <= 256) take(MidPlan{}, 2.1, 0.0);
+    else
+        for (const MidPlan& c : {MidPlan{2, 4, 1}, MidPlan{3, 4, 1}, MidPlan{4, 2, 1}, MidPlan{5, 2, 1}}) {
+            const size_t wgs = (units + (size_t)c.wn - 1) / (size_t)c.wn * segs;
+            take(c, (double)((wgs + cus - 1) / cus) * (c.wn + 1.2), 0.0);
+        }
+    for (size_t nks : {1, 2, 4, 8}) {
+        if (nks > 1 && (!slices || kt_n < 2 * nks)) continue;
+        const size_t per_cu = ((units + 3) / 4 * segs * nks + cus - 1) / cus, room = 10 / tt, gens = (per_cu + room - 1) / room;
+        if (nks > 1 && gens > 1) continue;
+        take(MidPlan{4, 1, nks}, (double)(gens * std::max<size_t>(2, std::min(per_cu, room))) * (nks > 1 ? 4.0 / (double)nks : 4.25),
+             nks > 1 ? 55.0 + 4.0 * (double)(nks * u) / 256.0 : 0.0);
     }
     return P;
+}
+
+extern "C" int w4a16_plan_stream(size_t n, size_t k, size_t t, int cu_count, int glu, int* waves_n, int* waves_k, int* k_slices) {
+    if (n == 0 || k == 0 || k % 128 != 0 || t == 0 || cu_count <= 0 || (glu && n % 32 != 0))
+        return w4_fail(W4A16_ERR_ARG, "plan_stream: n=%zu k=%zu t=%zu cus=%d glu=%d", n, k, t, cu_count, glu);
+    const size_t row_blocks = (n + 15) / 16, rows = t <= 32 ? 32 : t <= 48 ? 48 : 64;
+    const MidPlan P = plan_mid(glu ? row_blocks / 2 : (row_blocks + 1) / 2, (t + rows - 1) / rows, k / 128, t, (size_t)cu_count, 0, !glu);
+    if (waves_n) *waves_n = P.wn;
+    if (waves_k) *waves_k = P.wk;
+    if (k_slices) *k_slices = (int)P.nks;
+    return 0;
 }
 
 // glu_act >= 0: the linear is a fused gate|up projection and y receives f16 [t][n/2] = act(gate) * up on the f32 sums; the

@@ -388,6 +388,7 @@ __device__ __forceinline__ void mid_body(MID_PARAMS) {
     MID_KERNEL(PFX##_t##TT##_n3k4, G, SBF, false, TT, 3, 4)       \
     MID_KERNEL(PFX##_t##TT##_n3k4_glu, G, SBF, true, TT, 3, 4)    \
     MID_KERNEL(PFX##_t##TT##_n4k1, G, SBF, false, TT, 4, 1)       \
+    MID_KERNEL(PFX##_t##TT##_n4k1_glu, G, SBF, true, TT, 4, 1)    \
     MID_KERNEL(PFX##_t##TT##_n4k2, G, SBF, false, TT, 4, 2)       \
     MID_KERNEL(PFX##_t##TT##_n4k2_glu, G, SBF, true, TT, 4, 2)    \
     MID_KERNEL(PFX##_t##TT##_n5k2, G, SBF, false, TT, 5, 2)       \

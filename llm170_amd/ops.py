@@ -27,6 +27,13 @@ def plan_decode(n, k, group, t, cu_count=256, glu=False):
     return {"rows_per_wave": rows.value, "waves_per_block": waves.value, "k_slices": nks.value, "lds_bytes": lds.value}
 
 
+def plan_stream(n, k, t, cu_count=256, glu=False):
+    """Launch plan of the streaming path at 17..64 rows (no context, no GPU): dict of waves_n, waves_k, k_slices."""
+    wn, wk, nks = C.c_int(), C.c_int(), C.c_int()
+    ffi.check(ffi.load().w4a16_plan_stream(n, k, t, cu_count, int(bool(glu)), C.byref(wn), C.byref(wk), C.byref(nks)))
+    return {"waves_n": wn.value, "waves_k": wk.value, "k_slices": nks.value}
+
+
 def plan_prefill(t, n, k, cu_count=256, tile_rows=0, k_slices=0, group=128):
     """Launch plan of the prefill path (no context, no GPU): dict of tile_rows, k_slices, super_m, super_n, supers,
     price_us."""

@@ -161,3 +161,24 @@ def test_weights_between_2_and_4_gib(dec):
     bound = k * 2.0**-24 * (np.abs(x.astype(np.float64)) @ np.abs(w).T)
     assert np.all(np.abs(y - x.astype(np.float64) @ w.T) <= bound)
     assert np.all(y != 0)
+
+
+@pytest.mark.parametrize("group,bf16", [(128, False), (32, True)])
+@pytest.mark.parametrize("t", [20, 45, 64])
+def test_very_wide_outputs_walk_k_alone(dec, group, bf16, t):
+    """Workgroups of four waves along n whose waves walk the whole of k (one group, finished parts kept in LDS), plain and
+    gated: the last workgroup has surplus waves, k tiles (3) leave a part empty."""
+    n, k, cc = 65504, 384, dec.cc
+    x = _upload(dec, n, k, group, bf16)
+    want, _ = _run(dec, x, n, t, t * n, lambda xd, yd: dec.lin_forward("mid", xd, yd, t, path=ops.PATH_LANE))
+    f, sym = _run(dec, x, n, t, t * n, lambda xd, yd: dec.lin_forward("mid", xd, yd, t))
+    assert sym.endswith("_n4k1")
+    parity.assert_close(f.view(np.float32).reshape(t, n), want.view(np.float32).reshape(t, n), "wide t%d" % t)
+    fd, od = cc.to_device(f), cc.alloc(t * n)
+    dec.act_mul_f16(fd, n // 2, t, od)
+    want = cc.d2h(od, (t * n // 4,), np.uint32)
+    got, sym = _run(dec, x, n, t, t * n // 4, lambda xd, yd: dec.lin_forward_glu("mid", xd, yd, t))
+    cc.free(fd)
+    cc.free(od)
+    assert sym.endswith("_n4k1_glu")
+    assert np.array_equal(got, want)

@@ -136,3 +136,47 @@ def test_decode_plan_shrinks_to_fit_the_lds():
     for bad in [(0, 128, 128, 1), (64, 100, 128, 1), (64, 128, 64, 1), (64, 128, 128, 17)]:
         with pytest.raises(ops.W4a16Error):
             ops.plan_decode(*bad)
+
+
+def test_stream_plan_follows_the_sweep():
+    """17..64 rows, the shape that measured fastest (or within 4 % of it) at widths and k on both sides of the rule's lines,
+    among them those that a rule read from fewer widths gave a slower launch than the kernel before this one."""
+    want = {  # (n, k tiles, t) -> (waves along n, waves along k, k slices)
+        (13824, 136, 40): (4, 1, 4), (13824, 104, 64): (4, 1, 4), (13824, 40, 24): (2, 4, 1),  # 432 units: eight slices not resident
+        (12288, 160, 48): (4, 1, 8), (12288, 120, 56): (4, 1, 4),                              # 384: eight are, at three token blocks
+        (9216, 72, 24): (4, 1, 8), (9216, 86, 40): (4, 1, 8), (9216, 104, 64): (4, 1, 4), (9216, 40, 64): (2, 4, 1),
+        (11008, 104, 32): (4, 1, 8), (17408, 136, 40): (4, 1, 4), (17408, 136, 64): (3, 4, 1), (28672, 160, 56): (4, 1, 2),
+        (4096, 136, 24): (1, 4, 2), (3072, 136, 24): (1, 4, 2), (2560, 72, 24): (1, 4, 2), (2560, 33, 24): (1, 4, 1),
+        (5120, 40, 64): (1, 4, 1), (5120, 136, 64): (4, 1, 8), (8192, 64, 64): (1, 4, 1), (8192, 136, 24): (4, 1, 8),
+        (2048, 136, 24): (1, 4, 4), (2048, 16, 64): (1, 4, 1), (512, 136, 40): (1, 4, 8), (512, 16, 40): (1, 4, 1),
+    }
+    for (n, kt, t), shape in want.items():
+        p = ops.plan_stream(n, 128 * kt, t)
+        assert (p["waves_n"], p["waves_k"], p["k_slices"]) == shape, (n, kt, t, p)
+    for (n, shape) in [(8192, (1, 4, 1)), (8224, (2, 4, 1)), (22016, (3, 4, 1)), (28672, (4, 2, 1)), (34816, (5, 2, 1)), (65536, (4, 1, 1))]:
+        p = ops.plan_stream(n, 17408, 64, glu=True)  # the gated launch never splits
+        assert (p["waves_n"], p["waves_k"], p["k_slices"]) == shape, (n, p)
+
+
+def test_stream_plan_is_one_the_kernel_has():
+    """Every launch shape is built, its slices hold two k tiles or more and are resident at once where four units share a
+    workgroup, and a split launch needs less than 128 MiB of partial tiles, whatever the rows."""
+    built = {(1, 4), (2, 4), (3, 4), (4, 1), (4, 2), (5, 2)}
+    for n in list(range(16, 2100, 208)) + list(range(2100, 45000, 1337)) + [8224, 22016, 34816]:
+        for kt in (1, 2, 7, 18, 31, 64, 90, 136, 300):
+            for t in (1, 17, 33, 64, 65, 200, 1000):
+                p = ops.plan_stream(n, 128 * kt, t)
+                wn, wk, nks = p["waves_n"], p["waves_k"], p["k_slices"]
+                assert (wn, wk) in built and nks in (1, 2, 4, 8), p
+                assert nks == 1 or kt >= 2 * nks, p
+                tt = 2 if t <= 32 else 3 if t <= 48 else 4
+                groups = -(-((-(-n // 16) + 1) // 2) // wn) * -(-t // (16 * tt))
+                if (wn, wk) == (4, 1) and nks > 1:
+                    assert groups * nks <= 256 * (10 // tt), (n, kt, t, p)
+                assert nks == 1 or groups * wn * 2 * tt * 1024 * nks < 2**27, (n, kt, t, p)
+                if n % 32 == 0:
+                    p = ops.plan_stream(n, 128 * kt, t, glu=True)
+                    assert p["k_slices"] == 1 and (p["waves_n"], p["waves_k"]) in built, (n, kt, t, p)
+    for bad in [(0, 128, 17), (64, 100, 17), (64, 128, 0)]:
+        with pytest.raises(ops.W4a16Error):
+            ops.plan_stream(*bad)
