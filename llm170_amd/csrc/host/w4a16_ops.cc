@@ -526,6 +526,13 @@ static PrefillPlan plan_prefill_groups(const PrefillPlan& tiles, size_t t, size_
     return best;
 }
 
+// The launch's whole plan: everything that decides it is an argument.  `whole`: options that a split launch's second kernel does
+// not take at this shape keep k whole; the caller's pins (tile rows, slices) name the 256-column tiles.
+static PrefillPlan plan_prefill_launch(size_t t, size_t n, size_t k, size_t group, size_t cus, int tile_pin, int ksplit_pin, bool whole, bool glu) {
+    const PrefillPlan tiles = plan_prefill(t, n, k, group, cus, tile_pin, whole ? -1 : ksplit_pin, glu);
+    return tile_pin == 0 && ksplit_pin == 0 ? plan_prefill_groups(tiles, t, n, k, group, cus) : tiles;
+}
+
 extern "C" int w4a16_plan_prefill(size_t t, size_t n, size_t k, size_t group, int cu_count, int tile_rows, int k_slices,
                                   size_t out[5], double* price_us) {
     if (t == 0 || n == 0 || k == 0 || k % 128 != 0 || (group != 128 && group != 32) || cu_count <= 0 || !out ||
@@ -590,22 +597,17 @@ static int launch_prefill(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_t y
         return w4_fail(W4A16_ERR_SHAPE, "prefill: x or the tiled weights reach 2 GiB, beyond the buffer-descriptor range");
     // A split launch finishes in a second kernel.  With epilogue options that kernel works on whole 1024-column
     // chunks of a row; where the shape does not allow it (or for the gated form) the k range stays whole.
-    int ksplit = ctx->prefill_ksplit;
-    if (has_epi && (glu || L.n % 1024 != 0)) ksplit = -1;
-    // the plan depends on (t, n, k) and the pinned settings only and is kept per shape
-    PrefillPlan plan;
-    {
-        const auto key = std::make_tuple(t, L.n, L.k, ctx->prefill_tile_m + (glu ? 1000 : 0), ksplit);
-        const auto hit = ctx->prefill_plans.find(key);
-        if (hit != ctx->prefill_plans.end()) {
-            plan = PrefillPlan{hit->second[0], hit->second[1], PrefillSuper{hit->second[2], hit->second[3], hit->second[4], 0}, 0.0, hit->second[5]};
-        } else {
-            plan = plan_prefill(t, L.n, L.k, L.group, (size_t)std::max(ctx->cu_count, 1), ctx->prefill_tile_m, ksplit, glu);
-            if (ctx->prefill_tile_m == 0 && ctx->prefill_ksplit == 0)  // a pinned tile or slice count names the 256-column tiles
-                plan = plan_prefill_groups(plan, t, L.n, L.k, L.group, (size_t)std::max(ctx->cu_count, 1));
-            ctx->prefill_plans[key] = {plan.bm, plan.nks, plan.sup.sup_m, plan.sup.sup_n, plan.sup.supers, plan.wnw};
-        }
+    const bool whole = has_epi && (glu || L.n % 1024 != 0);
+    // kept per argument of the plan (one context, one CU count)
+    const auto key = std::make_tuple(t, L.n, L.k, L.group, ctx->prefill_tile_m, ctx->prefill_ksplit, (int)whole + 2 * (int)glu);
+    auto hit = ctx->prefill_plans.find(key);
+    if (hit == ctx->prefill_plans.end()) {
+        const PrefillPlan P = plan_prefill_launch(t, L.n, L.k, L.group, (size_t)std::max(ctx->cu_count, 1), ctx->prefill_tile_m,
+                                                  ctx->prefill_ksplit, whole, glu);
+        hit = ctx->prefill_plans.emplace(key, std::array<size_t, 6>{P.bm, P.nks, P.sup.sup_m, P.sup.sup_n, P.sup.supers, P.wnw}).first;
     }
+    const auto& kept = hit->second;
+    const PrefillPlan plan{kept[0], kept[1], PrefillSuper{kept[2], kept[3], kept[4], 0}, 0.0, kept[5]};
     const size_t bm = plan.bm, nks = plan.nks, sup_m = plan.sup.sup_m, sup_n = plan.sup.sup_n, supers = plan.sup.supers;
     const size_t grid = ((supers + 7) / 8) * (sup_m * sup_n) * 8;
     char sym[64];
