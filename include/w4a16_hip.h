@@ -194,13 +194,21 @@ int w4a16_plan_decode(size_t n, size_t k, size_t group, size_t t, int cu_count, 
  * workgroup along the output and along k, and k slices across workgroups.  `glu` != 0 plans the gated launch of
  * w4a16_lin_forward_glu (never split over k).  Needs neither a context nor a GPU.  Out pointers may be NULL. */
 int w4a16_plan_stream(size_t n, size_t k, size_t t, int cu_count, int glu, int* waves_n, int* waves_k, int* k_slices);
-/* The launch plan of the prefill path (W4A16_PATH_PREFILL) for t rows: out = {block tile rows (64, 96 or 128), k slices,
- * super-tile rows, super-tile columns, super-tile count}; `tile_rows` and `k_slices` pin a choice as
+/* The best launch of the prefill path (W4A16_PATH_PREFILL) on its 256-column block tiles for t rows: out = {block tile rows (64,
+ * 96 or 128), k slices, super-tile rows, super-tile columns, super-tile count}; `tile_rows` and `k_slices` pin a choice as
  * w4a16_set_prefill_tile / w4a16_set_prefill_ksplit do (0 = automatic); *price_us (may be NULL) receives the model's
- * estimate for the chosen plan.  Role of the reference's per-problem choice of thread-block shape
+ * estimate for the chosen plan.  With nothing pinned narrow outputs may run a k-group build instead: see
+ * w4a16_plan_prefill_launch.  Role of the reference's per-problem choice of thread-block shape
  * (kernels/marlin.rs:94-213).  Needs neither a context nor a GPU. */
 int w4a16_plan_prefill(size_t t, size_t n, size_t k, size_t group, int cu_count, int tile_rows, int k_slices,
                        size_t out[5], double* price_us);
+
+/* What the prefill path launches with nothing pinned: out = {block tile rows, block tile columns (256; 128 or 192 in a k-group
+ * build), k groups inside a workgroup (1 or 4), k slices, super-tile rows, super-tile columns, super-tile count}.  `glu` != 0: the
+ * gated launch.  `whole_k` != 0: a launch with the options of a deferred norm whose shape (gated, or n not a multiple of 1024)
+ * keeps k whole.  price_us as above (of the k-group build's own model where one is chosen). */
+int w4a16_plan_prefill_launch(size_t t, size_t n, size_t k, size_t group, int cu_count, int glu, int whole_k, size_t out[7],
+                              double* price_us);
 
 /* w4a16_lin_forward for callers that cannot allocate.  NO COUNTERPART IN THE REFERENCE: it exists for code under HIP graph
  * capture, tight serving loops and harnesses that forbid hipMalloc.  w4a16_lin_forward's decode launch, when it splits k

@@ -407,7 +407,8 @@ static int launch_decode_glu(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_
 }
 
 // Launch plan of the prefill GEMM (kernels/prefill.hip): a pure function of (t, n, k), the CU count and the pinned
-// settings, so that a CPU test can pin what it chooses at the layer shapes (w4a16_plan_prefill).
+// settings, so that a CPU test can pin what it chooses at the layer shapes (w4a16_plan_prefill); w4a16_plan_prefill_launch
+// also prices the k-group builds below.
 // Block tile 128 x 256 (two workgroups per CU), 96 x 256 or 64 x 256 (three per CU, 96 / 64 accumulator registers), the
 // k range whole or cut into 2, 3, 4, 6 or 8 slices (split-K: f32 partials in a context-owned workspace, added in slice order by a
 // second launch — deterministic), and the super-tile shape: every combination is priced and the cheapest runs.
@@ -502,14 +503,15 @@ static PrefillPlan plan_prefill(size_t t, size_t n, size_t k, size_t group, size
 // launch or a workspace, but keeps only 8 or 12 waves there, so it is a candidate only where the grid is one generation (a block
 // tile per CU at most; beyond that it loses: 5120 x 5120 t = 450 over 128 columns 48 us, 46 for the plan above).  Both sides
 // measured with weights from memory, 1489 shapes per group size (15 widths 512..22016, k = 640..11008, t = 17..1500), the plan
-// above / this one in us: group 128 5120 x 5120 t = 300 34.7 / 28.3, 7168 x 5120 t = 300 48.0 / 33.5 (192 columns), 4096 x 2048
-// t = 300 24.5 / 13.6, 1024 x 640 t = 100 13.8 / 7.9, group 32 5120 x 2048 t = 300 31.9 / 17.3; not chosen: 5120 x 5120 t = 65
+// above / this one in us: group 128 5120 x 5120 t = 300 32.0 / 27.4, 7168 x 5120 t = 300 43.5 / 34.6 (192 columns), 4096 x 2048
+// t = 300 26.3 / 12.9, 1024 x 640 t = 100 14.1 / 7.8, group 32 5120 x 2048 t = 300 32.1 / 16.1; not chosen: 5120 x 5120 t = 65
 // 22.7 / 23.7, 5120 x 17408 t = 128 43 / 74.
 // The price (fitted to the same sweep, 5 % rms): a fixed cost and one per k tile of a group's run, each growing with the part
 // of the chip in use.  The other plan's price is corrected before the two are compared, so that the choice is level or gains
 // at every shape of the sweep (2 %, the noise): + 3 us where its k range is whole (its fixed cost is low by 3..5 us at short k),
 // x 0.72 for up to four slices of up to four k tiles (they overlap better than priced), x 0.88 otherwise at group 128, whose
 // constants it was fitted with, 0.98 at group 32.  -13 % on average over the sweep; 1.6 % above the best choice for each shape.
+// (With the full wait at its barriers, since: 4096 x 5120 t = 300 25.8 / 26.8, 5120 x 5120 t = 256 26.7 / 27.5 are chosen and lose.)
 static PrefillPlan plan_prefill_groups(const PrefillPlan& tiles, size_t t, size_t n, size_t k, size_t group, size_t cus) {
     static const double price[2][2][4] = {{{4.6, 1.86, 1.0, 0.39}, {5.45, 2.13, 1.28, 0.65}},  // group 128: 128, 192 columns
                                           {{4.7, 2.53, 1.1, 0.27}, {5.4, 3.16, 1.4, 0.44}}};    // group 32
@@ -531,6 +533,17 @@ static PrefillPlan plan_prefill_groups(const PrefillPlan& tiles, size_t t, size_
 static PrefillPlan plan_prefill_launch(size_t t, size_t n, size_t k, size_t group, size_t cus, int tile_pin, int ksplit_pin, bool whole, bool glu) {
     const PrefillPlan tiles = plan_prefill(t, n, k, group, cus, tile_pin, whole ? -1 : ksplit_pin, glu);
     return tile_pin == 0 && ksplit_pin == 0 ? plan_prefill_groups(tiles, t, n, k, group, cus) : tiles;
+}
+
+extern "C" int w4a16_plan_prefill_launch(size_t t, size_t n, size_t k, size_t group, int cu_count, int glu, int whole_k, size_t out[7],
+                                         double* price_us) {
+    if (t == 0 || n == 0 || k == 0 || k % 128 != 0 || (group != 128 && group != 32) || cu_count <= 0 || !out || (glu && n % 32 != 0))
+        return w4_fail(W4A16_ERR_ARG, "plan_prefill_launch: t=%zu n=%zu k=%zu group=%zu cus=%d", t, n, k, group, cu_count);
+    const PrefillPlan P = plan_prefill_launch(t, n, k, group, (size_t)cu_count, 0, 0, whole_k != 0, glu != 0);
+    const size_t got[7] = {P.bm, P.wnw ? 64 * P.wnw : (size_t)kW4PfBn, P.wnw ? 4u : 1u, P.nks, P.sup.sup_m, P.sup.sup_n, P.sup.supers};
+    for (int i = 0; i < 7; i++) out[i] = got[i];
+    if (price_us) *price_us = P.us;
+    return 0;
 }
 
 extern "C" int w4a16_plan_prefill(size_t t, size_t n, size_t k, size_t group, int cu_count, int tile_rows, int k_slices,

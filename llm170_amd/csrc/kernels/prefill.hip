@@ -588,11 +588,11 @@ __device__ __forceinline__ bool pf_moe_tile(PfGroup<MODE>& gp, const int* num_po
 
 // k-group kernels, for outputs too narrow to fill the chip with 256-column tiles: 64 rows x 64 WNW columns, WNW waves along n times
 // four k groups in one workgroup (8 or 12 waves, 128 or 144 KiB of LDS: one workgroup per CU).  What bounds these launches is
-// not the matrix pipe but a chain per k tile (x by DMA, barrier, 16 MFMAs a wave) too few waves are there to hide, plus, when
+// not the matrix pipe but a chain per k tile (x by DMA, barrier, 32 MFMAs a wave) too few waves are there to hide, plus, when
 // k slices filled the chip instead, writing the slices' f32 sums to memory and a second launch that adds them.  Here each group
 // walks a quarter of k with x stages of its own, the groups' sums meet in LDS in group order (same bits on every run), and each
-// group runs the epilogue, options included, for a quarter of the rows.  5120 x 5120 t = 300 34.7 -> 28.3 us (200
-// workgroups instead of 400 and a second launch), 4096 x 2048 t = 300 24.5 -> 13.6, group 32 5120 x 2048 t = 300 31.9 -> 17.3.
+// group runs the epilogue, options included, for a quarter of the rows.  5120 x 5120 t = 300 32.0 -> 27.4 us (200
+// workgroups instead of 400 and a second launch), 4096 x 2048 t = 300 26.3 -> 12.9, group 32 5120 x 2048 t = 300 32.1 -> 16.1.
 // One wave along n (64 columns) needs twice the waves for the same x traffic and won 0.3 % over the range: not built.
 #define PREFILL_KG_KERNEL(NAME, G, SBF, WNW, MODE)                                                                    \
     extern "C" __global__ __launch_bounds__(64 * WNW * 4) __attribute__((amdgpu_waves_per_eu(WNW, WNW))) void NAME(       \

@@ -1,4 +1,4 @@
-"""Launch plans of the decode and prefill paths as pure functions (w4a16_plan_decode, w4a16_plan_prefill): no GPU.
+"""Launch plans of the decode, streaming and prefill paths as pure functions (w4a16_plan_*): no GPU.
 
 The prefill planner is a price model with constants fitted to measurements; the table of those measurements that is
 kept under profiles/ names, per layer shape, the (tile, k slices) that measured fastest.  This test feeds the planner
@@ -180,3 +180,39 @@ def test_stream_plan_is_one_the_kernel_has():
     for bad in [(0, 128, 17), (64, 100, 17), (64, 128, 0)]:
         with pytest.raises(ops.W4a16Error):
             ops.plan_stream(*bad)
+
+
+def test_prefill_launch_plan():
+    """What is launched with nothing pinned: k-group builds of 128 or 192 columns where the grid is at most one block tile per
+    CU and they are priced below the 256-column tiles, which are otherwise those of plan_prefill.  The scale group decides too."""
+    want = {  # (t, n, k, group) -> (columns, k groups, k slices)
+        (300, 5120, 5120, 128): (128, 4, 1), (300, 7168, 5120, 128): (192, 4, 1), (300, 4096, 2048, 128): (128, 4, 1),
+        (100, 1024, 640, 128): (128, 4, 1), (300, 5120, 2048, 32): (128, 4, 1), (65, 256, 512, 128): (128, 4, 1),
+        (200, 5120, 5120, 128): (128, 4, 1), (200, 5120, 5120, 32): (256, 1, 6),
+        (100, 5120, 2048, 128): (128, 4, 1), (100, 5120, 2048, 32): (256, 1, 4),
+        (128, 5120, 17408, 128): (256, 1, 8), (512, 34816, 5120, 128): (256, 1, 1), (4096, 5120, 17408, 128): (256, 1, 1),
+    }
+    for (t, n, k, g), shape in want.items():
+        p = ops.plan_prefill_launch(t, n, k, group=g)
+        assert (p["tile_cols"], p["k_groups"], p["k_slices"]) == shape, (t, n, k, g, p)
+    for t in (65, 100, 200, 300, 449, 640, 1000):
+        for n in (256, 1000, 4096, 5120, 7168, 12288, 34816):
+            for k in (128, 640, 2048, 5120, 17408):
+                for g in (128, 32):
+                    for glu in (False, True):
+                        if glu and n % 32:
+                            continue
+                        p = ops.plan_prefill_launch(t, n, k, group=g, glu=glu)
+                        tiles_m, tiles_n = -(-t // p["tile_rows"]), -(-n // p["tile_cols"])
+                        if p["k_groups"] == 4:
+                            assert p["tile_rows"] == 64 and p["k_slices"] == 1 and tiles_m * tiles_n <= 256, p
+                        elif not glu:
+                            q = ops.plan_prefill(t, n, k, group=g)
+                            assert p["tile_cols"] == 256 and all(p[f] == q[f] for f in q), (p, q)
+                        assert p["supers"] == -(-tiles_m // p["super_m"]) * -(-tiles_n // p["super_n"]), p
+                        assert ops.plan_prefill_launch(t, n, k, group=g, glu=glu, whole_k=True)["k_slices"] == 1
+    # a block tile per CU, and one more: 64 rows x 128 columns
+    assert ops.plan_prefill_launch(64 * 16, 128 * 16, 640)["k_groups"] == 4
+    assert ops.plan_prefill_launch(64 * 16 + 1, 128 * 16, 640)["tile_cols"] != 128
+    with pytest.raises(ops.W4a16Error):
+        ops.plan_prefill_launch(100, 1000, 640, glu=True)
