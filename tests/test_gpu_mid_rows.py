@@ -182,3 +182,22 @@ def test_very_wide_outputs_walk_k_alone(dec, group, bf16, t):
     cc.free(od)
     assert sym.endswith("_n4k1_glu")
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("group,bf16", [(128, False), (32, True)])
+@pytest.mark.parametrize("n,k,build", [(1, 640, "n1k4"), (19, 5120, "n1k4"), (423, 640, "n1k4"), (4097, 8448, "n4k1"), (8233, 640, "n2k4"),
+                                       (17002, 384, "n3k4"), (33009, 256, "n5k2")])
+def test_widths_that_are_no_multiple_of_four(dec, n, k, build, group, bf16):
+    """Rows of y start at any element: the four-column stores are unaligned and the last columns go out one by one; whole
+    and in k slices, f32 and f16."""
+    for t in (18, 33, 64):
+        print("odd width", n, k, t, group, bf16, flush=True)
+        x = _upload(dec, n, k, group, bf16)
+        want, _ = _run(dec, x, n, t, t * n, lambda xd, yd: dec.lin_forward("mid", xd, yd, t, path=ops.PATH_LANE))
+        got, sym = _run(dec, x, n, t, t * n, lambda xd, yd: dec.lin_forward("mid", xd, yd, t))
+        assert sym.endswith("_" + build)
+        parity.assert_close(got.view(np.float32).reshape(t, n), want.view(np.float32).reshape(t, n), "odd width %d t%d" % (n, t))
+        h, _ = _run(dec, x, n, t, (t * n + 1) // 2, lambda xd, yd: dec.lin_forward("mid", xd, yd, t, out_f16=True))
+        h = h.view(np.uint16)
+        assert np.array_equal(h[:t * n], gen.f32_to_f16_bits(got.view(np.float32)).reshape(-1))
+        assert t * n % 2 == 0 or h[t * n] == GUARD >> 16  # the half word behind the last element

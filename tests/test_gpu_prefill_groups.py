@@ -128,3 +128,18 @@ def test_options_of_a_deferred_norm(dec, n, k, t, cols):
     finally:
         for p in (px, pp, py, ps, pr, pw):
             cc.free(p)
+
+
+@pytest.mark.parametrize("group,bf16", [(128, False), (32, True)])
+@pytest.mark.parametrize("n,k,t,cols", [(1, 640, 65, 2), (67, 384, 100, 2), (1001, 640, 97, 2), (4103, 1152, 129, 2), (8234, 1152, 193, 3)])
+def test_widths_that_are_no_multiple_of_four(dec, n, k, t, cols, group, bf16):
+    print("odd width", n, k, t, group, bf16, flush=True)
+    x = _upload(dec, n, k, group, bf16, t)
+    want, _ = _run(dec, x, t * n, lambda xd, yd: dec.lin_forward("pg", xd, yd, t, path=ops.PATH_LANE))
+    got, sym = _run(dec, x, t * n, lambda xd, yd: dec.lin_forward("pg", xd, yd, t))
+    assert sym == _name(group, bf16, cols)
+    parity.assert_close(got.view(np.float32).reshape(t, n), want.view(np.float32).reshape(t, n), "odd width %d" % n)
+    h, _ = _run(dec, x, (t * n + 1) // 2, lambda xd, yd: dec.lin_forward("pg", xd, yd, t, out_f16=True))
+    h = h.view(np.uint16)
+    assert np.array_equal(h[:t * n], gen.f32_to_f16_bits(got.view(np.float32)).reshape(-1))
+    assert t * n % 2 == 0 or h[t * n] == GUARD >> 16  # the half word behind the last element
