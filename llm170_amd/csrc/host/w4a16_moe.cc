@@ -252,8 +252,10 @@ static int launch_moe_gemm(w4a16_ctx* ctx, const W4Experts& E, bool glu, uint64_
     const char* fam = E.tiled_bf16 ? "bf16" : "f16";
     if (tiled) {
         // MFMA-tiled grouped kernel (kernels/prefill.hip, MODE 1 / 2): block tile = one 64-slot segment x 256 columns
-        // (gate|up: 128 gate + the 128 matching up columns); LDS = two x stages of 64 rows x 64 k and the slot ids
+        // (gate|up: 128 gate + the 128 matching up columns); LDS = two x stages of 64 rows x 128 k, overlaid at the end by the
+        // waves' padded f16 tiles, then slot ids and routing weights; rows always leave as f16
         if (block != 64) return w4_fail(W4A16_ERR_ARG, "moe: the tiled grouped kernel needs 64-slot segments (got %zu)", block);
+        if (!y_f16) return w4_fail(W4A16_ERR_UNSUPPORTED, "moe: the tiled grouped kernel writes f16 rows only");
         const size_t cols = glu ? E.n_ff : n, per_tile = glu ? 128 : 256;
         snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_pf_%s", E.group, fam, glu ? "glu" : "lin");
         const size_t blocks = (max_segs + 7) / 8 * 8 * ((cols + per_tile - 1) / per_tile);

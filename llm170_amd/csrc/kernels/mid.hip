@@ -11,8 +11,10 @@
 //     The WN waves of a group share its staged x tile; the WK groups bring the waves that hide latency without more x.  WN is
 //     chosen so that one generation of workgroups covers the output evenly (the plan in w4a16_moe.cc); a grid a little over one
 //     workgroup per CU costs a second one (34816 x 5120 gated at t = 64: four waves along n 48 us, five 34);
-//   * x by LDS DMA, one k tile ahead, no registers held (128 VGPRs at four token blocks: four waves per SIMD); a lone wave
-//     along n (narrow outputs) stages its x through registers instead, needs no barrier and half the LDS;
+//   * x by LDS DMA, one k tile ahead, no registers held; a lone wave along n (narrow outputs) stages its x through registers
+//     instead and needs no barrier and half the LDS.  LDS sets how many waves a CU holds (at four token blocks: n5k2 160 KiB, ten
+//     waves; n4k2, n2k4 128 KiB, eight; n3k4 128 KiB, twelve; n1k4 68 KiB and n4k1 64 KiB, two workgroups, eight), two or three
+//     per SIMD; registers (at most 132, a lone wave 212) would allow as many;
 //   * scales: group 128 one load for both row blocks of a k tile (a quad's lanes fetch them alternately, DPP broadcasts).
 // Sums: a slice's k tiles are cut into MID_PARTS runs, each summed from zero and added in order.  WK groups take whole runs, so
 // every launch shape gives the same bits, and so do the gated and the plain launch and a slice of a split one.
@@ -203,8 +205,8 @@ __device__ __forceinline__ void mid_body(MID_PARAMS) {
     };
     const int iters = PPW * per;
     if constexpr (WN > 1) {
-        // one k tile ahead: its DMA and weights are issued ahead of this tile's MFMAs and waited for (vmcnt 0) at the
-        // barrier that ends them
+        // one k tile ahead: its DMA and weights are issued ahead of this tile's MFMAs and all waited for at the barrier that
+        // ends them
         load_x(kt0, 0);
         load_w(stage[0], kt0);
         w4_dma_barrier();

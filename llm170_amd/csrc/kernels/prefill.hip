@@ -6,8 +6,9 @@
 //     overlap the other's MFMAs;
 //   * x (the A operand) is staged through LDS a k tile at a time (in the 96-row tile, whose registers leave no room for the
 //     addresses, half of one), double buffered, by LDS DMA (buffer_load ... lds: no staging registers, no ds_write), one
-//     barrier per stage; stages of 64 k: 5120 x 34816 gated t = 300 113.5 -> 111.0 us, t = 4096 1158 -> 1151, 17408 x 5120
-//     t = 4096 618 -> 609; rows are unpadded and their 16-byte chunks swizzled by row so the ds_read_b128 fragment reads are
+//     barrier per stage; against stages of 64 k (us): 5120 x 34816 gated t = 300 114.8 -> 112.3; t = 4096, seven boxes, 1187 -> 1179,
+//     1166 -> 1157, 1187 -> 1178, 1204 -> 1200, 1251 -> 1253, 1219 -> 1210, 1172 -> 1161; group 32 1649 -> 1470 (its 256-register
+//     build spilled); 17408 x 5120 t = 4096 614 -> 608; but 17408 x 2560 t = 400 in eight slices 57.5 -> 61.7; rows are unpadded and their 16-byte chunks swizzled by row so the ds_read_b128 fragment reads are
 //     bank-conflict free; rows >= t come from out-of-range loads (zeros);
 //   * the weights (B operand) never touch LDS: the tiled layout of w4a16_common.hpp already is the MFMA B layout —
 //     lane (n = l % 32, khalf = l / 32) reads 16 B of tile lane g = 2h + khalf, r = n % 16 of its row block, dword w of
@@ -51,7 +52,7 @@ __device__ __forceinline__ float pf_ratio(float s_prev, float s_cur) {
 //   MODE 1 (gate|up, n = 2 n_ff): a wave's two 32-column sub-tiles are gate columns c.. and up columns n_ff + c.., so
 //     the lane that holds a gate sum holds the matching up sum; both are rounded to f16 (the reference materialises
 //     them as f16) and act[slot][c] = f16(act(gate) * up) is written, f16 [ns][n_ff];
-//   MODE 2 (down, n = hidden): y[slot][c] = sum * topw[slot] as f16 or f32 [ns][n].
+//   MODE 2 (down, n = hidden): y[slot][c] = f16(sum * topw[slot]), f16 [ns][n].
 //
 // Dense gated form (MODE 3): a fused gate|up linear (rows 0..n/2 gate, n/2..n up) with the element-wise kernel that
 // follows it in the reference's prefill chain (lin_forward + ew, w4a16_dec/prefill.rs:148-207, assets/ew.cu:9-57)
@@ -77,9 +78,8 @@ struct PfGroup {
 //   consumer side: stats_in [n_stats_in][ld_stats] are partial sums of squares of the INPUT rows left by the launch
 //     that produced x; the output row m is multiplied by 1/sqrt(sum_e stats_in[e][m] * inv_cols_in + 1e-6) * in_scale
 //     (in_scale = 2^e undoes the power-of-two factor x was handed over with); ldx = halves between x rows (0 = k);
-//   producer side: resid f32 [t][n] takes the output (v = resid + y, written back); stats_out[(tile_n*4 + wave)][m]
-//     receives this wave's partial sum of v^2 over its columns below stat_cols (one entry per wave and block tile
-//     column, no atomics); nw f32 [n] multiplies what y receives; out_scale = 2^-e is applied last.
+//   producer side: resid f32 [t][n] takes the output (v = resid + y, written back); stats_out[c / 64][m] receives
+//     the partial sum of v^2 over the 64 columns from c that a wave holds, those below stat_cols (no atomics); nw f32 [n] multiplies what y receives; out_scale = 2^-e is applied last.
 struct PfEpi {
     const float* stats_in;
     float* stats_out;
@@ -609,7 +609,7 @@ __device__ __forceinline__ bool pf_moe_tile(PfGroup<MODE>& gp, const int* num_po
     PREFILL_KG_KERNEL(PFX##_m64_n3k4_glu, G, SBF, 3, 3)
 
 // Grouped kernels for the expert FFN: same arguments as the streaming grouped kernels of moe.hip (blk must be 64, the
-// rows of a block tile; wpb is unused).
+// rows of a block tile, and y_f16 1: the host refuses others; wpb is unused).
 #define PREFILL_MOE_KERNEL(NAME, G, SBF, MODE)                                                                        \
     extern "C" __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(3, 3))) void NAME(            \
         const char* qa, const char* sa, unsigned long long q_stride, unsigned long long s_stride, const uint16_t* x,      \
