@@ -258,7 +258,7 @@ static int launch_moe_gemm(w4a16_ctx* ctx, const W4Experts& E, bool glu, uint64_
         if (!y_f16) return w4_fail(W4A16_ERR_UNSUPPORTED, "moe: the tiled grouped kernel writes f16 rows only");
         const size_t cols = glu ? E.n_ff : n, per_tile = glu ? 128 : 256;
         snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_pf_%s", E.group, fam, glu ? "glu" : "lin");
-        const size_t blocks = (max_segs + 7) / 8 * 8 * ((cols + per_tile - 1) / per_tile);
+        const size_t blocks = (max_segs * ((cols + per_tile - 1) / per_tile) + 7) / 8 * 8;
         if (blocks > 0x7fffffffu) return w4_fail(W4A16_ERR_SHAPE, "moe: %zu segments exceed the grid", max_segs);
         return w4_launch(ctx, sym, (unsigned)blocks, 1, 256, kW4PfMoeIdsAt + 64 * 8, p);
     }

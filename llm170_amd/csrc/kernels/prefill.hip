@@ -568,19 +568,22 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
         prefill_body<G, SBF, MI, 3>(qt, st, x, y, row_blocks, k, n, t, out_f16, sup_m, sup_n, gp, epi);                \
     }
 
-// Block tile of a grouped workgroup.  Every XCD (block b runs on XCD b % 8) takes an eighth of the live 64-slot segments in
-// order, column tiles fastest, so that the segments of one expert's run fetch its weights, and the column tiles of a segment
-// its x rows, into one L2 at about the same time (128 experts, T = 2048: -3 %).  Gate|up tiles span 128 gate and the 128
+// Block tile of a grouped workgroup.  Every XCD (block b runs on XCD b % 8) takes an eighth of the live block tiles, segments in
+// order and column tiles fastest, so that the segments of one expert's run fetch its weights, and the column tiles of a segment
+// its x rows, into one L2 at about the same time (128 experts, T = 2048: -3 %).  Dealt by whole segments, a count just over a
+// multiple of eight leaves most XCDs waiting for one (8 experts top-2, h 4096, n_ff 3584, us per FFN, by segments / by tiles:
+// group 32 T = 1024 298 / 272, group 128 T = 700 182 / 155; level elsewhere).  Gate|up tiles span 128 gate and the 128
 // matching up columns.  A segment whose second half is padding (its slots are a prefix of it) runs the 32-row body: an expert's
 // last segment is partly filled (T = 1536 246 -> 225 us per FFN, T = 2048 284 -> 264).
 template <int MODE>
 __device__ __forceinline__ bool pf_moe_tile(PfGroup<MODE>& gp, const int* num_post, int n, int* rows) {
     const int tiles = MODE == 1 ? ((n >> 1) + PF_BN / 2 - 1) / (PF_BN / 2) : (n + PF_BN - 1) / PF_BN;
-    const int segs = num_post[0] / 64, xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
-    const int seg = segs * xcd / 8 + j / tiles;
-    if (seg >= segs * (xcd + 1) / 8) return false;
+    const unsigned work = (unsigned)(num_post[0] / 64) * (unsigned)tiles, xcd = blockIdx.x & 7;
+    const unsigned at = (unsigned)((unsigned long long)work * xcd / 8) + (blockIdx.x >> 3);
+    if (at >= (unsigned)((unsigned long long)work * (xcd + 1) / 8)) return false;
+    const int seg = (int)(at / (unsigned)tiles);
     gp.m0 = seg * 64;
-    gp.n0 = (j % tiles) * (MODE == 1 ? PF_BN / 2 : PF_BN);
+    gp.n0 = (int)(at % (unsigned)tiles) * (MODE == 1 ? PF_BN / 2 : PF_BN);
     gp.expert = gp.expert_ids[seg];
     *rows = gp.sorted_ids[gp.m0 + 32] < gp.ns ? 64 : 32;
     return (unsigned)gp.expert < (unsigned)gp.n_exp;

@@ -1,5 +1,5 @@
 """The MFMA-tiled grouped kernels at the edges of their block tiles: runs that end just before and after 32 and 64 slots, empty
-and single experts, more segments than one per XCD and fewer, column tiles that are half empty."""
+and single experts, more segments than one per XCD and fewer, XCD shares that end inside a segment, column tiles that are half empty."""
 import numpy as np
 import pytest
 
@@ -21,7 +21,7 @@ def dec():
 @pytest.mark.parametrize("group", [32, 128])
 @pytest.mark.parametrize("h,n_ff,runs", [
     (128, 384, [1, 0, 32, 33, 0, 64, 65, 96, 97, 128, 129, 31]), (384, 128, [700]), (256, 256, [0, 0, 5]),
-    (640, 128, [63, 1, 64, 32] * 5)])
+    (640, 128, [63, 1, 64, 32] * 5), (640, 384, [64] * 9)])
 def test_tiled_runs_of_every_length(dec, orc, group, h, n_ff, runs):
     """top_k = 1, so that run lengths are what the list says; the slots of a run are scattered over the tokens.  silu only: the
     gelu's 1 + tanhf(..) cancels for gates below about -3, an error of up to 0.5 |g u| 2^-23 that the one-step envelope of the
