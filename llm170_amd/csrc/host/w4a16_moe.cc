@@ -274,8 +274,12 @@ static int launch_moe_gemm(w4a16_ctx* ctx, const W4Experts& E, bool glu, uint64_
     waves = ctx->moe_waves ? ctx->moe_waves : 4;
     waves = waves >= 8 ? 8 : 4;  // the x staging needs at least 4 waves
     const size_t blocks = max_segs * ((units + (size_t)waves - 1) / (size_t)waves);
-    snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_mm_%s_t%d", E.group, fam, glu ? "glu" : "lin", tt);
-    const unsigned shmem = (unsigned)(2 * 16 * tt * 256);  // two x tiles of 128 k
+    // Two k tiles per stage (kernels/moe.hip) at group 128 where the launch has at most three workgroups per CU and runs of up to
+    // 32 slots: 8 experts T = 100 62.5 -> 54.6 us per FFN, 32 experts top-4 n_ff 1024 T = 40 33.3 -> 30.8; beyond, the LDS they
+    // take costs more than the wait they hide (8 experts T = 256 91 / 101, 64 experts top-6 n_ff 1408 T = 24 57.4 / 59.9).
+    const bool two = E.group == 128 && tt <= 3 && ns < 32 * E.n_exp && blocks * (size_t)waves <= 12 * (size_t)std::max(ctx->cu_count, 1);
+    snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_mm_%s_t%d%s", E.group, fam, glu ? "glu" : "lin", tt, two ? "_k2" : "");
+    const unsigned shmem = (unsigned)((two ? 4 : 2) * 16 * tt * 256);  // two stages of one or two x tiles of 128 k
     return w4_launch(ctx, sym, (unsigned)blocks, 1, (unsigned)(waves * 64), shmem, p);
 }
 

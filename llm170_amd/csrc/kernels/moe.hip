@@ -429,10 +429,10 @@ struct MoeMmStage {
 };
 
 // One block = (segment of blk = 16*TT slots, group of W units); wave w owns unit group*W + w over the whole k range.
-// TT: the 16-slot blocks of the segment this workgroup multiplies (those that hold a slot).
-template <int G, bool SBF, bool GLU, int TT>
+// TT: the 16-slot blocks of the segment this workgroup multiplies (those that hold a slot).  KT: k tiles per stage.
+template <int G, bool SBF, bool GLU, int TT, int KT>
 __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
-    extern __shared__ _Float16 xs[];  // [2][16*TT][128]
+    extern __shared__ _Float16 xs[];  // [2][KT][16*TT][128]
     constexpr int GPT = W4_TILE_K / G;
     constexpr int ROWS = 16 * TT;
     const int tid = threadIdx.x, lane = tid & 63, W = wpb;
@@ -491,7 +491,7 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
     const unsigned sg = G == 32 ? (unsigned)(lane & 3) * 32u : 0u;
     const unsigned soff[2] = {(unsigned)rbA * (unsigned)kg_n * 32u + sg + (unsigned)q * 8u,
                               (unsigned)rbB * (unsigned)kg_n * 32u + sg + (unsigned)q * 8u};
-    MoeMmStage<2> stage[2];
+    MoeMmStage<2> stage[2][KT];
     auto load_w = [&](MoeMmStage<2>& s_, int kt) {
         const bool live = kt < kt_n;
         const __amdgpu_buffer_rsrc_t qr = w4_make_rsrc(qe, live ? q_bytes : 0u), sr = w4_make_rsrc(se, live ? s_bytes : 0u);
@@ -605,26 +605,33 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
         group(std::integral_constant<int, 7>{});
     };
 
-    // one k tile ahead: its DMA and weights are issued ahead of this tile's MFMAs and waited for (vmcnt 0) at the barrier
+    // one stage ahead: its DMA and weights are issued ahead of this stage's MFMAs and waited for (vmcnt 0) at the barrier
     // that ends them.  Few registers, many waves: x in flight in registers and weights two (group 32) or four (group 128) tiles
     // ahead, the wait for x behind the youngest weights, were slower throughout (128 experts, us per FFN: group 32 f16 T = 64
     // 75.6 -> 70.7, T = 517 117 -> 113; group 128 T = 64 74.9 -> 67.4, T = 517 111.5 -> 98.5).
-    load_x(0, 0);
-    load_w(stage[0], 0);
+    auto load_stage = [&](int kt, int d) {  // out of range past the last tile: zeros, no traffic
+#pragma unroll
+        for (int j = 0; j < KT; j++) {
+            load_x(kt + j, d * KT + j);
+            load_w(stage[d][j], kt + j);
+        }
+    };
+    load_stage(0, 0);
     w4_dma_barrier();
-    for (int kt0 = 0; kt0 < kt_n; kt0 += 2) {
+    for (int kt0 = 0; kt0 < kt_n; kt0 += 2 * KT) {
 #pragma unroll
         for (int d = 0; d < 2; d++) {
-            const int kt = kt0 + d;
-            load_x(kt + 1, d ^ 1);  // out of range past the last tile: zeros, no traffic
-            load_w(stage[d ^ 1], kt + 1);
+            const int kt = kt0 + d * KT;
+            load_stage(kt + KT, d ^ 1);
             __builtin_amdgcn_sched_barrier(0);
             // a wave that holds a landed tile issues ahead of the waves that are queueing loads (about 1 % at every T)
             __builtin_amdgcn_s_setprio(1);
-            if (kt < kt_n) {
-                if constexpr (G == 32 && TT <= 3) compute32(stage[d], d);
-                else compute(stage[d], d);
-            }
+#pragma unroll
+            for (int j = 0; j < KT; j++)
+                if (kt + j < kt_n) {
+                    if constexpr (G == 32 && TT <= 3) compute32(stage[d][j], d * KT + j);
+                    else compute(stage[d][j], d * KT + j);
+                }
             __builtin_amdgcn_s_setprio(0);
             w4_dma_barrier();
         }
@@ -644,20 +651,20 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
 // 16-slot block tells whether the block holds any: the workgroup runs the body built for the blocks that do, and the
 // MFMAs, scaled sums and x rows of all-padding blocks are never issued (128 experts, top-8, T = 512: runs of 32 +- 6
 // slots in 48-slot segments, every other expert fills two blocks of three).
-template <int G, bool SBF, bool GLU, int TT>
+template <int G, bool SBF, bool GLU, int TT, int KT = 1>
 __device__ __forceinline__ void moe_mm_entry(MOE_PARAMS) {
     if constexpr (TT == 1) {
-        moe_mm_body<G, SBF, GLU, 1>(MOE_ARGS);
+        moe_mm_body<G, SBF, GLU, 1, KT>(MOE_ARGS);
     } else {
         const int units = GLU ? row_blocks >> 1 : (row_blocks + 1) >> 1;
         const int seg = blockIdx.x / ((units + wpb - 1) / wpb);
         int live = 1;
 #pragma unroll
         for (int p = 1; p < TT; p++) live += sorted_ids[seg * blk + 16 * p] < ns ? 1 : 0;
-        if (live == 1) moe_mm_body<G, SBF, GLU, 1>(MOE_ARGS);
-        else if (TT == 2 || live == 2) moe_mm_body<G, SBF, GLU, 2>(MOE_ARGS);
-        else if (TT == 3 || live == 3) moe_mm_body<G, SBF, GLU, TT >= 3 ? 3 : 2>(MOE_ARGS);
-        else moe_mm_body<G, SBF, GLU, TT>(MOE_ARGS);
+        if (live == 1) moe_mm_body<G, SBF, GLU, 1, KT>(MOE_ARGS);
+        else if (TT == 2 || live == 2) moe_mm_body<G, SBF, GLU, 2, KT>(MOE_ARGS);
+        else if (TT == 3 || live == 3) moe_mm_body<G, SBF, GLU, TT >= 3 ? 3 : 2, KT>(MOE_ARGS);
+        else moe_mm_body<G, SBF, GLU, TT, KT>(MOE_ARGS);
     }
 }
 
@@ -665,9 +672,9 @@ __device__ __forceinline__ void moe_mm_entry(MOE_PARAMS) {
     extern "C" __global__ __launch_bounds__(512) void NAME(MOE_PARAMS) {              \
         moe_dec_body<G, SBF, GLU, XL, DEPTH>(MOE_ARGS);                               \
     }
-#define MOE_MM_KERNEL(NAME, G, SBF, GLU, TT)                                          \
+#define MOE_MM_KERNEL(NAME, G, SBF, GLU, ...)                                         \
     extern "C" __global__ __launch_bounds__(512) void NAME(MOE_PARAMS) {              \
-        moe_mm_entry<G, SBF, GLU, TT>(MOE_ARGS);                                      \
+        moe_mm_entry<G, SBF, GLU, __VA_ARGS__>(MOE_ARGS);                             \
     }
 // Ring depths of the streaming kernels, from sweeps on the 128-expert shape: the one-slot segments of the direct mode run
 // best with two k tiles in flight per wave (T = 4..12: 9-11 % faster than four: fewer registers, more waves resident at
@@ -690,6 +697,18 @@ MOE_FAMILY(w4a16_moe_g32_f16, 32, false)
 MOE_FAMILY(w4a16_moe_g32_bf16, 32, true)
 MOE_FAMILY(w4a16_moe_g128_f16, 128, false)
 MOE_FAMILY(w4a16_moe_g128_bf16, 128, true)
+
+// Two k tiles per stage, for launches of few workgroups (the rule is at the launch, w4a16_moe.cc): one tile in flight per wave
+// does not cover the trip to memory there.  Group 128, whose tiles take least time to multiply.  8 experts top-2, h 4096, n_ff
+// 3584, us per FFN, x and weights four tiles ahead in registers / one tile per stage / two: T = 16 52.5 / 57.8 / 49.2, T = 40
+// 50.3 / 57.3 / 45.7, T = 100 57.8 / 62.5 / 54.6; four tiles per stage lose (51.1, 49.4, 71.3).
+#define MOE_MM_KT2(PFX, G, SBF)                                \
+    MOE_MM_KERNEL(PFX##_mm_glu_t2_k2, G, SBF, true, 2, 2)      \
+    MOE_MM_KERNEL(PFX##_mm_glu_t3_k2, G, SBF, true, 3, 2)      \
+    MOE_MM_KERNEL(PFX##_mm_lin_t2_k2, G, SBF, false, 2, 2)     \
+    MOE_MM_KERNEL(PFX##_mm_lin_t3_k2, G, SBF, false, 3, 2)
+MOE_MM_KT2(w4a16_moe_g128_f16, 128, false)
+MOE_MM_KT2(w4a16_moe_g128_bf16, 128, true)
 
 // ---------------------------------------------------------------------------------------------------- routing
 // Routing rule of the reference (w4a16_dec/mod.rs:168-185, device counterpart assets/moe.cu:686-759): softmax over all
