@@ -427,11 +427,15 @@ struct PrefillPlan {
 // busiest XCD ends up with — counted exactly, partial super-tiles at the edges included — and the shape with the
 // lightest busiest XCD wins, the larger one on ties for L2 reuse.  (A fixed 8 along m left 10 tile rows as 8 + 2:
 // the XCDs that drew the 2-row super-tiles idled, 298 against 227 us on the down projection at t = 1280.)
-static PrefillSuper prefill_super(size_t tiles_m, size_t tiles_n) {
+// most_blocks: shapes that launch more blocks per XCD are left out, those past the output's edge counted.  A block past the edge
+// ends at once, but takes its place in the order in which an XCD's blocks are dealt to its CUs: a grid that holds one block per
+// CU has to count it (15 x 16 tiles in super-tiles of 7 x 2, 30 live blocks of 42: some CUs drew two, 32.1 us; 5 x 2, 18.8).
+static PrefillSuper prefill_super(size_t tiles_m, size_t tiles_n, size_t most_blocks = ~(size_t)0) {
     PrefillSuper best{std::min<size_t>(8, tiles_m), 8, 0, ~(size_t)0};
     for (size_t cm = std::min<size_t>(8, tiles_m); cm >= 1; cm--) {
         for (size_t cn : {8, 4, 2, 1}) {
             const size_t sm = (tiles_m + cm - 1) / cm, sn = (tiles_n + cn - 1) / cn, sp = sm * sn;
+            if ((sp + 7) / 8 * cm * cn > most_blocks) continue;
             size_t per_xcd[8] = {0, 0, 0, 0, 0, 0, 0, 0};
             for (size_t sidx = 0; sidx < sp; sidx++)
                 per_xcd[sidx & 7] += std::min(cm, tiles_m - (sidx % sm) * cm) * std::min(cn, tiles_n - (sidx / sm) * cn);
@@ -520,10 +524,10 @@ static PrefillPlan plan_prefill_groups(const PrefillPlan& tiles, size_t t, size_
     double us = tiles.nks == 1 ? tiles.us + 3.0 : tiles.us * (tiles.nks <= 4 && (kt_n + tiles.nks - 1) / tiles.nks <= 4 ? 0.72 : group == 32 ? 0.98 : 0.88);
     for (size_t w : {2, 3}) {
         const size_t tiles_n = (n + 64 * w - 1) / (64 * w);  // gated: as many pairs of 32 w gate and up columns
-        if (tiles_m * tiles_n > cus) continue;
+        if ((tiles_m * tiles_n + 7) / 8 * 8 > cus) continue;
         const double* c = price[group == 32][w - 2];
         const double full = (double)(tiles_m * tiles_n) / (double)cus, p = c[0] + c[2] * full + (c[1] + c[3] * full) * (double)run;
-        if (p < us) us = p, best = PrefillPlan{64, 1, prefill_super(tiles_m, tiles_n), p, w};
+        if (p < us) us = p, best = PrefillPlan{64, 1, prefill_super(tiles_m, tiles_n, cus / 8), p, w};
     }
     return best;
 }

@@ -195,8 +195,8 @@ def test_prefill_launch_plan():
     for (t, n, k, g), shape in want.items():
         p = ops.plan_prefill_launch(t, n, k, group=g)
         assert (p["tile_cols"], p["k_groups"], p["k_slices"]) == shape, (t, n, k, g, p)
-    for t in (65, 100, 200, 300, 449, 640, 1000):
-        for n in (256, 1000, 4096, 5120, 7168, 12288, 34816):
+    for t in (65, 100, 200, 300, 449, 640, 957, 1000):
+        for n in (256, 1000, 1928, 4096, 5120, 7168, 12288, 34816):
             for k in (128, 640, 2048, 5120, 17408):
                 for g in (128, 32):
                     for glu in (False, True):
@@ -206,6 +206,7 @@ def test_prefill_launch_plan():
                         tiles_m, tiles_n = -(-t // p["tile_rows"]), -(-n // p["tile_cols"])
                         if p["k_groups"] == 4:
                             assert p["tile_rows"] == 64 and p["k_slices"] == 1 and tiles_m * tiles_n <= 256, p
+                            assert -(-p["supers"] // 8) * p["super_m"] * p["super_n"] <= 32, p  # blocks of an XCD, empty ones too
                         elif not glu:
                             q = ops.plan_prefill(t, n, k, group=g)
                             assert p["tile_cols"] == 256 and all(p[f] == q[f] for f in q), (p, q)
