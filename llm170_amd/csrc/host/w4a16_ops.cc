@@ -510,24 +510,29 @@ static PrefillPlan plan_prefill(size_t t, size_t n, size_t k, size_t group, size
 // above / this one in us: group 128 5120 x 5120 t = 300 32.0 / 27.4, 7168 x 5120 t = 300 43.5 / 34.6 (192 columns), 4096 x 2048
 // t = 300 26.3 / 12.9, 1024 x 640 t = 100 14.1 / 7.8, group 32 5120 x 2048 t = 300 32.1 / 16.1; not chosen: 5120 x 5120 t = 65
 // 22.7 / 23.7, 5120 x 17408 t = 128 43 / 74.
-// The price (fitted to the same sweep, 5 % rms): a fixed cost and one per k tile of a group's run, each growing with the part
-// of the chip in use.  The other plan's price is corrected before the two are compared, so that the choice is level or gains
-// at every shape of the sweep (2 %, the noise): + 3 us where its k range is whole (its fixed cost is low by 3..5 us at short k),
-// x 0.72 for up to four slices of up to four k tiles (they overlap better than priced), x 0.88 otherwise at group 128, whose
-// constants it was fitted with, 0.98 at group 32.  -13 % on average over the sweep; 1.6 % above the best choice for each shape.
-// (With the full wait at its barriers, since: 4096 x 5120 t = 300 25.8 / 26.8, 5120 x 5120 t = 256 26.7 / 27.5 are chosen and lose.)
+// The price: a fixed cost and one per k tile of a group's run, each growing with the part of the chip in use (of the busiest XCD).
+// The other plan's is corrected before the two are compared, k whole and k in slices apart: its constants, fitted at group 128 over
+// wider outputs, are low at short k, and slices of the 64-row tile are faster than priced.  Fitted to both sides of 2186 launches
+// (96 linears of 512..23200 x 1024..17408, t = 65..2048, both groups, weights from memory), a quarter of them held out first: of
+// the launches that take a k-group build 0.7 % lose more than 2 % to the plan above (none of those held out; 23 % did under the
+// constants of the time when a counted wait stood at its barriers: 592 x 2560 t = 128 12.9 / 14.3 us, 7168 x 5120 t = 128 25.2 /
+// 27.8), and 3 % of those that do not would have gained more than 3 %.
 static PrefillPlan plan_prefill_groups(const PrefillPlan& tiles, size_t t, size_t n, size_t k, size_t group, size_t cus) {
-    static const double price[2][2][4] = {{{4.6, 1.86, 1.0, 0.39}, {5.45, 2.13, 1.28, 0.65}},  // group 128: 128, 192 columns
-                                          {{4.7, 2.53, 1.1, 0.27}, {5.4, 3.16, 1.4, 0.44}}};    // group 32
+    static const double price[2][2][4] = {{{5.738, 1.554, 0.8956, 0.3632}, {6.407, 1.616, 1.639, 0.5267}},   // group 128: 128, 192 columns
+                                          {{5.876, 2.025, 1.39, 0.2816}, {6.163, 2.427, 1.666, 0.5129}}};  // group 32
+    // factor and offset of the other plan's price: k whole, k in slices
+    static const double other[2][2][2] = {{{1.127, 3.319}, {0.8943, -1.773}}, {{0.9407, 4.859}, {1.099, -4.473}}};
     const size_t kt_n = k / 128, tiles_m = (t + 63) / 64, run = (kt_n + 3) / 4;
     PrefillPlan best = tiles;
-    double us = tiles.nks == 1 ? tiles.us + 3.0 : tiles.us * (tiles.nks <= 4 && (kt_n + tiles.nks - 1) / tiles.nks <= 4 ? 0.72 : group == 32 ? 0.98 : 0.88);
+    const double* o = other[group == 32][tiles.nks > 1];
+    double us = tiles.us * o[0] + o[1];
     for (size_t w : {2, 3}) {
         const size_t tiles_n = (n + 64 * w - 1) / (64 * w);  // gated: as many pairs of 32 w gate and up columns
         if ((tiles_m * tiles_n + 7) / 8 * 8 > cus) continue;
         const double* c = price[group == 32][w - 2];
-        const double full = (double)(tiles_m * tiles_n) / (double)cus, p = c[0] + c[2] * full + (c[1] + c[3] * full) * (double)run;
-        if (p < us) us = p, best = PrefillPlan{64, 1, prefill_super(tiles_m, tiles_n, cus / 8), p, w};
+        const PrefillSuper sup = prefill_super(tiles_m, tiles_n, cus / 8);
+        const double used = (double)(sup.load * 8) / (double)cus, p = c[0] + c[2] * used + (c[1] + c[3] * used) * (double)run;
+        if (p < us) us = p, best = PrefillPlan{64, 1, sup, p, w};
     }
     return best;
 }

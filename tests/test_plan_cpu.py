@@ -189,7 +189,7 @@ def test_prefill_launch_plan():
         (300, 5120, 5120, 128): (128, 4, 1), (300, 7168, 5120, 128): (192, 4, 1), (300, 4096, 2048, 128): (128, 4, 1),
         (100, 1024, 640, 128): (128, 4, 1), (300, 5120, 2048, 32): (128, 4, 1), (65, 256, 512, 128): (128, 4, 1),
         (200, 5120, 5120, 128): (128, 4, 1), (200, 5120, 5120, 32): (256, 1, 6),
-        (100, 5120, 2048, 128): (128, 4, 1), (100, 5120, 2048, 32): (256, 1, 4),
+        (100, 5120, 2048, 128): (128, 4, 1), (100, 5120, 2048, 32): (128, 4, 1), (128, 592, 2560, 128): (256, 1, 4), (80, 1768, 1920, 32): (256, 1, 3),
         (128, 5120, 17408, 128): (256, 1, 8), (512, 34816, 5120, 128): (256, 1, 1), (4096, 5120, 17408, 128): (256, 1, 1),
     }
     for (t, n, k, g), shape in want.items():
