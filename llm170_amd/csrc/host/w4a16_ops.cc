@@ -936,9 +936,10 @@ extern "C" int w4a16_lin_forward(w4a16_ctx* ctx, const char* name, uint64_t x_de
         else if (t <= 16)
             path = W4A16_PATH_DECODE;
         else if (t <= 64 || !L->scales_regular)
-            // a few dozen rows are still bound by the weight stream (measured on the 27B shapes: 33 vs 57 us at t = 32
-            // on gate|up, 22 vs 43 us on the down projection; level with the MFMA tiles at t = 128).  A linear with a
-            // zero or non-finite scale always comes here: the prefill kernel divides by scales.
+            // A few dozen rows are still bound by the weight stream.  us, this path / the MFMA tiles, group 128: 34816 x 5120 t = 32
+            // 31.1 / 32.8, t = 64 35.1 / 35.5, t = 65 63.0 / 53.0; 5120 x 17408 t = 32 23.3 / 27.0, t = 64 29.7 / 28.5, t = 65 43.1 /
+            // 39.8; 5120 x 5120 t = 64 14.0 / 18.2 (and t = 128 19.0 / 22.4: outputs of up to 7168 columns would gain here beyond 64
+            // rows too).  A linear with a zero or non-finite scale always comes here: the prefill kernel divides by scales.
             path = W4A16_PATH_STREAM;
         else
             path = W4A16_PATH_PREFILL;
