@@ -651,7 +651,7 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
 // 16-slot block tells whether the block holds any: the workgroup runs the body built for the blocks that do, and the
 // MFMAs, scaled sums and x rows of all-padding blocks are never issued (128 experts, top-8, T = 512: runs of 32 +- 6
 // slots in 48-slot segments, every other expert fills two blocks of three).
-template <int G, bool SBF, bool GLU, int TT, int KT = 1>
+template <int G, bool SBF, bool GLU, int TT, int KT>
 __device__ __forceinline__ void moe_mm_entry(MOE_PARAMS) {
     if constexpr (TT == 1) {
         moe_mm_body<G, SBF, GLU, 1, KT>(MOE_ARGS);
@@ -672,9 +672,9 @@ __device__ __forceinline__ void moe_mm_entry(MOE_PARAMS) {
     extern "C" __global__ __launch_bounds__(512) void NAME(MOE_PARAMS) {              \
         moe_dec_body<G, SBF, GLU, XL, DEPTH>(MOE_ARGS);                               \
     }
-#define MOE_MM_KERNEL(NAME, G, SBF, GLU, ...)                                         \
+#define MOE_MM_KERNEL(NAME, G, SBF, GLU, TT, KT)                                      \
     extern "C" __global__ __launch_bounds__(512) void NAME(MOE_PARAMS) {              \
-        moe_mm_entry<G, SBF, GLU, __VA_ARGS__>(MOE_ARGS);                             \
+        moe_mm_entry<G, SBF, GLU, TT, KT>(MOE_ARGS);                                  \
     }
 // Ring depths of the streaming kernels, from sweeps on the 128-expert shape: the one-slot segments of the direct mode run
 // best with two k tiles in flight per wave (T = 4..12: 9-11 % faster than four: fewer registers, more waves resident at
@@ -684,14 +684,14 @@ __device__ __forceinline__ void moe_mm_entry(MOE_PARAMS) {
     MOE_DEC_KERNEL(PFX##_dec_glu_x4, G, SBF, true, 4, 2)     \
     MOE_DEC_KERNEL(PFX##_dec_lin_x1, G, SBF, false, 1, 2)    \
     MOE_DEC_KERNEL(PFX##_dec_lin_x4, G, SBF, false, 4, 2)    \
-    MOE_MM_KERNEL(PFX##_mm_glu_t1, G, SBF, true, 1)    \
-    MOE_MM_KERNEL(PFX##_mm_glu_t2, G, SBF, true, 2)    \
-    MOE_MM_KERNEL(PFX##_mm_glu_t3, G, SBF, true, 3)    \
-    MOE_MM_KERNEL(PFX##_mm_glu_t4, G, SBF, true, 4)    \
-    MOE_MM_KERNEL(PFX##_mm_lin_t1, G, SBF, false, 1)   \
-    MOE_MM_KERNEL(PFX##_mm_lin_t2, G, SBF, false, 2)   \
-    MOE_MM_KERNEL(PFX##_mm_lin_t3, G, SBF, false, 3)   \
-    MOE_MM_KERNEL(PFX##_mm_lin_t4, G, SBF, false, 4)
+    MOE_MM_KERNEL(PFX##_mm_glu_t1, G, SBF, true, 1, 1)    \
+    MOE_MM_KERNEL(PFX##_mm_glu_t2, G, SBF, true, 2, 1)    \
+    MOE_MM_KERNEL(PFX##_mm_glu_t3, G, SBF, true, 3, 1)    \
+    MOE_MM_KERNEL(PFX##_mm_glu_t4, G, SBF, true, 4, 1)    \
+    MOE_MM_KERNEL(PFX##_mm_lin_t1, G, SBF, false, 1, 1)   \
+    MOE_MM_KERNEL(PFX##_mm_lin_t2, G, SBF, false, 2, 1)   \
+    MOE_MM_KERNEL(PFX##_mm_lin_t3, G, SBF, false, 3, 1)   \
+    MOE_MM_KERNEL(PFX##_mm_lin_t4, G, SBF, false, 4, 1)
 
 MOE_FAMILY(w4a16_moe_g32_f16, 32, false)
 MOE_FAMILY(w4a16_moe_g32_bf16, 32, true)
