@@ -71,25 +71,29 @@ static const char* const kPrefillSyms[] = {W4_PREFILL_KG("w4a16_prefill_g32_f16"
                                            "w4a16_prefill_g32_f16_m96_glu", "w4a16_prefill_g32_bf16_m96_glu",
                                            "w4a16_moe_g128_f16_pf_glu", "w4a16_moe_g128_f16_pf_lin", "w4a16_moe_g128_bf16_pf_glu",
                                            "w4a16_moe_g128_bf16_pf_lin", "w4a16_moe_g32_f16_pf_glu", "w4a16_moe_g32_f16_pf_lin",
-                                           "w4a16_moe_g32_bf16_pf_glu", "w4a16_moe_g32_bf16_pf_lin", nullptr};
+                                           "w4a16_moe_g32_bf16_pf_glu", "w4a16_moe_g32_bf16_pf_lin",
+                                           "w4a16_moe_g32_f16x_pf_glu", "w4a16_moe_g32_f16x_pf_lin", nullptr};
 // waves along n and k of a workgroup (kernels/mid.hip)
 #define W4_MID_BUILDS(P)                                                                                               \
     P "_n1k4", P "_n1k4_glu", P "_n2k4", P "_n2k4_glu", P "_n3k4", P "_n3k4_glu", P "_n4k1", P "_n4k1_glu", P "_n4k2", \
         P "_n4k2_glu", P "_n5k2", P "_n5k2_glu"
 #define W4_MID_FAMILY(P) W4_MID_BUILDS(P "_t2"), W4_MID_BUILDS(P "_t3"), W4_MID_BUILDS(P "_t4")
 static const char* const kMidSyms[] = {W4_MID_FAMILY("w4a16_mid_g128_f16"), W4_MID_FAMILY("w4a16_mid_g128_bf16"),
-                                       W4_MID_FAMILY("w4a16_mid_g32_f16"), W4_MID_FAMILY("w4a16_mid_g32_bf16"), nullptr};
+                                       W4_MID_FAMILY("w4a16_mid_g32_f16"), W4_MID_FAMILY("w4a16_mid_g32_bf16"),
+                                       W4_MID_FAMILY("w4a16_mid_g32_bf16x"), nullptr};
 static const char* const kUtilSyms[] = {"w4a16_fill0_u32", nullptr};
 static const char* const kGlueSyms[] = {"w4a16_rms_rescale_f16", "w4a16_silu_mul_f16", "w4a16_synth_q", "w4a16_synth_s",
                                         "w4a16_norm_resid", nullptr};
 #define W4_MOE_FAMILY(P)                                                                                      \
     P "_dec_glu_x1", P "_dec_glu_x4", P "_dec_lin_x1", P "_dec_lin_x4", P "_mm_glu_t1", P "_mm_glu_t2",       \
         P "_mm_glu_t3", P "_mm_glu_t4", P "_mm_lin_t1", P "_mm_lin_t2", P "_mm_lin_t3", P "_mm_lin_t4"
+#define W4_MOE_FOLD(P) P "_mm_glu_t2", P "_mm_glu_t3", P "_mm_glu_t4", P "_mm_lin_t2", P "_mm_lin_t3", P "_mm_lin_t4"
 #define W4_MOE_KT2(P) P "_mm_glu_t2_k2", P "_mm_glu_t3_k2", P "_mm_lin_t2_k2", P "_mm_lin_t3_k2"
 static const char* const kMoeSyms[] = {W4_MOE_FAMILY("w4a16_moe_g32_f16"),
                                        W4_MOE_FAMILY("w4a16_moe_g32_bf16"),
                                        W4_MOE_FAMILY("w4a16_moe_g128_f16"),
                                        W4_MOE_FAMILY("w4a16_moe_g128_bf16"),
+                                       W4_MOE_FOLD("w4a16_moe_g32_f16x"),
                                        W4_MOE_KT2("w4a16_moe_g128_f16"),
                                        W4_MOE_KT2("w4a16_moe_g128_bf16"),
                                        "w4a16_moe_g32_f16_down_sum",

@@ -24,6 +24,7 @@ struct W4Lin {
     int scale_bf16 = 0;
     size_t row_blocks = 0;
     bool scales_regular = true;  // every scale finite and non-zero (the MFMA prefill kernel divides by them)
+    bool fold = false;  // group 32, bf16 scales: f16 holds every weight times its scale exactly (w4_bf16_folds)
     float row_norm_max = -1.0f;  // largest row norm of the dequantised weights, computed on first request (< 0: not yet)
     std::vector<size_t> part_n;  // a fused linear: the rows of each part, in order (empty for a linear uploaded as one)
 };
@@ -36,6 +37,7 @@ struct W4Experts {
     int scale_bf16 = 0;
     size_t q13_stride = 0, s13_stride = 0, q2_stride = 0, s2_stride = 0;  // bytes per expert
     bool scales_regular = true;  // same rule as W4Lin::scales_regular, over both arenas: the MFMA-tiled grouped kernels need it
+    bool fold = false;        // as W4Lin::fold, over both arenas
     bool tiled_bf16 = false;  // the arenas hold bf16 scales (bf16 scales that f16 holds exactly are stored as f16)
 };
 
@@ -141,6 +143,10 @@ int w4_find_lin(w4a16_ctx* ctx, const char* name, W4Lin** out);
 bool w4_scales_regular(const uint16_t* s, size_t count, int scale_bf16);
 // true when every one of `count` bf16 scales is zero or a normal f16 number (2^-14 .. 2^16, 8 significant bits)
 bool w4_bf16_fits_f16(const uint16_t* s, size_t count);
+// true when every one of `count` bf16 scales s is what a symmetric quantiser writes, positive, and f16 holds (nibble - 8) * s
+// exactly: s a normal f16 number below 2^13 (its eight significant bits and three of the nibble are the eleven of an f16, and 8 * s
+// stays finite).  Zero or negative scales keep the kernels that scale group sums, whose bits do not depend on how scales are stored.
+bool w4_bf16_folds(const uint16_t* s, size_t count);
 int w4_ensure(w4a16_ctx* ctx, uint64_t* buf, size_t* cap, size_t bytes);
 // dense linear at 17..64 rows, or any number of rows (kernels/mid.hip).  glu_act >= 0: L is a fused gate|up linear and y_dev
 // receives f16 [t][n/2] = act(gate) * up on the f32 sums

@@ -84,8 +84,11 @@ extern "C" int w4a16_upload_experts(w4a16_ctx* ctx, const char* name, size_t n_e
     E.scales_regular = w4_scales_regular(static_cast<const uint16_t*>(s13), s13_bytes / 2, scale_bf16) &&
                        w4_scales_regular(static_cast<const uint16_t*>(s2), s2_bytes / 2, scale_bf16);
     // bf16 scales that f16 holds exactly are stored as f16: the f16 kernels read the same values without a conversion per scale
-    const bool to_f16 = scale_bf16 && w4_bf16_fits_f16(static_cast<const uint16_t*>(s13), s13_bytes / 2) &&
-                        w4_bf16_fits_f16(static_cast<const uint16_t*>(s2), s2_bytes / 2);
+    auto all = [&](bool (*test)(const uint16_t*, size_t)) {
+        return test(static_cast<const uint16_t*>(s13), s13_bytes / 2) && test(static_cast<const uint16_t*>(s2), s2_bytes / 2);
+    };
+    E.fold = scale_bf16 && group == 32 && all(w4_bf16_folds);
+    const bool to_f16 = E.fold || (scale_bf16 && all(w4_bf16_fits_f16));
     E.tiled_bf16 = scale_bf16 && !to_f16;
     int rc = tile_arena(ctx, q13, s13, n_experts, 2 * n_ff, h, group, to_f16, &E.q13, &E.s13, &E.q13_stride, &E.s13_stride);
     if (!rc) rc = tile_arena(ctx, q2, s2, n_experts, h, n_ff, group, to_f16, &E.q2, &E.s2, &E.q2_stride, &E.s2_stride);
@@ -257,7 +260,7 @@ static int launch_moe_gemm(w4a16_ctx* ctx, const W4Experts& E, bool glu, uint64_
         if (block != 64) return w4_fail(W4A16_ERR_ARG, "moe: the tiled grouped kernel needs 64-slot segments (got %zu)", block);
         if (!y_f16) return w4_fail(W4A16_ERR_UNSUPPORTED, "moe: the tiled grouped kernel writes f16 rows only");
         const size_t cols = glu ? E.n_ff : n, per_tile = glu ? 128 : 256;
-        snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_pf_%s", E.group, fam, glu ? "glu" : "lin");
+        snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_pf_%s", E.group, E.fold ? "f16x" : fam, glu ? "glu" : "lin");
         const size_t blocks = (max_segs * ((cols + per_tile - 1) / per_tile) + 7) / 8 * 8;
         if (blocks > 0x7fffffffu) return w4_fail(W4A16_ERR_SHAPE, "moe: %zu segments exceed the grid", max_segs);
         return w4_launch(ctx, sym, (unsigned)blocks, 1, 256, kW4PfMoeIdsAt + 64 * 8, p);
@@ -278,7 +281,8 @@ static int launch_moe_gemm(w4a16_ctx* ctx, const W4Experts& E, bool glu, uint64_
     // 32 slots: 8 experts T = 100 62.5 -> 54.6 us per FFN, 32 experts top-4 n_ff 1024 T = 40 33.3 -> 30.8; beyond, the LDS they
     // take costs more than the wait they hide (8 experts T = 256 91 / 101, 64 experts top-6 n_ff 1408 T = 24 57.4 / 59.9).
     const bool two = E.group == 128 && tt <= 3 && ns < 32 * E.n_exp && blocks * (size_t)waves <= 12 * (size_t)std::max(ctx->cu_count, 1);
-    snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_mm_%s_t%d%s", E.group, fam, glu ? "glu" : "lin", tt, two ? "_k2" : "");
+    const bool fold = E.fold && ns >= 8 * E.n_exp;  // figures at compute_fold, kernels/moe.hip
+    snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_mm_%s_t%d%s", E.group, fold ? "f16x" : fam, glu ? "glu" : "lin", tt, two ? "_k2" : "");
     const unsigned shmem = (unsigned)((two ? 4 : 2) * 16 * tt * 256);  // two stages of one or two x tiles of 128 k
     return w4_launch(ctx, sym, (unsigned)blocks, 1, (unsigned)(waves * 64), shmem, p);
 }
@@ -385,8 +389,15 @@ int w4_dense_mid(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_t y, size_t 
         ws = ctx->decode_ws;
         tk = ctx->decode_tickets;
     }
+    // At group 32 bf16 scales that fold (w4_bf16_folds) are multiplied into the weights (bf16x) where a slice has 24 k tiles or more,
+    // else group sums are scaled.  Folded sums round once per k tile instead of once per group but inside the MFMAs as well, which
+    // exact integer products do not: against 64-bit sums, folded / scaled, k = 2048 9.3e-8 / 8.5e-8, 3072 9.7e-8 / 9.9e-8, 5120
+    // 1.05e-7 / 1.22e-7, 17408 in eight slices 1.10e-7 / 1.22e-7 but 8192 in four 1.04e-7 / 8.8e-8: below 24 k tiles the folded ones
+    // are the less exact.
+    const bool fold = L.fold && L.k / 128 >= 24 * P.nks;
+    const char* fam = !L.scale_bf16 ? "f16" : fold ? "bf16x" : "bf16";
     char sym[64];
-    snprintf(sym, sizeof sym, "w4a16_mid_g%zu_%s_t%zu_n%dk%d%s", L.group, L.scale_bf16 ? "bf16" : "f16", tt, P.wn, P.wk, glu ? "_glu" : "");
+    snprintf(sym, sizeof sym, "w4a16_mid_g%zu_%s_t%zu_n%dk%d%s", L.group, fam, tt, P.wn, P.wk, glu ? "_glu" : "");
     // staged x (two buffers of unpadded rows; a lone wave along n: one of padded rows), overlaid by the groups' results; then,
     // where a wave sums several parts, its slot for the finished ones (kernels/mid.hip: XB, OB)
     const size_t xb = wk * 16 * tt * (wn > 1 ? 2 * 256 : 2 * (size_t)kW4MoeLdx), tiles = wk * wn * 2 * tt * 1024;
@@ -465,7 +476,13 @@ extern "C" int w4a16_moe_ffn_act(w4a16_ctx* ctx, const char* name, uint64_t x_de
     // n_ff 1024 T = 512 80 / 83, T = 600 96 / 88; group 128, 64 experts top-6 n_ff 1408 T = 600 133 / 134, T = 700 155 / 152).
     if (ctx->moe_tiled > 0 && !E->scales_regular)
         return w4_fail(W4A16_ERR_UNSUPPORTED, "moe_ffn %s: the MFMA-tiled grouped kernels were requested (set_moe_tiled 1) but the experts hold a zero, non-finite or out-of-range scale; the streaming kernels serve them", name);
-    const bool tiled = ctx->moe_tiled > 0 || (ctx->moe_tiled == 0 && ctx->moe_block == 0 && E->scales_regular && ns >= 68 * E->n_exp);
+    // At group 32, with two block tiles of the gate|up launch per CU from one segment per expert alone, earlier: from 60, and from 40
+    // with folded scales, whose tiled kernels are freed of the running unit (128 experts, folded, T = 640 112 / 111, T = 768 122 / 115,
+    // T = 1024 160 / 149; f16 T = 896 156 / 154, T = 1024 183 / 172; 64 experts top-6 n_ff 1408, folded, T = 426 106 / 99, T = 682
+    // 141 / 132; but 32 experts top-4 n_ff 1024, folded, T = 384 56 / 62, T = 512 64 / 65: one block tile per CU).
+    const bool many = E->group == 32 && E->n_exp * ((E->n_ff + 127) / 128) >= 2 * (size_t)std::max(ctx->cu_count, 1);
+    const size_t tiled_from = !many ? 68 : E->fold ? 40 : 60;
+    const bool tiled = ctx->moe_tiled > 0 || (ctx->moe_tiled == 0 && ctx->moe_block == 0 && E->scales_regular && ns >= tiled_from * E->n_exp);
     const size_t block = tiled ? 64 : pick_block(ctx, t, ns, E->n_exp, top_k);
     if (block != 1 && block != 4 && block != 16 && block != 32 && block != 48 && block != 64)
         return w4_fail(W4A16_ERR_ARG, "moe_ffn %s: segment size %zu not in {1,4,16,32,48,64}", name, block);

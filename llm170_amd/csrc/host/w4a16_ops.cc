@@ -698,16 +698,17 @@ extern "C" int w4a16_gemm_host(w4a16_ctx* ctx, const uint16_t* x_f16, size_t t, 
 }
 
 // ------------------------------------------------------------------------------------------------ registration
-// Every magnitude m (bits without the sign) has lo <= m < hi, or is zero where zero_ok.  Four scales per 64-bit word: bit 15 of a
-// lane of m + 0x8000 - b is set exactly where m >= b, and no lane carries into the next.  (A model's scales are scanned on each
+// Every magnitude m (bits without the sign) has lo <= m < hi, or is zero where zero_ok; no sign is set where positive.  Four scales
+// per 64-bit word: bit 15 of a lane of m + 0x8000 - b is set exactly where m >= b, and no lane carries into the next.  (A model's scales are scanned on each
 // upload: 38 M of them, two expert layers, 13 ms; one at a time 41.)
-static bool scales_within(const uint16_t* sp, size_t count, unsigned lo, unsigned hi, bool zero_ok) {
+static bool scales_within(const uint16_t* sp, size_t count, unsigned lo, unsigned hi, bool zero_ok, bool positive = false) {
     constexpr uint64_t one = 0x0001000100010001ull, top = one << 15;
     const uint64_t from = one * (0x8000u - lo), to = one * (0x8000u - hi), nonzero = one * 0x7FFFu;
     uint64_t bad = 0;
     auto look = [&](uint64_t w) {
         const uint64_t m = w & ~top;
         bad |= (~(m + from) | (m + to)) & (zero_ok ? m + nonzero : top) & top;
+        if (positive) bad |= w & top;
     };
     size_t i = 0;
     for (; i + 4 <= count && !bad; i += 4) {
@@ -732,6 +733,8 @@ bool w4_bf16_fits_f16(const uint16_t* sp, size_t count) {
     // normal in f16: exponent 2^-14 .. 2^15, biased with 127; its seven mantissa bits always fit
     return scales_within(sp, count, (127u - 14u) << 7, (127u + 16u) << 7, true);
 }
+
+bool w4_bf16_folds(const uint16_t* sp, size_t count) { return scales_within(sp, count, (127u - 14u) << 7, (127u + 13u) << 7, false, true); }
 
 static void free_lin(w4a16_ctx* ctx, W4Lin& L) {
     (void)w4a16_free(ctx, L.q_raw);
@@ -759,6 +762,7 @@ extern "C" int w4a16_upload_lin(w4a16_ctx* ctx, const char* name, const void* q,
     // "regular": what the MFMA prefill kernel can carry as a running unit (w4_scales_regular).  Other linears are served
     // by the streaming kernels, which only ever multiply by a scale.
     L.scales_regular = w4_scales_regular(static_cast<const uint16_t*>(s), slen_bytes / 2, scale_bf16);
+    L.fold = scale_bf16 && group == 32 && w4_bf16_folds(static_cast<const uint16_t*>(s), slen_bytes / 2);
     int rc = w4a16_alloc(ctx, qlen_bytes, &L.q_raw);
     if (!rc) rc = w4a16_alloc(ctx, slen_bytes, &L.s_raw);
     if (!rc) rc = w4a16_h2d(ctx, L.q_raw, q, qlen_bytes);
@@ -792,6 +796,7 @@ extern "C" int w4a16_lin_fuse(w4a16_ctx* ctx, const char* name, const char* cons
             F.k = L.k;
             F.group = L.group;
             F.scale_bf16 = L.scale_bf16;
+            F.fold = L.fold;
         } else if (L.k != F.k || L.group != F.group || L.scale_bf16 != F.scale_bf16) {
             return w4_fail(W4A16_ERR_SHAPE, "lin_fuse %s: part %s (k=%zu g=%zu bf16=%d) does not match k=%zu g=%zu bf16=%d",
                            name, parts[i], L.k, L.group, L.scale_bf16, F.k, F.group, F.scale_bf16);
@@ -799,6 +804,7 @@ extern "C" int w4a16_lin_fuse(w4a16_ctx* ctx, const char* name, const char* cons
         F.n += L.n;
         F.part_n.push_back(L.n);
         F.scales_regular = F.scales_regular && L.scales_regular;
+        F.fold = F.fold && L.fold;
     }
     if (F.n > 0x7fffffffu) return w4_fail(W4A16_ERR_SHAPE, "lin_fuse %s: n=%zu too large", name, F.n);
     const size_t q_row = F.k / 2, s_row = (F.k / F.group) * 2;

@@ -21,6 +21,10 @@
 // Measured against the grouped expert kernel that served these rows before (us, before / now): gated 34816 x 5120 t = 64
 // 49.8 / 34.7, t = 32 34.3 / 27.8; gated 22016 x 4096 t = 64 30.3 / 20.9; 16384 x 4096 t = 40 21.7 / 15.5; 5120 x 5120 t = 64
 // 18.6 / 14.5; 5120 x 2048 group 32 t = 37 12.8 / 7.1; 17408 x 5120 t = 64 35.8 / 24.9; 512 x 17408 t = 40 20.4 / 10.7.
+// FOLD (group 32, bf16 scales; rule at the launch, w4a16_moe.cc): scales multiplied into the weights (w4_deq8_scaled), a k tile's four
+// MFMAs summed from zero and added once, a quarter of the additions and no scale to spread over the accumulators.  us, scaled sums /
+// folded: 34816 x 5120 t = 64 52.5 / 45.5, t = 48 43.3 / 36.9, t = 20 33.4 / 30.9; gated 22016 x 4096 t = 40 20.9 / 18.9; 7168 x 5120
+// t = 30 10.66 / 10.65.
 // (The full wait at the barriers costs the gated 34816 x 5120 at t = 64 1 us, the other shapes of the timing cases nothing.)
 #include "w4a16_common.hpp"
 
@@ -51,7 +55,7 @@ __device__ __forceinline__ f4_t mid_scale4(unsigned d0, unsigned d1) {
         int row_blocks, int k, int n, int t, int out_f16, int act_kind, f4_t *ws, int *tickets, int nks, int gp
 #define MID_ARGS qt, st, x, y, row_blocks, k, n, t, out_f16, act_kind, ws, tickets, nks, gp
 
-template <int G, bool SBF, bool GLU, int TT, int WN, int WK>
+template <int G, bool SBF, bool GLU, int TT, int WN, int WK, bool FOLD>
 __device__ __forceinline__ void mid_body(MID_PARAMS) {
     extern __shared__ __attribute__((aligned(16))) _Float16 xs[];
     constexpr int GPT = W4_TILE_K / G, ROWS = 16 * TT, XL = (4 * TT + WN - 1) / WN, NBUF = WN > 1 ? 2 : 1;
@@ -81,9 +85,12 @@ __device__ __forceinline__ void mid_body(MID_PARAMS) {
     const unsigned qoff[2] = {(unsigned)rbA * (unsigned)kt_n * 1024u + (unsigned)lane * 16u,
                               (unsigned)rbB * (unsigned)kt_n * 1024u + (unsigned)lane * 16u};
     // scale loads: group 128: one, lane l of a quad fetches row block l & 1; group 32: one per row block, lane l of a quad
-    // fetches group l of the k tile
+    // fetches group l of the k tile; FOLD: one per row block, one of the k tile's 64 scales per lane
     unsigned soff[SL];
-    if constexpr (G == 128) {
+    if constexpr (FOLD) {
+        soff[0] = (unsigned)rbA * (unsigned)kg_n * 32u + (unsigned)lane * 2u;
+        soff[1] = (unsigned)rbB * (unsigned)kg_n * 32u + (unsigned)lane * 2u;
+    } else if constexpr (G == 128) {
         soff[0] = (unsigned)((lane & 1) ? rbB : rbA) * (unsigned)kg_n * 32u + (unsigned)q * 8u;
     } else {
         soff[0] = (unsigned)rbA * (unsigned)kg_n * 32u + (unsigned)(lane & 3) * 32u + (unsigned)q * 8u;
@@ -118,7 +125,10 @@ __device__ __forceinline__ void mid_body(MID_PARAMS) {
 #pragma unroll
         for (int rb = 0; rb < 2; rb++) s_.q[rb] = __builtin_amdgcn_raw_buffer_load_b128(qr, qoff[rb], kt * 1024, 2);
 #pragma unroll
-        for (int l = 0; l < SL; l++) s_.s[l] = __builtin_amdgcn_raw_buffer_load_b64(sr, soff[l], kt * (GPT * 32), 0);
+        for (int l = 0; l < SL; l++) {
+            if constexpr (FOLD) s_.s[l][0] = __builtin_amdgcn_raw_buffer_load_b16(sr, soff[l], kt * (GPT * 32), 0);
+            else s_.s[l] = __builtin_amdgcn_raw_buffer_load_b64(sr, soff[l], kt * (GPT * 32), 0);
+        }
     };
     auto load_x = [&](int kt, int buf) {
         const __amdgpu_buffer_rsrc_t xr = w4_make_rsrc(x, kt < kt1 ? x_bytes : 0u);
@@ -148,6 +158,11 @@ __device__ __forceinline__ void mid_body(MID_PARAMS) {
         const _Float16* xb = xg + buf * (ROWS * LDX);
         const f4_t zero = {0.f, 0.f, 0.f, 0.f};
         f4_t part[2][TT];
+        unsigned fold[2][4];  // FOLD: f16 scales of the lane's weight row, per row block and MFMA
+        if constexpr (FOLD) {
+#pragma unroll
+            for (int rb = 0; rb < 2; rb++) w4_spread_groups(SBF ? w4_bf16_to_f16(s_.s[rb][0]) : s_.s[rb][0], fold[rb]);
+        }
         auto scaled = [&](int rb, unsigned d0, unsigned d1) {
             const f4_t sc = mid_scale4<SBF>(d0, d1);
 #pragma unroll
@@ -160,12 +175,19 @@ __device__ __forceinline__ void mid_body(MID_PARAMS) {
             for (int tt = 0; tt < TT; tt++) b[tt] = *reinterpret_cast<const h8_t*>(xb + x_get[w] + tt * 16 * LDX);
 #pragma unroll
             for (int rb = 0; rb < 2; rb++) {
+                if constexpr (FOLD) {
+                    const h8_t a = w4_deq8_scaled(s_.q[rb][w], fold[rb][w]);
+#pragma unroll
+                    for (int tt = 0; tt < TT; tt++)
+                        part[rb][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[tt], w == 0 ? zero : part[rb][tt], 0, 0, 0);
+                    continue;
+                }
                 const h8_t a = w4_deq8(s_.q[rb][w]);
 #pragma unroll
                 for (int tt = 0; tt < TT; tt++)
                     part[rb][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[tt], (G == 32 || w == 0) ? zero : part[rb][tt], 0, 0, 0);
             }
-            if constexpr (G == 32) {
+            if constexpr (G == 32 && !FOLD) {
 #pragma unroll
                 for (int rb = 0; rb < 2; rb++) {
                     const u2_t s2 = s_.s[rb];
@@ -177,6 +199,12 @@ __device__ __forceinline__ void mid_body(MID_PARAMS) {
                     scaled(rb, d0, d1);
                 }
             }
+        }
+        if constexpr (FOLD) {
+#pragma unroll
+            for (int rb = 0; rb < 2; rb++)
+#pragma unroll
+                for (int tt = 0; tt < TT; tt++) acc[rb][tt] += part[rb][tt];
         }
         if constexpr (G == 128) {
             scaled(0, mid_quad_bcast<0>(s_.s[0][0]), mid_quad_bcast<0>(s_.s[0][1]));
@@ -376,27 +404,28 @@ __device__ __forceinline__ void mid_body(MID_PARAMS) {
     }
 }
 
-#define MID_KERNEL(NAME, G, SBF, GLU, TT, WN, WK)                                                                      \
+#define MID_KERNEL(NAME, G, SBF, GLU, TT, WN, WK, FOLD)                                                                \
     extern "C" __global__ __launch_bounds__(WN * WK * 64) __attribute__((amdgpu_waves_per_eu(MID_WPE(WN, WK)))) void NAME( \
         MID_PARAMS) {                                                                                                      \
-        mid_body<G, SBF, GLU, TT, WN, WK>(MID_ARGS);                                                                       \
+        mid_body<G, SBF, GLU, TT, WN, WK, FOLD>(MID_ARGS);                                                                       \
     }
 #define MID_WPE(WN, WK) (WN * WK > 8 ? 3 : 2)
-#define MID_FAMILY(PFX, G, SBF, TT)                               \
-    MID_KERNEL(PFX##_t##TT##_n1k4, G, SBF, false, TT, 1, 4)       \
-    MID_KERNEL(PFX##_t##TT##_n1k4_glu, G, SBF, true, TT, 1, 4)    \
-    MID_KERNEL(PFX##_t##TT##_n2k4, G, SBF, false, TT, 2, 4)       \
-    MID_KERNEL(PFX##_t##TT##_n2k4_glu, G, SBF, true, TT, 2, 4)    \
-    MID_KERNEL(PFX##_t##TT##_n3k4, G, SBF, false, TT, 3, 4)       \
-    MID_KERNEL(PFX##_t##TT##_n3k4_glu, G, SBF, true, TT, 3, 4)    \
-    MID_KERNEL(PFX##_t##TT##_n4k1, G, SBF, false, TT, 4, 1)       \
-    MID_KERNEL(PFX##_t##TT##_n4k1_glu, G, SBF, true, TT, 4, 1)    \
-    MID_KERNEL(PFX##_t##TT##_n4k2, G, SBF, false, TT, 4, 2)       \
-    MID_KERNEL(PFX##_t##TT##_n4k2_glu, G, SBF, true, TT, 4, 2)    \
-    MID_KERNEL(PFX##_t##TT##_n5k2, G, SBF, false, TT, 5, 2)       \
-    MID_KERNEL(PFX##_t##TT##_n5k2_glu, G, SBF, true, TT, 5, 2)
-#define MID_FAMILIES(PFX, G, SBF) MID_FAMILY(PFX, G, SBF, 2) MID_FAMILY(PFX, G, SBF, 3) MID_FAMILY(PFX, G, SBF, 4)
-MID_FAMILIES(w4a16_mid_g128_f16, 128, false)
-MID_FAMILIES(w4a16_mid_g128_bf16, 128, true)
-MID_FAMILIES(w4a16_mid_g32_f16, 32, false)
-MID_FAMILIES(w4a16_mid_g32_bf16, 32, true)
+#define MID_FAMILY(PFX, G, SBF, TT, FOLD)                         \
+    MID_KERNEL(PFX##_t##TT##_n1k4, G, SBF, false, TT, 1, 4, FOLD)       \
+    MID_KERNEL(PFX##_t##TT##_n1k4_glu, G, SBF, true, TT, 1, 4, FOLD)    \
+    MID_KERNEL(PFX##_t##TT##_n2k4, G, SBF, false, TT, 2, 4, FOLD)       \
+    MID_KERNEL(PFX##_t##TT##_n2k4_glu, G, SBF, true, TT, 2, 4, FOLD)    \
+    MID_KERNEL(PFX##_t##TT##_n3k4, G, SBF, false, TT, 3, 4, FOLD)       \
+    MID_KERNEL(PFX##_t##TT##_n3k4_glu, G, SBF, true, TT, 3, 4, FOLD)    \
+    MID_KERNEL(PFX##_t##TT##_n4k1, G, SBF, false, TT, 4, 1, FOLD)       \
+    MID_KERNEL(PFX##_t##TT##_n4k1_glu, G, SBF, true, TT, 4, 1, FOLD)    \
+    MID_KERNEL(PFX##_t##TT##_n4k2, G, SBF, false, TT, 4, 2, FOLD)       \
+    MID_KERNEL(PFX##_t##TT##_n4k2_glu, G, SBF, true, TT, 4, 2, FOLD)    \
+    MID_KERNEL(PFX##_t##TT##_n5k2, G, SBF, false, TT, 5, 2, FOLD)       \
+    MID_KERNEL(PFX##_t##TT##_n5k2_glu, G, SBF, true, TT, 5, 2, FOLD)
+#define MID_FAMILIES(PFX, G, SBF, FOLD) MID_FAMILY(PFX, G, SBF, 2, FOLD) MID_FAMILY(PFX, G, SBF, 3, FOLD) MID_FAMILY(PFX, G, SBF, 4, FOLD)
+MID_FAMILIES(w4a16_mid_g128_f16, 128, false, false)
+MID_FAMILIES(w4a16_mid_g128_bf16, 128, true, false)
+MID_FAMILIES(w4a16_mid_g32_f16, 32, false, false)
+MID_FAMILIES(w4a16_mid_g32_bf16, 32, true, false)
+MID_FAMILIES(w4a16_mid_g32_bf16x, 32, true, true)

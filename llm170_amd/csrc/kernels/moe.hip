@@ -422,15 +422,15 @@ MOE_DOWN_SUM_KERNEL(w4a16_moe_g128_f16_down_sum1, 128, false, 1)
 MOE_DOWN_SUM_KERNEL(w4a16_moe_g128_bf16_down_sum1, 128, true, 1)
 
 // ---------------------------------------------------------------------------------------------------- moe_mm
-template <int RB>
+template <int RB, bool FOLD>
 struct MoeMmStage {
     u4_t q[RB];
-    u2_t s[RB];
+    typename std::conditional<FOLD, unsigned, u2_t>::type s[RB];
 };
 
 // One block = (segment of blk = 16*TT slots, group of W units); wave w owns unit group*W + w over the whole k range.
 // TT: the 16-slot blocks of the segment this workgroup multiplies (those that hold a slot).  KT: k tiles per stage.
-template <int G, bool SBF, bool GLU, int TT, int KT>
+template <int G, bool SBF, bool GLU, int TT, int KT, bool FOLD>
 __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
     extern __shared__ _Float16 xs[];  // [2][KT][16*TT][128]
     constexpr int GPT = W4_TILE_K / G;
@@ -488,17 +488,21 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
 
     const unsigned qoff[2] = {(unsigned)rbA * (unsigned)kt_n * 1024u + (unsigned)lane * 16u,
                               (unsigned)rbB * (unsigned)kt_n * 1024u + (unsigned)lane * 16u};
-    const unsigned sg = G == 32 ? (unsigned)(lane & 3) * 32u : 0u;
-    const unsigned soff[2] = {(unsigned)rbA * (unsigned)kg_n * 32u + sg + (unsigned)q * 8u,
-                              (unsigned)rbB * (unsigned)kg_n * 32u + sg + (unsigned)q * 8u};
-    MoeMmStage<2> stage[2][KT];
-    auto load_w = [&](MoeMmStage<2>& s_, int kt) {
+    // scales: FOLD: one of the k tile's 64 per lane; else the four rows of the lane's results, group 32: of group lane % 4
+    const unsigned sg = FOLD ? (unsigned)lane * 2u : (G == 32 ? (unsigned)(lane & 3) * 32u : 0u) + (unsigned)q * 8u;
+    const unsigned soff[2] = {(unsigned)rbA * (unsigned)kg_n * 32u + sg, (unsigned)rbB * (unsigned)kg_n * 32u + sg};
+    typedef MoeMmStage<2, FOLD> Stage;
+    Stage stage[2][KT];
+    auto load_w = [&](Stage& s_, int kt) {
         const bool live = kt < kt_n;
         const __amdgpu_buffer_rsrc_t qr = w4_make_rsrc(qe, live ? q_bytes : 0u), sr = w4_make_rsrc(se, live ? s_bytes : 0u);
 #pragma unroll
         for (int rb = 0; rb < 2; rb++) s_.q[rb] = __builtin_amdgcn_raw_buffer_load_b128(qr, qoff[rb], kt * 1024, 2);
 #pragma unroll
-        for (int rb = 0; rb < 2; rb++) s_.s[rb] = __builtin_amdgcn_raw_buffer_load_b64(sr, soff[rb], kt * (GPT * 32), 0);
+        for (int rb = 0; rb < 2; rb++) {
+            if constexpr (FOLD) s_.s[rb] = __builtin_amdgcn_raw_buffer_load_b16(sr, soff[rb], kt * (GPT * 32), 0);
+            else s_.s[rb] = __builtin_amdgcn_raw_buffer_load_b64(sr, soff[rb], kt * (GPT * 32), 0);
+        }
     };
 
     f4_t acc[2][TT];
@@ -507,7 +511,7 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
 #pragma unroll
         for (int tt = 0; tt < TT; tt++) acc[rb][tt] = (f4_t){0.f, 0.f, 0.f, 0.f};
 
-    auto compute = [&](const MoeMmStage<2>& s_, int buf) {
+    auto compute = [&](const auto& s_, int buf) {
         const _Float16* xb = xs + buf * (ROWS * 128);
         const f4_t zero = {0.f, 0.f, 0.f, 0.f};
         f4_t part[2][TT];
@@ -561,7 +565,7 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
     // MFMA for the other waves to fill).  Scheduling barriers hold the phases in this order; one group's results are
     // live at a time.  128 experts, top-8: T = 64 77.6 -> 76.1 us, T = 512 117.9 -> 115.6 us; with four blocks the
     // extra registers cost a wave per SIMD (T = 1024 +2 %), so 64-slot segments keep the plain order.
-    auto compute32 = [&](const MoeMmStage<2>& s_, int buf) {
+    auto compute32 = [&](const auto& s_, int buf) {
         const _Float16* xb = xs + buf * (ROWS * 128);
         const f4_t zero = {0.f, 0.f, 0.f, 0.f};
         h8_t b[TT];
@@ -605,6 +609,38 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
         group(std::integral_constant<int, 7>{});
     };
 
+    // FOLD: scaled weights (w4_deq8_scaled), sums straight in the accumulators: at three 16-slot blocks a third of the vector ALU work of
+    // scaled group sums is gone.  A k tile is eight groups (32 k x one row block), issued like those of compute32: a group's MFMAs, then
+    // the next group's unpack, the B operands of the next 32 k one group early (in the order the compiler finds by itself 128 experts
+    // top-8 take 74.2 instead of 71.7 us per FFN at T = 64).  Scaled sums / folded, us per FFN: 128 experts T = 200 83.2 / 81.8, T = 517
+    // 119.6 / 108.9, T = 800 152 / 132; 8 experts top-2 n_ff 3584 T = 64 67.1 / 62.7, T = 150 82.9 / 72.1; T = 64 71.4 / 71.7, T = 32 69.6
+    // / 70.0, so runs below eight slots per expert keep the scaled sums (rule at the launch).  The results' distance from 64-bit sums is
+    // that of the f16 intermediates, 4.0e-4, to four digits either way.
+    auto compute_fold = [&](const auto& s_, int buf) {
+        const _Float16* xb = xs + buf * (ROWS * 128);
+        unsigned sc[2][4];
+        h8_t b[2][TT];
+#pragma unroll
+        for (int tt = 0; tt < TT; tt++) b[0][tt] = *reinterpret_cast<const h8_t*>(xb + x_get[0] + tt * 16 * 128);
+#pragma unroll
+        for (int rb = 0; rb < 2; rb++) w4_spread_groups(s_.s[rb], sc[rb]);
+        h8_t a = w4_deq8_scaled(s_.q[0][0], sc[0][0]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int g = 0; g < 8; g++) {
+            const int w = g >> 1, rb = g & 1;
+            if (rb == 0 && w < 3) {
+#pragma unroll
+                for (int tt = 0; tt < TT; tt++) b[(w + 1) & 1][tt] = *reinterpret_cast<const h8_t*>(xb + x_get[w + 1] + tt * 16 * 128);
+            }
+#pragma unroll
+            for (int tt = 0; tt < TT; tt++) acc[rb][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[w & 1][tt], acc[rb][tt], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (g < 7) a = w4_deq8_scaled(s_.q[(g + 1) & 1][(g + 1) >> 1], sc[(g + 1) & 1][(g + 1) >> 1]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
     // one stage ahead: its DMA and weights are issued ahead of this stage's MFMAs and waited for (vmcnt 0) at the barrier
     // that ends them.  Few registers, many waves: x in flight in registers and weights two (group 32) or four (group 128) tiles
     // ahead, the wait for x behind the youngest weights, were slower throughout (128 experts, us per FFN: group 32 f16 T = 64
@@ -629,7 +665,8 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
 #pragma unroll
             for (int j = 0; j < KT; j++)
                 if (kt + j < kt_n) {
-                    if constexpr (G == 32 && TT <= 3) compute32(stage[d][j], d * KT + j);
+                    if constexpr (FOLD) compute_fold(stage[d][j], d * KT + j);
+                    else if constexpr (G == 32 && TT <= 3) compute32(stage[d][j], d * KT + j);
                     else compute(stage[d][j], d * KT + j);
                 }
             __builtin_amdgcn_s_setprio(0);
@@ -651,20 +688,20 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
 // 16-slot block tells whether the block holds any: the workgroup runs the body built for the blocks that do, and the
 // MFMAs, scaled sums and x rows of all-padding blocks are never issued (128 experts, top-8, T = 512: runs of 32 +- 6
 // slots in 48-slot segments, every other expert fills two blocks of three).
-template <int G, bool SBF, bool GLU, int TT, int KT>
+template <int G, bool SBF, bool GLU, int TT, int KT, bool FOLD>
 __device__ __forceinline__ void moe_mm_entry(MOE_PARAMS) {
     if constexpr (TT == 1) {
-        moe_mm_body<G, SBF, GLU, 1, KT>(MOE_ARGS);
+        moe_mm_body<G, SBF, GLU, 1, KT, FOLD>(MOE_ARGS);
     } else {
         const int units = GLU ? row_blocks >> 1 : (row_blocks + 1) >> 1;
         const int seg = blockIdx.x / ((units + wpb - 1) / wpb);
         int live = 1;
 #pragma unroll
         for (int p = 1; p < TT; p++) live += sorted_ids[seg * blk + 16 * p] < ns ? 1 : 0;
-        if (live == 1) moe_mm_body<G, SBF, GLU, 1, KT>(MOE_ARGS);
-        else if (TT == 2 || live == 2) moe_mm_body<G, SBF, GLU, 2, KT>(MOE_ARGS);
-        else if (TT == 3 || live == 3) moe_mm_body<G, SBF, GLU, TT >= 3 ? 3 : 2, KT>(MOE_ARGS);
-        else moe_mm_body<G, SBF, GLU, TT, KT>(MOE_ARGS);
+        if (live == 1) moe_mm_body<G, SBF, GLU, 1, KT, FOLD>(MOE_ARGS);
+        else if (TT == 2 || live == 2) moe_mm_body<G, SBF, GLU, 2, KT, FOLD>(MOE_ARGS);
+        else if (TT == 3 || live == 3) moe_mm_body<G, SBF, GLU, TT >= 3 ? 3 : 2, KT, FOLD>(MOE_ARGS);
+        else moe_mm_body<G, SBF, GLU, TT, KT, FOLD>(MOE_ARGS);
     }
 }
 
@@ -672,10 +709,11 @@ __device__ __forceinline__ void moe_mm_entry(MOE_PARAMS) {
     extern "C" __global__ __launch_bounds__(512) void NAME(MOE_PARAMS) {              \
         moe_dec_body<G, SBF, GLU, XL, DEPTH>(MOE_ARGS);                               \
     }
-#define MOE_MM_KERNEL(NAME, G, SBF, GLU, TT, KT)                                      \
+#define MOE_MM_BUILD(NAME, G, SBF, GLU, TT, KT, FOLD)                                 \
     extern "C" __global__ __launch_bounds__(512) void NAME(MOE_PARAMS) {              \
-        moe_mm_entry<G, SBF, GLU, TT, KT>(MOE_ARGS);                                  \
+        moe_mm_entry<G, SBF, GLU, TT, KT, FOLD>(MOE_ARGS);                            \
     }
+#define MOE_MM_KERNEL(NAME, G, SBF, GLU, TT, KT) MOE_MM_BUILD(NAME, G, SBF, GLU, TT, KT, false)
 // Ring depths of the streaming kernels, from sweeps on the 128-expert shape: the one-slot segments of the direct mode run
 // best with two k tiles in flight per wave (T = 4..12: 9-11 % faster than four: fewer registers, more waves resident at
 // once); so do the segments of up to 16 slots (5 % faster than three).
@@ -697,6 +735,16 @@ MOE_FAMILY(w4a16_moe_g32_f16, 32, false)
 MOE_FAMILY(w4a16_moe_g32_bf16, 32, true)
 MOE_FAMILY(w4a16_moe_g128_f16, 128, false)
 MOE_FAMILY(w4a16_moe_g128_bf16, 128, true)
+
+// Folded scales (f16x: arenas of bf16 scales kept as f16, W4Experts::fold)
+#define MOE_MM_FOLD(PFX)                                    \
+    MOE_MM_BUILD(PFX##_mm_glu_t2, 32, false, true, 2, 1, true)   \
+    MOE_MM_BUILD(PFX##_mm_glu_t3, 32, false, true, 3, 1, true)   \
+    MOE_MM_BUILD(PFX##_mm_glu_t4, 32, false, true, 4, 1, true)   \
+    MOE_MM_BUILD(PFX##_mm_lin_t2, 32, false, false, 2, 1, true)  \
+    MOE_MM_BUILD(PFX##_mm_lin_t3, 32, false, false, 3, 1, true)  \
+    MOE_MM_BUILD(PFX##_mm_lin_t4, 32, false, false, 4, 1, true)
+MOE_MM_FOLD(w4a16_moe_g32_f16x)
 
 // Two k tiles per stage, for launches of few workgroups (the rule is at the launch, w4a16_moe.cc): one tile in flight per wave
 // does not cover the trip to memory there.  Group 128, whose tiles take least time to multiply.  8 experts top-2, h 4096, n_ff

@@ -89,7 +89,11 @@ struct PfEpi {
     float inv_cols_in, in_scale, out_scale;
 };
 
-template <int G, bool SBF, int MI, int MODE = 0, int WNW = 4, int KG = 1>
+// FOLD (grouped form, group 32): scales multiplied into the weights (w4_deq8_scaled), no running unit: 7 instead of 18 vector ALU
+// instructions per MFMA.  128 experts top-8 n_ff 768, us per FFN: T = 2048 265 -> 232, T = 1152 188 -> 168.  Dense linears keep the
+// unit: their f32 results would lie 15 % further from 64-bit sums (5120 x 5120 t = 1024 2.6e-7 instead of 2.3e-7), which the f16
+// rows of the expert FFN do not show (4.0e-4 either way).  us they would save: 34816 x 5120 t = 2048 773 -> 657.
+template <int G, bool SBF, int MI, int MODE = 0, int WNW = 4, int KG = 1, bool FOLD = false>
 __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const uint16_t* __restrict__ st,
                                              const uint16_t* __restrict__ x, void* __restrict__ y, int row_blocks,
                                              int k, int n, int t, int out_f16, int sup_m, int sup_n,
@@ -290,7 +294,7 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
                 // scheduler the same lost 0.4-0.9 % on the faster boxes).  Group 32 rescales inside the stage and has no
                 // such stretch.
                 if (PF_WAVE_PRIO && kbl == 0) __builtin_amdgcn_s_setprio(1);
-                const bool boundary32 = G == 32 && h == 0;
+                const bool boundary32 = G == 32 && h == 0 && !FOLD;
                 float ratio[2] = {1.f, 1.f};
                 if (boundary32) {
 #pragma unroll
@@ -324,7 +328,9 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
                 }
 #pragma unroll
                 for (int ni = 0; ni < 2; ni++) {
-                    const h8_t b = w4_deq8(bq[ni][h][w]);
+                    h8_t b;
+                    if constexpr (FOLD) b = w4_deq8_scaled(bq[ni][h][w], sc[ni][w]);
+                    else b = w4_deq8(bq[ni][h][w]);
 #pragma unroll
                     for (int mi = 0; mi < MI; mi++) {
                         if (boundary32) acc[mi][ni] *= ratio[ni];
@@ -613,7 +619,7 @@ __device__ __forceinline__ bool pf_moe_tile(PfGroup<MODE>& gp, const int* num_po
 
 // Grouped kernels for the expert FFN: same arguments as the streaming grouped kernels of moe.hip (blk must be 64, the
 // rows of a block tile, and y_f16 1: the host refuses others; wpb is unused).
-#define PREFILL_MOE_KERNEL(NAME, G, SBF, MODE)                                                                        \
+#define PREFILL_MOE_BUILD(NAME, G, SBF, MODE, FOLD)                                                                   \
     extern "C" __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(3, 3))) void NAME(            \
         const char* qa, const char* sa, unsigned long long q_stride, unsigned long long s_stride, const uint16_t* x,      \
         int x_rows, int x_div, void* y, int y_f16, const float* topw, const int* sorted_ids, const int* expert_ids,      \
@@ -635,9 +641,11 @@ __device__ __forceinline__ bool pf_moe_tile(PfGroup<MODE>& gp, const int* num_po
         if (!pf_moe_tile<MODE>(gp, num_post, n, &rows)) return;                                                          \
         const u4_t* qt = reinterpret_cast<const u4_t*>(qa);                                                              \
         const uint16_t* st = reinterpret_cast<const uint16_t*>(sa);                                                      \
-        if (rows <= 32) prefill_body<G, SBF, 1, MODE>(qt, st, x, y, row_blocks, k, n, 0, y_f16, 1, 1, gp);         \
-        else prefill_body<G, SBF, 2, MODE>(qt, st, x, y, row_blocks, k, n, 0, y_f16, 1, 1, gp);                    \
+        if (rows <= 32) prefill_body<G, SBF, 1, MODE, 4, 1, FOLD>(qt, st, x, y, row_blocks, k, n, 0, y_f16, 1, 1, gp);         \
+        else prefill_body<G, SBF, 2, MODE, 4, 1, FOLD>(qt, st, x, y, row_blocks, k, n, 0, y_f16, 1, 1, gp);                    \
     }
+
+#define PREFILL_MOE_KERNEL(NAME, G, SBF, MODE) PREFILL_MOE_BUILD(NAME, G, SBF, MODE, false)
 
 // This file builds two code objects.  Compiled on its own it holds everything but the dense group-128 kernels;
 // prefill_g128.hip includes it with PF_DENSE_G128 defined and holds those (the k-group ones as well), built with the backend's max-ILP
@@ -775,6 +783,8 @@ PREFILL_MOE_KERNEL(w4a16_moe_g128_bf16_pf_glu, 128, true, 1)
 PREFILL_MOE_KERNEL(w4a16_moe_g128_bf16_pf_lin, 128, true, 2)
 PREFILL_MOE_KERNEL(w4a16_moe_g32_f16_pf_glu, 32, false, 1)
 PREFILL_MOE_KERNEL(w4a16_moe_g32_f16_pf_lin, 32, false, 2)
+PREFILL_MOE_BUILD(w4a16_moe_g32_f16x_pf_glu, 32, false, 1, true)
+PREFILL_MOE_BUILD(w4a16_moe_g32_f16x_pf_lin, 32, false, 2, true)
 PREFILL_MOE_KERNEL(w4a16_moe_g32_bf16_pf_glu, 32, true, 1)
 PREFILL_MOE_KERNEL(w4a16_moe_g32_bf16_pf_lin, 32, true, 2)
 #endif

@@ -58,6 +58,33 @@ __device__ __forceinline__ h8_t w4_deq8(unsigned w) {
     return r;
 }
 
+// The eight weights of a dword times their scale, (nibble - 8) * s, as f16: exact where every scale has at most eight significant
+// bits (bf16) and is a normal f16 number below 8192, or zero: |nibble - 8| <= 7 adds three bits, 8 is a power of two, and an f16
+// holds eleven.  Such weights enter the MFMA as they are and no sum is scaled afterwards.  s: f16 bits in the low half.
+// 13 VALU ops per dword.
+__device__ __forceinline__ h8_t w4_deq8_scaled(unsigned w, unsigned s) {
+    const _Float16 v = __builtin_bit_cast(_Float16, (unsigned short)s);
+    return w4_deq8(w) * (h8_t){v, v, v, v, v, v, v, v};
+}
+
+// bf16 bits -> f16 bits, exact for the scales w4_deq8_scaled takes.
+__device__ __forceinline__ unsigned w4_bf16_to_f16(unsigned b) {
+    return __builtin_bit_cast(unsigned short, (_Float16)__builtin_bit_cast(float, b << 16));
+}
+
+// The four scale groups of a k tile of one row block at group 32 (64 scales, [4 groups][16 rows]), one scale per lane in: out[w] =
+// lane l's row (l % 16) of group w, so a lane holds what its weight row is multiplied by.  Rows of 16 lanes are exchanged by
+// v_permlane32_swap / v_permlane16_swap.
+__device__ __forceinline__ void w4_spread_groups(unsigned v, unsigned (&out)[4]) {
+    const auto half = __builtin_amdgcn_permlane32_swap(v, v, false, false);  // lanes rows {0, 1, 0, 1}, {2, 3, 2, 3}
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const auto row = __builtin_amdgcn_permlane16_swap(half[i], half[i], false, false);
+        out[2 * i] = row[0];
+        out[2 * i + 1] = row[1];
+    }
+}
+
 // Raw buffer descriptor over [base, base + bytes): loads whose byte offset falls outside return 0 and touch no
 // memory, which gives branch-free predication of per-lane loads.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t w4_make_rsrc(const void* base, unsigned bytes) {
