@@ -79,15 +79,15 @@ extern "C" int w4a16_upload_experts(w4a16_ctx* ctx, const char* name, size_t n_e
     E.n_ff = n_ff;
     E.group = group;
     E.scale_bf16 = scale_bf16 ? 1 : 0;
-    // the MFMA-tiled grouped kernels carry the running unit of the prefill kernel: they are taken only for arenas
-    // whose every scale that kernel can divide by (the streaming kernels only multiply by scales and take any)
-    E.scales_regular = w4_scales_regular(static_cast<const uint16_t*>(s13), s13_bytes / 2, scale_bf16) &&
-                       w4_scales_regular(static_cast<const uint16_t*>(s2), s2_bytes / 2, scale_bf16);
-    // bf16 scales that f16 holds exactly are stored as f16: the f16 kernels read the same values without a conversion per scale
     auto all = [&](bool (*test)(const uint16_t*, size_t)) {
         return test(static_cast<const uint16_t*>(s13), s13_bytes / 2) && test(static_cast<const uint16_t*>(s2), s2_bytes / 2);
     };
-    E.fold = scale_bf16 && group == 32 && all(w4_bf16_folds);
+    E.fold = scale_bf16 && group == 32 && all(w4_bf16_folds);  // the narrowest range: no further scan
+    // the MFMA-tiled grouped kernels carry the running unit of the prefill kernel: they are taken only for arenas
+    // whose every scale that kernel can divide by (the streaming kernels only multiply by scales and take any)
+    E.scales_regular = E.fold || (w4_scales_regular(static_cast<const uint16_t*>(s13), s13_bytes / 2, scale_bf16) &&
+                                  w4_scales_regular(static_cast<const uint16_t*>(s2), s2_bytes / 2, scale_bf16));
+    // bf16 scales that f16 holds exactly are stored as f16: the f16 kernels read the same values without a conversion per scale
     const bool to_f16 = E.fold || (scale_bf16 && all(w4_bf16_fits_f16));
     E.tiled_bf16 = scale_bf16 && !to_f16;
     int rc = tile_arena(ctx, q13, s13, n_experts, 2 * n_ff, h, group, to_f16, &E.q13, &E.s13, &E.q13_stride, &E.s13_stride);

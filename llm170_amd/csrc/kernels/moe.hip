@@ -488,9 +488,10 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
 
     const unsigned qoff[2] = {(unsigned)rbA * (unsigned)kt_n * 1024u + (unsigned)lane * 16u,
                               (unsigned)rbB * (unsigned)kt_n * 1024u + (unsigned)lane * 16u};
-    // scales: FOLD: one of the k tile's 64 per lane; else the four rows of the lane's results, group 32: of group lane % 4
-    const unsigned sg = FOLD ? (unsigned)lane * 2u : (G == 32 ? (unsigned)(lane & 3) * 32u : 0u) + (unsigned)q * 8u;
-    const unsigned soff[2] = {(unsigned)rbA * (unsigned)kg_n * 32u + sg, (unsigned)rbB * (unsigned)kg_n * 32u + sg};
+    // scales: the four rows of the lane's results (group 32: of group lane % 4); FOLD: one of the k tile's 64 per lane
+    const unsigned sg = G == 32 ? (unsigned)(lane & 3) * 32u : 0u;
+    const unsigned soff[2] = {FOLD ? (unsigned)rbA * (unsigned)kg_n * 32u + (unsigned)lane * 2u : (unsigned)rbA * (unsigned)kg_n * 32u + sg + (unsigned)q * 8u,
+                              FOLD ? (unsigned)rbB * (unsigned)kg_n * 32u + (unsigned)lane * 2u : (unsigned)rbB * (unsigned)kg_n * 32u + sg + (unsigned)q * 8u};
     typedef MoeMmStage<2, FOLD> Stage;
     Stage stage[2][KT];
     auto load_w = [&](Stage& s_, int kt) {
