@@ -309,7 +309,7 @@ def plan_sweep(out_path):
         for t in PLAN_SWEEP_T:
             rows = []
             for tile in (64, 96, 128):
-                for ks in (1, 2, 3, 4, 6, 8):
+                for ks in (1, 2, 3, 4, 5, 6, 7, 8):
                     if ks > 1 and ks > (k // 128) // 4:
                         continue
                     dec.set_prefill_tile(tile)

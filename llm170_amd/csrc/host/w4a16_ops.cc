@@ -410,7 +410,7 @@ static int launch_decode_glu(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_
 // settings, so that a CPU test can pin what it chooses at the layer shapes (w4a16_plan_prefill); w4a16_plan_prefill_launch
 // also prices the k-group builds below.
 // Block tile 128 x 256 (two workgroups per CU), 96 x 256 or 64 x 256 (three per CU, 96 / 64 accumulator registers), the
-// k range whole or cut into 2, 3, 4, 6 or 8 slices (split-K: f32 partials in a context-owned workspace, added in slice order by a
+// k range whole or cut into 2 to 8 slices (split-K: f32 partials in a context-owned workspace, added in slice order by a
 // second launch — deterministic), and the super-tile shape: every combination is priced and the cheapest runs.
 struct PrefillSuper {
     size_t sup_m, sup_n, supers, load;
@@ -422,64 +422,86 @@ struct PrefillPlan {
     size_t wnw = 0;  // 2 or 3: the k-group build with 64 * wnw columns per block tile; 0: the 256-column tiles
 };
 
-// Super-tile shape for a grid of tiles_m x tiles_n block tiles: sup_m <= 8 along m, sup_n in {8, 4, 2, 1} along n.
-// Super-tiles are dealt round-robin to the 8 XCDs (m fastest), so every candidate is priced by the block tiles its
-// busiest XCD ends up with — counted exactly, partial super-tiles at the edges included — and the shape with the
-// lightest busiest XCD wins, the larger one on ties for L2 reuse.  (A fixed 8 along m left 10 tile rows as 8 + 2:
-// the XCDs that drew the 2-row super-tiles idled, 298 against 227 us on the down projection at t = 1280.)
-// most_blocks: shapes that launch more blocks per XCD are left out, those past the output's edge counted.  A block past the edge
-// ends at once, but takes its place in the order in which an XCD's blocks are dealt to its CUs: a grid that holds one block per
-// CU has to count it (15 x 16 tiles in super-tiles of 7 x 2, 30 live blocks of 42: some CUs drew two, 32.1 us; 5 x 2, 18.8).
+// Super-tile shape for a grid of tiles_m x tiles_n block tiles: sup_m <= 8 along m, sup_n in {8, 4, 2, 1} along n, the largest (L2
+// reuse).  It decides only the order in which an XCD walks its tiles: the kernel numbers the live ones without gaps and every XCD takes
+// an eighth of them (load).  most_blocks: super-tiles that would hold more blocks per XCD, edges counted, are left out.
 static PrefillSuper prefill_super(size_t tiles_m, size_t tiles_n, size_t most_blocks = ~(size_t)0) {
-    PrefillSuper best{std::min<size_t>(8, tiles_m), 8, 0, ~(size_t)0};
+    PrefillSuper best{0, 0, 0, (tiles_m * tiles_n + 7) / 8};
     for (size_t cm = std::min<size_t>(8, tiles_m); cm >= 1; cm--) {
         for (size_t cn : {8, 4, 2, 1}) {
-            const size_t sm = (tiles_m + cm - 1) / cm, sn = (tiles_n + cn - 1) / cn, sp = sm * sn;
-            if ((sp + 7) / 8 * cm * cn > most_blocks) continue;
-            size_t per_xcd[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-            for (size_t sidx = 0; sidx < sp; sidx++)
-                per_xcd[sidx & 7] += std::min(cm, tiles_m - (sidx % sm) * cm) * std::min(cn, tiles_n - (sidx / sm) * cn);
-            const size_t load = *std::max_element(per_xcd, per_xcd + 8);
-            if (load < best.load || (load == best.load && cm * cn > best.sup_m * best.sup_n)) best = PrefillSuper{cm, cn, sp, load};
+            const size_t supers = ((tiles_m + cm - 1) / cm) * ((tiles_n + cn - 1) / cn);
+            if ((supers + 7) / 8 * cm * cn > most_blocks || cm * cn <= best.sup_m * best.sup_n) continue;
+            best.sup_m = cm, best.sup_n = cn, best.supers = supers;
         }
     }
     return best;
 }
 
+// How the kernel walks the block tiles (its sup_m, sup_n; negative: bands of rows).  x_tile, w_tile: bytes per k tile of a tile's x rows and
+// weight columns; resident: blocks an XCD holds at once.  Where all blocks of an XCD's eighth are resident it is one block of tiles, as
+// many rows as leave it the fewest bytes to read, walked in bands.  Else super-tiles of the plan's shape, in panels or bands, whichever
+// leaves the eighth the fewer bytes.  (848 x 2048 t = 2982, 47 x 5 tiles: the shape's panels of one column 21.0 us, bands of six rows
+// 19.0.)
+static std::pair<int, int> prefill_walk(size_t m_tiles, size_t n_tiles, size_t nks, size_t x_tile, size_t w_tile, const PrefillSuper& sup, size_t resident) {
+    const size_t share = std::max<size_t>(1, (m_tiles * n_tiles + 7) / 8);
+    if (share * nks <= resident) {
+        size_t rows = (size_t)std::lround(std::sqrt(2.0 * (double)share * (double)w_tile / (double)x_tile));
+        rows = std::max((share + n_tiles - 1) / n_tiles, std::min(std::max<size_t>(rows, 1), m_tiles));
+        return {(int)rows, -8};
+    }
+    auto read = [&](size_t inner, size_t outer_width, size_t inner_bytes, size_t outer_bytes) {
+        const size_t wide = std::max<size_t>(1, std::min(outer_width, share));
+        return share >= inner * wide ? inner * inner_bytes + share / inner * outer_bytes : share / wide * inner_bytes + wide * outer_bytes;
+    };
+    const bool bands = read(n_tiles, std::min(sup.sup_m, m_tiles), w_tile, x_tile) < read(m_tiles, std::min(sup.sup_n, n_tiles), x_tile, w_tile);
+    return {(int)sup.sup_m, bands ? -(int)sup.sup_n : (int)sup.sup_n};
+}
+
+// Price of a launch in microseconds, from measurements on MI355X.  A CU holds `room` workgroups at once; j of them per CU, an even share
+// (the kernel numbers the block tiles without gaps), take per k tile of a slice:
+//   up to a generation, first[ceil(j) - 1]: between two whole numbers from the time just above the lower one over the middle to the
+//   upper one (some CUs already hold a workgroup more; a workgroup alone runs nearly twice as fast as one of a full set);
+//   in the second, `full` for the first and more[] (at steps of half a workgroup) for the rest;
+//   from there `steady` per generation: workgroups have drifted apart and no generation ends as one (`later` for its fixed part).
+// Plus a fixed cost per launch and per generation, and for a split launch one and the time of its partial sums (us per MB written and read).
+// Fitted to 1056 launches per group (167 linears of 512..40000 x 1024..17408, t = 65..4096; every tile, one to eight slices and the
+// k-group builds timed, weights from memory): least squares on the times, then by the time lost against the best choice.  Over 405
+// launches of 62 other linears the plans lose 0.5 % to the best of each shape and take 0.936 (group 128) and 0.943 (group 32) of the
+// time of those they replaced (whole super-tiles dealt to the XCDs; 2, 3, 4, 6 or 8 slices): of the 810 19 are more than 3 % slower,
+// 8 more than 5, 12 at worst.  5120 x 17408 t = 300 73.7 -> 65 us in five slices, 5120 x 5120 t = 1568 101 -> 82.
+struct TilePrice {
+    int room;
+    double first[3][3], more[7], full, launch, generation, split, per_mb, steady, later;
+    double us(size_t kt_slice, double per_cu, size_t nks, double mb) const {
+        double gens = std::ceil(per_cu / room - 1e-9), f;
+        if (gens > 2.0) {
+            const double past = per_cu / room - 2.0;
+            f = 2.0 * full + steady * past;
+            gens = 2.0 + later / generation * past;
+        } else if (gens <= 1.0) {
+            const int m = std::max(0, (int)std::ceil(per_cu - 1e-9) - 1);
+            const double at = (per_cu - m) * 2.0;
+            f = at <= 1.0 ? first[m][0] + (first[m][1] - first[m][0]) * at : first[m][1] + (first[m][2] - first[m][1]) * (at - 1.0);
+        } else {
+            const double rem = (per_cu - room) * 2.0;
+            const int i = std::min((int)rem, 2 * room - 1);
+            f = full + more[i] + (more[i + 1] - more[i]) * (rem - i);
+        }
+        return (double)kt_slice * f + launch + generation * gens + (nks > 1 ? split + per_mb * mb : 0.0);
+    }
+};
+static const TilePrice kTilePrice[2][3] = {  // group 128, 32; 64, 96, 128 rows (the 96-row tile is not chosen at group 32)
+    {{3, {{0.728, 0.968, 1.172}, {1.427, 1.554, 1.794}, {2.239, 2.453, 2.733}}, {0.0, 0.687, 0.961, 1.256, 1.623, 2.773, 2.628}, 2.823, 3.855, 5.632, 0.0, 0.0938, 2.496, 9.27},
+     {3, {{1.184, 1.486, 1.619}, {2.114, 2.291, 2.688}, {3.259, 3.569, 3.887}}, {0.0, 0.729, 1.249, 1.938, 2.473, 3.61, 3.656}, 3.958, 0.939, 10.895, 0.057, 0.0806, 3.306, 19.52},
+     {2, {{1.445, 1.803, 1.947}, {2.619, 2.861, 3.32}}, {0.0, 1.16, 2.04, 2.726, 2.838}, 3.62, 0.843, 11.275, 0.001, 0.0836, 2.950, 16.80}},
+    {{3, {{0.786, 1.396, 1.553}, {2.216, 2.244, 2.376}, {3.004, 3.31, 3.539}}, {0.0, 0.699, 0.908, 1.774, 1.992, 3.283, 3.205}, 3.739, 7.362, 2.375, 0.0, 0.0921, 3.463, 5.90},
+     {3, {{1.184, 1.486, 1.619}, {2.114, 2.291, 2.688}, {3.259, 3.569, 3.887}}, {0.0, 0.729, 1.249, 1.938, 2.473, 3.61, 3.656}, 3.958, 0.939, 10.895, 0.057, 0.0806, 3.306, 19.52},
+     {2, {{2.003, 2.38, 2.515}, {3.674, 3.71, 4.246}}, {0.0, 1.442, 1.998, 3.493, 3.565}, 4.611, 5.478, 6.669, 0.0, 0.0778, 4.022, 13.77}}};
+
 static PrefillPlan plan_prefill(size_t t, size_t n, size_t k, size_t group, size_t cus, int tile_m_forced, int ksplit_forced,
                                 bool glu = false) {
     // a gated launch tiles the n/2 output columns by 128 (each block tile holds the matching 128 up columns as well)
     const size_t tiles_n = glu ? (n / 2 + kW4PfBn / 2 - 1) / (kW4PfBn / 2) : (n + kW4PfBn - 1) / kW4PfBn, kt_n = k / 128;
-    // Price of a launch in microseconds, from measurements on MI355X (grids of exactly 256 x j workgroups of each tile,
-    // k = 17408 and 5120).  A CU holds c workgroups at once (3 of the 64-row tile, 2 of the 128-row tile); j workgroups
-    // per CU (of the busiest XCD) run as floor(j / c) full generations, `full` microseconds per k tile each, and a last
-    // partial one whose cost depends on how many workgroups share the CU — a workgroup alone runs nearly twice as fast
-    // as one of a full set (the chip is power-limited under this kernel), so the cost of a partial generation starts at
-    // more than half a full one and grows from there.  Plus a fixed cost per generation (first loads, epilogue), and for a
-    // split launch the second launch and the partial sums written and read back.  The constants started from those
-    // measurements and were then fitted to a sweep of tile x slices over 108 (n, k, t) shapes (nine linears, t = 128
-    // to 4096), minimising the time lost against the best choice of the sweep: 0.8 % lost on average, 9 % at worst,
-    // where the earlier rule (generations x slice length x a tile factor, slices by doubling) lost 3 % and 22 %; fitted
-    // on four of the linears only it lost 0.9 % / 11 % on the other five.  The 96-row tile joined later with constants of
-    // its own fitted to a sweep of that tile over the same 108 shapes (the others kept): the plans gain 0.5 % on average,
-    // up to 14 % where its grid fills the generations better (11008 x 4096 at t = 1536, 17408 x 5120 at t = 1024,
-    // 5120 x 34816 at t = 1024: 4 %), and lose at most 3 % against the two-tile plans.
-    auto us_per_k_tile = [](size_t rows, double per_cu) {
-        static const double at[7] = {0.0, 0.5, 1.0, 1.5, 2.0, 2.5, 3.0};
-        static const double part64[7] = {1.0, 1.006, 1.595, 1.738, 1.95, 2.552, 2.903}, part128[5] = {1.5, 1.6, 2.416, 2.9, 3.37},
-                            part96[7] = {1.25, 1.258, 1.994, 2.494, 2.729, 3.787, 4.077};
-        const double c = rows == 128 ? 2.0 : 3.0, full = rows == 64 ? 2.745 : rows == 96 ? 4.126 : 3.497;
-        const double* part = rows == 64 ? part64 : rows == 96 ? part96 : part128;
-        const double gens = std::floor(per_cu / c), rem = per_cu - gens * c;
-        double us = gens * full;
-        if (rem > 1e-9) {
-            const int last = rows == 128 ? 4 : 6;
-            int i = 1;
-            while (i < last && rem > at[i]) i++;
-            us += part[i - 1] + (part[i] - part[i - 1]) * (rem - at[i - 1]) / (at[i] - at[i - 1]);
-        }
-        return us;
-    };
     PrefillPlan best{128, 1, PrefillSuper{1, 1, 0, 0}, 1e30};
     for (size_t rows : {(size_t)128, (size_t)96, (size_t)64}) {
         if (tile_m_forced && (size_t)tile_m_forced != rows) continue;
@@ -487,15 +509,14 @@ static PrefillPlan plan_prefill(size_t t, size_t n, size_t k, size_t group, size
         const size_t tiles_m = (t + rows - 1) / rows;
         const PrefillSuper sup = prefill_super(tiles_m, tiles_n);
         const size_t forced = ksplit_forced > 0 ? std::max<size_t>(1, std::min<size_t>((size_t)ksplit_forced, kt_n / 4)) : 0;
-        for (size_t cand : {1, 2, 3, 4, 6, 8}) {
+        for (size_t cand : {1, 2, 3, 4, 5, 6, 7, 8}) {
             const size_t nks = forced ? forced : cand;  // a pinned slice count is the only candidate
             if (forced && cand != 1) break;
             if (ksplit_forced < 0 && nks != 1) continue;
             if (!forced && nks > 1 && (n % (glu ? 8 : 4) != 0 || nks > kt_n / 4)) continue;
-            const double per_cu = (double)(sup.load * nks) * 8.0 / (double)cus;  // of the busiest XCD
-            const double gens = std::ceil(per_cu / (rows == 128 ? 2.0 : 3.0));
-            double us = (double)((kt_n + nks - 1) / nks) * us_per_k_tile(rows, per_cu) + 5.7 * gens;
-            if (nks > 1) us += 6.0 + (double)nks * (double)t * (double)n * 8.0 / 9.76e6;
+            if (!forced && (nks == 5 || nks == 7) && nks * 5 > kt_n) continue;  // no gain from slices of four k tiles
+            const double per_cu = (double)((tiles_m * tiles_n * nks + 7) / 8 * 8) / (double)cus;
+            const double us = kTilePrice[group == 32][rows / 32 - 2].us((kt_n + nks - 1) / nks, per_cu, nks, (double)nks * (double)t * (double)n * 8.0 / 1e6);
             if (us < best.us) best = PrefillPlan{rows, nks, sup, us};
         }
     }
@@ -510,22 +531,14 @@ static PrefillPlan plan_prefill(size_t t, size_t n, size_t k, size_t group, size
 // above / this one in us: group 128 5120 x 5120 t = 300 32.0 / 27.4, 7168 x 5120 t = 300 43.5 / 34.6 (192 columns), 4096 x 2048
 // t = 300 26.3 / 12.9, 1024 x 640 t = 100 14.1 / 7.8, group 32 5120 x 2048 t = 300 32.1 / 16.1; not chosen: 5120 x 5120 t = 65
 // 22.7 / 23.7, 5120 x 17408 t = 128 43 / 74.
-// The price: a fixed cost and one per k tile of a group's run, each growing with the part of the chip in use (of the busiest XCD).
-// The other plan's is corrected before the two are compared, k whole and k in slices apart: its constants, fitted at group 128 over
-// wider outputs, are low at short k, and slices of the 64-row tile are faster than priced.  Fitted to both sides of 2186 launches
-// (96 linears of 512..23200 x 1024..17408, t = 65..2048, both groups, weights from memory), a quarter of them held out first: of
-// the launches that take a k-group build 0.7 % lose more than 2 % to the plan above (none of those held out; 23 % did under the
-// constants of the time when a counted wait stood at its barriers: 592 x 2560 t = 128 12.9 / 14.3 us, 7168 x 5120 t = 128 25.2 /
-// 27.8), and 3 % of those that do not would have gained more than 3 %.
+// The price: a fixed cost and one per k tile of a group's run, each growing with the part of the chip in use; fitted with the tiles' above
+// to the 1149 launches per group where the grid fits.
 static PrefillPlan plan_prefill_groups(const PrefillPlan& tiles, size_t t, size_t n, size_t k, size_t group, size_t cus) {
-    static const double price[2][2][4] = {{{5.738, 1.554, 0.8956, 0.3632}, {6.407, 1.616, 1.639, 0.5267}},   // group 128: 128, 192 columns
-                                          {{5.876, 2.025, 1.39, 0.2816}, {6.163, 2.427, 1.666, 0.5129}}};  // group 32
-    // factor and offset of the other plan's price: k whole, k in slices
-    static const double other[2][2][2] = {{{1.127, 3.319}, {0.8943, -1.773}}, {{0.9407, 4.859}, {1.099, -4.473}}};
+    static const double price[2][2][4] = {{{5.687, 1.647, 1.243, 0.4823}, {6.55, 2.041, 1.814, 0.6567}},   // group 128: 128, 192 columns
+                                          {{5.872, 2.428, 0.806, 0.4374}, {7.53, 2.966, 1.746, 0.6738}}};  // group 32
     const size_t kt_n = k / 128, tiles_m = (t + 63) / 64, run = (kt_n + 3) / 4;
     PrefillPlan best = tiles;
-    const double* o = other[group == 32][tiles.nks > 1];
-    double us = tiles.us * o[0] + o[1];
+    double us = tiles.us;
     for (size_t w : {2, 3}) {
         const size_t tiles_n = (n + 64 * w - 1) / (64 * w);  // gated: as many pairs of 32 w gate and up columns
         if ((tiles_m * tiles_n + 7) / 8 * 8 > cus) continue;
@@ -630,8 +643,7 @@ static int launch_prefill(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_t y
     }
     const auto& kept = hit->second;
     const PrefillPlan plan{kept[0], kept[1], PrefillSuper{kept[2], kept[3], kept[4], 0}, 0.0, kept[5]};
-    const size_t bm = plan.bm, nks = plan.nks, sup_m = plan.sup.sup_m, sup_n = plan.sup.sup_n, supers = plan.sup.supers;
-    const size_t grid = ((supers + 7) / 8) * (sup_m * sup_n) * 8;
+    const size_t bm = plan.bm, nks = plan.nks;
     char sym[64];
     snprintf(sym, sizeof sym, "w4a16_prefill_g%zu_%s%s%s%s", L.group, L.scale_bf16 ? "bf16" : "f16", bm == 64 ? "_m64" : bm == 96 ? "_m96" : "",
              plan.wnw == 2 ? "_n2k4" : plan.wnw == 3 ? "_n3k4" : "", glu ? "_glu" : "");
@@ -642,10 +654,15 @@ static int launch_prefill(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_t y
     const unsigned shmem = (unsigned)(plan.wnw ? std::max<size_t>(4 * stages, plan.wnw * 12 * 4 * 1024) : stages) + threads * 4;
     uint64_t qt = L.q_tiled, st = L.s_tiled;
     int row_blocks = (int)L.row_blocks, ki = (int)L.k, ni = (int)L.n, ti = (int)t, of = (out_f16 || glu) ? 1 : 0;
-    int spm = (int)sup_m, spn = (int)sup_n, act = glu ? glu_act : 0, glu_i = glu ? 1 : 0;
+    const size_t cols = plan.wnw ? 64 * plan.wnw : kW4PfBn, n_tiles = glu ? (L.n / 2 + cols / 2 - 1) / (cols / 2) : (L.n + cols - 1) / cols;
+    const size_t grid = ((t + bm - 1) / bm * n_tiles * nks + 7) / 8 * 8;
+    const auto walk = prefill_walk((t + bm - 1) / bm, n_tiles, nks, bm * 256, cols * 64, plan.sup, 32 * (plan.wnw ? 1 : bm == 128 ? 2 : 3));
+    int spm = walk.first, spn = walk.second, act = glu ? glu_act : 0, glu_i = glu ? 1 : 0;
+    int nksi = (int)nks;
+    if (grid > 0x7fffffffu) return w4_fail(W4A16_ERR_SHAPE, "prefill: t=%zu n=%zu exceed the grid", t, L.n);
     if (nks == 1) {
         if (norm && epi.stats_out) norm->n_stats_out = ((size_t)epi.stat_cols + 63) / 64;  // one entry per wave's 64 columns
-        void* params[] = {&qt, &st, &x, &y, &row_blocks, &ki, &ni, &ti, &of, &spm, &spn, &act, &epi};
+        void* params[] = {&qt, &st, &x, &y, &row_blocks, &ki, &ni, &ti, &of, &spm, &spn, &nksi, &act, &epi};
         return w4_launch(ctx, sym, (unsigned)grid, 1, threads, shmem, params);
     }
     if (L.n % (glu ? 8 : 4) != 0) return w4_fail(W4A16_ERR_UNSUPPORTED, "prefill: split-K needs n %% %d == 0", glu ? 8 : 4);
@@ -655,9 +672,8 @@ static int launch_prefill(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_t y
     int zero = 0;
     PfEpiHost slice_epi;  // the slices only need the row stride of x; the finish kernel applies the options
     slice_epi.ldx = (int)ldx;
-    void* params[] = {&qt, &st, &x, &ws, &row_blocks, &ki, &ni, &ti, &zero, &spm, &spn, &act, &slice_epi};
-    W4_TRY(w4_launch(ctx, sym, (unsigned)grid, (unsigned)nks, kW4PfThreads, shmem, params));
-    int nksi = (int)nks;
+    void* params[] = {&qt, &st, &x, &ws, &row_blocks, &ki, &ni, &ti, &zero, &spm, &spn, &nksi, &act, &slice_epi};
+    W4_TRY(w4_launch(ctx, sym, (unsigned)grid, 1, kW4PfThreads, shmem, params));
     if (has_epi) {
         if (t * (L.n / 1024) > 0x7fffffffu) return w4_fail(W4A16_ERR_SHAPE, "prefill: t=%zu n=%zu exceed the finish launch", t, L.n);
         if (norm && epi.stats_out) norm->n_stats_out = ((size_t)epi.stat_cols + 1023) / 1024;  // one entry per 1024-column chunk
@@ -761,8 +777,8 @@ extern "C" int w4a16_upload_lin(w4a16_ctx* ctx, const char* name, const void* q,
     L.scale_bf16 = scale_bf16 ? 1 : 0;
     // "regular": what the MFMA prefill kernel can carry as a running unit (w4_scales_regular).  Other linears are served
     // by the streaming kernels, which only ever multiply by a scale.
-    L.scales_regular = w4_scales_regular(static_cast<const uint16_t*>(s), slen_bytes / 2, scale_bf16);
-    L.fold = scale_bf16 && group == 32 && w4_bf16_folds(static_cast<const uint16_t*>(s), slen_bytes / 2);
+    L.fold = scale_bf16 && group == 32 && w4_bf16_folds(static_cast<const uint16_t*>(s), slen_bytes / 2);  // a narrower range: no second scan
+    L.scales_regular = L.fold || w4_scales_regular(static_cast<const uint16_t*>(s), slen_bytes / 2, scale_bf16);
     int rc = w4a16_alloc(ctx, qlen_bytes, &L.q_raw);
     if (!rc) rc = w4a16_alloc(ctx, slen_bytes, &L.s_raw);
     if (!rc) rc = w4a16_h2d(ctx, L.q_raw, q, qlen_bytes);

@@ -96,7 +96,7 @@ struct PfEpi {
 template <int G, bool SBF, int MI, int MODE = 0, int WNW = 4, int KG = 1, bool FOLD = false>
 __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const uint16_t* __restrict__ st,
                                              const uint16_t* __restrict__ x, void* __restrict__ y, int row_blocks,
-                                             int k, int n, int t, int out_f16, int sup_m, int sup_n,
+                                             int k, int n, int t, int out_f16, int sup_m, int sup_n, int nks,
                                              const PfGroup<MODE> gp = PfGroup<MODE>(), const PfEpi epi = PfEpi()) {
     extern __shared__ _Float16 lds[];  // 2 stages x [PF_BM][KS]; then row factors, a word per thread (dense) / slot ids, weights (grouped)
     constexpr int GPT = W4_TILE_K / G;
@@ -111,22 +111,32 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
     const int wn = KG > 1 ? wave % WNW : wave, kg = KG > 1 ? wave / WNW : 0;
     const int kt_n = k / W4_TILE_K, kg_n = kt_n * GPT;
 
-    // XCD-aware tile numbering.  Block b runs on XCD b % 8 and is the (b / 8)-th block of that XCD; consecutive
-    // blocks of an XCD walk one super-tile of sup_m x sup_n block tiles (m fastest), so the blocks resident on an XCD
-    // at a time share x slabs and weight panels through its L2.  Super-tiles are dealt round-robin to the XCDs.  The
-    // host picks the super-tile shape: 8 x 8 on large grids, smaller on small ones so that every XCD gets work.
-    int m0, n0;
+    // XCD-aware tile numbering.  Block b runs on XCD b % 8 and is the (b / 8)-th block of that XCD.  The live block tiles are numbered
+    // without gaps: panels of sup_n tile columns, in a panel super-tiles of sup_m tile rows, in a super-tile m fastest (sup_n < 0:
+    // bands of sup_m tile rows, in a band super-tiles of -sup_n columns), and a tile's k slices one after the other.  Every XCD
+    // takes an eighth of the numbers, one run, so the blocks resident on it at a time share x slabs and weight panels through its L2,
+    // and no XCD and no CU has more block tiles than an even share.  (Whole super-tiles dealt round-robin, those at the edges
+    // partly empty, left some CUs with a block more: 5120 x 5120 t = 1568 99 us, now 80; 14336 x 5248 t = 1041 203 / 144; over 256
+    // shapes of 65..4096 rows 5 % on average.  Slices as the outermost dimension cost launches of one block per CU two us: 2448 x 8064
+    // t = 177 in eight slices 27.3 / 24.6.)
+    int m0, n0, slice = 0;
     constexpr bool DENSE = MODE == 0 || MODE == 3, PAIRED = MODE == 1 || MODE == 3;  // PAIRED: gate and up columns per wave
     if (DENSE) {
         const int tiles_m = (t + PF_BM - 1) / PF_BM,
                   tiles_n = MODE == 3 ? ((n >> 1) + BN / 2 - 1) / (BN / 2) : (n + BN - 1) / BN;
-        const int sm_n = (tiles_m + sup_m - 1) / sup_m, sn_n = (tiles_n + sup_n - 1) / sup_n;
-        const int per = sup_m * sup_n;
-        const int j = blockIdx.x >> 3;
-        const int super = (blockIdx.x & 7) + 8 * (j / per), within = j % per;
-        if (super >= sm_n * sn_n) return;  // uniform for the whole block
-        const int tm = (super % sm_n) * sup_m + within % sup_m, tn = (super / sm_n) * sup_n + within / sup_m;
-        if (tm >= tiles_m || tn >= tiles_n) return;
+        const unsigned work = (unsigned)(tiles_m * tiles_n) * (unsigned)nks, xcd = blockIdx.x & 7;
+        const unsigned at = (unsigned)((unsigned long long)work * xcd / 8) + (blockIdx.x >> 3);
+        if (at >= (unsigned)((unsigned long long)work * (xcd + 1) / 8)) return;  // uniform for the whole block
+        const int r = (int)(at / (unsigned)nks);
+        slice = (int)(at - (unsigned)(r * nks));
+        // outer: the dimension cut into panels or bands, inner: the one walked within
+        const bool bands = sup_n < 0;
+        const int so = bands ? sup_m : sup_n, si = bands ? -sup_n : sup_m, to = bands ? tiles_m : tiles_n, ti = bands ? tiles_n : tiles_m;
+        const int o = r / (ti * so), in_o = r - o * (ti * so), wide = min(so, to - o * so);
+        const int super = in_o / (si * wide), in_super = in_o - super * (si * wide), deep = min(si, ti - super * si);
+        // m fastest inside a super-tile
+        const int rows = bands ? wide : deep, i_n = in_super / rows, i_m = in_super - i_n * rows;
+        const int tm = (bands ? o * so : super * si) + i_m, tn = (bands ? super * si : o * so) + i_n;
         m0 = tm * PF_BM;
         n0 = tn * (MODE == 3 ? BN / 2 : BN);
     } else {
@@ -239,12 +249,12 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
     float unit[2] = {1.f, 1.f};  // scale the accumulator of sub-tile ni is currently expressed in
 
     const int a_row = nl;  // + mi * 32
-    // split-K over gridDim.y (narrow outputs at moderate t, where the tile grid alone cannot fill the chip): this
+    // split-K over nks slices (narrow outputs at moderate t, where the tile grid alone cannot fill the chip): this
     // block covers k tiles [kt_lo, kt_hi) and writes an f32 partial; a second launch adds the partials in order
     // KG > 1: the k range is dealt to the groups of the workgroup's waves instead, contiguous runs of equal length (the last
     // shorter or empty); every group runs as many iterations, for the barriers, and skips those past its run
-    const int kt_a = DENSE && KG == 1 ? (kt_n * (int)blockIdx.y) / (int)gridDim.y : 0,
-              kt_b = DENSE && KG == 1 ? (kt_n * ((int)blockIdx.y + 1)) / (int)gridDim.y : kt_n;
+    const int kt_a = DENSE && KG == 1 ? (kt_n * slice) / nks : 0,
+              kt_b = DENSE && KG == 1 ? (kt_n * (slice + 1)) / nks : kt_n;
     const int per = (kt_b - kt_a + KG - 1) / KG;
     const int kt_lo = kt_a + kg * per, kt_hi = KG > 1 ? min(kt_b, kt_lo + per) : kt_b;
     const int stages = SPT * kt_hi;
@@ -439,7 +449,7 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
     }
     // x arrived as its true value times 1/in_scale and (with input statistics) un-normalised: one factor per row
     const bool use_fac = DENSE && (has_stats || (epi.in_scale != 1.0f && epi.in_scale != 0.0f));
-    if (MODE == 3 && (KG > 1 || gridDim.y == 1)) {
+    if (MODE == 3 && (KG > 1 || nks == 1)) {
         const int n_ff = n >> 1, col = n0 + wn * 32 + nl;
         if (col >= n_ff) return;
 #pragma unroll
@@ -467,8 +477,8 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
         }
         return;
     }
-    if (KG == 1 && gridDim.y > 1) {  // partial (f32) of a split launch: w4a16_prefill_splitk_sum finishes (activation, epilogue options)
-        y = reinterpret_cast<float*>(y) + (size_t)blockIdx.y * (size_t)t * (size_t)n;
+    if (KG == 1 && nks > 1) {  // partial (f32) of a split launch: w4a16_prefill_splitk_sum finishes (activation, epilogue options)
+        y = reinterpret_cast<float*>(y) + (size_t)slice * (size_t)t * (size_t)n;
 #pragma unroll
         for (int ni = 0; ni < 2; ni++) {
             const int col = MODE == 3 ? ni * (n >> 1) + n0 + wn * 32 + nl : n0 + wn * 64 + ni * 32 + nl;
@@ -558,9 +568,9 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
 #define PREFILL_KERNEL(NAME, G, SBF, MI, WPE)                                                                      \
     extern "C" __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void NAME(      \
         const u4_t* qt, const uint16_t* st, const uint16_t* x, void* y, int row_blocks, int k, int n, int t,          \
-        int out_f16, int sup_m, int sup_n, int act_kind, PfEpi epi) {                                                  \
+        int out_f16, int sup_m, int sup_n, int nks, int act_kind, PfEpi epi) {                                                  \
         (void)act_kind;                                                                                                \
-        prefill_body<G, SBF, MI>(qt, st, x, y, row_blocks, k, n, t, out_f16, sup_m, sup_n, PfGroup<0>(), epi);         \
+        prefill_body<G, SBF, MI>(qt, st, x, y, row_blocks, k, n, t, out_f16, sup_m, sup_n, nks, PfGroup<0>(), epi);         \
     }
 
 // Dense gated kernels: same arguments (the plain kernels ignore act_kind, W4A16_ACT_*); y is f16 [t][n/2], or the f32
@@ -568,10 +578,10 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
 #define PREFILL_GLU_KERNEL(NAME, G, SBF, MI, WPE)                                                                  \
     extern "C" __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void NAME(      \
         const u4_t* qt, const uint16_t* st, const uint16_t* x, void* y, int row_blocks, int k, int n, int t,          \
-        int out_f16, int sup_m, int sup_n, int act_kind, PfEpi epi) {                                                  \
+        int out_f16, int sup_m, int sup_n, int nks, int act_kind, PfEpi epi) {                                                  \
         PfGroup<3> gp;                                                                                                 \
         gp.act_kind = act_kind;                                                                                        \
-        prefill_body<G, SBF, MI, 3>(qt, st, x, y, row_blocks, k, n, t, out_f16, sup_m, sup_n, gp, epi);                \
+        prefill_body<G, SBF, MI, 3>(qt, st, x, y, row_blocks, k, n, t, out_f16, sup_m, sup_n, nks, gp, epi);                \
     }
 
 // Block tile of a grouped workgroup.  Every XCD (block b runs on XCD b % 8) takes an eighth of the live block tiles, segments in
@@ -606,10 +616,10 @@ __device__ __forceinline__ bool pf_moe_tile(PfGroup<MODE>& gp, const int* num_po
 #define PREFILL_KG_KERNEL(NAME, G, SBF, WNW, MODE)                                                                    \
     extern "C" __global__ __launch_bounds__(64 * WNW * 4) __attribute__((amdgpu_waves_per_eu(WNW, WNW))) void NAME(       \
         const u4_t* qt, const uint16_t* st, const uint16_t* x, void* y, int row_blocks, int k, int n, int t,          \
-        int out_f16, int sup_m, int sup_n, int act_kind, PfEpi epi) {                                                  \
+        int out_f16, int sup_m, int sup_n, int nks, int act_kind, PfEpi epi) {                                                  \
         PfGroup<MODE> gp;                                                                                              \
         gp.act_kind = act_kind;                                                                                        \
-        prefill_body<G, SBF, 2, MODE, WNW, 4>(qt, st, x, y, row_blocks, k, n, t, out_f16, sup_m, sup_n, gp, epi);      \
+        prefill_body<G, SBF, 2, MODE, WNW, 4>(qt, st, x, y, row_blocks, k, n, t, out_f16, sup_m, sup_n, nks, gp, epi);      \
     }
 #define PREFILL_KG_FAMILY(PFX, G, SBF)                    \
     PREFILL_KG_KERNEL(PFX##_m64_n2k4, G, SBF, 2, 0)       \
@@ -641,8 +651,8 @@ __device__ __forceinline__ bool pf_moe_tile(PfGroup<MODE>& gp, const int* num_po
         if (!pf_moe_tile<MODE>(gp, num_post, n, &rows)) return;                                                          \
         const u4_t* qt = reinterpret_cast<const u4_t*>(qa);                                                              \
         const uint16_t* st = reinterpret_cast<const uint16_t*>(sa);                                                      \
-        if (rows <= 32) prefill_body<G, SBF, 1, MODE, 4, 1, FOLD>(qt, st, x, y, row_blocks, k, n, 0, y_f16, 1, 1, gp);         \
-        else prefill_body<G, SBF, 2, MODE, 4, 1, FOLD>(qt, st, x, y, row_blocks, k, n, 0, y_f16, 1, 1, gp);                    \
+        if (rows <= 32) prefill_body<G, SBF, 1, MODE, 4, 1, FOLD>(qt, st, x, y, row_blocks, k, n, 0, y_f16, 1, 1, 1, gp);         \
+        else prefill_body<G, SBF, 2, MODE, 4, 1, FOLD>(qt, st, x, y, row_blocks, k, n, 0, y_f16, 1, 1, 1, gp);                    \
     }
 
 #define PREFILL_MOE_KERNEL(NAME, G, SBF, MODE) PREFILL_MOE_BUILD(NAME, G, SBF, MODE, false)
