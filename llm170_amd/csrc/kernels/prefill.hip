@@ -18,9 +18,8 @@
 //     holds sum / s_g; at each group boundary it is multiplied by s_prev / s_cur and the new group's integer products
 //     are added by the MFMA itself; the epilogue multiplies by the last scale.  No weight is rounded to f16 and no
 //     second accumulator set is needed.  (Linears with a zero or non-finite scale are not routed here.)
-//   * workgroups are numbered so that the blocks resident on one XCD form a super-tile (8 x 8 block tiles on large
-//     grids: each x slab and each weight panel is fetched into that L2 once per eight uses; smaller on small grids so
-//     that all eight XCDs get work).
+//   * the live block tiles are numbered without gaps and every XCD takes an eighth of them, neighbours in super-tiles (8 x 8 block
+//     tiles on large grids: each x slab and each weight panel is fetched into that L2 once per eight uses).
 #include "w4a16_common.hpp"
 
 // s_prev / s_cur of a group boundary: the hardware reciprocal (1 ulp) and one Newton step on the quotient (the residual
