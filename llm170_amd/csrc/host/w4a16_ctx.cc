@@ -96,6 +96,8 @@ static const char* const kMoeSyms[] = {W4_MOE_FAMILY("w4a16_moe_g32_f16"),
                                        W4_MOE_FOLD("w4a16_moe_g32_f16x"),
                                        W4_MOE_KT2("w4a16_moe_g128_f16"),
                                        W4_MOE_KT2("w4a16_moe_g128_bf16"),
+                                       W4_MOE_KT2("w4a16_moe_g32_f16"),
+                                       W4_MOE_KT2("w4a16_moe_g32_f16x"),
                                        "w4a16_moe_g32_f16_down_sum",
                                        "w4a16_moe_g32_bf16_down_sum",
                                        "w4a16_moe_g128_f16_down_sum",

@@ -277,10 +277,15 @@ static int launch_moe_gemm(w4a16_ctx* ctx, const W4Experts& E, bool glu, uint64_
     waves = ctx->moe_waves ? ctx->moe_waves : 4;
     waves = waves >= 8 ? 8 : 4;  // the x staging needs at least 4 waves
     const size_t blocks = max_segs * ((units + (size_t)waves - 1) / (size_t)waves);
-    // Two k tiles per stage (kernels/moe.hip) at group 128 where the launch has at most three workgroups per CU and runs of up to
-    // 32 slots: 8 experts T = 100 62.5 -> 54.6 us per FFN, 32 experts top-4 n_ff 1024 T = 40 33.3 -> 30.8; beyond, the LDS they
-    // take costs more than the wait they hide (8 experts T = 256 91 / 101, 64 experts top-6 n_ff 1408 T = 24 57.4 / 59.9).
-    const bool two = E.group == 128 && tt <= 3 && ns < 32 * E.n_exp && blocks * (size_t)waves <= 12 * (size_t)std::max(ctx->cu_count, 1);
+    // Two k tiles per stage (kernels/moe.hip) for runs of up to 32 slots, at group 128 where the launch has at most three workgroups
+    // per CU: 8 experts T = 100 62.5 -> 54.6 us per FFN, 32 experts top-4 n_ff 1024 T = 40 33.3 -> 30.8; beyond, the LDS they
+    // take costs more than the wait they hide (8 experts T = 256 91 / 101, 64 experts top-6 n_ff 1408 T = 24 57.4 / 59.9).  At group
+    // 32 (f16 scales or bf16 kept as f16), whose tiles take longer to multiply, where one segment per expert gives at most one
+    // workgroup per CU (folded / f16 scales, 128 or 256 of them: 4 experts h 4096 n_ff 3584 T = 16 51.6 -> 40.8 / 54.5 -> 43.4, 8 experts
+    // n_ff 2048 T = 24 45.5 -> 39.1 / 45.9 -> 38.8, T = 100 47.9 -> 45.3 / 56.8 -> 57.2; 384: 12 experts T = 24 50.6 / 51.2, T = 100
+    // 56.2 / 58.5 / 61.5 / 64.2).
+    const size_t few = E.group == 128 ? blocks * (size_t)waves : E.tiled_bf16 ? ~(size_t)0 : 3 * E.n_exp * (blocks / max_segs) * (size_t)waves;
+    const bool two = tt <= 3 && ns < 32 * E.n_exp && few <= 12 * (size_t)std::max(ctx->cu_count, 1);
     const bool fold = E.fold && ns >= 8 * E.n_exp;  // figures at compute_fold, kernels/moe.hip
     snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_mm_%s_t%d%s", E.group, fold ? "f16x" : fam, glu ? "glu" : "lin", tt, two ? "_k2" : "");
     const unsigned shmem = (unsigned)((two ? 4 : 2) * 16 * tt * 256);  // two stages of one or two x tiles of 128 k

@@ -748,16 +748,19 @@ MOE_FAMILY(w4a16_moe_g128_bf16, 128, true)
 MOE_MM_FOLD(w4a16_moe_g32_f16x)
 
 // Two k tiles per stage, for launches of few workgroups (the rule is at the launch, w4a16_moe.cc): one tile in flight per wave
-// does not cover the trip to memory there.  Group 128, whose tiles take least time to multiply.  8 experts top-2, h 4096, n_ff
+// does not cover the trip to memory there.  Same sums in the same order.  Group 128, 8 experts top-2, h 4096, n_ff
 // 3584, us per FFN, x and weights four tiles ahead in registers / one tile per stage / two: T = 16 52.5 / 57.8 / 49.2, T = 40
-// 50.3 / 57.3 / 45.7, T = 100 57.8 / 62.5 / 54.6; four tiles per stage lose (51.1, 49.4, 71.3).
-#define MOE_MM_KT2(PFX, G, SBF)                                \
-    MOE_MM_KERNEL(PFX##_mm_glu_t2_k2, G, SBF, true, 2, 2)      \
-    MOE_MM_KERNEL(PFX##_mm_glu_t3_k2, G, SBF, true, 3, 2)      \
-    MOE_MM_KERNEL(PFX##_mm_lin_t2_k2, G, SBF, false, 2, 2)     \
-    MOE_MM_KERNEL(PFX##_mm_lin_t3_k2, G, SBF, false, 3, 2)
-MOE_MM_KT2(w4a16_moe_g128_f16, 128, false)
-MOE_MM_KT2(w4a16_moe_g128_bf16, 128, true)
+// 50.3 / 57.3 / 45.7, T = 100 57.8 / 62.5 / 54.6; four tiles per stage lose (51.1, 49.4, 71.3).  Group
+// 32, folded bf16 / f16 scales, one tile / two: same shape T = 16 58.3 / 52.4 and 57.9 / 52.3, T = 100 66.0 / 63.4 and 69.3 / 67.6.
+#define MOE_MM_KT2(PFX, G, SBF, FOLD)                              \
+    MOE_MM_BUILD(PFX##_mm_glu_t2_k2, G, SBF, true, 2, 2, FOLD)     \
+    MOE_MM_BUILD(PFX##_mm_glu_t3_k2, G, SBF, true, 3, 2, FOLD)     \
+    MOE_MM_BUILD(PFX##_mm_lin_t2_k2, G, SBF, false, 2, 2, FOLD)    \
+    MOE_MM_BUILD(PFX##_mm_lin_t3_k2, G, SBF, false, 3, 2, FOLD)
+MOE_MM_KT2(w4a16_moe_g128_f16, 128, false, false)
+MOE_MM_KT2(w4a16_moe_g128_bf16, 128, true, false)
+MOE_MM_KT2(w4a16_moe_g32_f16, 32, false, false)
+MOE_MM_KT2(w4a16_moe_g32_f16x, 32, false, true)
 
 // ---------------------------------------------------------------------------------------------------- routing
 // Routing rule of the reference (w4a16_dec/mod.rs:168-185, device counterpart assets/moe.cu:686-759): softmax over all
