@@ -286,7 +286,12 @@ static int launch_moe_gemm(w4a16_ctx* ctx, const W4Experts& E, bool glu, uint64_
     // 56.2 / 58.5 / 61.5 / 64.2).
     const size_t few = E.group == 128 ? blocks * (size_t)waves : E.tiled_bf16 ? ~(size_t)0 : 3 * E.n_exp * (blocks / max_segs) * (size_t)waves;
     const bool two = tt <= 3 && ns < 32 * E.n_exp && few <= 12 * (size_t)std::max(ctx->cu_count, 1);
-    const bool fold = E.fold && ns >= 8 * E.n_exp;  // figures at compute_fold, kernels/moe.hip
+    // Folded scales (compute_fold, kernels/moe.hip) from eight k tiles, below which folded sums are the less exact, and eight slots per
+    // expert; in segments of two 16-slot blocks only where one segment per expert gives at most 20 waves per CU: the folded build
+    // has registers for five waves per SIMD, the other for six (128 experts top-8 n_ff 768 T = 200 scaled / folded 77.2 / 83.4 us,
+    // 64 experts top-6 n_ff 1408 T = 100 67.4 / 71.9; 32 experts top-4 n_ff 1024 T = 100 38.3 / 37.2, 8 experts n_ff 3584 T = 100 65.5 / 57.6).
+    const bool fold = E.fold && kt_n >= 8 && ns >= 8 * E.n_exp &&
+                      (tt > 2 || E.n_exp * (blocks / max_segs) * (size_t)waves <= 20 * (size_t)std::max(ctx->cu_count, 1));
     snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_mm_%s_t%d%s", E.group, fold ? "f16x" : fam, glu ? "glu" : "lin", tt, two ? "_k2" : "");
     const unsigned shmem = (unsigned)((two ? 4 : 2) * 16 * tt * 256);  // two stages of one or two x tiles of 128 k
     return w4_launch(ctx, sym, (unsigned)blocks, 1, (unsigned)(waves * 64), shmem, p);

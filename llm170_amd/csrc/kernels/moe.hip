@@ -610,15 +610,19 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
         group(std::integral_constant<int, 7>{});
     };
 
-    // FOLD: scaled weights (w4_deq8_scaled), sums straight in the accumulators: at three 16-slot blocks a third of the vector ALU work of
-    // scaled group sums is gone.  A k tile is eight groups (32 k x one row block), issued like those of compute32: a group's MFMAs, then
-    // the next group's unpack, the B operands of the next 32 k one group early (in the order the compiler finds by itself 128 experts
-    // top-8 take 74.2 instead of 71.7 us per FFN at T = 64).  Scaled sums / folded, us per FFN: 128 experts T = 200 83.2 / 81.8, T = 517
-    // 119.6 / 108.9, T = 800 152 / 132; 8 experts top-2 n_ff 3584 T = 64 67.1 / 62.7, T = 150 82.9 / 72.1; T = 64 71.4 / 71.7, T = 32 69.6
-    // / 70.0, so runs below eight slots per expert keep the scaled sums (rule at the launch).  The results' distance from 64-bit sums is
-    // that of the f16 intermediates, 4.0e-4, to four digits either way.
+    // FOLD: scaled weights (w4_deq8_scaled); a k tile's four MFMAs are summed from zero and added once, so an accumulator rounds as often
+    // as there are k tiles and not at every MFMA: at three 16-slot blocks a quarter of the vector ALU work of scaled group sums is gone.
+    // A k tile is eight groups (32 k x one row block), issued like those of compute32: a group's MFMAs, then the next group's unpack,
+    // the B operands of the next 32 k one group early (in the order the compiler finds by itself 128 experts top-8 take 74.2 instead
+    // of 71.7 us per FFN at T = 64).  Mean distance from 64-bit sums over their rms, scaled group sums / MFMAs chained straight into the
+    // accumulators / this: k = 512 0.67e-7 / - / 0.73e-7, 768 0.76e-7 / 1.32e-7 / 0.83e-7, 1024 0.90e-7 / 1.65e-7 / 0.80e-7, 2048
+    // 1.09e-7 / 2.1e-7 / 0.93e-7, 3584 1.40e-7 / 2.7e-7 / 1.0e-7: below eight k tiles the launch keeps scaled sums.  us per FFN,
+    // scaled / this (gate and up; down where it has eight k tiles): 128 experts top-8 n_ff 768 T = 517 114.4 / 109.2, T = 640 125.8 / 118.5;
+    // 8 experts top-2 n_ff 3584 T = 64 62.1 / 56.4, T = 250 108.1 / 93.2; runs below eight slots per expert gain nothing (T = 64 71.4 / 71.7).
     auto compute_fold = [&](const auto& s_, int buf) {
         const _Float16* xb = xs + buf * (ROWS * 128);
+        const f4_t zero = {0.f, 0.f, 0.f, 0.f};
+        f4_t part[2][TT];
         unsigned sc[2][4];
         h8_t b[2][TT];
 #pragma unroll
@@ -635,11 +639,15 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
                 for (int tt = 0; tt < TT; tt++) b[(w + 1) & 1][tt] = *reinterpret_cast<const h8_t*>(xb + x_get[w + 1] + tt * 16 * 128);
             }
 #pragma unroll
-            for (int tt = 0; tt < TT; tt++) acc[rb][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[w & 1][tt], acc[rb][tt], 0, 0, 0);
+            for (int tt = 0; tt < TT; tt++) part[rb][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[w & 1][tt], w == 0 ? zero : part[rb][tt], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
             if (g < 7) a = w4_deq8_scaled(s_.q[(g + 1) & 1][(g + 1) >> 1], sc[(g + 1) & 1][(g + 1) >> 1]);
             __builtin_amdgcn_sched_barrier(0);
         }
+#pragma unroll
+        for (int rb = 0; rb < 2; rb++)
+#pragma unroll
+            for (int tt = 0; tt < TT; tt++) acc[rb][tt] += part[rb][tt];
     };
 
     // one stage ahead: its DMA and weights are issued ahead of this stage's MFMAs and waited for (vmcnt 0) at the barrier

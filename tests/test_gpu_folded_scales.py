@@ -148,3 +148,51 @@ def test_experts(dec, block, runs, wide):
         assert np.all(np.abs(af[rows] - silu * u) <= err), (e, "act")
         down, bd = af[rows] @ w2.T, _bound(af[rows], w2)
         assert np.all(np.abs(y[rows] - down) <= bd + 2.0 ** -11 * (np.abs(down) + bd) + 2.0 ** -25), (e, "down")
+
+
+def _misrounded(dec, name, x, idx, h, n_ff, q2, s2):
+    """Number of f16 rows' values that are not the nearest f16 to the 64-bit sum of the device's activation and w2 (values of at least
+    half the rms).  A sum that is off by err lands on the wrong side of a rounding boundary with a chance of err / ulp, so the number
+    grows in proportion to the mean distance of the f32 sums from 64-bit ones."""
+    t, cc = len(idx), dec.cc
+    bufs = [cc.to_device(x), cc.to_device(idx), cc.to_device(np.ones((t, 1), np.float32)), cc.to_device(np.zeros((t, h), np.float32))]
+    try:
+        dec.moe_ffn(name, *bufs[:3], t, 1, bufs[3])
+        y, act = cc.d2h(bufs[3], (t, h), np.float32), dec.moe_scratch(3, np.uint16)[0].reshape(t, n_ff)
+    finally:
+        for b in bufs:
+            cc.free(b)
+    count = 0
+    for e in np.unique(idx):
+        rows = np.nonzero(idx[:, 0] == e)[0]
+        ref = gen.f16_bits_to_f32(act[rows]).astype(np.float64) @ _weights(q2[e], s2[e], n_ff).T
+        wrong = y[rows] != ref.astype(np.float16).astype(np.float32)
+        count += int(np.count_nonzero(wrong & (np.abs(ref) > 0.5 * np.sqrt(np.mean(ref * ref)))))
+    return count
+
+
+@pytest.mark.parametrize("block", [32, 48, 64, 0])
+@pytest.mark.parametrize("n_ff", [768, 1024, 3584])
+def test_expert_sums_no_further_from_64_bits(dec, n_ff, block):
+    """Experts whose scales fold against the same experts next to one that has a negative scale and no token, which run the builds that
+    do not fold.  Misrounded values are independent rare events: five standard deviations of the difference of two equal counts.
+    Block 0: the MFMA-tiled kernels."""
+    print("fold sums", n_ff, block, flush=True)
+    E, t, h = 3, 1024, 4096
+    q13, s13, q2, s2 = gen.make_experts(E, h, n_ff, 32, seed=gen.GATE_SEED + 31)
+    s13, s2 = ((gen.f16_bits_to_f32(s).view(np.uint32) >> 16).astype(np.uint16) for s in (s13, s2))
+    x, idx = gen.normal_f16(81, (t, h)), (np.arange(t, dtype=np.int32) % 2)[:, None].copy()
+    counts = []
+    for negative in (False, True):
+        s13[2, 0, 0] = (s13[2, 0, 0] & 0x7FFF) | (0x8000 if negative else 0)
+        dec.upload_experts("sums", q13, s13, q2, s2, E, h, n_ff, 32, True)
+        dec.set_moe_shape(block, 0)
+        dec.set_moe_tiled(0 if block else 1)
+        try:
+            counts.append(_misrounded(dec, "sums", x, idx, h, n_ff, q2, s2))
+        finally:
+            dec.set_moe_shape(0, 0)
+            dec.set_moe_tiled(0)
+    fold, scaled = counts
+    print("misrounded: folded %d, scaled %d" % (fold, scaled), flush=True)
+    assert fold <= scaled + 5.0 * np.sqrt(2.0 * scaled)
