@@ -414,8 +414,7 @@ int w4a16_set_moe_shape(w4a16_ctx* ctx, int block, int waves);
 /* The MFMA-tiled grouped kernels (the role of the reference's grouped Marlin GEMM at prefill sizes, assets/moe.cu:686-759
  * via kernels/marlin_moe.rs:290-422): workgroup = one 64-slot segment x 256 output columns on 32x32x16 MFMA tiles, the
  * segment's x rows gathered into LDS, expert weights as the B operand straight from the arena.  0 = automatic (mean run
- * per expert of at least 68 slots, i.e. t * top_k >= 68 * n_experts, and no segment size forced; at group 32 with n_experts *
- * ceil(n_ff / 128) >= two per CU from 60, with bf16 scales that are all in [2^-14, 2^13) from 40), -1 = never, 1 =
+ * per expert of at least 68 slots, i.e. t * top_k >= 68 * n_experts, and no segment size forced), -1 = never, 1 =
  * always (64-slot segments whatever t).  Same results as the streaming kernels up to the order of the f32 sums. */
 int w4a16_set_moe_tiled(w4a16_ctx* ctx, int mode);
 /* Timed back-to-back w4a16_moe_ffn calls (as w4a16_bench_forward); call i uses experts names[i % n_names]. */

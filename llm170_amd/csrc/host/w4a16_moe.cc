@@ -486,13 +486,10 @@ extern "C" int w4a16_moe_ffn_act(w4a16_ctx* ctx, const char* name, uint64_t x_de
     // n_ff 1024 T = 512 80 / 83, T = 600 96 / 88; group 128, 64 experts top-6 n_ff 1408 T = 600 133 / 134, T = 700 155 / 152).
     if (ctx->moe_tiled > 0 && !E->scales_regular)
         return w4_fail(W4A16_ERR_UNSUPPORTED, "moe_ffn %s: the MFMA-tiled grouped kernels were requested (set_moe_tiled 1) but the experts hold a zero, non-finite or out-of-range scale; the streaming kernels serve them", name);
-    // At group 32, with two block tiles of the gate|up launch per CU from one segment per expert alone, earlier: from 60, and from 40
-    // with folded scales, whose tiled kernels are freed of the running unit (128 experts, folded, T = 640 112 / 111, T = 768 122 / 115,
-    // T = 1024 160 / 149; f16 T = 896 156 / 154, T = 1024 183 / 172; 64 experts top-6 n_ff 1408, folded, T = 426 106 / 99, T = 682
-    // 141 / 132; but 32 experts top-4 n_ff 1024, folded, T = 384 56 / 62, T = 512 64 / 65: one block tile per CU).
-    const bool many = E->group == 32 && E->n_exp * ((E->n_ff + 127) / 128) >= 2 * (size_t)std::max(ctx->cu_count, 1);
-    const size_t tiled_from = !many ? 68 : E->fold ? 40 : 60;
-    const bool tiled = ctx->moe_tiled > 0 || (ctx->moe_tiled == 0 && ctx->moe_block == 0 && E->scales_regular && ns >= tiled_from * E->n_exp);
+    // Folded scales gain there too, and earlier (128 experts, T = 768 129 / 124, T = 1024 174 / 156), but the tiled kernels' sums, one
+    // chain of MFMAs over all of k, lie about twice as far from 64-bit sums as the streaming ones (k = 2048 2.2e-7 and 1.0e-7 of
+    // their rms): the line stays.
+    const bool tiled = ctx->moe_tiled > 0 || (ctx->moe_tiled == 0 && ctx->moe_block == 0 && E->scales_regular && ns >= 68 * E->n_exp);
     const size_t block = tiled ? 64 : pick_block(ctx, t, ns, E->n_exp, top_k);
     if (block != 1 && block != 4 && block != 16 && block != 32 && block != 48 && block != 64)
         return w4_fail(W4A16_ERR_ARG, "moe_ffn %s: segment size %zu not in {1,4,16,32,48,64}", name, block);

@@ -150,7 +150,7 @@ def test_experts(dec, block, runs, wide):
         assert np.all(np.abs(y[rows] - down) <= bd + 2.0 ** -11 * (np.abs(down) + bd) + 2.0 ** -25), (e, "down")
 
 
-def _misrounded(dec, name, x, idx, h, n_ff, q2, s2):
+def _misrounded(dec, name, x, idx, h, n_ff, w2):
     """Number of f16 rows' values that are not the nearest f16 to the 64-bit sum of the device's activation and w2 (values of at least
     half the rms).  A sum that is off by err lands on the wrong side of a rounding boundary with a chance of err / ulp, so the number
     grows in proportion to the mean distance of the f32 sums from 64-bit ones."""
@@ -165,7 +165,7 @@ def _misrounded(dec, name, x, idx, h, n_ff, q2, s2):
     count = 0
     for e in np.unique(idx):
         rows = np.nonzero(idx[:, 0] == e)[0]
-        ref = gen.f16_bits_to_f32(act[rows]).astype(np.float64) @ _weights(q2[e], s2[e], n_ff).T
+        ref = gen.f16_bits_to_f32(act[rows]).astype(np.float64) @ w2(e).T
         wrong = y[rows] != ref.astype(np.float16).astype(np.float32)
         count += int(np.count_nonzero(wrong & (np.abs(ref) > 0.5 * np.sqrt(np.mean(ref * ref)))))
     return count
@@ -189,10 +189,34 @@ def test_expert_sums_no_further_from_64_bits(dec, n_ff, block):
         dec.set_moe_shape(block, 0)
         dec.set_moe_tiled(0 if block else 1)
         try:
-            counts.append(_misrounded(dec, "sums", x, idx, h, n_ff, q2, s2))
+            counts.append(_misrounded(dec, "sums", x, idx, h, n_ff, lambda e: _weights(q2[e], s2[e], n_ff)))
         finally:
             dec.set_moe_shape(0, 0)
             dec.set_moe_tiled(0)
     fold, scaled = counts
     print("misrounded: folded %d, scaled %d" % (fold, scaled), flush=True)
     assert fold <= scaled + 5.0 * np.sqrt(2.0 * scaled)
+
+
+@pytest.mark.parametrize("bf16,run", [(True, 50), (False, 64), (False, 67)])
+def test_expert_route_of_medium_runs_keeps_the_sums(dec, bf16, run):
+    """Mean runs of 40 to 67 slots, as many block tiles as any rule asks for: left to the library the sums are no further from 64 bits
+    than those of the streaming kernels (64-slot segments pinned).  Bounds as above."""
+    print("medium runs", bf16, run, flush=True)
+    E, h, n_ff = 32, 1024, 2048
+    q13, s13, q2, s2 = gen.make_experts(E, h, n_ff, 32, seed=gen.GATE_SEED + 37)
+    if bf16:
+        s13, s2 = ((gen.f16_bits_to_f32(s).view(np.uint32) >> 16).astype(np.uint16) for s in (s13, s2))
+    value = (lambda s: (s.astype(np.uint32) << 16).view(np.float32)) if bf16 else gen.f16_bits_to_f32
+    w2 = lambda e: gen.unpack_nibbles(q2[e], n_ff).astype(np.float64) * np.repeat(value(s2[e]).astype(np.float64), 32, axis=-1)
+    x, idx = gen.normal_f16(82, (E * run, h)), (np.arange(E * run, dtype=np.int32) % E)[:, None].copy()
+    dec.upload_experts("medium", q13, s13, q2, s2, E, h, n_ff, 32, bf16)
+    counts = []
+    for block in (0, 64):
+        dec.set_moe_shape(block, 0)
+        try:
+            counts.append(_misrounded(dec, "medium", x, idx, h, n_ff, w2))
+        finally:
+            dec.set_moe_shape(0, 0)
+    print("misrounded: automatic %d, streaming %d" % tuple(counts), flush=True)
+    assert counts[0] <= counts[1] + 5.0 * np.sqrt(2.0 * counts[1])
