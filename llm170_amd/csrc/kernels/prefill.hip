@@ -476,7 +476,10 @@ __device__ __forceinline__ void prefill_body(const u4_t* __restrict__ qt, const 
         }
         return;
     }
-    if (KG == 1 && nks > 1) {  // partial (f32) of a split launch: w4a16_prefill_splitk_sum finishes (activation, epilogue options)
+    // a partial (f32) of a split launch: w4a16_prefill_splitk_sum finishes (activation, epilogue options).  Gated launches end here or
+    // above; said without nks, or the compiler keeps the plain epilogue for them too, which doubles their code (55 KB instead of 30 at
+    // 64 rows) and what a launch fetches of it.
+    if (KG == 1 && (MODE == 3 || nks > 1)) {
         y = reinterpret_cast<float*>(y) + (size_t)slice * (size_t)t * (size_t)n;
 #pragma unroll
         for (int ni = 0; ni < 2; ni++) {
