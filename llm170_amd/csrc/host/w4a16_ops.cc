@@ -657,12 +657,12 @@ static int launch_prefill(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_t y
     const size_t cols = plan.wnw ? 64 * plan.wnw : kW4PfBn, n_tiles = glu ? (L.n / 2 + cols / 2 - 1) / (cols / 2) : (L.n + cols - 1) / cols;
     const size_t grid = ((t + bm - 1) / bm * n_tiles * nks + 7) / 8 * 8;
     const auto walk = prefill_walk((t + bm - 1) / bm, n_tiles, nks, bm * 256, cols * 64, plan.sup, 32 * (plan.wnw ? 1 : bm == 128 ? 2 : 3));
-    int spm = walk.first, spn = walk.second, act = glu ? glu_act : 0, glu_i = glu ? 1 : 0;
+    int walk_arg = (walk.first & 0xffff) | (int)((unsigned)walk.second << 16), act = glu ? glu_act : 0, glu_i = glu ? 1 : 0;
     int nksi = (int)nks;
     if (grid > 0x7fffffffu) return w4_fail(W4A16_ERR_SHAPE, "prefill: t=%zu n=%zu exceed the grid", t, L.n);
     if (nks == 1) {
         if (norm && epi.stats_out) norm->n_stats_out = ((size_t)epi.stat_cols + 63) / 64;  // one entry per wave's 64 columns
-        void* params[] = {&qt, &st, &x, &y, &row_blocks, &ki, &ni, &ti, &of, &spm, &spn, &nksi, &act, &epi};
+        void* params[] = {&qt, &st, &x, &y, &row_blocks, &ki, &ni, &ti, &of, &walk_arg, &nksi, &act, &epi};
         return w4_launch(ctx, sym, (unsigned)grid, 1, threads, shmem, params);
     }
     if (L.n % (glu ? 8 : 4) != 0) return w4_fail(W4A16_ERR_UNSUPPORTED, "prefill: split-K needs n %% %d == 0", glu ? 8 : 4);
@@ -672,7 +672,7 @@ static int launch_prefill(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_t y
     int zero = 0;
     PfEpiHost slice_epi;  // the slices only need the row stride of x; the finish kernel applies the options
     slice_epi.ldx = (int)ldx;
-    void* params[] = {&qt, &st, &x, &ws, &row_blocks, &ki, &ni, &ti, &zero, &spm, &spn, &nksi, &act, &slice_epi};
+    void* params[] = {&qt, &st, &x, &ws, &row_blocks, &ki, &ni, &ti, &zero, &walk_arg, &nksi, &act, &slice_epi};
     W4_TRY(w4_launch(ctx, sym, (unsigned)grid, 1, kW4PfThreads, shmem, params));
     if (has_epi) {
         if (t * (L.n / 1024) > 0x7fffffffu) return w4_fail(W4A16_ERR_SHAPE, "prefill: t=%zu n=%zu exceed the finish launch", t, L.n);

@@ -1,7 +1,9 @@
-"""Sizes of the built tiled kernels.  A gated launch has one epilogue, or stores partial sums: its code is no longer than that of the
-plain kernel of the same tile, which has more (launches of ten microseconds feel every further line that they fetch)."""
+"""Sizes of the built tiled kernels: what a launch of ten microseconds fetches cold.  A gated launch has one epilogue, or stores partial sums: its code is no longer than that of the
+plain kernel of the same tile, which has more.  The arguments fill two lines of 64 bytes."""
 import os
+import re
 import struct
+import subprocess
 
 import pytest
 
@@ -35,3 +37,16 @@ def test_gated_kernels_are_no_longer_than_plain_ones(asset):
     assert len(pairs) >= 10, sizes
     for plain, gated in pairs:
         assert sizes[gated] <= sizes[plain], (plain, sizes[plain], sizes[gated])
+
+
+@pytest.mark.parametrize("asset", ["prefill", "prefill_g128"])
+def test_arguments_fill_two_lines(asset):
+    notes = subprocess.run([os.path.join(build.ROCM, "llvm", "bin", "llvm-readelf"), "--notes", os.path.join(build.ASSET_DIR, asset + ".hsaco")],
+                           capture_output=True, text=True, check=True).stdout
+    found = []
+    for kernel in re.split(r"- \.agpr_count", notes)[1:]:
+        name = re.search(r"\.symbol:\s*(\w+)\.kd", kernel).group(1)
+        if name.startswith("w4a16_prefill_g"):
+            found.append((name, int(re.search(r"\.kernarg_segment_size:\s*(\d+)", kernel).group(1))))
+    assert len(found) == 20, found
+    assert all(size <= 128 for _, size in found), found
