@@ -195,7 +195,8 @@ int w4a16_plan_decode(size_t n, size_t k, size_t group, size_t t, int cu_count, 
  * w4a16_lin_forward_glu (never split over k).  Needs neither a context nor a GPU.  Out pointers may be NULL. */
 int w4a16_plan_stream(size_t n, size_t k, size_t t, int cu_count, int glu, int* waves_n, int* waves_k, int* k_slices);
 /* The best launch of the prefill path (W4A16_PATH_PREFILL) on its 256-column block tiles for t rows: out = {block tile rows (64,
- * 96 or 128), k slices, super-tile rows, super-tile columns, super-tile count}; `tile_rows` and `k_slices` pin a choice as
+ * 96 or 128), k slices, block tile rows and columns of a super-tile, 1 where super-tiles follow one another in bands of rows and 0 in
+ * panels of columns}; `tile_rows` and `k_slices` pin a choice as
  * w4a16_set_prefill_tile / w4a16_set_prefill_ksplit do (0 = automatic); *price_us (may be NULL) receives the model's
  * estimate for the chosen plan.  With nothing pinned narrow outputs may run a k-group build instead: see
  * w4a16_plan_prefill_launch.  Role of the reference's per-problem choice of thread-block shape
@@ -204,8 +205,8 @@ int w4a16_plan_prefill(size_t t, size_t n, size_t k, size_t group, int cu_count,
                        size_t out[5], double* price_us);
 
 /* What the prefill path launches with nothing pinned: out = {block tile rows, block tile columns (256; 128 or 192 in a k-group
- * build), k groups inside a workgroup (1 or 4), k slices, super-tile rows, super-tile columns, super-tile count}.  `glu` != 0: the
- * gated launch.  `whole_k` != 0: a launch with the options of a deferred norm whose shape (gated, or n not a multiple of 1024)
+ * build), k groups inside a workgroup (1 or 4), k slices, super-tile rows, super-tile columns, bands}, the last three as above.  `glu` != 0:
+ * the gated launch.  `whole_k` != 0: a launch with the options of a deferred norm whose shape (gated, or n not a multiple of 1024)
  * keeps k whole.  price_us as above (of the k-group build's own model where one is chosen). */
 int w4a16_plan_prefill_launch(size_t t, size_t n, size_t k, size_t group, int cu_count, int glu, int whole_k, size_t out[7],
                               double* price_us);

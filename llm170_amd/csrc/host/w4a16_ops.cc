@@ -411,50 +411,43 @@ static int launch_decode_glu(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_
 // also prices the k-group builds below.
 // Block tile 128 x 256 (two workgroups per CU), 96 x 256 or 64 x 256 (three per CU, 96 / 64 accumulator registers), the
 // k range whole or cut into 2 to 8 slices (split-K: f32 partials in a context-owned workspace, added in slice order by a
-// second launch — deterministic), and the super-tile shape: every combination is priced and the cheapest runs.
-struct PrefillSuper {
-    size_t sup_m, sup_n, supers, load;
+// second launch — deterministic): every combination is priced and the cheapest runs.
+struct PrefillWalk {
+    size_t rows, cols;  // block tiles of a super-tile
+    bool bands;         // super-tiles follow one another in bands of rows, else in panels of columns
 };
 struct PrefillPlan {
     size_t bm, nks;
-    PrefillSuper sup;
     double us;       // the price it won with
     size_t wnw = 0;  // 2 or 3: the k-group build with 64 * wnw columns per block tile; 0: the 256-column tiles
+    PrefillWalk walk{1, 1, false};
+    size_t tiles_m(size_t t) const { return (t + bm - 1) / bm; }
+    // a gated launch tiles the n/2 output columns by half a block tile (each block tile holds the matching up columns as well)
+    size_t cols() const { return wnw ? 64 * wnw : (size_t)kW4PfBn; }
+    size_t tiles_n(size_t n, bool glu) const { return glu ? (n / 2 + cols() / 2 - 1) / (cols() / 2) : (n + cols() - 1) / cols(); }
+    // workgroups of the kernel that a CU holds at once
+    size_t room() const { return wnw ? 1 : bm == 128 ? 2 : 3; }
 };
 
-// Super-tile shape for a grid of tiles_m x tiles_n block tiles: sup_m <= 8 along m, sup_n in {8, 4, 2, 1} along n, the largest (L2
-// reuse).  It decides only the order in which an XCD walks its tiles: the kernel numbers the live ones without gaps and every XCD takes
-// an eighth of them (load).  most_blocks: super-tiles that would hold more blocks per XCD, edges counted, are left out.
-static PrefillSuper prefill_super(size_t tiles_m, size_t tiles_n, size_t most_blocks = ~(size_t)0) {
-    PrefillSuper best{0, 0, 0, (tiles_m * tiles_n + 7) / 8};
-    for (size_t cm = std::min<size_t>(8, tiles_m); cm >= 1; cm--) {
-        for (size_t cn : {8, 4, 2, 1}) {
-            const size_t supers = ((tiles_m + cm - 1) / cm) * ((tiles_n + cn - 1) / cn);
-            if ((supers + 7) / 8 * cm * cn > most_blocks || cm * cn <= best.sup_m * best.sup_n) continue;
-            best.sup_m = cm, best.sup_n = cn, best.supers = supers;
-        }
-    }
-    return best;
-}
-
-// How the kernel walks the block tiles (its sup_m, sup_n; negative: bands of rows).  x_tile, w_tile: bytes per k tile of a tile's x rows and
-// weight columns; resident: blocks an XCD holds at once.  Where all blocks of an XCD's eighth are resident it is one block of tiles, as
-// many rows as leave it the fewest bytes to read, walked in bands.  Else super-tiles of the plan's shape, in panels or bands, whichever
-// leaves the eighth the fewer bytes.  (848 x 2048 t = 2982, 47 x 5 tiles: the shape's panels of one column 21.0 us, bands of six rows
-// 19.0.)
-static std::pair<int, int> prefill_walk(size_t m_tiles, size_t n_tiles, size_t nks, size_t x_tile, size_t w_tile, const PrefillSuper& sup, size_t resident) {
+// How the kernel walks the block tiles: the order only, every XCD takes an eighth of them.  x_tile, w_tile: bytes per k tile of a tile's
+// x rows and weight columns; resident: blocks an XCD holds at once.  Where all blocks of an XCD's eighth are resident it is one run in
+// bands of as many rows as leave it the fewest bytes to read, rows * x_tile + share / rows * w_tile, a weight byte counted twice: it
+// comes from HBM and x mostly from a cache (330 launches with it counted once 0.5 % slower on average, four times 0.4 % faster: flat).
+// Else super-tiles of 8 x 8 (fewer tile rows where there are fewer) in panels or bands, whichever leaves the eighth the fewer bytes.
+// (848 x 2048 t = 2982, 47 x 5 tiles: panels of one column 21.0 us, bands of six rows 19.0.)
+static PrefillWalk prefill_walk(size_t m_tiles, size_t n_tiles, size_t nks, size_t x_tile, size_t w_tile, size_t resident) {
     const size_t share = std::max<size_t>(1, (m_tiles * n_tiles + 7) / 8);
     if (share * nks <= resident) {
         size_t rows = (size_t)std::lround(std::sqrt(2.0 * (double)share * (double)w_tile / (double)x_tile));
         rows = std::max((share + n_tiles - 1) / n_tiles, std::min(std::max<size_t>(rows, 1), m_tiles));
-        return {(int)rows, -8};
+        return {rows, 8, true};
     }
     auto read = [&](size_t inner, size_t outer_width, size_t inner_bytes, size_t outer_bytes) {
         const size_t wide = std::max<size_t>(1, std::min(outer_width, share));
         return share >= inner * wide ? inner * inner_bytes + share / inner * outer_bytes : share / wide * inner_bytes + wide * outer_bytes;
     };
-    const bool bands = read(n_tiles, std::min(sup.sup_m, m_tiles), w_tile, x_tile) < read(m_tiles, std::min(sup.sup_n, n_tiles), x_tile, w_tile);
-    return {(int)sup.sup_m, bands ? -(int)sup.sup_n : (int)sup.sup_n};
+    const size_t sup_m = std::min<size_t>(8, m_tiles);
+    return {sup_m, 8, read(n_tiles, sup_m, w_tile, x_tile) < read(m_tiles, std::min<size_t>(8, n_tiles), x_tile, w_tile)};
 }
 
 // Price of a launch in microseconds, from measurements on MI355X.  A CU holds `room` workgroups at once; j of them per CU, an even share
@@ -500,14 +493,12 @@ static const TilePrice kTilePrice[2][3] = {  // group 128, 32; 64, 96, 128 rows 
 
 static PrefillPlan plan_prefill(size_t t, size_t n, size_t k, size_t group, size_t cus, int tile_m_forced, int ksplit_forced,
                                 bool glu = false) {
-    // a gated launch tiles the n/2 output columns by 128 (each block tile holds the matching 128 up columns as well)
-    const size_t tiles_n = glu ? (n / 2 + kW4PfBn / 2 - 1) / (kW4PfBn / 2) : (n + kW4PfBn - 1) / kW4PfBn, kt_n = k / 128;
-    PrefillPlan best{128, 1, PrefillSuper{1, 1, 0, 0}, 1e30};
+    PrefillPlan best{128, 1, 1e30};
+    const size_t tiles_n = best.tiles_n(n, glu), kt_n = k / 128;
     for (size_t rows : {(size_t)128, (size_t)96, (size_t)64}) {
         if (tile_m_forced && (size_t)tile_m_forced != rows) continue;
         if (rows == 96 && group != 128 && !tile_m_forced) continue;  // the group-32 builds of that tile spill: only when pinned
         const size_t tiles_m = (t + rows - 1) / rows;
-        const PrefillSuper sup = prefill_super(tiles_m, tiles_n);
         const size_t forced = ksplit_forced > 0 ? std::max<size_t>(1, std::min<size_t>((size_t)ksplit_forced, kt_n / 4)) : 0;
         for (size_t cand : {1, 2, 3, 4, 5, 6, 7, 8}) {
             const size_t nks = forced ? forced : cand;  // a pinned slice count is the only candidate
@@ -517,7 +508,7 @@ static PrefillPlan plan_prefill(size_t t, size_t n, size_t k, size_t group, size
             if (!forced && (nks == 5 || nks == 7) && nks * 5 > kt_n) continue;  // no gain from slices of four k tiles
             const double per_cu = (double)((tiles_m * tiles_n * nks + 7) / 8 * 8) / (double)cus;
             const double us = kTilePrice[group == 32][rows / 32 - 2].us((kt_n + nks - 1) / nks, per_cu, nks, (double)nks * (double)t * (double)n * 8.0 / 1e6);
-            if (us < best.us) best = PrefillPlan{rows, nks, sup, us};
+            if (us < best.us) best = PrefillPlan{rows, nks, us};
         }
     }
     return best;
@@ -543,9 +534,8 @@ static PrefillPlan plan_prefill_groups(const PrefillPlan& tiles, size_t t, size_
         const size_t tiles_n = (n + 64 * w - 1) / (64 * w);  // gated: as many pairs of 32 w gate and up columns
         if ((tiles_m * tiles_n + 7) / 8 * 8 > cus) continue;
         const double* c = price[group == 32][w - 2];
-        const PrefillSuper sup = prefill_super(tiles_m, tiles_n, cus / 8);
-        const double used = (double)(sup.load * 8) / (double)cus, p = c[0] + c[2] * used + (c[1] + c[3] * used) * (double)run;
-        if (p < us) us = p, best = PrefillPlan{64, 1, sup, p, w};
+        const double used = (double)((tiles_m * tiles_n + 7) / 8 * 8) / (double)cus, p = c[0] + c[2] * used + (c[1] + c[3] * used) * (double)run;
+        if (p < us) us = p, best = PrefillPlan{64, 1, p, w};
     }
     return best;
 }
@@ -553,8 +543,10 @@ static PrefillPlan plan_prefill_groups(const PrefillPlan& tiles, size_t t, size_
 // The launch's whole plan: everything that decides it is an argument.  `whole`: options that a split launch's second kernel does
 // not take at this shape keep k whole; the caller's pins (tile rows, slices) name the 256-column tiles.
 static PrefillPlan plan_prefill_launch(size_t t, size_t n, size_t k, size_t group, size_t cus, int tile_pin, int ksplit_pin, bool whole, bool glu) {
-    const PrefillPlan tiles = plan_prefill(t, n, k, group, cus, tile_pin, whole ? -1 : ksplit_pin, glu);
-    return tile_pin == 0 && ksplit_pin == 0 ? plan_prefill_groups(tiles, t, n, k, group, cus) : tiles;
+    PrefillPlan P = plan_prefill(t, n, k, group, cus, tile_pin, whole ? -1 : ksplit_pin, glu);
+    if (tile_pin == 0 && ksplit_pin == 0) P = plan_prefill_groups(P, t, n, k, group, cus);
+    P.walk = prefill_walk(P.tiles_m(t), P.tiles_n(n, glu), P.nks, P.bm * 256, P.cols() * 64, cus / 8 * P.room());
+    return P;
 }
 
 extern "C" int w4a16_plan_prefill_launch(size_t t, size_t n, size_t k, size_t group, int cu_count, int glu, int whole_k, size_t out[7],
@@ -562,7 +554,7 @@ extern "C" int w4a16_plan_prefill_launch(size_t t, size_t n, size_t k, size_t gr
     if (t == 0 || n == 0 || k == 0 || k % 128 != 0 || (group != 128 && group != 32) || cu_count <= 0 || !out || (glu && n % 32 != 0))
         return w4_fail(W4A16_ERR_ARG, "plan_prefill_launch: t=%zu n=%zu k=%zu group=%zu cus=%d", t, n, k, group, cu_count);
     const PrefillPlan P = plan_prefill_launch(t, n, k, group, (size_t)cu_count, 0, 0, whole_k != 0, glu != 0);
-    const size_t got[7] = {P.bm, P.wnw ? 64 * P.wnw : (size_t)kW4PfBn, P.wnw ? 4u : 1u, P.nks, P.sup.sup_m, P.sup.sup_n, P.sup.supers};
+    const size_t got[7] = {P.bm, P.cols(), P.wnw ? 4u : 1u, P.nks, P.walk.rows, P.walk.cols, P.walk.bands ? 1u : 0u};
     for (int i = 0; i < 7; i++) out[i] = got[i];
     if (price_us) *price_us = P.us;
     return 0;
@@ -573,12 +565,13 @@ extern "C" int w4a16_plan_prefill(size_t t, size_t n, size_t k, size_t group, in
     if (t == 0 || n == 0 || k == 0 || k % 128 != 0 || (group != 128 && group != 32) || cu_count <= 0 || !out ||
         (tile_rows != 0 && tile_rows != 64 && tile_rows != 96 && tile_rows != 128) || k_slices < -1 || k_slices > 16)
         return w4_fail(W4A16_ERR_ARG, "plan_prefill: t=%zu n=%zu k=%zu cus=%d tile=%d slices=%d", t, n, k, cu_count, tile_rows, k_slices);
-    const PrefillPlan P = plan_prefill(t, n, k, group, (size_t)cu_count, tile_rows, k_slices);
+    PrefillPlan P = plan_prefill(t, n, k, group, (size_t)cu_count, tile_rows, k_slices);
+    P.walk = prefill_walk(P.tiles_m(t), P.tiles_n(n, false), P.nks, P.bm * 256, P.cols() * 64, (size_t)cu_count / 8 * P.room());
     out[0] = P.bm;
     out[1] = P.nks;
-    out[2] = P.sup.sup_m;
-    out[3] = P.sup.sup_n;
-    out[4] = P.sup.supers;
+    out[2] = P.walk.rows;
+    out[3] = P.walk.cols;
+    out[4] = P.walk.bands ? 1 : 0;
     if (price_us) *price_us = P.us;
     return 0;
 }
@@ -639,10 +632,10 @@ static int launch_prefill(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_t y
     if (hit == ctx->prefill_plans.end()) {
         const PrefillPlan P = plan_prefill_launch(t, L.n, L.k, L.group, (size_t)std::max(ctx->cu_count, 1), ctx->prefill_tile_m,
                                                   ctx->prefill_ksplit, whole, glu);
-        hit = ctx->prefill_plans.emplace(key, std::array<size_t, 6>{P.bm, P.nks, P.sup.sup_m, P.sup.sup_n, P.sup.supers, P.wnw}).first;
+        hit = ctx->prefill_plans.emplace(key, std::array<size_t, 6>{P.bm, P.nks, P.wnw, P.walk.rows, P.walk.cols, P.walk.bands}).first;
     }
     const auto& kept = hit->second;
-    const PrefillPlan plan{kept[0], kept[1], PrefillSuper{kept[2], kept[3], kept[4], 0}, 0.0, kept[5]};
+    const PrefillPlan plan{kept[0], kept[1], 0.0, kept[2], PrefillWalk{kept[3], kept[4], kept[5] != 0}};
     const size_t bm = plan.bm, nks = plan.nks;
     char sym[64];
     snprintf(sym, sizeof sym, "w4a16_prefill_g%zu_%s%s%s%s", L.group, L.scale_bf16 ? "bf16" : "f16", bm == 64 ? "_m64" : bm == 96 ? "_m96" : "",
@@ -654,10 +647,10 @@ static int launch_prefill(w4a16_ctx* ctx, const W4Lin& L, uint64_t x, uint64_t y
     const unsigned shmem = (unsigned)(plan.wnw ? std::max<size_t>(4 * stages, plan.wnw * 12 * 4 * 1024) : stages) + threads * 4;
     uint64_t qt = L.q_tiled, st = L.s_tiled;
     int row_blocks = (int)L.row_blocks, ki = (int)L.k, ni = (int)L.n, ti = (int)t, of = (out_f16 || glu) ? 1 : 0;
-    const size_t cols = plan.wnw ? 64 * plan.wnw : kW4PfBn, n_tiles = glu ? (L.n / 2 + cols / 2 - 1) / (cols / 2) : (L.n + cols - 1) / cols;
-    const size_t grid = ((t + bm - 1) / bm * n_tiles * nks + 7) / 8 * 8;
-    const auto walk = prefill_walk((t + bm - 1) / bm, n_tiles, nks, bm * 256, cols * 64, plan.sup, 32 * (plan.wnw ? 1 : bm == 128 ? 2 : 3));
-    int walk_arg = (walk.first & 0xffff) | (int)((unsigned)walk.second << 16), act = glu ? glu_act : 0, glu_i = glu ? 1 : 0;
+    const size_t grid = (plan.tiles_m(t) * plan.tiles_n(L.n, glu) * nks + 7) / 8 * 8;
+    // rows in the low 16 bits, columns, negative for bands, in the high ones
+    const int walk_cols = plan.walk.bands ? -(int)plan.walk.cols : (int)plan.walk.cols;
+    int walk_arg = (int)(plan.walk.rows | (size_t)(uint16_t)walk_cols << 16), act = glu ? glu_act : 0, glu_i = glu ? 1 : 0;
     int nksi = (int)nks;
     if (grid > 0x7fffffffu) return w4_fail(W4A16_ERR_SHAPE, "prefill: t=%zu n=%zu exceed the grid", t, L.n);
     if (nks == 1) {

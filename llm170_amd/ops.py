@@ -36,21 +36,21 @@ def plan_stream(n, k, t, cu_count=256, glu=False):
 
 def plan_prefill(t, n, k, cu_count=256, tile_rows=0, k_slices=0, group=128):
     """Best launch of the prefill path on its 256-column tiles (no context, no GPU): dict of tile_rows, k_slices, super_m,
-    super_n, supers, price_us."""
+    super_n, bands, price_us."""
     out = (C.c_size_t * 5)()
     us = C.c_double()
     ffi.check(ffi.load().w4a16_plan_prefill(t, n, k, group, cu_count, tile_rows, k_slices, out, C.byref(us)))
-    return {"tile_rows": out[0], "k_slices": out[1], "super_m": out[2], "super_n": out[3], "supers": out[4],
+    return {"tile_rows": out[0], "k_slices": out[1], "super_m": out[2], "super_n": out[3], "bands": out[4],
             "price_us": us.value}
 
 
 def plan_prefill_launch(t, n, k, cu_count=256, group=128, glu=False, whole_k=False):
     """What the prefill path launches with nothing pinned (no context, no GPU): dict of tile_rows, tile_cols, k_groups,
-    k_slices, super_m, super_n, supers, price_us."""
+    k_slices, super_m, super_n, bands, price_us."""
     out = (C.c_size_t * 7)()
     us = C.c_double()
     ffi.check(ffi.load().w4a16_plan_prefill_launch(t, n, k, group, cu_count, int(bool(glu)), int(bool(whole_k)), out, C.byref(us)))
-    keys = ("tile_rows", "tile_cols", "k_groups", "k_slices", "super_m", "super_n", "supers")
+    keys = ("tile_rows", "tile_cols", "k_groups", "k_slices", "super_m", "super_n", "bands")
     return dict(zip(keys, out), price_us=us.value)
 
 

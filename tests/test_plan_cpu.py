@@ -40,12 +40,41 @@ def test_prefill_plan_is_the_sweeps_winner_at_the_layer_shapes():
         assert cand[pick] <= 1.03 * best, (n, k, t, pick, cand[pick], best)
 
 
-def test_prefill_plan_super_tiles_cover_the_grid_and_pins_are_honoured():
-    for (t, n, k) in [(4096, 34816, 5120), (1280, 5120, 17408), (100, 7168, 5120), (65, 256, 512)]:
+def visited(tiles_m, tiles_n, slices, sup_m, sup_n, bands):
+    """(tile row, tile column, slice) of every workgroup, XCD by XCD, as kernels/prefill.hip numbers them (prefill_body)."""
+    work, out = tiles_m * tiles_n * slices, []
+    for xcd in range(8):
+        run = []
+        for b in range(-(-work // 8)):
+            at = work * xcd // 8 + b
+            if at >= work * (xcd + 1) // 8:
+                continue
+            r, sl = divmod(at, slices)
+            so, si, to, ti = (sup_m, sup_n, tiles_m, tiles_n) if bands else (sup_n, sup_m, tiles_n, tiles_m)
+            o, in_o = divmod(r, ti * so)
+            wide = min(so, to - o * so)
+            sup, in_super = divmod(in_o, si * wide)
+            deep = min(si, ti - sup * si)
+            i_n, i_m = divmod(in_super, wide if bands else deep)
+            run.append(((o * so if bands else sup * si) + i_m, (sup * si if bands else o * so) + i_n, sl))
+        out.append(run)
+    return out
+
+
+def check_walk(p, t, n, glu=False):
+    cols = p.get("tile_cols", 256)
+    tiles_m, tiles_n = -(-t // p["tile_rows"]), -(-(n // 2) // (cols // 2)) if glu else -(-n // cols)
+    runs = visited(tiles_m, tiles_n, p["k_slices"], p["super_m"], p["super_n"], p["bands"])
+    seen = [v for run in runs for v in run]
+    assert len(set(seen)) == len(seen) == tiles_m * tiles_n * p["k_slices"], (t, n, p)
+    assert all(0 <= m < tiles_m and 0 <= c < tiles_n for m, c, _ in seen), (t, n, p)
+    assert max(map(len, runs)) - min(map(len, runs)) <= 1 and p["super_m"] < 2**15, (t, n, p)
+
+
+def test_prefill_plan_walks_every_tile_and_pins_are_honoured():
+    for (t, n, k) in [(4096, 34816, 5120), (1280, 5120, 17408), (100, 7168, 5120), (65, 256, 512), (2982, 848, 2048), (40000, 16, 512)]:
         p = ops.plan_prefill(t, n, k)
-        tiles_m, tiles_n = -(-t // p["tile_rows"]), -(-n // 256)
-        sm, sn = -(-tiles_m // p["super_m"]), -(-tiles_n // p["super_n"])
-        assert p["supers"] == sm * sn and 1 <= p["super_m"] <= 8 and p["super_n"] in (1, 2, 4, 8)
+        check_walk(p, t, n)
         assert p["k_slices"] == 1 or p["k_slices"] <= (k // 128) // 4
     assert ops.plan_prefill(4096, 34816, 5120, tile_rows=64)["tile_rows"] == 64
     assert ops.plan_prefill(4096, 34816, 5120, tile_rows=96)["tile_rows"] == 96
@@ -182,6 +211,13 @@ def test_stream_plan_is_one_the_kernel_has():
             ops.plan_stream(*bad)
 
 
+def test_prefill_walk_where_an_xcds_eighth_is_resident():
+    """The chip's own size decides what is resident at once: 3 x 256 blocks of the 64-row tile on 256 CUs, 3 x 128 on 128."""
+    walk = lambda cus: {f: ops.plan_prefill(640, 12288, 512, cu_count=cus, tile_rows=64, k_slices=-1)[f] for f in ("super_m", "super_n", "bands")}
+    assert walk(256) == {"super_m": 10, "super_n": 8, "bands": 1}  # 10 x 48 tiles, all rows in one band
+    assert walk(128)["super_m"] == 8                               # 60 per XCD, 48 resident: super-tiles
+
+
 def test_prefill_launch_plan():
     """What is launched with nothing pinned: k-group builds of 128 or 192 columns where the grid is at most one block tile per
     CU and they are priced below the 256-column tiles, which are otherwise those of plan_prefill.  The scale group decides too."""
@@ -206,11 +242,11 @@ def test_prefill_launch_plan():
                         tiles_m, tiles_n = -(-t // p["tile_rows"]), -(-n // p["tile_cols"])
                         if p["k_groups"] == 4:
                             assert p["tile_rows"] == 64 and p["k_slices"] == 1 and tiles_m * tiles_n <= 256, p
-                            assert -(-p["supers"] // 8) * p["super_m"] * p["super_n"] <= 32, p  # blocks of an XCD, empty ones too
+                            assert p["bands"] == 1, p  # an XCD's eighth is resident: one band
                         elif not glu:
                             q = ops.plan_prefill(t, n, k, group=g)
                             assert p["tile_cols"] == 256 and all(p[f] == q[f] for f in q), (p, q)
-                        assert p["supers"] == -(-tiles_m // p["super_m"]) * -(-tiles_n // p["super_n"]), p
+                        check_walk(p, t, n, glu)
                         assert ops.plan_prefill_launch(t, n, k, group=g, glu=glu, whole_k=True)["k_slices"] == 1
     # a block tile per CU, and one more: 64 rows x 128 columns
     assert ops.plan_prefill_launch(64 * 16, 128 * 16, 640)["k_groups"] == 4
