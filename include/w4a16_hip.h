@@ -418,6 +418,12 @@ int w4a16_set_moe_shape(w4a16_ctx* ctx, int block, int waves);
  * per expert of at least 68 slots, i.e. t * top_k >= 68 * n_experts, and no segment size forced), -1 = never, 1 =
  * always (64-slot segments whatever t).  Same results as the streaming kernels up to the order of the f32 sums. */
 int w4a16_set_moe_tiled(w4a16_ctx* ctx, int mode);
+/* The launch plan of w4a16_moe_ffn with every setting automatic, for experts whose every scale the MFMA-tiled kernels take: *segment
+ * receives the slots per segment (1: the direct mode of up to 15 tokens, which has no aligned GEMMs and leaves the names empty),
+ * gate_up and down the kernels of the two grouped GEMMs.  `scales`: 0 = f16, or bf16 that f16 holds; 1 = bf16; 2 (group 32) = bf16, all
+ * in [2^-14, 2^13).  `cap`: bytes of each name, at least 80.  Needs neither a context nor a GPU. */
+int w4a16_plan_moe(size_t t, size_t top_k, size_t n_experts, size_t h, size_t n_ff, size_t group, int scales, int cu_count,
+                   size_t* segment, char* gate_up, char* down, size_t cap);
 /* Timed back-to-back w4a16_moe_ffn calls (as w4a16_bench_forward); call i uses experts names[i % n_names]. */
 int w4a16_bench_moe(w4a16_ctx* ctx, const char* const* names, size_t n_names, uint64_t x_dev, uint64_t idx_dev,
                     uint64_t wt_dev, size_t t, size_t top_k, uint64_t y_dev, size_t warmup, size_t reps,

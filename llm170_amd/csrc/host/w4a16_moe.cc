@@ -223,8 +223,7 @@ int w4_ensure(w4a16_ctx* ctx, uint64_t* buf, size_t* cap, size_t bytes) {
 // 16/32/48/64 that the mean run fills to under 90 % (kernels/marlin_moe.rs:309-315); measured here (128 experts,
 // top-8, T = 16..1024) 32-slot segments beat 16-slot ones at every T, and the larger sizes win once most experts would
 // need a second segment.
-static size_t pick_block(const w4a16_ctx* ctx, size_t t, size_t ns, size_t n_exp, size_t top_k) {
-    if (ctx->moe_block) return (size_t)ctx->moe_block;
+static size_t pick_block(size_t t, size_t ns, size_t n_exp, size_t top_k) {
     // direct mode (no alignment, two launches, see w4a16_moe_ffn): streams an expert once per token that chose it,
     // which still beats the two extra launches up to fifteen tokens (128 experts, top-8: 35.6 vs 52.9 us at t = 8,
     // 49.3 vs 61.3 us at t = 12, 62.9 vs 64.7 us at t = 15, level at t = 16, 79.3 vs 65.4 us at t = 20)
@@ -235,48 +234,58 @@ static size_t pick_block(const w4a16_ctx* ctx, size_t t, size_t ns, size_t n_exp
     return mean < 24.0 ? 32 : mean < 40.0 ? 48 : 64;
 }
 
-static int launch_moe_gemm(w4a16_ctx* ctx, const W4Experts& E, bool glu, uint64_t x, size_t x_rows, size_t x_div,
-                           uint64_t y, int y_f16, uint64_t topw, size_t ns, size_t block, size_t max_segs,
-                           uint64_t sorted, uint64_t eids, uint64_t npost, bool tiled = false) {
-    const size_t n = glu ? 2 * E.n_ff : E.h, k = glu ? E.h : E.n_ff;
-    const size_t row_blocks = (n + 15) / 16, kt_n = k / 128;
-    const size_t units = glu ? row_blocks / 2 : (row_blocks + 1) / 2;
-    if (x_rows * k * 2 >= 0x80000000ull)
-        return w4_fail(W4A16_ERR_SHAPE, "moe: activations reach 2 GiB, beyond the buffer-descriptor range");
-    uint64_t qa = glu ? E.q13 : E.q2, sa = glu ? E.s13 : E.s2;
-    unsigned long long qs = glu ? E.q13_stride : E.q2_stride, ss = glu ? E.s13_stride : E.s2_stride;
-    int xr = (int)x_rows, xd = (int)x_div, yf = y_f16, blk = (int)block, nsi = (int)ns, rbi = (int)row_blocks,
-        ki = (int)k, ni = (int)n, nei = (int)E.n_exp;
-    int waves = 0;  // set below, before the launch reads it
-    int act_kind = ctx->moe_act_kind;  // read by the gate|up kernels only
-    void* p[] = {&qa, &sa, &qs, &ss, &x, &xr, &xd, &y, &yf, &topw, &sorted, &eids, &npost, &blk, &nsi, &rbi, &ki, &ni, &nei,
-                 &waves, &act_kind};
+// What an expert launch makes of its scales: f16 (or bf16 kept as f16), bf16, folded (W4Experts::fold).
+enum MoeScales { kMoeF16 = 0, kMoeBf16 = 1, kMoeFold = 2 };
+static MoeScales moe_scales(const W4Experts& E) { return E.fold ? kMoeFold : E.tiled_bf16 ? kMoeBf16 : kMoeF16; }
+
+// Every expert's run is padded to a multiple of block: at most ns / block full segments plus one partial per expert.
+static size_t moe_max_segs(size_t ns, size_t block, size_t n_exp) { return std::min(ns, ns / block + n_exp); }
+
+// Segment size of an expert FFN (1: the direct mode, no alignment), and whether its GEMMs are the MFMA-tiled kernels.
+struct MoeRoute {
+    size_t block;
+    bool tiled;
+};
+
+static MoeRoute plan_moe_route(size_t t, size_t top_k, size_t n_exp, bool scales_regular, int block_pin, int tiled_pin) {
+    const size_t ns = t * top_k;
+    // Where 64-slot segments are mostly full the MFMA-tiled grouped kernel (one segment x 256 columns per workgroup, x through
+    // LDS, 32x32x16 tiles) takes over from the streaming kernels.  Mean run per expert from which it wins: 68 slots (us per FFN,
+    // streaming / tiled: group 32, 128 experts top-8 h 2048 n_ff 768, T = 850 163 / 160, T = 1024 201 / 184; 32 experts top-4
+    // n_ff 1024 T = 512 80 / 83, T = 600 96 / 88; group 128, 64 experts top-6 n_ff 1408 T = 600 133 / 134, T = 700 155 / 152).
+    // Folded scales gain there too, and earlier (128 experts, T = 768 129 / 124, T = 1024 174 / 156), but the tiled kernels' sums, one
+    // chain of MFMAs over all of k, lie about twice as far from 64-bit sums as the streaming ones (k = 2048 2.2e-7 and 1.0e-7 of
+    // their rms): the line stays.
+    const bool tiled = tiled_pin > 0 || (tiled_pin == 0 && block_pin == 0 && scales_regular && ns >= 68 * n_exp);
+    return {tiled ? 64 : block_pin ? (size_t)block_pin : pick_block(t, ns, n_exp, top_k), tiled};
+}
+
+// The build of one aligned expert GEMM: gate|up (glu) or down.
+struct MoeBuild {
     char sym[80];
-    const char* fam = E.tiled_bf16 ? "bf16" : "f16";
+    int waves;  // per workgroup
+    bool two;   // two k tiles per stage
+};
+
+static MoeBuild plan_moe_build(bool glu, size_t n_exp, size_t h, size_t n_ff, size_t group, MoeScales scales, size_t ns, size_t block, bool tiled,
+                               int waves_pin, size_t cus) {
+    const size_t n = glu ? 2 * n_ff : h, kt_n = (glu ? h : n_ff) / 128;
+    const char *kind = glu ? "glu" : "lin", *fam = scales == kMoeBf16 ? "bf16" : "f16";
+    MoeBuild P{{0}, waves_pin ? waves_pin : 4, false};
     if (tiled) {
-        // MFMA-tiled grouped kernel (kernels/prefill.hip, MODE 1 / 2): block tile = one 64-slot segment x 256 columns
-        // (gate|up: 128 gate + the 128 matching up columns); LDS = two x stages of 64 rows x 128 k, overlaid at the end by the
-        // waves' padded f16 tiles, then slot ids and routing weights; rows always leave as f16
-        if (block != 64) return w4_fail(W4A16_ERR_ARG, "moe: the tiled grouped kernel needs 64-slot segments (got %zu)", block);
-        if (!y_f16) return w4_fail(W4A16_ERR_UNSUPPORTED, "moe: the tiled grouped kernel writes f16 rows only");
-        const size_t cols = glu ? E.n_ff : n, per_tile = glu ? 128 : 256;
-        snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_pf_%s", E.group, E.fold ? "f16x" : fam, glu ? "glu" : "lin");
-        const size_t blocks = (max_segs * ((cols + per_tile - 1) / per_tile) + 7) / 8 * 8;
-        if (blocks > 0x7fffffffu) return w4_fail(W4A16_ERR_SHAPE, "moe: %zu segments exceed the grid", max_segs);
-        return w4_launch(ctx, sym, (unsigned)blocks, 1, 256, kW4PfMoeIdsAt + 64 * 8, p);
+        snprintf(P.sym, sizeof P.sym, "w4a16_moe_g%zu_%s_pf_%s", group, scales == kMoeFold ? "f16x" : fam, kind);
+        return P;
     }
     if (block <= 16) {
         // in-block split-K: each wave needs at least one k tile
-        waves = ctx->moe_waves ? ctx->moe_waves : 4;
-        waves = std::max(1, std::min(std::min(waves, 8), (int)kt_n));
-        snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_dec_%s_x%d", E.group, fam, glu ? "glu" : "lin", block <= 4 ? 1 : 4);
-        const unsigned shmem = waves > 1 ? (unsigned)(waves * 2 * 64 * 16) : 0;
-        return w4_launch(ctx, sym, (unsigned)(max_segs * units), 1, (unsigned)(waves * 64), shmem, p);
+        P.waves = std::max(1, std::min(std::min(P.waves, 8), (int)kt_n));
+        snprintf(P.sym, sizeof P.sym, "w4a16_moe_g%zu_%s_dec_%s_x%d", group, fam, kind, block <= 4 ? 1 : 4);
+        return P;
     }
+    P.waves = P.waves >= 8 ? 8 : 4;  // the x staging needs at least 4 waves
     const int tt = (int)(block / 16);
-    waves = ctx->moe_waves ? ctx->moe_waves : 4;
-    waves = waves >= 8 ? 8 : 4;  // the x staging needs at least 4 waves
-    const size_t blocks = max_segs * ((units + (size_t)waves - 1) / (size_t)waves);
+    const size_t row_blocks = (n + 15) / 16, units = glu ? row_blocks / 2 : (row_blocks + 1) / 2, waves = (size_t)P.waves;
+    const size_t max_segs = moe_max_segs(ns, block, n_exp), wide = (units + waves - 1) / waves * waves;  // waves of a segment's workgroups
     // Two k tiles per stage (kernels/moe.hip) for runs of up to 32 slots, at group 128 where the launch has at most three workgroups
     // per CU: 8 experts T = 100 62.5 -> 54.6 us per FFN, 32 experts top-4 n_ff 1024 T = 40 33.3 -> 30.8; beyond, the LDS they
     // take costs more than the wait they hide (8 experts T = 256 91 / 101, 64 experts top-6 n_ff 1408 T = 24 57.4 / 59.9).  At group
@@ -284,17 +293,53 @@ static int launch_moe_gemm(w4a16_ctx* ctx, const W4Experts& E, bool glu, uint64_
     // workgroup per CU (folded / f16 scales, 128 or 256 of them: 4 experts h 4096 n_ff 3584 T = 16 51.6 -> 40.8 / 54.5 -> 43.4, 8 experts
     // n_ff 2048 T = 24 45.5 -> 39.1 / 45.9 -> 38.8, T = 100 47.9 -> 45.3 / 56.8 -> 57.2; 384: 12 experts T = 24 50.6 / 51.2, T = 100
     // 56.2 / 58.5 / 61.5 / 64.2).
-    const size_t few = E.group == 128 ? blocks * (size_t)waves : E.tiled_bf16 ? ~(size_t)0 : 3 * E.n_exp * (blocks / max_segs) * (size_t)waves;
-    const bool two = tt <= 3 && ns < 32 * E.n_exp && few <= 12 * (size_t)std::max(ctx->cu_count, 1);
+    const size_t few = group == 128 ? max_segs * wide : scales == kMoeBf16 ? ~(size_t)0 : 3 * n_exp * wide;
+    P.two = tt <= 3 && ns < 32 * n_exp && few <= 12 * cus;
     // Folded scales (compute_fold, kernels/moe.hip) from eight k tiles, below which folded sums are the less exact, and eight slots per
     // expert; in segments of two 16-slot blocks only where one segment per expert gives at most 20 waves per CU: the folded build
     // has registers for five waves per SIMD, the other for six (128 experts top-8 n_ff 768 T = 200 scaled / folded 77.2 / 83.4 us,
     // 64 experts top-6 n_ff 1408 T = 100 67.4 / 71.9; 32 experts top-4 n_ff 1024 T = 100 38.3 / 37.2, 8 experts n_ff 3584 T = 100 65.5 / 57.6).
-    const bool fold = E.fold && kt_n >= 8 && ns >= 8 * E.n_exp &&
-                      (tt > 2 || E.n_exp * (blocks / max_segs) * (size_t)waves <= 20 * (size_t)std::max(ctx->cu_count, 1));
-    snprintf(sym, sizeof sym, "w4a16_moe_g%zu_%s_mm_%s_t%d%s", E.group, fold ? "f16x" : fam, glu ? "glu" : "lin", tt, two ? "_k2" : "");
-    const unsigned shmem = (unsigned)((two ? 4 : 2) * 16 * tt * 256);  // two stages of one or two x tiles of 128 k
-    return w4_launch(ctx, sym, (unsigned)blocks, 1, (unsigned)(waves * 64), shmem, p);
+    const bool fold = scales == kMoeFold && kt_n >= 8 && ns >= 8 * n_exp &&
+                      (tt > 2 || n_exp * wide <= 20 * cus);
+    snprintf(P.sym, sizeof P.sym, "w4a16_moe_g%zu_%s_mm_%s_t%d%s", group, fold ? "f16x" : fam, kind, tt, P.two ? "_k2" : "");
+    return P;
+}
+
+static int launch_moe_gemm(w4a16_ctx* ctx, const W4Experts& E, bool glu, uint64_t x, size_t x_rows, size_t x_div,
+                           uint64_t y, int y_f16, uint64_t topw, size_t ns, size_t block, size_t max_segs,
+                           uint64_t sorted, uint64_t eids, uint64_t npost, bool tiled = false) {
+    const size_t n = glu ? 2 * E.n_ff : E.h, k = glu ? E.h : E.n_ff;
+    const size_t row_blocks = (n + 15) / 16;
+    const size_t units = glu ? row_blocks / 2 : (row_blocks + 1) / 2;
+    if (x_rows * k * 2 >= 0x80000000ull)
+        return w4_fail(W4A16_ERR_SHAPE, "moe: activations reach 2 GiB, beyond the buffer-descriptor range");
+    uint64_t qa = glu ? E.q13 : E.q2, sa = glu ? E.s13 : E.s2;
+    unsigned long long qs = glu ? E.q13_stride : E.q2_stride, ss = glu ? E.s13_stride : E.s2_stride;
+    int xr = (int)x_rows, xd = (int)x_div, yf = y_f16, blk = (int)block, nsi = (int)ns, rbi = (int)row_blocks,
+        ki = (int)k, ni = (int)n, nei = (int)E.n_exp;
+    const MoeBuild P = plan_moe_build(glu, E.n_exp, E.h, E.n_ff, E.group, moe_scales(E), ns, block, tiled, ctx->moe_waves, (size_t)std::max(ctx->cu_count, 1));
+    int waves = P.waves;
+    int act_kind = ctx->moe_act_kind;  // read by the gate|up kernels only
+    void* p[] = {&qa, &sa, &qs, &ss, &x, &xr, &xd, &y, &yf, &topw, &sorted, &eids, &npost, &blk, &nsi, &rbi, &ki, &ni, &nei,
+                 &waves, &act_kind};
+    if (tiled) {
+        // MFMA-tiled grouped kernel (kernels/prefill.hip, MODE 1 / 2): block tile = one 64-slot segment x 256 columns
+        // (gate|up: 128 gate + the 128 matching up columns); LDS = two x stages of 64 rows x 128 k, overlaid at the end by the
+        // waves' padded f16 tiles, then slot ids and routing weights; rows always leave as f16
+        if (block != 64) return w4_fail(W4A16_ERR_ARG, "moe: the tiled grouped kernel needs 64-slot segments (got %zu)", block);
+        if (!y_f16) return w4_fail(W4A16_ERR_UNSUPPORTED, "moe: the tiled grouped kernel writes f16 rows only");
+        const size_t cols = glu ? E.n_ff : n, per_tile = glu ? 128 : 256;
+        const size_t blocks = (max_segs * ((cols + per_tile - 1) / per_tile) + 7) / 8 * 8;
+        if (blocks > 0x7fffffffu) return w4_fail(W4A16_ERR_SHAPE, "moe: %zu segments exceed the grid", max_segs);
+        return w4_launch(ctx, P.sym, (unsigned)blocks, 1, 256, kW4PfMoeIdsAt + 64 * 8, p);
+    }
+    if (block <= 16) {
+        const unsigned shmem = waves > 1 ? (unsigned)(waves * 2 * 64 * 16) : 0;
+        return w4_launch(ctx, P.sym, (unsigned)(max_segs * units), 1, (unsigned)(waves * 64), shmem, p);
+    }
+    const size_t blocks = max_segs * ((units + (size_t)waves - 1) / (size_t)waves);
+    const unsigned shmem = (unsigned)((P.two ? 4 : 2) * block * 256);  // two stages of one or two x tiles of 128 k
+    return w4_launch(ctx, P.sym, (unsigned)blocks, 1, (unsigned)(waves * 64), shmem, p);
 }
 
 // Launch plan of the 17..64-row kernel (kernels/mid.hip): waves along n and k of a workgroup, k slices across workgroups.
@@ -463,6 +508,24 @@ static int moe_ffn_direct(w4a16_ctx* ctx, const char* name, const W4Experts& E, 
     return w4_launch(ctx, sym, (unsigned)(t * units), 1, (unsigned)(top_k * 64), (unsigned)(top_k * rbu * 64 * 16), p);
 }
 
+extern "C" int w4a16_plan_moe(size_t t, size_t top_k, size_t n_exp, size_t h, size_t n_ff, size_t group, int scales, int cu_count,
+                              size_t* segment, char* gate_up, char* down, size_t cap) {
+    if (t == 0 || top_k == 0 || top_k > n_exp || t > 0x3fffffffu / top_k || h == 0 || n_ff == 0 || h % 128 != 0 || n_ff % 128 != 0 ||
+        (group != 128 && group != 32) || scales < kMoeF16 || scales > kMoeFold || (scales == kMoeFold && group != 32) || cu_count <= 0 ||
+        !segment || !gate_up || !down || cap < sizeof(MoeBuild::sym))
+        return w4_fail(W4A16_ERR_ARG, "plan_moe: t=%zu top_k=%zu experts=%zu h=%zu n_ff=%zu group=%zu scales=%d cus=%d", t, top_k, n_exp, h, n_ff, group,
+                       scales, cu_count);
+    const MoeRoute R = plan_moe_route(t, top_k, n_exp, true, 0, 0);
+    *segment = R.block;
+    gate_up[0] = down[0] = 0;
+    if (R.block == 1) return 0;
+    for (bool glu : {true, false}) {
+        const MoeBuild P = plan_moe_build(glu, n_exp, h, n_ff, group, (MoeScales)scales, t * top_k, R.block, R.tiled, 0, (size_t)cu_count);
+        std::memcpy(glu ? gate_up : down, P.sym, sizeof P.sym);
+    }
+    return 0;
+}
+
 extern "C" int w4a16_moe_ffn(w4a16_ctx* ctx, const char* name, uint64_t x_dev, uint64_t idx_dev, uint64_t wt_dev,
                              size_t t, size_t top_k, uint64_t y_dev) {
     return w4a16_moe_ffn_act(ctx, name, x_dev, idx_dev, wt_dev, t, top_k, y_dev, W4A16_ACT_SILU);
@@ -480,22 +543,15 @@ extern "C" int w4a16_moe_ffn_act(w4a16_ctx* ctx, const char* name, uint64_t x_de
         return w4_fail(W4A16_ERR_SHAPE, "moe_ffn %s: t=%zu top_k=%zu experts=%zu", name, t, top_k, E->n_exp);
     W4_TRY(w4_hip(hipSetDevice(ctx->device), "hipSetDevice"));
     const size_t ns = t * top_k;
-    // Where 64-slot segments are mostly full the MFMA-tiled grouped kernel (one segment x 256 columns per workgroup, x through
-    // LDS, 32x32x16 tiles) takes over from the streaming kernels.  Mean run per expert from which it wins: 68 slots (us per FFN,
-    // streaming / tiled: group 32, 128 experts top-8 h 2048 n_ff 768, T = 850 163 / 160, T = 1024 201 / 184; 32 experts top-4
-    // n_ff 1024 T = 512 80 / 83, T = 600 96 / 88; group 128, 64 experts top-6 n_ff 1408 T = 600 133 / 134, T = 700 155 / 152).
     if (ctx->moe_tiled > 0 && !E->scales_regular)
         return w4_fail(W4A16_ERR_UNSUPPORTED, "moe_ffn %s: the MFMA-tiled grouped kernels were requested (set_moe_tiled 1) but the experts hold a zero, non-finite or out-of-range scale; the streaming kernels serve them", name);
-    // Folded scales gain there too, and earlier (128 experts, T = 768 129 / 124, T = 1024 174 / 156), but the tiled kernels' sums, one
-    // chain of MFMAs over all of k, lie about twice as far from 64-bit sums as the streaming ones (k = 2048 2.2e-7 and 1.0e-7 of
-    // their rms): the line stays.
-    const bool tiled = ctx->moe_tiled > 0 || (ctx->moe_tiled == 0 && ctx->moe_block == 0 && E->scales_regular && ns >= 68 * E->n_exp);
-    const size_t block = tiled ? 64 : pick_block(ctx, t, ns, E->n_exp, top_k);
+    const MoeRoute R = plan_moe_route(t, top_k, E->n_exp, E->scales_regular, ctx->moe_block, ctx->moe_tiled);
+    const bool tiled = R.tiled;
+    const size_t block = R.block;
     if (block != 1 && block != 4 && block != 16 && block != 32 && block != 48 && block != 64)
         return w4_fail(W4A16_ERR_ARG, "moe_ffn %s: segment size %zu not in {1,4,16,32,48,64}", name, block);
     if (block == 1) return moe_ffn_direct(ctx, name, *E, x_dev, idx_dev, wt_dev, t, top_k, y_dev);
-    // every expert's run is padded to a multiple of block: at most ns/block full segments plus one partial per expert
-    const size_t max_segs = std::min(ns, ns / block + E->n_exp);
+    const size_t max_segs = moe_max_segs(ns, block, E->n_exp);
     W4MoeScratch& S = ctx->moe;
     S.block = block;
     S.sorted_len = (ns + E->n_exp * block) * 4;

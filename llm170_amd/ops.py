@@ -54,6 +54,14 @@ def plan_prefill_launch(t, n, k, cu_count=256, group=128, glu=False, whole_k=Fal
     return dict(zip(keys, out), price_us=us.value)
 
 
+def plan_moe(t, top_k, n_experts, h, n_ff, group=32, scales=0, cu_count=256):
+    """Launch plan of moe_ffn (no context, no GPU): dict of segment (slots; 1 = the direct mode) and the kernels of its grouped GEMMs,
+    gate_up and down.  scales: 0 = f16, or bf16 that f16 holds; 1 = bf16; 2 = bf16, all in [2^-14, 2^13)."""
+    seg, names = C.c_size_t(), [C.create_string_buffer(80) for _ in range(2)]
+    ffi.check(ffi.load().w4a16_plan_moe(t, top_k, n_experts, h, n_ff, group, scales, cu_count, C.byref(seg), names[0], names[1], 80))
+    return {"segment": seg.value, "gate_up": names[0].value.decode(), "down": names[1].value.decode()}
+
+
 def check_shapes(t, qlen, slen, xlen, n, k, group):
     """gptq4.rs:31-58.  Raises W4a16Error(ERR_SHAPE) on violation."""
     ffi.check(ffi.load().w4a16_check_shapes(t, qlen, slen, xlen, n, k, group))

@@ -253,3 +253,58 @@ def test_prefill_launch_plan():
     assert ops.plan_prefill_launch(64 * 16 + 1, 128 * 16, 640)["tile_cols"] != 128
     with pytest.raises(ops.W4a16Error):
         ops.plan_prefill_launch(100, 1000, 640, glu=True)
+
+
+def test_expert_plan_segments_and_tiled_line():
+    """Mean runs on both sides of 24, 40 and 68 slots per expert, whatever the scales; the direct mode up to 15 tokens of top-8."""
+    for scales, fam in ((0, "f16"), (1, "bf16"), (2, "f16x")):
+        for t, seg in [(15, 1), (16, 32), (383, 32), (384, 48), (639, 48), (640, 64), (1087, 64), (1088, 64)]:
+            p = ops.plan_moe(t, 8, 128, 2048, 768, 32, scales)
+            assert p["segment"] == seg, (t, scales, p)
+            tiled = t >= 1088
+            if tiled:
+                assert (p["gate_up"], p["down"]) == ("w4a16_moe_g32_%s_pf_glu" % fam, "w4a16_moe_g32_%s_pf_lin" % fam), p
+            elif seg > 1:
+                assert "_mm_glu_t%d" % (seg // 16) in p["gate_up"] and "_mm_lin_t%d" % (seg // 16) in p["down"], p
+    assert ops.plan_moe(8, 9, 32, 2048, 768)["segment"] == 16 and ops.plan_moe(4, 9, 32, 2048, 768)["segment"] == 4
+    for bad in [(0, 1, 4, 128, 128), (4, 5, 4, 128, 128), (4, 1, 4, 100, 128)]:
+        with pytest.raises(ops.W4a16Error):
+            ops.plan_moe(*bad)
+    with pytest.raises(ops.W4a16Error):
+        ops.plan_moe(100, 1, 4, 128, 128, 128, 2)
+
+
+def test_expert_plan_folds_from_eight_k_tiles_and_eight_slots():
+    def folds(t, n_exp, h, n_ff, top_k=8):
+        p = ops.plan_moe(t, top_k, n_exp, h, n_ff, 32, 2)
+        return "_f16x_" in p["gate_up"], "_f16x_" in p["down"]
+
+    assert folds(517, 128, 2048, 768) == (True, False)                              # down: six k tiles
+    assert folds(517, 128, 896, 1024) == (False, True)                              # gate|up: seven
+    assert folds(517, 128, 1024, 896) == (True, False)
+    assert folds(31, 32, 2048, 1024) == (False, False) and folds(32, 32, 2048, 1024) == (True, True)  # 248 and 256 slots
+    # 32-slot segments: 20 waves per CU from one segment per expert, 5120 waves (units of 32 rows; 40 experts of 128 waves)
+    assert folds(100, 40, 4096, 2048) == (True, True) and folds(100, 41, 4096, 2048) == (False, False)
+    assert folds(240, 41, 4096, 2048) == (True, True)                               # 48-slot segments: however many
+    for scales in (0, 1):
+        p = ops.plan_moe(517, 8, 128, 2048, 1024, 32, scales)
+        assert "f16x" not in p["gate_up"] + p["down"], p
+
+
+def test_expert_plan_two_k_tiles_per_stage():
+    def two(t, n_exp, h, n_ff, group, scales, top_k):
+        p = ops.plan_moe(t, top_k, n_exp, h, n_ff, group, scales)
+        return p["gate_up"].endswith("_k2"), p["down"].endswith("_k2")
+
+    # group 32: one segment per expert at most one workgroup of four waves per CU (256 of them; n_ff 4096: 64 per expert, h 4096: 32)
+    for scales in (0, 2):
+        assert two(24, 4, 4096, 4096, 32, scales, 2) == (True, True)
+        assert two(24, 5, 4096, 4096, 32, scales, 2) == (False, True)
+        assert two(24, 8, 4096, 2048, 32, scales, 2) == (True, True) and two(24, 9, 4096, 2048, 32, scales, 2) == (False, False)
+    assert two(24, 4, 4096, 4096, 32, 1, 2) == (False, False)                       # bf16 arenas: never
+    # runs of 32 slots on: one tile
+    assert two(127, 8, 4096, 2048, 32, 0, 2) == (True, True) and two(128, 8, 4096, 2048, 32, 0, 2) == (False, False)
+    # group 128: at most three workgroups per CU, segments counted (768; 24 and 25 of them at n_ff 2048 and h 4096: 32 per segment)
+    for scales in (0, 1):
+        assert two(88, 19, 4096, 2048, 128, scales, 2) == (True, True)              # 176 slots: 5 + 19 segments
+        assert two(96, 19, 4096, 2048, 128, scales, 2) == (False, False)            # 192: 6 + 19
