@@ -699,19 +699,15 @@ __device__ __forceinline__ void moe_mm_body(MOE_PARAMS) {
 // slots in 48-slot segments, every other expert fills two blocks of three).
 template <int G, bool SBF, bool GLU, int TT, int KT, bool FOLD>
 __device__ __forceinline__ void moe_mm_entry(MOE_PARAMS) {
-    if constexpr (TT == 1) {
-        moe_mm_body<G, SBF, GLU, 1, KT, FOLD>(MOE_ARGS);
-    } else {
-        const int units = GLU ? row_blocks >> 1 : (row_blocks + 1) >> 1;
-        const int seg = blockIdx.x / ((units + wpb - 1) / wpb);
-        int live = 1;
+    const int units = GLU ? row_blocks >> 1 : (row_blocks + 1) >> 1;
+    const int seg = blockIdx.x / ((units + wpb - 1) / wpb);
+    int live = 1;
 #pragma unroll
-        for (int p = 1; p < TT; p++) live += sorted_ids[seg * blk + 16 * p] < ns ? 1 : 0;
-        if (live == 1) moe_mm_body<G, SBF, GLU, 1, KT, FOLD>(MOE_ARGS);
-        else if (TT == 2 || live == 2) moe_mm_body<G, SBF, GLU, 2, KT, FOLD>(MOE_ARGS);
-        else if (TT == 3 || live == 3) moe_mm_body<G, SBF, GLU, TT >= 3 ? 3 : 2, KT, FOLD>(MOE_ARGS);
-        else moe_mm_body<G, SBF, GLU, TT, KT, FOLD>(MOE_ARGS);
-    }
+    for (int p = 1; p < TT; p++) live += sorted_ids[seg * blk + 16 * p] < ns ? 1 : 0;
+    if (live == 1) moe_mm_body<G, SBF, GLU, 1, KT, FOLD>(MOE_ARGS);
+    else if (TT == 2 || live == 2) moe_mm_body<G, SBF, GLU, 2, KT, FOLD>(MOE_ARGS);
+    else if (TT == 3 || live == 3) moe_mm_body<G, SBF, GLU, TT >= 3 ? 3 : 2, KT, FOLD>(MOE_ARGS);
+    else moe_mm_body<G, SBF, GLU, TT, KT, FOLD>(MOE_ARGS);
 }
 
 #define MOE_DEC_KERNEL(NAME, G, SBF, GLU, XL, DEPTH)                                  \
@@ -731,11 +727,9 @@ __device__ __forceinline__ void moe_mm_entry(MOE_PARAMS) {
     MOE_DEC_KERNEL(PFX##_dec_glu_x4, G, SBF, true, 4, 2)     \
     MOE_DEC_KERNEL(PFX##_dec_lin_x1, G, SBF, false, 1, 2)    \
     MOE_DEC_KERNEL(PFX##_dec_lin_x4, G, SBF, false, 4, 2)    \
-    MOE_MM_KERNEL(PFX##_mm_glu_t1, G, SBF, true, 1, 1)    \
     MOE_MM_KERNEL(PFX##_mm_glu_t2, G, SBF, true, 2, 1)    \
     MOE_MM_KERNEL(PFX##_mm_glu_t3, G, SBF, true, 3, 1)    \
     MOE_MM_KERNEL(PFX##_mm_glu_t4, G, SBF, true, 4, 1)    \
-    MOE_MM_KERNEL(PFX##_mm_lin_t1, G, SBF, false, 1, 1)   \
     MOE_MM_KERNEL(PFX##_mm_lin_t2, G, SBF, false, 2, 1)   \
     MOE_MM_KERNEL(PFX##_mm_lin_t3, G, SBF, false, 3, 1)   \
     MOE_MM_KERNEL(PFX##_mm_lin_t4, G, SBF, false, 4, 1)
