@@ -82,6 +82,33 @@ def test_streaming_rows(dec, n, k, t, wide):
     assert dec.cc.last_launch_symbol().startswith("w4a16_mid_g32_%s_t" % ("bf16x" if folds else "bf16"))
 
 
+@pytest.mark.parametrize("n,k", [(4104, 3200), (17000, 3328), (27016, 3072), (33008, 3072), (2048, 17408)])
+@pytest.mark.parametrize("t", [17, 64])
+def test_streaming_sums_no_further_from_64_bits(dec, n, k, t):
+    """The distance that decides where linears fold, on the rows of ordinary scales: over the rms of the sums, of the builds left to the
+    library and of those a single scale that does not fold selects.  4 k / 128 additions of group sums, each rounding a partial sum that
+    grows as a random walk by 2^-24 / sqrt 3 at most, are sqrt(2 k / 128) of them; the two distances are equal to the spread of an rms
+    over 400 columns x 17 rows (1 %) where few k tiles are folded, a tenth is allowed."""
+    print("fold distance", n, k, t, flush=True)
+    far = []
+    for wide in (False, True):
+        q, s, x = _linear(n, k, t, wide)
+        dec.upload_lin_g("far", q, s, n, k, 32, True)
+        xd, yd = dec.cc.to_device(x), dec.cc.alloc(t * n * 4)
+        try:
+            dec.lin_forward("far", xd, yd, t)
+            y = dec.cc.d2h(yd, (t, n), np.float32)
+        finally:
+            dec.cc.free(xd)
+            dec.cc.free(yd)
+        cols = np.unique(np.random.default_rng(n).integers(2, n - 1, 400))
+        ref = gen.f16_bits_to_f32(x).astype(np.float64) @ _weights(q[cols], s[cols], k).T
+        far.append(float(np.sqrt(np.mean((y[:, cols] - ref) ** 2) / np.mean(ref ** 2))))
+    print("distance: %.3g, scaled sums %.3g" % tuple(far), flush=True)
+    assert max(far) <= np.sqrt(2.0 * k / 128) * 2.0 ** -24 / np.sqrt(3.0)
+    assert far[0] <= 1.1 * far[1]
+
+
 @pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("t", [17, 40, 64])
 def test_gated(dec, t, wide):
