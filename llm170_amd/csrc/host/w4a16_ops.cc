@@ -457,11 +457,12 @@ static PrefillWalk prefill_walk(size_t m_tiles, size_t n_tiles, size_t nks, size
 //   in the second, `full` for the first and more[] (at steps of half a workgroup) for the rest;
 //   from there `steady` per generation: workgroups have drifted apart and no generation ends as one (`later` for its fixed part).
 // Plus a fixed cost per launch and per generation, and for a split launch one and the time of its partial sums (us per MB written and read).
-// Fitted to 1056 launches per group (167 linears of 512..40000 x 1024..17408, t = 65..4096; every tile, one to eight slices and the
-// k-group builds timed, weights from memory): least squares on the times, then by the time lost against the best choice.  Over 405
-// launches of 62 other linears the plans lose 0.5 % to the best of each shape and take 0.936 (group 128) and 0.943 (group 32) of the
-// time of those they replaced (whole super-tiles dealt to the XCDs; 2, 3, 4, 6 or 8 slices): of the 810 19 are more than 3 % slower,
-// 8 more than 5, 12 at worst.  5120 x 17408 t = 300 73.7 -> 65 us in five slices, 5120 x 5120 t = 1568 101 -> 82.
+// Fitted, with the k groups below, to 6000 shapes (512..128256 x 1024..53248, gated and not, t = 65..16384; every tile, one to eight slices
+// and the k-group builds timed, weights from memory, launches of 60 us on under sustained load: in short bursts 64 rows look better than
+// they are) by the time lost against the best choice, weighted up beyond 2 % and where an earlier plan was faster.  A fit to three
+// quarters lost 0.37 % on the others, 4.4 % of them more than 3 %; a fit to 167 linears before it 0.8 and 10 %, up to 17 % (22016 x 4096
+// t = 542 gated 119 us, now 104; 4096 x 4096 t = 193 21.8, 18.8).  Of 3500 drawn shapes outside the fit 390 changed plan: 0.976 of the
+// time, 28 more than 3 % slower, 9.5 at worst; 81 of them had been more than 3 % slower than the plans before that fit, now 4.
 struct TilePrice {
     int room;
     double first[3][3], more[7], full, launch, generation, split, per_mb, steady, later;
@@ -484,12 +485,12 @@ struct TilePrice {
     }
 };
 static const TilePrice kTilePrice[2][3] = {  // group 128, 32; 64, 96, 128 rows (the 96-row tile is not chosen at group 32)
-    {{3, {{0.728, 0.968, 1.172}, {1.427, 1.554, 1.794}, {2.239, 2.453, 2.733}}, {0.0, 0.687, 0.961, 1.256, 1.623, 2.773, 2.628}, 2.823, 3.855, 5.632, 0.0, 0.0938, 2.496, 9.27},
-     {3, {{1.184, 1.486, 1.619}, {2.114, 2.291, 2.688}, {3.259, 3.569, 3.887}}, {0.0, 0.729, 1.249, 1.938, 2.473, 3.61, 3.656}, 3.958, 0.939, 10.895, 0.057, 0.0806, 3.306, 19.52},
-     {2, {{1.445, 1.803, 1.947}, {2.619, 2.861, 3.32}}, {0.0, 1.16, 2.04, 2.726, 2.838}, 3.62, 0.843, 11.275, 0.001, 0.0836, 2.950, 16.80}},
-    {{3, {{0.786, 1.396, 1.553}, {2.216, 2.244, 2.376}, {3.004, 3.31, 3.539}}, {0.0, 0.699, 0.908, 1.774, 1.992, 3.283, 3.205}, 3.739, 7.362, 2.375, 0.0, 0.0921, 3.463, 5.90},
-     {3, {{1.184, 1.486, 1.619}, {2.114, 2.291, 2.688}, {3.259, 3.569, 3.887}}, {0.0, 0.729, 1.249, 1.938, 2.473, 3.61, 3.656}, 3.958, 0.939, 10.895, 0.057, 0.0806, 3.306, 19.52},
-     {2, {{2.003, 2.38, 2.515}, {3.674, 3.71, 4.246}}, {0.0, 1.442, 1.998, 3.493, 3.565}, 4.611, 5.478, 6.669, 0.0, 0.0778, 4.022, 13.77}}};
+    {{3, {{0.4218, 0.9117, 1.072}, {1.473, 1.508, 1.63}, {2.202, 2.321, 2.512}}, {0.0, 0.7227, 0.9575, 0.9315, 1.269, 2.425, 2.453}, 2.923, 7.259, 2.063, 0.0, 0.1236, 2.792, 1.653},
+     {3, {{0.9083, 1.447, 1.574}, {2.16, 2.203, 2.433}, {3.056, 3.546, 3.46}}, {0.0, 0.3873, 1.22, 1.627, 2.374, 3.332, 3.019}, 4.028, 6.025, 5.676, 0.00193, 0.1074, 3.969, 0.7899},
+     {2, {{2.112, 1.633, 1.856}, {2.585, 2.679, 2.988}}, {0.0, 1.206, 1.731, 2.48, 2.733}, 3.723, 7.779, 5.398, 0.0001395, 0.1102, 3.238, 9.579}},
+    {{3, {{0.6343, 1.324, 1.475}, {2.223, 2.217, 2.321}, {3.373, 3.272, 3.583}}, {0.0, 0.7727, 1.142, 1.518, 2.006, 3.018, 3.246}, 3.698, 1.449, 7.917, 1.349, 0.06999, 4.199, 0.1875},
+     {3, {{0.9083, 1.447, 1.574}, {2.16, 2.203, 2.433}, {3.056, 3.546, 3.46}}, {0.0, 0.3873, 1.22, 1.627, 2.374, 3.332, 3.019}, 4.028, 6.025, 5.676, 0.00193, 0.1074, 3.969, 0.7899},
+     {2, {{2.493, 2.255, 2.248}, {3.694, 3.582, 3.895}}, {0.0, 0.9294, 1.777, 3.628, 2.874}, 4.783, 5.478, 9.689, 5.425e-05, 0.07507, 4.629, 0.7141}}};
 
 static PrefillPlan plan_prefill(size_t t, size_t n, size_t k, size_t group, size_t cus, int tile_m_forced, int ksplit_forced,
                                 bool glu = false) {
@@ -522,11 +523,10 @@ static PrefillPlan plan_prefill(size_t t, size_t n, size_t k, size_t group, size
 // above / this one in us: group 128 5120 x 5120 t = 300 32.0 / 27.4, 7168 x 5120 t = 300 43.5 / 34.6 (192 columns), 4096 x 2048
 // t = 300 26.3 / 12.9, 1024 x 640 t = 100 14.1 / 7.8, group 32 5120 x 2048 t = 300 32.1 / 16.1; not chosen: 5120 x 5120 t = 65
 // 22.7 / 23.7, 5120 x 17408 t = 128 43 / 74.
-// The price: a fixed cost and one per k tile of a group's run, each growing with the part of the chip in use; fitted with the tiles' above
-// to the 1149 launches per group where the grid fits.
+// The price: a fixed cost and one per k tile of a group's run, each growing with the part of the chip in use; fitted with the tiles' above.
 static PrefillPlan plan_prefill_groups(const PrefillPlan& tiles, size_t t, size_t n, size_t k, size_t group, size_t cus) {
-    static const double price[2][2][4] = {{{5.687, 1.647, 1.243, 0.4823}, {6.55, 2.041, 1.814, 0.6567}},   // group 128: 128, 192 columns
-                                          {{5.872, 2.428, 0.806, 0.4374}, {7.53, 2.966, 1.746, 0.6738}}};  // group 32
+    static const double price[2][2][4] = {{{5.585, 1.61, 0.04486, 0.5213}, {5.848, 2.155, 0.2861, 0.4314}},   // group 128: 128, 192 columns
+                                          {{5.305, 2.591, 0.03913, 0.03608}, {7.122, 3.027, 0.7626, 0.2271}}};  // group 32
     const size_t kt_n = k / 128, tiles_m = (t + 63) / 64, run = (kt_n + 3) / 4;
     PrefillPlan best = tiles;
     double us = tiles.us;
